@@ -91,6 +91,22 @@ WZ_D void lift_tile(const T* src, uint64_t base, uint64_t stride, T* dst, uint64
     }
 }
 
+// Index in its half of the even / odd sample of pair k of a line of n samples,
+// mirrored at the line's ends. One reflection on each side: exact for n >= 9
+// on the four samples past either end that a lifted sample reads; farther
+// positions (the last tile's, whose outputs do not exist) only stay in range.
+// No branch or division, unlike reflect_pos, which shorter lines take.
+WZ_D int32_t pair_even(int32_t k, int32_t n) {
+    if (n < 9) return int32_t(reflect_pos(2 * k, uint32_t(n)) >> 1);
+    const int32_t m = k < 0 ? -k : k;
+    return max(min(m, n - 1 - m), 0);
+}
+WZ_D int32_t pair_odd(int32_t k, int32_t n) {
+    if (n < 9) return int32_t(reflect_pos(2 * k + 1, uint32_t(n)) >> 1);
+    const int32_t m = max(k, -k - 1);
+    return max(min(m, n - 2 - m), 0);
+}
+
 // Threads of a workgroup that runs lds_pass.
 constexpr uint32_t kLdsThreads = 512;
 

@@ -23,6 +23,7 @@
 #include <tuple>
 #include <type_traits>
 
+#include "buffer.hpp"
 #include "common.hpp"
 #include "fused.hpp"
 #include "launch.hpp"
@@ -182,72 +183,170 @@ bool plane_pair(const T* src, T* dst, Dims full, Dims act, int a0, int a1, uint3
     return true;
 }
 
-// Every Z level of the plane schedule in one pass (its Z phase): one
-// workgroup per row of 64 columns stages the columns, all z, in LDS, runs the
-// levels' Z lifting there (lds_pass: the tiles and arithmetic of the Z axis
-// passes, so the same bits) and writes them once. src may equal dst; status:
-// screen for non-finite samples the forward's input (its first pass) or the
-// inverse's output (its last).
-constexpr uint32_t kZColBytes = 66560;
-constexpr uint32_t kZColumns = 64;
-bool zcol_fits(uint32_t nz, unsigned width) { return nz <= kZColBytes / kZColumns / width; }
+// Every Z level of the plane schedule in one pass (its Z phase). A workgroup
+// of four waves owns a row of 64 columns, all z; a wave takes one tile of the
+// 64 columns at a time, a lane a column, so that a tile's rows, their
+// mirrored places and its tests are wave-uniform (scalar): per sample only the
+// lifting itself and its loads and stores reach the vector unit. The finest
+// level reads (forward) or writes (inverse) the field and every high band
+// goes between registers and the volume directly; only the low boxes between
+// the levels pass through LDS, alternating between two buffers (box 1 in the
+// first, ceil(nz/2) rows, box 2 in the second, box 3 in the first again), with
+// one barrier per level. Tiles and arithmetic are those of the Z axis passes
+// (lift_forward / lift_inverse folded), so the same bits. src != dst; status:
+// screen for non-finite samples the forward's input or the inverse's output.
+// Bound by memory: it reads and writes the field once, at 3.3-4.0 TB/s. With
+// every column staged in LDS and per-lane index arithmetic it was bound by
+// vector issue: 500x500x100 float 108 -> 55 us (forward), 127 -> 61 us
+// (inverse), 384x384x96 double 70 -> 56 us, 73 -> 67 us.
+constexpr uint32_t kZColumns = 64, kZThreads = 256;
+uint64_t zcol_lds_bytes(uint32_t nz, unsigned levels, unsigned width) {
+    if (levels < 2) return 0;
+    const uint32_t n1 = half_len(nz), n2 = levels > 2 ? half_len(n1) : 0u;
+    return uint64_t(n1 + n2) * kZColumns * width;
+}
+// 64 KiB of LDS: nz up to 341 (float) or 170 (double) whatever the levels
+bool zcol_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5, width) <= 65536; }
 
 template <class T, bool Inverse>
-__global__ void __launch_bounds__(kLdsThreads) zcol_levels_kernel(const T* src, T* dst, Dims full, uint32_t levels,
-                                                                  uint32_t* __restrict__ status) {
-    constexpr int ZTile = Inverse ? (sizeof(T) == 4 ? 16 : 8) : 8;
-    __shared__ T A[kZColBytes / sizeof(T)];
-    const uint32_t t = threadIdx.x;
+__global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(const T* __restrict__ src, T* __restrict__ dst,
+                                                                Dims full, uint32_t levels,
+                                                                uint32_t* __restrict__ status) {
+    constexpr int Tile = sizeof(T) == 4 ? 16 : 8, P = Tile / 2 + 4;  // (the inverse's is part of the format)
+    constexpr uint32_t W = kZThreads / 64;
+    extern __shared__ __attribute__((aligned(16))) uint8_t zlds[];
+    T* const box0 = reinterpret_cast<T*>(zlds);
+    T* const box1 = box0 + uint64_t(half_len(full.nz)) * kZColumns;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const uint32_t xb = (full.nx + kZColumns - 1) / kZColumns;
-    const uint32_t y = blockIdx.x / xb, x0 = (blockIdx.x - y * xb) * kZColumns;
-    const uint32_t cols = min(kZColumns, full.nx - x0), cells = cols * full.nz;
-    const uint64_t plane = uint64_t(full.nx) * full.ny, base = uint64_t(y) * full.nx + x0;
-    const FastDiv by_cols(cols);  // cells fit LDS: exact
-    // every thread issues kBurst loads before it writes any of them to LDS
-    constexpr uint32_t kBurst = 8;
-    bool ok = true;
-    for (uint32_t i0 = 0; i0 < cells; i0 += kBurst * kLdsThreads) {
-        T v[kBurst];
-#pragma unroll
-        for (uint32_t k = 0; k < kBurst; ++k) {
-            const uint32_t i = i0 + k * kLdsThreads + t, r = by_cols.div(i);
-            v[k] = i < cells ? src[uint64_t(r) * plane + base + (i - r * cols)] : T(0);
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kBurst; ++k) {
-            const uint32_t i = i0 + k * kLdsThreads + t, r = by_cols.div(i);
-            if (i < cells) {
-                ok = ok && (Inverse || !status || __builtin_isfinite(v[k]));
-                A[r * kZColumns + (i - r * cols)] = v[k];
-            }
-        }
-    }
-    if (__ballot(!ok) && (t & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteInput));
-    __syncthreads();
-    uint32_t ex[5];
-    ex[0] = full.nz;
-    for (uint32_t l = 1; l < 5; ++l) ex[l] = half_len(ex[l - 1]);
+    // consecutive column rows go to one XCD (workgroups are dealt to the eight
+    // in turn): rows are no multiple of a cache line in general, and
+    // neighbours share the lines at their ends
+    const uint32_t total = xb * full.ny, per = (total + 7) / 8;
+    const uint32_t id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+    if (id >= total) return;
+    const uint32_t y = id / xb, x = (id - y * xb) * kZColumns + lane;
+    const bool in = x < full.nx;
+    // byte offsets: the field's bytes fit 32 bits
+    const uint32_t plane = full.nx * full.ny * uint32_t(sizeof(T));
+    const uint32_t col = (y * full.nx + (in ? x : full.nx - 1u)) * uint32_t(sizeof(T));
+    const auto ws = window(src), wd = window(dst);
+    bool fin = true;
     for (uint32_t k = 0; k < levels; ++k) {
         const uint32_t l = Inverse ? levels - 1 - k : k;
-        lds_pass<T, Inverse, 2, ZTile>(A, kZColumns, ex[l], cols);  // ends with a barrier
+        uint32_t m = full.nz;
+        for (uint32_t i = 0; i < l; ++i) m = half_len(m);
+        const int32_t n = int32_t(m), h = int32_t(half_len(m));
+        const bool finest = l == 0, coarsest = l + 1 == levels;
+        // this level's box (l >= 1) and the next coarser one
+        T* const own = (l & 1u) ? box0 : box1;
+        T* const low = (l & 1u) ? box1 : box0;
+        for (uint32_t tile = wave; int32_t(tile) * Tile < n; tile += W) {
+            T e[P], o[P];
+            const int32_t k0 = int32_t(tile) * (Tile / 2) - 2;
+            const bool inner = k0 >= 0 && 2 * (k0 + P) <= n;  // no mirrored position
+            if constexpr (!Inverse) {
+                if (finest) {
+                    if (inner) {
+                        uint32_t at = uint32_t(2 * k0) * plane;
+#pragma unroll
+                        for (int j = 0; j < P; ++j) {
+                            e[j] = buf_load_at(T(0), ws, col, at);
+                            o[j] = buf_load_at(T(0), ws, col, at + plane);
+                            at += 2 * plane;
+                        }
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < P; ++j) {
+                            e[j] = buf_load_at(T(0), ws, col, uint32_t(2 * pair_even(k0 + j, n)) * plane);
+                            o[j] = buf_load_at(T(0), ws, col, uint32_t(2 * pair_odd(k0 + j, n) + 1) * plane);
+                        }
+                    }
+                    if (status) {
+#pragma unroll
+                        for (int j = 2; j < P - 2; ++j) fin = fin && finite_value(e[j]) && finite_value(o[j]);
+                    }
+                } else {
+                    const T* b = own + lane;
+#pragma unroll
+                    for (int j = 0; j < P; ++j) {
+                        e[j] = b[uint32_t(2 * pair_even(k0 + j, n)) * kZColumns];
+                        o[j] = b[uint32_t(2 * pair_odd(k0 + j, n) + 1) * kZColumns];
+                    }
+                }
+                lift_forward<T, P>(e, o);
+                T* b = low + uint32_t(k0 + 2) * kZColumns + lane;
+                uint32_t at = uint32_t(k0 + 2) * plane, up = uint32_t(k0 + 2 + h) * plane;
+#pragma unroll
+                for (int j = 2; j < P - 2; ++j) {
+                    if (2 * (k0 + j) < n) {
+                        if (!coarsest) b[uint32_t(j - 2) * kZColumns] = e[j];
+                        else if (in) buf_store_at(e[j], wd, col, at);
+                    }
+                    if (2 * (k0 + j) + 1 < n && in) buf_store_at(o[j], wd, col, up);
+                    at += plane;
+                    up += plane;
+                }
+            } else {
+                if (inner) {
+                    uint32_t at = uint32_t(k0) * plane, up = uint32_t(k0 + h) * plane;
+#pragma unroll
+                    for (int j = 0; j < P; ++j) {
+                        if (coarsest) e[j] = buf_load_at(T(0), ws, col, at);
+                        o[j] = buf_load_at(T(0), ws, col, up);
+                        at += plane;
+                        up += plane;
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < P; ++j) {
+                        if (coarsest) e[j] = buf_load_at(T(0), ws, col, uint32_t(pair_even(k0 + j, n)) * plane);
+                        o[j] = buf_load_at(T(0), ws, col, uint32_t(h + pair_odd(k0 + j, n)) * plane);
+                    }
+                }
+                if (!coarsest) {
+                    const T* b = low + lane;
+#pragma unroll
+                    for (int j = 0; j < P; ++j) e[j] = b[uint32_t(pair_even(k0 + j, n)) * kZColumns];
+                }
+                lift_inverse<T, P, true>(e, o);
+                T* b = own + uint32_t(2 * (k0 + 2)) * kZColumns + lane;
+                uint32_t at = uint32_t(2 * (k0 + 2)) * plane;
+#pragma unroll
+                for (int j = 2; j < P - 2; ++j) {
+                    const int32_t q = 2 * (k0 + j);
+                    if (q < n) {
+                        if (!finest) b[uint32_t(2 * (j - 2)) * kZColumns] = e[j];
+                        else if (in) buf_store_at(e[j], wd, col, at);
+                    }
+                    if (q + 1 < n) {
+                        if (!finest) b[uint32_t(2 * (j - 2) + 1) * kZColumns] = o[j];
+                        else if (in) buf_store_at(o[j], wd, col, at + plane);
+                    }
+                    if (finest && status) {
+                        if (q < n) fin = fin && finite_value(e[j]);
+                        if (q + 1 < n) fin = fin && finite_value(o[j]);
+                    }
+                    at += 2 * plane;
+                }
+            }
+        }
+        __syncthreads();
     }
-    bool fin = true;
-    for (uint32_t i = t; i < cells; i += kLdsThreads) {
-        const uint32_t r = by_cols.div(i), c = i - r * cols;
-        const T v = A[r * kZColumns + c];
-        if (Inverse && status) fin = fin && __builtin_isfinite(v);
-        dst[uint64_t(r) * plane + base + c] = v;
-    }
-    if (__ballot(!fin) && (t & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteOutput));
+    if (status && __ballot(!fin) && lane == 0)
+        atomicOr(status, uint32_t(Inverse ? kNonFiniteOutput : kNonFiniteInput));
 }
 
 template <class T, bool Inverse>
 void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* status, hipStream_t s) {
-    if (!zcol_fits(full.nz, sizeof(T)) || levels > 5) throw std::logic_error("Z phase does not fit LDS");
-    const uint64_t blocks = uint64_t(full.ny) * ((full.nx + kZColumns - 1) / kZColumns);
-    check_launch_size(blocks * kLdsThreads);
-    hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse>), dim3(uint32_t(blocks)), dim3(kLdsThreads), 0, s, src, dst,
-                       full, uint32_t(levels), status);
+    if (!zcol_fits(full.nz, sizeof(T)) || levels < 1 || levels > 5 || src == dst)
+        throw std::logic_error("Z phase does not fit LDS");
+    const uint64_t total = uint64_t(full.ny) * ((full.nx + kZColumns - 1) / kZColumns);
+    const uint64_t blocks = 8 * ((total + 7) / 8);
+    check_launch_size(blocks * kZThreads);
+    hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse>), dim3(uint32_t(blocks)), dim3(kZThreads),
+                       uint32_t(zcol_lds_bytes(full.nz, levels, sizeof(T))), s, src, dst, full, uint32_t(levels),
+                       status);
 }
 
 // One XY level of the plane schedule per launch: a workgroup of 256 threads
@@ -809,7 +908,7 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
     }
     static const int zonly[1] = {2};
     static const int yx[2] = {1, 0};
-    // every XY level as one fused launch: the Z phase (one LDS-staged pass)
+    // every XY level as one fused launch: the Z phase (one pass)
     // into tmp1, then level l reads its box (tmp1, then the compact boxes in
     // tmp0) and writes its high bands into coeff and its low band into the
     // next box (coeff for the last level)
@@ -841,7 +940,7 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
         return;
     }
     Dims act = full;
-    if (lz && zcol_fits(full.nz, sizeof(T))) {  // the Z phase in one LDS-staged pass
+    if (lz && zcol_fits(full.nz, sizeof(T)) && p.first_src != coeff) {  // the Z phase in one pass
         StageClock clock("forward_Z", s);
         zcol_levels<T, false>(p.first_src, coeff, full, lz, status, s);
         p.first = false;
@@ -898,7 +997,7 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
     // every XY level as one fused launch: level l reads coeff's bands and the
     // coarser reconstruction (coeff's low quadrant for the coarsest level,
     // then the compact boxes in tmp0) and writes its box to tmp0, the finest
-    // into tmp1, from which the Z phase (one LDS-staged pass) writes output
+    // into tmp1, from which the Z phase (one pass) writes output
     if (lxy && (lz ? zcol_fits(full.nz, sizeof(T)) : output != coeff)) {
         // the Z phase screens the output when asked (no repairs to fold here)
         uint32_t* screen = emit && emit->mode == kEmitStoreScreen && !emit->np && lz ? emit->status : nullptr;
@@ -930,7 +1029,7 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         return screen != nullptr;
     }
     for (int l = int(lxy) - 1; l >= 0; --l) p.level(full, xy[l], xyo, 2, lz == 0 && l == 0, unsigned(l));
-    if (lz && zcol_fits(full.nz, sizeof(T))) {  // the Z phase in one LDS-staged pass
+    if (lz && zcol_fits(full.nz, sizeof(T)) && (p.first ? p.first_src : p.home) != output) {  // in one pass
         StageClock clock("inverse_Z", s);
         zcol_levels<T, true>(p.first ? p.first_src : p.home, output, full, lz, nullptr, s);
     } else {
