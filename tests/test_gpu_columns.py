@@ -32,3 +32,23 @@ def test_column_pass_bitwise(oracle, case, dtype):
     assert np.array_equal(c.view(np.uint8), want.view(np.uint8))
     back = stages.transform(torch.from_numpy(want).cuda(), lxy, lz, False, True).cpu().numpy()
     assert np.array_equal(back.view(np.uint8), oracle.transform(want, lxy, lz, False, True).view(np.uint8))
+
+
+# rows whose flag words are shared with their neighbours (x not a multiple of
+# 32), partial column blocks, one Z level and several, few and many repairs
+@pytest.mark.parametrize("shape", [(9, 40, 33), (10, 17, 65), (12, 33, 20), (17, 70, 96), (33, 150, 130),
+                                   (80, 160, 64), (100, 300, 18)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("bound", [0.5, 2e-4])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+def test_repairs_of_the_column_pass(oracle, shape, bound, dtype):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import waltz_amd
+    nx, ny, nz = reversed(shape)
+    lx, lz, dyadic, _ = oracle.geometry(nx, ny, nz)
+    assert lz and not dyadic
+    x = field(shape, "noise", dtype) * 30 + field(shape, "checker", dtype)
+    want = oracle.compress(x, bound)
+    assert int.from_bytes(want[24:28], "little") > 0  # repairs
+    got = waltz_amd.compress(torch.from_numpy(x).cuda(), abs_error=bound).cpu().numpy().tobytes()
+    assert got == want

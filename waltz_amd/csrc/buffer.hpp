@@ -62,6 +62,13 @@ WZ_D float buf_load_at(float, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t 
 WZ_D double buf_load_at(double, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, int(voff), int(soff), 0));
 }
+// (read exactly once: non-temporal, as buf_load_nt)
+WZ_D float buf_load_at_nt(float, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, int(voff), int(soff), 2));
+}
+WZ_D double buf_load_at_nt(double, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, int(voff), int(soff), 2));
+}
 WZ_D void buf_store_at(float v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, int(voff), int(soff), 0);
 }

@@ -194,8 +194,8 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     const WzpShape ws = wzp_shape(n);
     const uint32_t nq = qcap(n);
     const uint32_t rtiles = (n + kRepairTile - 1) / kRepairTile;
-    uint32_t fsegs = 0, fcap = 0;  // repair segments of a fused finest inverse level
-    level0_repair_segments(g.d, g.lx, g.dyadic, sizeof(T), &fsegs, &fcap);
+    uint32_t fsegs = 0, fcap = 0;  // repair segments of the last inverse pass, when it detects them
+    level0_repair_segments(g.d, g.lx, g.lz, g.dyadic, sizeof(T), &fsegs, &fcap);
     const uint64_t rslots = std::max<uint64_t>(uint64_t(rtiles) * kRepairTile, uint64_t(fsegs) * fcap);
     const uint32_t rsegs = std::max(rtiles, fsegs);
 
@@ -208,6 +208,8 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     // other fields of full bricks quantize inside the encoder too
     const bool ranks = rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz);
     const bool fusedq = pairs || ranks;
+    // rows that share flag words: set by atomics, cleared beforehand
+    const bool shared_words = fsegs && (g.d.nx & 31u);
     auto plan = [&](Carve& c) {
         struct P {
             T *coeff, *t0, *t1, *rec;
@@ -221,10 +223,10 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         p.coeff = c.take<T>(n);
         p.t0 = c.take<T>(n);
         p.t1 = c.take<T>(n);
-        // the reconstruction of an unfused finest level and the encoder's
-        // staging slots: one region with a fused finest level (which never
-        // writes the reconstruction), else two, so that the WZP group pass
-        // can run beside the inverse
+        // the reconstruction and the encoder's staging slots: one region when
+        // the last inverse pass detects the repairs (the reconstruction is
+        // never written then), else two, so that the WZP group pass can run
+        // beside the inverse
         if (fsegs) {
             p.rec = reinterpret_cast<T*>(
                 c.take<uint8_t>(std::max<uint64_t>(uint64_t(n) * sizeof(T), wzp_staging_bytes(ws.chunks))));
@@ -237,15 +239,16 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         p.ridx = c.take<uint32_t>(rslots);
         p.rerr = c.take<T>(rslots);
         p.rcount = c.take<uint32_t>(rsegs);
-        p.rbm = c.take<uint32_t>(words);
+        if (!shared_words) p.rbm = c.take<uint32_t>(words);
         p.qidx = c.take<uint32_t>(nq);
         p.qval = c.take<uint32_t>(nq);
         p.seg = c.take<uint32_t>(finish_scratch_words(n));
         p.size = c.take<uint32_t>(ws.chunks);
-        // zero-initialised region: sign, q bitmap, lookback descriptors, counters
+        // zero-initialised region: sign, bitmaps, lookback descriptors, counters
         const size_t z0 = c.used;
         p.sign = c.take<uint32_t>(fusedq ? 0 : words);
         p.qbm = c.take<uint32_t>(words);
+        if (shared_words) p.rbm = c.take<uint32_t>(words);
         p.desc = c.take<unsigned long long>(ws.chunks);
         p.counters = c.take<uint32_t>(4);  // ticket, q count, repair total
         p.zeroed = reinterpret_cast<uint32_t*>(c.base + z0);
@@ -267,7 +270,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     // with the fused repair emitter and a quantizing encoder the finest
     // level's high bands stay unquantized in coeff; that kernel requantizes
     // them on load
-    const bool requant = fsegs && fusedq;
+    const bool requant = g.dyadic && fsegs && fusedq;
     // The group pass runs on the side stream beside the inverse levels (the
     // staging slots it reads are never written by them); the archive sections
     // wait for it.
@@ -302,8 +305,8 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         StageClock c("wzp_encode", s);
         wzp_encode(p.mag, p.sign, n, archive + 32, capacity - 32, wsc, &res->wzp_bytes, status, s, side);
     }
-    // finest inverse level with native repair detection fused in when that
-    // level runs as a fused kernel; otherwise reconstruct, then a repair pass
+    // the last inverse pass detects the native repairs where it can (fsegs);
+    // otherwise reconstruct, then a repair pass
     Level0Emit<T> emit{kEmitRepair, status, input, abs_bound, SegList{p.rbm, p.ridx, p.rerr, p.rcount, fsegs, fcap},
                        requant ? quantum : 0.0};
     SegList rp = emit.rep;

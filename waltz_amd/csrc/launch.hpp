@@ -22,16 +22,18 @@ inline void check_launch_size(uint64_t total) {
 template <class T>
 void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz,
                        bool dyadic, uint32_t* status, hipStream_t s);
-// What the last (finest) inverse level does with its reconstruction when it
-// runs as a fused kernel: store it (optionally screening for non-finite
-// samples) or, without storing, derive native repairs against `orig`.
+// What the last inverse pass (the fused finest level of a dyadic field, the Z
+// phase of a plane-schedule one) does with its reconstruction: store it
+// (optionally screening for non-finite samples) or, without storing, derive
+// native repairs against `orig`.
 template <class T>
 struct Level0Emit {
     int mode;          // InvEmit (fused.hpp)
     uint32_t* status;
     const T* orig;
     double bound;
-    SegList rep;       // segments/cap per level0_repair_segments()
+    SegList rep;       // segments/cap per level0_repair_segments(); its bitmap
+                       // cleared by the caller unless rows are whole words (nx % 32 == 0)
     double quantum;    // kEmitRepair: > 0 when the finest level's high bands hold the
                        // unquantized coefficients (quantized and dequantized on load)
     // kEmitStoreScreen: a repair list (strictly increasing indices, np > 0
@@ -51,8 +53,7 @@ struct Level0Emit {
 // tile), or 0 when a list of np entries of `width`-byte values cannot be
 // folded into the finest level's stores for this geometry.
 uint64_t patch_table_words(Dims full, uint32_t np, unsigned width);
-// Returns true when `emit` was carried out inside the fused finest level;
-// false means the caller must run the equivalent separate pass on `output`.
+// Returns true when `emit` was carried out inside the last pass; false means the caller must run the equivalent separate pass on `output`.
 // requant > 0 (plane-schedule fields with plane_fused_fits only): coeff holds
 // the unquantized coefficients, quantized with this quantum and dequantized
 // as the levels load them.
@@ -105,9 +106,9 @@ void inverse_coarse_requant(const T* coeff, T* t0, T* t1, Dims full, unsigned lx
 template <class T>
 void inverse_finest_requant(const T* coeff, const T* t0, Dims full, unsigned lxy, const Level0Emit<T>& emit,
                             hipStream_t s);
-// Segments and per-segment capacity the fused finest inverse level uses for
-// repairs (0 segments when that level is not fused for this geometry).
-void level0_repair_segments(Dims full, unsigned lxy, bool dyadic, unsigned width, uint32_t* segments,
+// Segments and per-segment capacity the last inverse pass uses for repairs
+// (0 segments when it does not detect them for this geometry).
+void level0_repair_segments(Dims full, unsigned lxy, unsigned lz, bool dyadic, unsigned width, uint32_t* segments,
                             uint32_t* cap);
 
 

@@ -15,6 +15,7 @@
 // Y and Z lines map consecutive lanes to consecutive x, so every register load
 // is a fully coalesced 256 B (f32) / 512 B (f64) wave access; X lines map lanes
 // to consecutive tiles of one row (overlapping 64 B windows served from L1).
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <map>
@@ -208,10 +209,94 @@ uint64_t zcol_lds_bytes(uint32_t nz, unsigned levels, unsigned width) {
 // 64 KiB of LDS: nz up to 341 (float) or 170 (double) whatever the levels
 bool zcol_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5, width) <= 65536; }
 
-template <class T, bool Inverse>
+//
+// Repair (inverse, compress): the reconstruction is not written; each sample
+// is compared with the original as its tile is lifted, and the native repair
+// records and flag bits go out (one segment per workgroup, columns x nz slots).
+// That drops a write and a read of the field and one launch: 384x384x96
+// double, inverse and repair passes 67 + 47 us before.
+template <class T>
+struct ZRepair {
+    const T* orig;
+    double bound;
+    T bound_lo;  // the largest T <= bound
+    SegList rep;
+};
+// Decides the samples v[j] (rows z + j of column x, row y) of a wave's tile
+// against their originals, sets their flag bits and appends their records to
+// segment `id`; false when a lane's sample cannot meet the bound. Wave masks
+// as in the fused finest level: the rounded difference of the final value and
+// the original settles the strict bound unless it is not below it.
+template <class T, int Tile>
+WZ_D bool zcol_repairs(const T (&v)[Tile], const T (&ref)[Tile], const ZRepair<T>& rp, Dims full, uint32_t x,
+                       uint32_t y, uint32_t z, bool in, uint32_t id, uint32_t* seg_fill) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const unsigned long long in_m = __ballot(in);
+    const T nb = T(rp.bound);
+    bool ok = true;
+    unsigned long long masks[Tile];
+    T err[Tile];
+    uint32_t total = 0;
+#pragma unroll
+    for (int j = 0; j < Tile; ++j) {
+        masks[j] = 0;
+        err[j] = v[j] - ref[j];
+        if (z + uint32_t(j) >= full.nz) continue;  // (wave-uniform)
+        const T e = err[j];
+        const bool p = abs_t(e) > nb;
+        const T d = p ? (v[j] - e) - ref[j] : e;
+        const bool fast = abs_t(d) < rp.bound_lo;
+        masks[j] = __ballot(p) & in_m;
+        if (in_m & ~__ballot(fast)) {  // a tie at the bound or a non-finite sample: the full test
+            bool okj = true;
+            T ej;
+            const bool pj = repair_decision<T>(v[j], ref[j], nb, rp.bound, &ej, &okj);
+            masks[j] = __ballot(pj) & in_m;
+            ok = ok && (!in || okj);
+        }
+        total += uint32_t(__popcll(masks[j]));
+    }
+    uint32_t base = 0;
+    if (total && lane == 0) base = atomicAdd(seg_fill, total);
+    base = __builtin_amdgcn_readfirstlane(base);
+    const uint32_t row_words = (full.nx & 31u) == 0;
+    uint32_t at = uint32_t((uint64_t(z) * full.ny + y) * full.nx) + x;  // sample index of row z
+    uint32_t* const index = rp.rep.index + uint64_t(id) * rp.rep.cap;
+    T* const payload = static_cast<T*>(rp.rep.payload) + uint64_t(id) * rp.rep.cap;
+#pragma unroll
+    for (int j = 0; j < Tile; ++j) {
+        if (z + uint32_t(j) >= full.nz) continue;
+        const unsigned long long m = masks[j];
+        const uint32_t first = at - lane;  // sample of lane 0
+        if (row_words) {  // the row's 64 samples own whole words
+            if (lane < 2 && x - lane + 32u * lane < full.nx)
+                rp.rep.bitmap[(first >> 5) + lane] = uint32_t(m >> (32u * lane));
+        } else if (m && lane < 3) {  // shared words of a cleared bitmap
+            const uint32_t s = first & 31u;
+            const unsigned long long lo = m << s;
+            const uint32_t w = lane == 0   ? uint32_t(lo)
+                               : lane == 1 ? uint32_t(lo >> 32)
+                               : s         ? uint32_t(m >> (64u - s))
+                                           : 0u;
+            if (w) atomicOr(&rp.rep.bitmap[(first >> 5) + lane], w);
+        }
+        if ((m >> lane) & 1ull) {
+            const uint32_t k = base + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+            index[k] = at;
+            payload[k] = err[j];
+        }
+        base += uint32_t(__popcll(m));
+        at += full.nx * full.ny;
+    }
+    return ok;
+}
+
+template <class T, bool Inverse, bool Repair>
 __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(const T* __restrict__ src, T* __restrict__ dst,
                                                                 Dims full, uint32_t levels,
-                                                                uint32_t* __restrict__ status) {
+                                                                uint32_t* __restrict__ status, ZRepair<T> rp) {
+    static_assert(Inverse || !Repair, "repairs follow the inverse");
+    __shared__ uint32_t seg_fill;  // repair entries of this workgroup
     constexpr int Tile = sizeof(T) == 4 ? 16 : 8, P = Tile / 2 + 4;  // (the inverse's is part of the format)
     constexpr uint32_t W = kZThreads / 64;
     extern __shared__ __attribute__((aligned(16))) uint8_t zlds[];
@@ -230,8 +315,12 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(const T* __restr
     // byte offsets: the field's bytes fit 32 bits
     const uint32_t plane = full.nx * full.ny * uint32_t(sizeof(T));
     const uint32_t col = (y * full.nx + (in ? x : full.nx - 1u)) * uint32_t(sizeof(T));
-    const auto ws = window(src), wd = window(dst);
+    const auto ws = window(src), wd = window(Repair ? rp.orig : dst);
     bool fin = true;
+    if constexpr (Repair) {  // (a tile's entries are counted after at least one barrier)
+        if (threadIdx.x == 0) seg_fill = 0;
+        if (levels == 1) __syncthreads();
+    }
     for (uint32_t k = 0; k < levels; ++k) {
         const uint32_t l = Inverse ? levels - 1 - k : k;
         uint32_t m = full.nz;
@@ -304,12 +393,36 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(const T* __restr
                         o[j] = buf_load_at(T(0), ws, col, uint32_t(h + pair_odd(k0 + j, n)) * plane);
                     }
                 }
+                T ref[Repair ? Tile : 1];  // the tile's originals, in flight with its coefficients
+                if constexpr (Repair) {
+                    if (finest) {
+                        uint32_t at = tile * uint32_t(Tile) * plane;
+#pragma unroll
+                        for (int j = 0; j < Tile; ++j) {
+                            ref[j] = buf_load_at_nt(T(0), wd, col, int32_t(tile) * Tile + j < n ? at : 0u);
+                            at += plane;
+                        }
+                    }
+                }
                 if (!coarsest) {
                     const T* b = low + lane;
 #pragma unroll
                     for (int j = 0; j < P; ++j) e[j] = b[uint32_t(pair_even(k0 + j, n)) * kZColumns];
                 }
                 lift_inverse<T, P, true>(e, o);
+                if constexpr (Repair) {
+                    if (finest) {
+                        T v[Tile];
+#pragma unroll
+                        for (int j = 0; j < Tile / 2; ++j) {
+                            v[2 * j] = e[j + 2];
+                            v[2 * j + 1] = o[j + 2];
+                        }
+                        const uint32_t z = tile * uint32_t(Tile);
+                        fin = zcol_repairs<T, Tile>(v, ref, rp, full, x, y, z, in, id, &seg_fill) && fin;
+                        continue;
+                    }
+                }
                 T* b = own + uint32_t(2 * (k0 + 2)) * kZColumns + lane;
                 uint32_t at = uint32_t(2 * (k0 + 2)) * plane;
 #pragma unroll
@@ -334,19 +447,33 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(const T* __restr
         __syncthreads();
     }
     if (status && __ballot(!fin) && lane == 0)
-        atomicOr(status, uint32_t(Inverse ? kNonFiniteOutput : kNonFiniteInput));
+        atomicOr(status, uint32_t(Repair ? kRepairBound : Inverse ? kNonFiniteOutput : kNonFiniteInput));
+    if constexpr (Repair) {
+        if (threadIdx.x == 0) rp.rep.count[id] = seg_fill;
+    }
 }
 
 template <class T, bool Inverse>
-void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* status, hipStream_t s) {
+void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* status, hipStream_t s,
+                 const ZRepair<T>* repair = nullptr) {
     if (!zcol_fits(full.nz, sizeof(T)) || levels < 1 || levels > 5 || src == dst)
         throw std::logic_error("Z phase does not fit LDS");
     const uint64_t total = uint64_t(full.ny) * ((full.nx + kZColumns - 1) / kZColumns);
     const uint64_t blocks = 8 * ((total + 7) / 8);
     check_launch_size(blocks * kZThreads);
-    hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse>), dim3(uint32_t(blocks)), dim3(kZThreads),
-                       uint32_t(zcol_lds_bytes(full.nz, levels, sizeof(T))), s, src, dst, full, uint32_t(levels),
-                       status);
+    const dim3 grid{uint32_t(blocks)};
+    const uint32_t lds = uint32_t(zcol_lds_bytes(full.nz, levels, sizeof(T)));
+    if constexpr (Inverse) {
+        if (repair) {
+            if (repair->rep.segments != total || repair->rep.cap < uint64_t(std::min(full.nx, kZColumns)) * full.nz)
+                throw std::logic_error("repair segments do not match the Z phase's launch");
+            hipLaunchKernelGGL((zcol_levels_kernel<T, true, true>), grid, dim3(kZThreads), lds, s, src, dst, full,
+                               uint32_t(levels), status, *repair);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse, false>), grid, dim3(kZThreads), lds, s, src, dst, full,
+                       uint32_t(levels), status, ZRepair<T>{});
 }
 
 // One XY level of the plane schedule per launch: a workgroup of 256 threads
@@ -817,8 +944,6 @@ void launch_finest(const T* coeff, const T* lo, uint32_t lpy, uint32_t lpz, T* o
             if (a.sz % 16 || inv_segments(full, a.sz) != emit->rep.segments)
                 throw std::logic_error("repair segments do not match the finest level's launch");
         }
-        if (repairs && (full.nx & 31u))  // atomics path needs a clean bitmap
-            zero_words(emit->rep.bitmap, (uint64_t(full.nx) * full.ny * full.nz + 31) / 32, s);
     }
     launch_inv_level<T>(a, s);
 }
@@ -862,10 +987,15 @@ void fused_inverse(T* coeff, T* output, T* tmp0, Dims full, unsigned levels, con
     launch_finest<T>(coeff, low.p, low.py, low.pz, output, full, tu.sz[0], emit, s, names[base]);
 }
 
-void level0_repair_segments(Dims full, unsigned lxy, bool dyadic, unsigned width, uint32_t* segments,
+void level0_repair_segments(Dims full, unsigned lxy, unsigned lz, bool dyadic, unsigned width, uint32_t* segments,
                             uint32_t* cap) {
     *segments = 0;
     *cap = 0;
+    if (!dyadic && plane_fused_fits(full, lxy, lz, width)) {  // the Z phase detects them, by rows of columns
+        *segments = full.ny * ((full.nx + kZColumns - 1) / kZColumns);
+        *cap = std::min(full.nx, kZColumns) * full.nz;
+        return;
+    }
     if (!dyadic || !lxy) return;
     const Tuning tu = tuning_for(full, lxy, width, true);
     if (!tu.fused) return;
@@ -1001,6 +1131,7 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
     if (lxy && (lz ? zcol_fits(full.nz, sizeof(T)) : output != coeff)) {
         // the Z phase screens the output when asked (no repairs to fold here)
         uint32_t* screen = emit && emit->mode == kEmitStoreScreen && !emit->np && lz ? emit->status : nullptr;
+        const bool repair = emit && emit->mode == kEmitRepair && lz;
         static const char* names[] = {"inverse_L0", "inverse_L1", "inverse_L2", "inverse_L3", "inverse_L4"};
         const T* lo = coeff;
         uint64_t lpy = full.nx, lpz = uint64_t(full.nx) * full.ny;
@@ -1024,9 +1155,16 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         }
         if (lz) {
             StageClock clock("inverse_Z", s);
-            zcol_levels<T, true>(tmp1, output, full, lz, screen, s);
+            if (repair) {
+                T lo = T(emit->bound);
+                if (double(lo) > emit->bound) lo = std::nextafter(lo, T(0));
+                const ZRepair<T> z{emit->orig, emit->bound, lo, emit->rep};
+                zcol_levels<T, true>(tmp1, output, full, lz, emit->status, s, &z);
+            } else {
+                zcol_levels<T, true>(tmp1, output, full, lz, screen, s);
+            }
         }
-        return screen != nullptr;
+        return screen != nullptr || repair;
     }
     for (int l = int(lxy) - 1; l >= 0; --l) p.level(full, xy[l], xyo, 2, lz == 0 && l == 0, unsigned(l));
     if (lz && zcol_fits(full.nz, sizeof(T)) && (p.first ? p.first_src : p.home) != output) {  // in one pass
