@@ -30,6 +30,7 @@
 #include "launch.hpp"
 #include "lifting.hpp"
 #include "profile.hpp"
+#include "xystrip.hpp"
 
 namespace wz {
 
@@ -476,203 +477,65 @@ void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* sta
                        uint32_t(levels), status, ZRepair<T>{});
 }
 
-// One XY level of the plane schedule per launch: a workgroup of 256 threads
-// owns a 64 x 32 tile of one plane, runs the level's first pass (inverse: X,
-// forward: Y) over the tile and the halo the second pass reads, keeps the
-// results in LDS and runs the second pass from there, so the level reads its
-// input once (halos aside) and writes once. Tiles and arithmetic are those of
-// lift_tile (inverse Y tile 8 folded, every other tile 8 and unfolded), so
-// every value equals the per-axis passes'.
-constexpr uint32_t kXYW = 64, kXYH = 32, kXYThreads = 256;
-
-struct XYTile {
-    uint32_t x0, y0, z;
-};
-// Tile of this workgroup: consecutive tiles go to one XCD (workgroups are
-// dealt to the eight XCDs in turn), so neighbours' halos meet in its L2.
-WZ_D bool xy_tile(Dims n, XYTile& t) {
-    const uint32_t tx = (n.nx + kXYW - 1) / kXYW, ty = (n.ny + kXYH - 1) / kXYH;
-    const uint32_t total = tx * ty * n.nz, per = (total + 7) / 8;
+// One XY level (of the plane schedule, or of a dyadic level that runs as
+// passes) per launch, four strips of planes per workgroup. Consecutive items
+// go to one XCD (workgroups are dealt to the eight XCDs in turn), so that
+// neighbours' halos and warm-up rows meet in its L2.
+WZ_D bool strip_of_wave(const StripPlan& p, uint32_t& item) {
+    const uint32_t total = uint32_t(p.items()), groups = (total + 3) / 4, per = (groups + 7) / 8;
     const uint32_t id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
-    if (id >= total) return false;
-    t.x0 = (id % tx) * kXYW;
-    t.y0 = ((id / tx) % ty) * kXYH;
-    t.z = id / (tx * ty);
-    return true;
+    item = 4 * id + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    return id < groups && item < total;
 }
-uint32_t xy_blocks(Dims n) {
-    const uint64_t total = uint64_t((n.nx + kXYW - 1) / kXYW) * ((n.ny + kXYH - 1) / kXYH) * n.nz;
-    check_launch_size(8 * ((total + 7) / 8) * kXYThreads);
-    return uint32_t(8 * ((total + 7) / 8));
+template <class T, bool Requant>
+__global__ void __launch_bounds__(kStripThreads) xy_inverse_kernel(XYInverse<T> a, StripPlan p) {
+    uint32_t item;
+    if (strip_of_wave(p, item)) strip_inverse<T, Requant>(a, p, item);
 }
-
 template <class T>
-struct XYInverse {
-    const T* hi;  // the level's coefficients outside its low box
-    uint64_t hpy, hpz;
-    const T* lo;  // its low box [0, ceil(nx/2)) x [0, ceil(ny/2)): the coarser reconstruction
-    uint64_t lpy, lpz;
-    T* out;  // the level's reconstruction (natural layout)
-    uint64_t opy, opz;
-    Dims n;  // level box: nx x ny, every plane
-    // q > 0: the coefficients hold unquantized values, quantized and
-    // dequantized as they load (the low box too when lo_coeff: the coarsest
-    // level, whose low box is the coefficient volume's)
-    T q, inv;
-    uint32_t lo_coeff;
-};
-
-template <class T>
-__global__ void __launch_bounds__(kXYThreads) xy_inverse_kernel(XYInverse<T> a) {
-    constexpr int TX = 8, P = TX / 2 + 4;  // X tiles
-    constexpr uint32_t R = kXYH + 8;       // y positions y0 - 4 .. y0 + 35 (interleaved)
-    constexpr uint32_t kTiles = kXYW / TX;
-    __shared__ T S[R][kXYW + 1];
-    XYTile tl;
-    if (!xy_tile(a.n, tl)) return;
-    const uint32_t t = threadIdx.x, nx = a.n.nx, ny = a.n.ny, hx = half_len(nx), hy = half_len(ny);
-    const T* hiz = a.hi + uint64_t(tl.z) * a.hpz;
-    const T* loz = a.lo + uint64_t(tl.z) * a.lpz;
-    // X: row r of S is y position y0 - 4 + r, read from its split row
-    for (uint32_t item = t; item < R * kTiles; item += kXYThreads) {
-        const uint32_t r = item / kTiles, k = item % kTiles, start = tl.x0 + k * TX;
-        if (start >= nx) continue;
-        const uint32_t sr = split_pos(int32_t(tl.y0) - 4 + int32_t(r), ny);
-        const T* hrow = hiz + uint64_t(sr) * a.hpy;
-        const T* lrow = loz + uint64_t(sr) * a.lpy;
-        const bool lowrow = sr < hy;
-        T e[P], o[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const int32_t q = int32_t(start) - 4 + 2 * j;
-            const uint32_t ce = split_pos(q, nx), co = split_pos(q + 1, nx);
-            const bool le = lowrow && ce < hx, lo_ = lowrow && co < hx;
-            e[j] = le ? lrow[ce] : hrow[ce];
-            o[j] = lo_ ? lrow[co] : hrow[co];
-            if (a.q > T(0)) {  // (wave-uniform)
-                if (!le || a.lo_coeff) e[j] = requantize<T>(e[j], a.q, a.inv);
-                if (!lo_ || a.lo_coeff) o[j] = requantize<T>(o[j], a.q, a.inv);
-            }
-        }
-        lift_inverse<T, P, false>(e, o);
-#pragma unroll
-        for (int j = 2; j < P - 2; ++j) {
-            const uint32_t q = start + 2u * uint32_t(j - 2);
-            if (q < nx) S[r][q - tl.x0] = e[j];
-            if (q + 1 < nx) S[r][q + 1 - tl.x0] = o[j];
-        }
-    }
-    __syncthreads();
-    // Y (tile 8, folded): one (column, tile) per thread, lanes 64 consecutive x
-    constexpr int PY = 8;
-    const uint32_t c = t & 63u, k = t >> 6, x = tl.x0 + c, start = tl.y0 + 8 * k;
-    if (x >= nx || start >= ny) return;
-    T e[PY], o[PY];
-#pragma unroll
-    for (int j = 0; j < PY; ++j) {
-        e[j] = S[8 * k + 2 * j][c];
-        o[j] = S[8 * k + 2 * j + 1][c];
-    }
-    lift_inverse<T, PY, true>(e, o);
-    T* col = a.out + uint64_t(tl.z) * a.opz + x;
-#pragma unroll
-    for (int j = 2; j < PY - 2; ++j) {
-        const uint32_t q = start + 2u * uint32_t(j - 2);
-        if (q < ny) col[uint64_t(q) * a.opy] = e[j];
-        if (q + 1 < ny) col[uint64_t(q + 1) * a.opy] = o[j];
-    }
+__global__ void __launch_bounds__(kStripThreads) xy_forward_kernel(XYForward<T> a, StripPlan p) {
+    uint32_t item;
+    if (strip_of_wave(p, item)) strip_forward<T>(a, p, item);
 }
-
-template <class T>
-struct XYForward {
-    const T* src;  // the level's input (natural layout)
-    uint64_t spy, spz;
-    T* hi;  // where the three high bands go
-    uint64_t hpy, hpz;
-    T* lo;  // where the low band [0, ceil(nx/2)) x [0, ceil(ny/2)) goes
-    uint64_t lpy, lpz;
-    Dims n;
-    uint32_t* status;  // non-null: screen the input for non-finite samples
-};
-
-template <class T>
-__global__ void __launch_bounds__(kXYThreads) xy_forward_kernel(XYForward<T> a) {
-    constexpr int TL = 8, P = TL / 2 + 4;  // Y and X tiles
-    constexpr uint32_t C = kXYW + 8;       // x positions x0 - 4 .. x0 + 67 (reflected)
-    __shared__ T S[kXYH][C + 1];
-    XYTile tl;
-    if (!xy_tile(a.n, tl)) return;
-    const uint32_t t = threadIdx.x, nx = a.n.nx, ny = a.n.ny, hx = half_len(nx), hy = half_len(ny);
-    const T* srcz = a.src + uint64_t(tl.z) * a.spz;
-    // Y: column c of S is x position x0 - 4 + c (its reflected column); row r
-    // is the Y output of y position y0 + r (its split row)
-    bool ok = true;
-    for (uint32_t item = t; item < C * (kXYH / TL); item += kXYThreads) {
-        const uint32_t c = item % C, k = item / C, start = tl.y0 + k * TL;
-        if (start >= ny) continue;
-        const T* col = srcz + reflect_pos(int32_t(tl.x0) - 4 + int32_t(c), nx);
-        T e[P], o[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const int32_t q = int32_t(start) - 4 + 2 * j;
-            e[j] = col[uint64_t(reflect_pos(q, ny)) * a.spy];
-            o[j] = col[uint64_t(reflect_pos(q + 1, ny)) * a.spy];
-        }
-        if (a.status) {  // input screen (cpu/src/codec.cpp:183)
-#pragma unroll
-            for (int j = 0; j < P; ++j) ok = ok && finite_value(e[j]) && finite_value(o[j]);
-        }
-        lift_forward<T, P>(e, o);
-#pragma unroll
-        for (int j = 2; j < P - 2; ++j) {
-            const uint32_t q = start + 2u * uint32_t(j - 2);
-            if (q < ny) S[q - tl.y0][c] = e[j];
-            if (q + 1 < ny) S[q + 1 - tl.y0][c] = o[j];
-        }
-    }
-    if (a.status && !ok) atomicOr(a.status, uint32_t(kNonFiniteInput));
-    __syncthreads();
-    // X: one (row, tile) per thread; row r is split row sy of y = y0 + r
-    constexpr uint32_t kTiles = kXYW / TL;
-    for (uint32_t item = t; item < kXYH * kTiles; item += kXYThreads) {
-        const uint32_t r = item / kTiles, k = item % kTiles, y = tl.y0 + r, start = tl.x0 + k * TL;
-        if (y >= ny || start >= nx) continue;
-        const uint32_t sy = (y & 1u) ? hy + (y >> 1) : (y >> 1);
-        T e[P], o[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const uint32_t q = start + 2u * uint32_t(j) - tl.x0;  // S column of x position start - 4 + 2j
-            e[j] = S[r][q];
-            o[j] = S[r][q + 1];
-        }
-        lift_forward<T, P>(e, o);
-        const bool lowrow = sy < hy;
-        T* hrow = a.hi + uint64_t(tl.z) * a.hpz + uint64_t(sy) * a.hpy;
-        T* lrow = a.lo + uint64_t(tl.z) * a.lpz + uint64_t(sy) * a.lpy;
-#pragma unroll
-        for (int j = 2; j < P - 2; ++j) {
-            const uint32_t q = start + 2u * uint32_t(j - 2), ce = q >> 1, co = hx + (q >> 1);
-            if (q < nx) (lowrow && ce < hx ? lrow : hrow)[ce] = e[j];
-            if (q + 1 < nx) hrow[co] = o[j];
-        }
-    }
+uint32_t strip_blocks(const StripPlan& p) {
+    const uint64_t groups = (p.items() + 3) / 4, blocks = 8 * ((groups + 7) / 8);
+    check_launch_size(blocks * kStripThreads);
+    return uint32_t(blocks);
 }
+// Whether every XY level of an nx x ny plane runs as strips: no line of one
+// sample, and a plane inside one 32-bit window.
+bool strips_fit(Dims n, uint64_t pitch, uint64_t rows, unsigned levels, unsigned width) {
+    for (unsigned l = 0; l < levels; ++l) {
+        if (n.nx < 2 || n.ny < 2) return false;
+        n = shrink(n, true, false);
+    }
+    return fused_plane_fits(pitch, rows, width);
+}
+// Lines share a wave only while the planes of a group (at most eight) share a
+// window.
+bool strips_pack(uint64_t plane, unsigned width) { return fused_plane_fits(8 * plane, 1, width); }
 
 template <class T>
 void xy_inverse(const XYInverse<T>& a, hipStream_t s) {
-    hipLaunchKernelGGL((xy_inverse_kernel<T>), dim3(xy_blocks(a.n)), dim3(kXYThreads), 0, s, a);
+    const StripPlan p = strip_plan(a.n, strips_pack(std::max({a.hpz, a.lpz, a.opz}), sizeof(T)));
+    if (a.q > T(0))
+        hipLaunchKernelGGL((xy_inverse_kernel<T, true>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s, a, p);
+    else
+        hipLaunchKernelGGL((xy_inverse_kernel<T, false>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s, a, p);
 }
 template <class T>
 void xy_forward(const XYForward<T>& a, hipStream_t s) {
-    hipLaunchKernelGGL((xy_forward_kernel<T>), dim3(xy_blocks(a.n)), dim3(kXYThreads), 0, s, a);
+    const StripPlan p = strip_plan(a.n, strips_pack(std::max({a.hpz, a.lpz, a.spz}), sizeof(T)));
+    hipLaunchKernelGGL((xy_forward_kernel<T>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s, a, p);
 }
 
 // The X and Y passes of box `act` (in full-pitched arrays, src != dst) as one
-// tiled launch, in the order the tiled kernels lift (forward Y then X,
-// inverse X then Y); false for the other order.
+// launch, in the order the strips lift (forward Y then X, inverse X then Y);
+// false for the other order and for boxes that strips do not take.
 template <class T, bool Inverse>
 bool xy_pair(const T* src, T* dst, Dims full, Dims act, int a0, hipStream_t s) {
     const uint64_t py = full.nx, pz = uint64_t(full.nx) * full.ny;
+    if (!strips_fit(act, full.nx, full.ny, 1, sizeof(T))) return false;
     if constexpr (Inverse) {
         if (a0 != 0) return false;
         xy_inverse<T>(XYInverse<T>{src, py, pz, src, py, pz, dst, py, pz, act, T(0), T(0), 0u}, s);
@@ -1042,7 +905,8 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
     // into tmp1, then level l reads its box (tmp1, then the compact boxes in
     // tmp0) and writes its high bands into coeff and its low band into the
     // next box (coeff for the last level)
-    if (lxy && (lz ? zcol_fits(full.nz, sizeof(T)) : input != coeff)) {
+    if (strips_fit(full, full.nx, full.ny, lxy, sizeof(T)) && lxy &&
+        (lz ? zcol_fits(full.nz, sizeof(T)) : input != coeff)) {
         const T* src = input;
         uint64_t spy = full.nx, spz = uint64_t(full.nx) * full.ny;
         if (lz) {
@@ -1128,7 +992,8 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
     // coarser reconstruction (coeff's low quadrant for the coarsest level,
     // then the compact boxes in tmp0) and writes its box to tmp0, the finest
     // into tmp1, from which the Z phase (one pass) writes output
-    if (lxy && (lz ? zcol_fits(full.nz, sizeof(T)) : output != coeff)) {
+    if (strips_fit(full, full.nx, full.ny, lxy, sizeof(T)) && lxy &&
+        (lz ? zcol_fits(full.nz, sizeof(T)) : output != coeff)) {
         // the Z phase screens the output when asked (no repairs to fold here)
         uint32_t* screen = emit && emit->mode == kEmitStoreScreen && !emit->np && lz ? emit->status : nullptr;
         const bool repair = emit && emit->mode == kEmitRepair && lz;
@@ -1225,7 +1090,7 @@ bool transform_inverse_preserving(const T* coeff, T* output, T* tmp0, T* tmp1, D
 }
 
 bool plane_fused_fits(Dims full, unsigned lxy, unsigned lz, unsigned width) {
-    return lxy && lz && zcol_fits(full.nz, width);
+    return lxy && lz && zcol_fits(full.nz, width) && strips_fit(full, full.nx, full.ny, lxy, width);
 }
 
 bool coarse_split_fits(Dims full, unsigned lxy, unsigned width) {

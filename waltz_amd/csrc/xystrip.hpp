@@ -1,0 +1,368 @@
+// X and Y lifting of one level of a stack of planes in registers (no LDS, no
+// barrier), shared by the single-field and batched transforms.
+//
+// A wave owns a strip of a plane and walks it along y, two rows (one sample
+// pair) per step. A lane holds one (even, odd) sample pair of its line in x:
+// X lifting takes the neighbouring pairs' values from the neighbouring lanes
+// (one cross-lane move each), Y lifting streams down the strip with five live
+// values per column. So every value is loaded once (strip ends and the
+// warm-up rows of a strip's y segment aside), all loads and stores are whole
+// row segments, and a sample costs about 9 vector operations for X and 7 for
+// Y, well below what memory takes. Every value is the same sequence of
+// operations on the same operands as in lift_tile (inverse Y tile 8 folded,
+// X unfolded), so the same bits.
+//
+// Lines of up to 62 pairs, or of exactly 64, take one strip; longer ones
+// strips of 62, then 60 pairs with two pairs of halo on each side. Narrow
+// lines share a wave: groups of 8, 16 or 32 lanes take consecutive planes.
+// Mirroring: lanes past a line's end load the mirrored samples, so two such
+// lanes give the last pair its neighbours; at lane 0 of a line, and at the
+// last lane of a line of even length that fills its group, the neighbour's
+// value is the lane's own (the lifted extension keeps the symmetry).
+#pragma once
+
+#include <type_traits>
+
+#include "buffer.hpp"
+#include "common.hpp"
+#include "lifting.hpp"
+
+namespace wz {
+
+struct StripPlan {
+    uint32_t lw;      // log2 of the lanes of one line (3 .. 6)
+    uint32_t strips;  // strips of a line
+    uint32_t sy;      // rows of a y segment (a multiple of 8)
+    uint32_t segs;    // y segments
+    uint32_t zgroups; // groups of 64 >> lw planes
+    WZ_HD uint64_t items() const { return uint64_t(strips) * segs * zgroups; }  // waves
+};
+constexpr uint32_t kStripThreads = 256;
+
+// The plan of an nx x ny box of nz planes; `pack`: lines may share a wave
+// (false: the planes of a group would not fit one 32-bit window).
+WZ_HD StripPlan strip_plan(Dims n, bool pack) {
+    StripPlan p;
+    const uint32_t np = half_len(n.nx);
+    auto fits = [&](uint32_t w) { return np + 2 <= w || (np == w && !(n.nx & 1u)); };
+    p.lw = 6;
+    if (pack)
+        while (p.lw > 3 && fits(1u << (p.lw - 1))) --p.lw;
+    p.strips = fits(1u << p.lw) ? 1u : 1u + (np - 62u + 59u) / 60u;
+    p.zgroups = (n.nz + (64u >> p.lw) - 1) >> (6 - p.lw);
+    // long segments (few warm-up rows), halved while the waves are too few to
+    // keep memory busy
+    p.sy = 128;
+    auto waves = [&] { return uint64_t(p.strips) * p.zgroups * ((n.ny + p.sy - 1) / p.sy); };
+    while (p.sy > 32 && waves() < 4096) p.sy >>= 1;
+    if (waves() < 1024) p.sy = 16;
+    p.segs = (n.ny + p.sy - 1) / p.sy;
+    return p;
+}
+
+// The value of the lane before / after (cross-lane move over the wave), or the
+// lane's own at the end of its line.
+WZ_D float lane_prev(float v, bool own) {
+    const int x = __builtin_bit_cast(int, v);
+    const float r = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, 0x138, 0xf, 0xf, true));
+    return own ? v : r;
+}
+WZ_D float lane_next(float v, bool own) {
+    const int x = __builtin_bit_cast(int, v);
+    const float r = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, 0x130, 0xf, 0xf, true));
+    return own ? v : r;
+}
+WZ_D double lane_prev(double v, bool own) {
+    const int2 x = __builtin_bit_cast(int2, v);
+    const int2 r = make_int2(__builtin_amdgcn_update_dpp(0, x.x, 0x138, 0xf, 0xf, true),
+                             __builtin_amdgcn_update_dpp(0, x.y, 0x138, 0xf, 0xf, true));
+    return own ? v : __builtin_bit_cast(double, r);
+}
+WZ_D double lane_next(double v, bool own) {
+    const int2 x = __builtin_bit_cast(int2, v);
+    const int2 r = make_int2(__builtin_amdgcn_update_dpp(0, x.x, 0x130, 0xf, 0xf, true),
+                             __builtin_amdgcn_update_dpp(0, x.y, 0x130, 0xf, 0xf, true));
+    return own ? v : __builtin_bit_cast(double, r);
+}
+
+// Inverse / forward X lifting of a row, one pair per lane.
+template <class T>
+WZ_D void strip_x_inverse(T& e, T& o, bool first, bool last) {
+    using C = Lift<T>;
+    const T o0 = o * (-C::k), e0 = e * C::ik;
+    const T e1 = fmadd(-C::d, lane_prev(o0, first) + o0, e0);
+    const T o2 = fmadd(-C::g, e1 + lane_next(e1, last), o0);
+    e = fmadd(-C::b, lane_prev(o2, first) + o2, e1);
+    o = fmadd(-C::a, e + lane_next(e, last), o2);
+}
+template <class T>
+WZ_D void strip_x_forward(T& e, T& o, bool first, bool last) {
+    using C = Lift<T>;
+    const T o1 = fmadd(C::a, e + lane_next(e, last), o);
+    const T e2 = fmadd(C::b, lane_prev(o1, first) + o1, e);
+    const T o3 = fmadd(C::g, e2 + lane_next(e2, last), o1);
+    const T e4 = fmadd(C::d, lane_prev(o3, first) + o3, e2);
+    e = e4 * C::k;
+    o = o3 * (-C::ik);
+}
+
+// Two consecutive samples (dword-aligned).
+WZ_D void buf_load_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, float& a, float& b) {
+    using F2 = float __attribute__((ext_vector_type(2)));
+    const F2 v = __builtin_bit_cast(F2, __builtin_amdgcn_raw_buffer_load_b64(r, int(voff), int(soff), 0));
+    a = v.x;
+    b = v.y;
+}
+WZ_D void buf_load_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, double& a, double& b) {
+    using D2 = double __attribute__((ext_vector_type(2)));
+    const D2 v = __builtin_bit_cast(D2, __builtin_amdgcn_raw_buffer_load_b128(r, int(voff), int(soff), 0));
+    a = v.x;
+    b = v.y;
+}
+WZ_D void buf_store_pair(float a, float b, __amdgpu_buffer_rsrc_t r, uint32_t voff) {
+    using F2 = float __attribute__((ext_vector_type(2)));
+    using U2 = unsigned __attribute__((ext_vector_type(2)));
+    const F2 v = {a, b};
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), r, int(voff), 0, 0);
+}
+WZ_D void buf_store_pair(double a, double b, __amdgpu_buffer_rsrc_t r, uint32_t voff) {
+    using D2 = double __attribute__((ext_vector_type(2)));
+    using U4 = unsigned __attribute__((ext_vector_type(4)));
+    const D2 v = {a, b};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, v), r, int(voff), 0, 0);
+}
+
+// A wave's item: its strip, y segment and planes, and each lane's pair.
+struct StripItem {
+    uint32_t z0, zl;  // first plane, and the lane's plane less it (in range)
+    uint32_t ys, blocks;  // first row, blocks of 8 rows
+    uint32_t kp;      // the lane's pair in x
+    bool own;         // the lane's pair is the strip's to write
+    bool first, last; // line ends at this lane's group edges
+};
+WZ_D StripItem strip_item(const StripPlan& p, Dims n, uint32_t item) {
+    StripItem it;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t strip = item % p.strips, r = item / p.strips, seg = r % p.segs, zg = r / p.segs;
+    const uint32_t group = lane >> p.lw, w = 1u << p.lw, k = lane & (w - 1u), per = 64u >> p.lw;
+    it.z0 = zg * per;
+    const uint32_t z = it.z0 + group;
+    it.zl = min(z, n.nz - 1u) - it.z0;
+    it.ys = seg * p.sy;
+    it.blocks = (min(p.sy, n.ny - it.ys) + 7) / 8;
+    const uint32_t np = half_len(n.nx);
+    const uint32_t b0 = strip ? 62u + 60u * (strip - 1u) : 0u;
+    const uint32_t b1 = p.strips == 1 ? np : min(np, strip ? b0 + 60u : 62u);
+    it.kp = (strip ? b0 - 2u : 0u) + k;
+    it.own = z < n.nz && it.kp >= b0 && it.kp < b1;
+    it.first = k == 0;
+    it.last = k == w - 1u;
+    return it;
+}
+
+template <class T>
+struct XYInverse {
+    const T* hi;  // the level's coefficients outside its low box
+    uint64_t hpy, hpz;
+    const T* lo;  // its low box [0, ceil(nx/2)) x [0, ceil(ny/2)): the coarser reconstruction
+    uint64_t lpy, lpz;
+    T* out;  // the level's reconstruction (natural layout)
+    uint64_t opy, opz;
+    Dims n;  // level box: nx x ny, every plane
+    // q > 0: the coefficients hold unquantized values, quantized and
+    // dequantized as they load (the low box too when lo_coeff: the coarsest
+    // level, whose low box is the coefficient volume's)
+    T q, inv;
+    uint32_t lo_coeff;
+};
+
+// One item of an inverse level (nx, ny >= 2): the step of pair g loads pair
+// g + 2 and emits rows 2 (g - 2) and 2 (g - 2) + 1; the segment's first four
+// steps only warm the Y pipeline up. Four steps are one block (the fold phases
+// of the Y tile of 8 rows are then fixed).
+template <class T, bool Requant>
+WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item) {
+    using C = Lift<T>;
+    constexpr uint32_t S = sizeof(T);
+    const Dims n = a.n;
+    const StripItem it = strip_item(p, n, item);
+    const uint32_t hy = half_len(n.ny);
+    const int32_t ny = int32_t(n.ny);
+    const uint32_t ce = split_pos(int32_t(2 * it.kp), n.nx), co = split_pos(int32_t(2 * it.kp + 1), n.nx);
+    const auto wh = window(a.hi + uint64_t(it.z0) * a.hpz), wl = window(a.lo + uint64_t(it.z0) * a.lpz);
+    const uint32_t hrow = uint32_t(a.hpy) * S, lrow = uint32_t(a.lpy) * S, orow = uint32_t(a.opy) * S;
+    const uint32_t lv = (it.zl * uint32_t(a.lpz) + ce) * S, hv = it.zl * uint32_t(a.hpz) * S;
+    const uint32_t he = hv + ce * S, ho = hv + co * S;
+    // stores: lanes and rows outside go past the window's range (dropped)
+    const auto wo = window_n(a.out + uint64_t(it.z0) * a.opz,
+                             uint32_t((uint64_t(min(64u >> p.lw, n.nz - it.z0) - 1u) * a.opz +
+                                       uint64_t(n.ny - 1u) * a.opy + n.nx) * S));
+    const uint32_t ov = (it.zl * uint32_t(a.opz) + 2 * it.kp) * S;
+    const bool both = it.own && 2 * it.kp + 1 < n.nx, half = it.own && !both;
+    auto load = [&](int32_t g, T (&v)[4]) {  // pair g of rows: (low, high) of its even and of its odd row
+        const uint32_t se = uint32_t(pair_even(g, ny)), so = hy + uint32_t(pair_odd(g, ny));
+        v[0] = buf_load_at(T(0), wl, lv, se * lrow);
+        v[1] = buf_load_at(T(0), wh, ho, se * hrow);
+        v[2] = buf_load_at(T(0), wh, he, so * hrow);
+        v[3] = buf_load_at(T(0), wh, ho, so * hrow);
+    };
+    T OS[2], EA[2], OB[2], EC[2], SF[2];  // Y state, as the fused level's Z synthesis
+#pragma unroll
+    for (int c = 0; c < 2; ++c) OS[c] = EA[c] = OB[c] = EC[c] = SF[c] = T(0);
+    T buf[4][4];
+    int32_t g = int32_t(it.ys / 2) - 2;
+    load(g, buf[0]);
+    load(g + 1, buf[1]);
+    auto block = [&](auto emit_c) {
+        constexpr bool emit = decltype(emit_c)::value;
+#pragma unroll
+        for (int u = 0; u < 4; ++u, ++g) {
+            load(g + 2, buf[(u + 2) & 3]);
+            T(&v)[4] = buf[u];
+            if constexpr (Requant) {
+                if (a.lo_coeff) v[0] = requantize<T>(v[0], a.q, a.inv);
+#pragma unroll
+                for (int i = 1; i < 4; ++i) v[i] = requantize<T>(v[i], a.q, a.inv);
+            }
+            strip_x_inverse(v[0], v[1], it.first, it.last);
+            strip_x_inverse(v[2], v[3], it.first, it.last);
+            const int phase = (u + 2) & 3;
+            T re[2], ro[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const T oraw = v[2 + c];
+                const T es = v[c] * C::ik, os = oraw * (-C::k);
+                const T eA = fmadd(-C::d, OS[c] + os, es);
+                const T oB = fmadd(-C::g, EA[c] + eA, OS[c]);
+                const T eC = fmadd(-C::b, OB[c] + oB, EA[c]);
+                re[c] = EC[c];
+                ro[c] = fmadd(-C::a, EC[c] + eC, OB[c]);
+                if (phase == 3) {  // g = B - 1: fold of tile B's first pair
+                    SF[c] = fmadd(-C::d, fmadd(SF[c], -C::k, os), es);
+                } else if (phase == 0) {
+                    SF[c] = fmadd(-C::g, SF[c] + eA, OS[c]);
+                } else if (phase == 1) {  // and the tile before's last sample
+                    SF[c] = fmadd(-C::b, SF[c] + oB, EA[c]);
+                    const T eAe = fmadd(-C::d, fmadd(oraw, -C::k, OS[c]), es);
+                    const T oBe = fmadd(-C::g, EA[c] + eAe, OS[c]);
+                    const T eCe = fmadd(-C::b, OB[c] + oBe, EA[c]);
+                    ro[c] = fmadd(-C::a, EC[c] + eCe, OB[c]);
+                } else {  // g = B + 2: tile B's first two samples; o_raw[B' - 2] for the next fold
+                    re[c] = SF[c];
+                    ro[c] = fmadd(-C::a, SF[c] + eC, OB[c]);
+                    SF[c] = oraw;
+                }
+                OS[c] = os;
+                EA[c] = eA;
+                OB[c] = oB;
+                EC[c] = eC;
+            }
+            if constexpr (emit) {
+                const uint32_t y = 2 * uint32_t(g - 2);
+                buf_store_pair(re[0], re[1], wo, both && y < n.ny ? ov + y * orow : kOutside);
+                buf_store_pair(ro[0], ro[1], wo, both && y + 1 < n.ny ? ov + (y + 1) * orow : kOutside);
+                if (n.nx & 1u) {  // the last sample of an odd line
+                    buf_store(re[0], wo, half && y < n.ny ? ov + y * orow : kOutside);
+                    buf_store(ro[0], wo, half && y + 1 < n.ny ? ov + (y + 1) * orow : kOutside);
+                }
+            }
+        }
+    };
+    block(std::false_type{});
+    for (uint32_t b = 0; b < it.blocks; ++b) block(std::true_type{});
+}
+
+template <class T>
+struct XYForward {
+    const T* src;  // the level's input (natural layout)
+    uint64_t spy, spz;
+    T* hi;  // where the three high bands go
+    uint64_t hpy, hpz;
+    T* lo;  // where the low band [0, ceil(nx/2)) x [0, ceil(ny/2)) goes
+    uint64_t lpy, lpz;
+    Dims n;
+    uint32_t* status;  // non-null: screen the input for non-finite samples
+};
+
+// One item of a forward level (nx, ny >= 2): the step of row pair g loads pair
+// g + 2 and emits the low and high row g - 2 of the split.
+template <class T>
+WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item) {
+    using C = Lift<T>;
+    constexpr uint32_t S = sizeof(T);
+    const Dims n = a.n;
+    const StripItem it = strip_item(p, n, item);
+    const uint32_t hx = half_len(n.nx), hy = half_len(n.ny);
+    const int32_t ny = int32_t(n.ny);
+    // the pair's two samples are neighbours also where they are mirrored, then
+    // in the other order
+    const uint32_t xe = reflect_pos(int32_t(2 * it.kp), n.nx), xo = reflect_pos(int32_t(2 * it.kp + 1), n.nx);
+    const bool swap = xo < xe;
+    const auto ws = window(a.src + uint64_t(it.z0) * a.spz);
+    const uint32_t sv = (it.zl * uint32_t(a.spz) + min(xe, xo)) * S, srow = uint32_t(a.spy) * S;
+    const uint32_t planes = min(64u >> p.lw, n.nz - it.z0) - 1u;
+    const auto wl = window_n(a.lo + uint64_t(it.z0) * a.lpz,
+                             uint32_t((uint64_t(planes) * a.lpz + uint64_t(hy - 1u) * a.lpy + hx) * S));
+    const auto wh = window_n(a.hi + uint64_t(it.z0) * a.hpz,
+                             uint32_t((uint64_t(planes) * a.hpz + uint64_t(n.ny - 1u) * a.hpy + n.nx) * S));
+    const uint32_t hrow = uint32_t(a.hpy) * S, lrow = uint32_t(a.lpy) * S;
+    const uint32_t lv = (it.zl * uint32_t(a.lpz) + it.kp) * S, hv = (it.zl * uint32_t(a.hpz) + it.kp) * S;
+    const bool odd = it.own && 2 * it.kp + 1 < n.nx;
+    bool ok = true;
+    auto load = [&](int32_t g, T (&v)[4]) {  // pair g of rows, two samples of each
+        buf_load_pair(ws, sv, uint32_t(2 * pair_even(g, ny)) * srow, v[0], v[1]);
+        buf_load_pair(ws, sv, uint32_t(2 * pair_odd(g, ny) + 1) * srow, v[2], v[3]);
+    };
+    T E[2], O[2], O1[2], E2[2], O3[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) E[c] = O[c] = O1[c] = E2[c] = O3[c] = T(0);
+    T buf[4][4];
+    int32_t g = int32_t(it.ys / 2) - 2;
+    load(g, buf[0]);
+    load(g + 1, buf[1]);
+    auto block = [&](auto emit_c) {
+        constexpr bool emit = decltype(emit_c)::value;
+#pragma unroll
+        for (int u = 0; u < 4; ++u, ++g) {
+            load(g + 2, buf[(u + 2) & 3]);
+            const T(&v)[4] = buf[u];
+            if (a.status) {  // input screen (cpu/src/codec.cpp:183)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ok = ok && finite_value(v[i]);
+            }
+            T le[2], hi[2];  // the two columns of the low and of the high row
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const bool other = (c != 0) != swap;
+                const T ev = other ? v[1] : v[0], ov = other ? v[3] : v[2];
+                const T o1 = fmadd(C::a, E[c] + ev, O[c]);
+                const T e2 = fmadd(C::b, O1[c] + o1, E[c]);
+                const T o3 = fmadd(C::g, E2[c] + e2, O1[c]);
+                const T e4 = fmadd(C::d, O3[c] + o3, E2[c]);
+                le[c] = e4 * C::k;
+                hi[c] = o3 * (-C::ik);
+                E[c] = ev;
+                O[c] = ov;
+                O1[c] = o1;
+                E2[c] = e2;
+                O3[c] = o3;
+            }
+            if constexpr (emit) {
+                strip_x_forward(le[0], le[1], it.first, it.last);
+                strip_x_forward(hi[0], hi[1], it.first, it.last);
+                const uint32_t iy = uint32_t(g - 2);
+                const bool low = 2 * iy < n.ny, high = 2 * iy + 1 < n.ny;
+                const uint32_t at = hv + iy * hrow, up = hv + (hy + iy) * hrow;
+                buf_store(le[0], wl, it.own && low ? lv + iy * lrow : kOutside);
+                buf_store(le[1], wh, odd && low ? at + hx * S : kOutside);
+                buf_store(hi[0], wh, it.own && high ? up : kOutside);
+                buf_store(hi[1], wh, odd && high ? up + hx * S : kOutside);
+            }
+        }
+    };
+    block(std::false_type{});
+    for (uint32_t b = 0; b < it.blocks; ++b) block(std::true_type{});
+    if (a.status && __ballot(!ok) && (threadIdx.x & 63u) == 0) atomicOr(a.status, uint32_t(kNonFiniteInput));
+}
+
+}  // namespace wz
