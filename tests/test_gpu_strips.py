@@ -45,3 +45,24 @@ def test_line_counts(oracle, ny, dtype):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 def test_levels(oracle, shape, lxy, dtype):
     check(oracle, shape, lxy, dtype)
+
+
+# one batch whose jobs take every schedule: columns too tall for one pass, no Z
+# level, no XY level, several strips, dyadic boxes, odd extents
+BATCH = [(400, 9, 20), (180, 10, 33), (1, 40, 50), (40, 5, 30), (20, 20, 300), (33, 17, 65), (40, 48, 56), (9, 9, 9)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+def test_batch_schedules(oracle, dtype):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from waltz_amd import batch
+    fields = [field(s, "smooth", dtype, seed=k + 1) for k, s in enumerate(BATCH)]
+    dec = batch.BatchDecoder(BATCH, torch.float32 if dtype is np.float32 else torch.float64)
+    arcs, spans = dec.compress(dec.flatten([torch.from_numpy(f).cuda() for f in fields]), 1e-2)
+    tiles = dec.views(dec.decode(arcs, spans))
+    for k, (f, (at, size)) in enumerate(zip(fields, spans.view(-1, 2).tolist())):
+        want = oracle.compress(f, 1e-2)
+        assert arcs[at:at + size].cpu().numpy().tobytes() == want, BATCH[k]
+        got = tiles[k].cpu().numpy()
+        assert np.array_equal(got.view(np.uint8), oracle.decompress(want, f.shape, dtype).view(np.uint8)), BATCH[k]

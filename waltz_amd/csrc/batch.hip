@@ -40,9 +40,12 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "bricks.hpp"
+#include "fused.hpp"
 #include "lifting.hpp"
 #include "sections.hpp"
 #include "wzp_encode.hpp"
+#include "xystrip.hpp"
+#include "zcolumns.hpp"
 
 namespace wz {
 namespace {
@@ -79,10 +82,14 @@ struct JobRun {
 };
 
 struct Pass {
-    uint8_t kind, src, dst, pad;
+    uint8_t kind, src, dst, levels;  // levels: of a column pass
+    // volume of a strip pass: 0 the bank's at the job's pitches, l >= 1 the
+    // compact XY box of level l in the tmp0 bank
+    uint8_t src_box, low_box, dst_box, pad;
     Dims act;           // box of this pass
     uint32_t ntiles;    // tiles per line
-    uint32_t work;      // work items (threads)
+    uint32_t work;      // work items: threads, or workgroups of a strip / column pass
+    StripPlan strip;
 };
 
 struct Banks {
@@ -857,28 +864,14 @@ __global__ void __launch_bounds__(256) batch_place_kernel(const JobShape* __rest
     }
 }
 
-// ------------------------------------------------------------------ LDS-staged passes
-// Two pass kinds that stage a whole piece of the box in LDS and run several
-// lifting passes there, reading and writing the box once:
-//   kPassXYPlane  one workgroup per z plane of the box: the X and Y passes of
-//                 `levels` XY levels (Pass::pad) in canonical order (inverse:
-//                 coarse to fine, X then Y; forward: fine to coarse, Y then X);
-//   kPassZCol     one workgroup per row of 64 columns: the Z passes of
-//                 `levels` Z levels (the plane schedule's whole Z phase).
-// Tiles and arithmetic are those of the per-axis passes (lift_tile), so every
-// value is the same. In place is allowed (src may equal dst).
-enum : uint8_t { kPassXYPlane = 6, kPassZCol = 7 };
-constexpr uint32_t kColumns = 64;          // columns of a kPassZCol workgroup
-// Samples of the one LDS buffer a workgroup stages (odd plane pitches: rows
-// of up to 128 + 1 samples for the large variant).
-template <class T, bool Large>
-struct PlaneCap {
-    static constexpr uint32_t value = (Large ? 66560u : 16640u) / sizeof(T);
-};
-template <class T>
-constexpr uint32_t zcol_cap() { return PlaneCap<T, true>::value / kColumns; }  // z extent of a column row
+// Strip passes (one XY level of a job's box, xystrip.hpp) and column passes
+// (Z levels, zcolumns.hpp) over all jobs, each one launch per step. Bound by
+// memory; staging whole planes and columns in LDS was bound by vector issue:
+// 256 chunks (94 M float samples) decoded 1310 -> 862 us, 64 chunks compressed
+// 765 -> 550 us.
+enum : uint8_t { kPassStrip = 6, kPassZCol = 7 };
 
-// Banks of the LDS passes: input (compress forward), the three work banks, the
+// Banks of these passes: input (compress forward), the three work banks, the
 // output (decode) or reconstruction (compress inverse), and where failures go.
 struct StageBanks {
     const void* input;
@@ -888,107 +881,94 @@ struct StageBanks {
     void* out;
     EncodeResult* res;  // compress: per-job status; decode: null (status word)
 };
-
 template <class T>
-WZ_D T* stage_bank(const StageBanks& b, const JobShape& sh, uint8_t id) {
-    if (id == kInput) return const_cast<T*>(static_cast<const T*>(b.input)) + sh.out;
-    return static_cast<T*>(id == kHome ? b.home : id == kTmp0 ? b.tmp0 : b.tmp1) + sh.bank;
+struct Volume {
+    T* p;
+    uint64_t py, pz;
+};
+template <class T>
+WZ_D Volume<T> volume_of(const StageBanks& b, const JobShape& sh, uint8_t id, uint8_t box) {
+    if (box) {  // odd levels at offset 0, even ones after the level-1 box (the two never alias)
+        uint32_t nx = sh.d.nx, ny = sh.d.ny;
+        for (uint8_t l = 0; l < box; ++l) {
+            nx = half_len(nx);
+            ny = half_len(ny);
+        }
+        const uint64_t first = (box & 1u) ? 0u : uint64_t(half_len(sh.d.nx)) * half_len(sh.d.ny) * sh.d.nz;
+        return {static_cast<T*>(b.tmp0) + sh.bank + first, nx, uint64_t(nx) * ny};
+    }
+    const uint64_t py = sh.d.nx, pz = uint64_t(sh.d.nx) * sh.d.ny;
+    if (id == kInput) return {const_cast<T*>(static_cast<const T*>(b.input)) + sh.out, py, pz};
+    if (id == kOutput) return {static_cast<T*>(b.out) + sh.out, sh.opy, sh.opz};
+    return {static_cast<T*>(id == kHome ? b.home : id == kTmp0 ? b.tmp0 : b.tmp1) + sh.bank, py, pz};
 }
 
-template <class T, bool Large, bool Inverse>
-__global__ void __launch_bounds__(kLdsThreads) batch_lds_kernel(const JobShape* __restrict__ shape,
-                                                                const JobRun* __restrict__ run,
-                                                                const Pass* __restrict__ pass,
-                                                                const uint32_t* __restrict__ pfx, uint32_t jobs,
-                                                                StageBanks b, T fill, uint32_t* status) {
-    constexpr uint32_t Cap = PlaneCap<T, Large>::value;
-    constexpr int ZTile = Inverse ? (sizeof(T) == 4 ? 16 : 8) : 8;
-    __shared__ T A[Cap];
-    const uint32_t j = job_of_wave(pfx, jobs, blockIdx.x);
-    const Pass ps = pass[j];
-    if (ps.kind != kPassXYPlane && ps.kind != kPassZCol) return;
+// This workgroup's place in a grid of a multiple of eight workgroups over
+// `total` items: each XCD (workgroups are dealt to the eight in turn) takes a
+// contiguous range.
+WZ_D uint32_t xcd_place(uint32_t total) { return (blockIdx.x & 7u) * ((total + 7) / 8) + (blockIdx.x >> 3); }
+
+template <class T, bool Inverse>
+__global__ void __launch_bounds__(kStripThreads) batch_strip_kernel(const JobShape* __restrict__ shape,
+                                                                    const JobRun* __restrict__ run,
+                                                                    const Pass* __restrict__ pass,
+                                                                    const uint32_t* __restrict__ pfx, uint32_t jobs,
+                                                                    StageBanks b, T fill, uint32_t* status) {
+    const uint32_t id = xcd_place(pfx[jobs]);
+    if (id >= pfx[jobs]) return;
+    const uint32_t j = __builtin_amdgcn_readfirstlane(job_of_wave(pfx, jobs, id));
+    const Pass& ps = pass[j];
     const uint32_t state = run ? run[j].state : uint32_t(kJobOk);
     if (state == kJobBad || (state == kJobHole && ps.dst != kOutput)) return;
     const JobShape& sh = shape[j];
-    const uint32_t t = threadIdx.x, item = blockIdx.x - pfx[j];
-    const Dims full = sh.d, act = ps.act;
-    const uint64_t plane = uint64_t(full.nx) * full.ny;
-    const T* src = stage_bank<T>(b, sh, ps.src);
-    const bool screen = ps.src == kInput;
-    const bool xy = ps.kind == kPassXYPlane;
-    // the staged piece: plane z (rows of act.nx samples at an odd pitch), or
-    // columns x0.. of row y (rows of up to 64 z-ordered columns)
-    const uint32_t z = item, y = xy ? 0u : item % act.ny, x0 = xy ? 0u : (item / act.ny) * kColumns;
-    const uint32_t cols = xy ? act.nx : min(kColumns, act.nx - x0);
-    const uint32_t rows = xy ? act.ny : act.nz;
-    const uint32_t pitch = xy ? (act.nx | 1u) : kColumns;
-    const uint32_t cells = cols * rows;
-    const FastDiv by_cols(cols);  // cells fit LDS: exact
-    auto gat = [&](uint32_t c, uint32_t r) -> uint64_t {  // global index of staged cell (c, r)
-        return xy ? uint64_t(z) * plane + uint64_t(r) * full.nx + c
-                  : uint64_t(r) * plane + uint64_t(y) * full.nx + x0 + c;
-    };
-    // staging: every thread issues kBurst loads before it writes any of them to LDS
-    constexpr uint32_t kBurst = 8;
-    bool ok = true;
-    for (uint32_t i0 = 0; i0 < cells; i0 += kBurst * kLdsThreads) {
-        T v[kBurst];
-#pragma unroll
-        for (uint32_t k = 0; k < kBurst; ++k) {
-            const uint32_t i = i0 + k * kLdsThreads + t;
-            const uint32_t r = by_cols.div(i);
-            v[k] = i < cells ? src[gat(i - r * cols, r)] : T(0);
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kBurst; ++k) {
-            const uint32_t i = i0 + k * kLdsThreads + t;
-            if (i < cells) {
-                ok = ok && (!screen || __builtin_isfinite(v[k]));
-                const uint32_t r = by_cols.div(i);
-                A[r * pitch + (i - r * cols)] = v[k];
-            }
-        }
-    }
-    __syncthreads();
-    const uint32_t levels = ps.pad;
-    uint32_t ex[5], ey[5];  // extents of each level inside the piece
-    ex[0] = xy ? act.nx : act.nz;
-    ey[0] = act.ny;
-    for (uint32_t l = 1; l < 5; ++l) {
-        ex[l] = half_len(ex[l - 1]);
-        ey[l] = half_len(ey[l - 1]);
-    }
-    for (uint32_t k = 0; k < levels; ++k) {
-        const uint32_t l = Inverse ? levels - 1 - k : k;
-        if (xy) {
-            if constexpr (Inverse) {
-                lds_pass<T, true, 0, 8>(A, pitch, ex[l], ey[l]);  // X (unfolded), rows of the level box
-                lds_pass<T, true, 1, 8>(A, pitch, ey[l], ex[l]);  // Y (folded), its columns
-            } else {
-                lds_pass<T, false, 1, 8>(A, pitch, ey[l], ex[l]);  // Y
-                lds_pass<T, false, 0, 8>(A, pitch, ex[l], ey[l]);  // X
-            }
-        } else {
-            lds_pass<T, Inverse, 2, ZTile>(A, pitch, ex[l], cols);  // Z (folded) of every column
-        }
-    }
-    bool fin = true;
-    if (ps.dst == kOutput) {
-        const Put<T> put{nullptr, static_cast<T*>(b.out), &sh, state == kJobHole, fill};
-        for (uint32_t i = t; i < cells; i += kLdsThreads) {
-            const uint32_t r = by_cols.div(i), c = i - r * cols;
-            const uint32_t X = xy ? c : x0 + c, Y = xy ? r : y, Zc = xy ? z : r;
-            fin = put(gat(c, r), X, Y, Zc, A[r * pitch + c]) && fin;
-        }
-        if (__ballot(!fin) && (t & 63u) == 0 && status) atomicOr(status, uint32_t(kNonFiniteOutput));
+    const uint32_t item = 4 * (id - pfx[j]) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const StripPlan plan = ps.strip;
+    if (item >= plan.items()) return;
+    const Volume<T> src = volume_of<T>(b, sh, ps.src, ps.src_box), dst = volume_of<T>(b, sh, ps.dst, ps.dst_box);
+    const Volume<T> low = ps.low_box ? volume_of<T>(b, sh, kTmp0, ps.low_box) : Inverse ? src : dst;
+    if constexpr (Inverse) {
+        const bool last = ps.dst == kOutput;
+        StripOutput<T> out{last ? sh.clip : ps.act, state == kJobHole, fill};
+        strip_inverse<T, false>(XYInverse<T>{src.p, src.py, src.pz, low.p, low.py, low.pz, dst.p, dst.py, dst.pz,
+                                             ps.act, T(0), T(0), 0u},
+                                plan, item, out);
+        if (last && __ballot(!out.finite) && (threadIdx.x & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteOutput));
     } else {
-        T* dst = stage_bank<T>(b, sh, ps.dst);
-        for (uint32_t i = t; i < cells; i += kLdsThreads) {
-            const uint32_t r = by_cols.div(i), c = i - r * cols;
-            dst[gat(c, r)] = A[r * pitch + c];
-        }
+        strip_forward<T>(XYForward<T>{src.p, src.py, src.pz, dst.p, dst.py, dst.pz, low.p, low.py, low.pz, ps.act,
+                                      ps.src == kInput ? &b.res[j].status : nullptr},
+                         plan, item);
     }
-    if (screen && __ballot(!ok) && (t & 63u) == 0 && b.res) atomicOr(&b.res[j].status, uint32_t(kNonFiniteInput));
+}
+
+template <class T, bool Inverse>
+__global__ void __launch_bounds__(kZThreads) batch_zcol_kernel(const JobShape* __restrict__ shape,
+                                                               const JobRun* __restrict__ run,
+                                                               const Pass* __restrict__ pass,
+                                                               const uint32_t* __restrict__ pfx, uint32_t jobs,
+                                                               StageBanks b, T fill, uint32_t* status) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t zlds[];
+    const uint32_t id = xcd_place(pfx[jobs]);
+    if (id >= pfx[jobs]) return;
+    const uint32_t j = __builtin_amdgcn_readfirstlane(job_of_wave(pfx, jobs, id));
+    const Pass& ps = pass[j];
+    const uint32_t state = run ? run[j].state : uint32_t(kJobOk);
+    if (state == kJobBad || (state == kJobHole && ps.dst != kOutput)) return;
+    const JobShape& sh = shape[j];
+    const Dims act = ps.act;
+    const Volume<T> src = volume_of<T>(b, sh, ps.src, 0), dst = volume_of<T>(b, sh, ps.dst, 0);
+    T* const box0 = reinterpret_cast<T*>(zlds);
+    T* const box1 = box0 + uint64_t(half_len(act.nz)) * kZColumns;
+    const uint32_t xb = (act.nx + kZColumns - 1) / kZColumns, item = id - pfx[j], y = item / xb;
+    const bool last = ps.dst == kOutput, screen = Inverse ? last : ps.src == kInput;
+    const bool fin = zcol_columns<T, Inverse, false>(
+        ZColumnsOf<T>{src.p, uint32_t(src.py), uint32_t(src.pz), dst.p, uint32_t(dst.py), uint32_t(dst.pz), act,
+                      ps.levels},
+        y, (item - y * xb) * kZColumns, box0, box1, screen,
+        ZOutput<T>{last ? sh.clip : act, screen, state == kJobHole, fill}, ZRepair<T>{}, 0u, nullptr);
+    if (screen && __ballot(!fin) && (threadIdx.x & 63u) == 0) {
+        if constexpr (Inverse) atomicOr(status, uint32_t(kNonFiniteOutput));
+        else atomicOr(&b.res[j].status, uint32_t(kNonFiniteInput));
+    }
 }
 
 // ------------------------------------------------------------------ host plan
@@ -1020,199 +1000,220 @@ Pass make_pass(uint8_t kind, uint8_t src, uint8_t dst, Dims act, unsigned width)
     return p;
 }
 
-// Whether a box's XY planes / Z columns fit the LDS-staged passes.
-bool plane_fits(Dims act, unsigned width) {
-    // rows at an odd pitch; every tile column of a line fits one lds_pass group
-    const uint64_t cap = width == 4 ? PlaneCap<float, true>::value : PlaneCap<double, true>::value;
-    const uint64_t k = width == 4 ? 4 : 2;
-    return uint64_t(act.nx | 1u) * act.ny <= cap && (act.nx + 7) / 8 <= k * kLdsThreads &&
-           (act.ny + 7) / 8 <= k * kLdsThreads;
-}
-bool zcol_fits(Dims act, unsigned width) { return act.nz <= (width == 4 ? zcol_cap<float>() : zcol_cap<double>()); }
-
-Pass lds_pass(uint8_t kind, uint8_t src, uint8_t dst, Dims act, uint32_t levels) {
+// Strip pass over box `act` of a job. `jobs`: of the plan (a batch's waves fill
+// the device together, so each job's strips may be long).
+Pass strip_pass(const JobShape& sh, uint8_t src, uint8_t src_box, uint8_t low_box, uint8_t dst, uint8_t dst_box,
+                Dims act, unsigned width, uint32_t jobs) {
     Pass p{};
-    p.kind = kind;
+    p.kind = kPassStrip;
     p.src = src;
     p.dst = dst;
-    p.pad = uint8_t(levels);
+    p.src_box = src_box;
+    p.low_box = low_box;
+    p.dst_box = dst_box;
     p.act = act;
     p.ntiles = 1;
-    p.work = kind == kPassXYPlane ? act.nz : act.ny * ((act.nx + kColumns - 1) / kColumns);  // workgroups
+    const uint64_t plane = uint64_t(sh.d.nx) * sh.d.ny;
+    p.strip = strip_plan(act, fused_plane_fits(8 * (dst == kOutput ? std::max(plane, sh.opz) : plane), 1, width),
+                         std::max(64u, 4096u / jobs));
+    p.work = uint32_t((p.strip.items() + 3) / 4);
+    return p;
+}
+Pass column_pass(uint8_t src, uint8_t dst, Dims act, unsigned levels) {
+    Pass p{};
+    p.kind = kPassZCol;
+    p.src = src;
+    p.dst = dst;
+    p.levels = uint8_t(levels);
+    p.act = act;
+    p.ntiles = 1;
+    p.work = act.ny * ((act.nx + kZColumns - 1) / kZColumns);
     return p;
 }
 
-// The inverse schedule of transform_inverse (cpu/src/transform.cpp:409-447):
-// every level ends in the home bank, the very last pass writes the output.
-// A dyadic level is its Z pass and one XY-plane pass (X then Y) when the
-// level's planes fit LDS; the plane schedule is one XY-plane pass for all XY
-// levels and one Z-column pass for all Z levels when they fit. Otherwise per
-// axis passes through the scratch banks (copied back to home).
-std::vector<Pass> inverse_schedule(const JobShape& sh, unsigned width) {
+// Whether a tile's planes fit the 32-bit windows of the strip and column
+// passes (else per-axis passes), and whether their last pass may write the
+// output frame itself (else into the home bank, copied from there).
+bool windows_fit(const JobShape& sh, unsigned width) { return fused_plane_fits(sh.d.nx, sh.d.ny, width); }
+bool strip_output_fits(const JobShape& sh, unsigned width) { return fused_plane_fits(sh.opz, 1, width); }
+bool column_output_fits(const JobShape& sh, unsigned width) { return fused_plane_fits(16 * sh.opz, 1, width); }
+
+// The extents of every lifted box, finest first.
+std::vector<Dims> boxes_of(Dims d, unsigned levels, bool xy, bool z) {
+    std::vector<Dims> v;
+    for (unsigned l = 0; l < levels; ++l) {
+        v.push_back(d);
+        d = halve(d, xy, z);
+    }
+    return v;
+}
+
+// One level as per-axis passes through the scratch banks, from `src` (home or
+// the input) into `fin` (home or the output; copied there when needed).
+void axis_level(std::vector<Pass>& out, Dims act, std::initializer_list<uint8_t> axes, uint8_t src, uint8_t fin,
+                unsigned width) {
+    size_t a = 0;
+    for (uint8_t k : axes) {
+        uint8_t dst = ++a == axes.size() ? fin : src == kTmp0 ? uint8_t(kTmp1) : uint8_t(kTmp0);
+        if (dst == src) dst = kTmp0;
+        out.push_back(make_pass(k, src, dst, act, width));
+        src = dst;
+    }
+    if (src != fin) out.push_back(make_pass(kPassCopy, src, fin, act, width));
+}
+
+// The inverse schedule of transform_inverse (cpu/src/transform.cpp:409-447),
+// the very last pass writing the output. A dyadic level is a column pass (its
+// Z) into scratch and a strip pass (X then Y) back into the home bank. The
+// plane schedule is a strip pass per XY level, through compact boxes, and one
+// column pass for all Z levels when they fit its LDS, else one per level.
+std::vector<Pass> inverse_schedule(const JobShape& sh, unsigned width, uint32_t jobs) {
     std::vector<Pass> out;
     if (sh.lx == 0 && sh.lz == 0) {
         out.push_back(make_pass(kPassCopy, kHome, kOutput, sh.d, width));
         return out;
     }
-    struct Op {
-        uint8_t kind;
-        Dims act;
-        uint32_t levels;
-    };
-    std::vector<std::vector<Op>> levels;  // ops of each level (one level ends in home)
-    auto axes = [&](Dims act, std::initializer_list<uint8_t> ks) {
-        std::vector<Op> v;
-        for (uint8_t k : ks) v.push_back({k, act, 1});
-        return v;
-    };
+    const bool win = windows_fit(sh, width);
     if (sh.dyadic) {
-        Dims sizes[5], act = sh.d;
-        for (unsigned l = 0; l < sh.lx; ++l) {
-            sizes[l] = act;
-            act = halve(act, true, true);
-        }
+        const std::vector<Dims> box = boxes_of(sh.d, sh.lx, true, true);
         for (int l = int(sh.lx) - 1; l >= 0; --l) {
-            if (plane_fits(sizes[l], width)) levels.push_back({{kPassZ, sizes[l], 1}, {kPassXYPlane, sizes[l], 1}});
-            else levels.push_back(axes(sizes[l], {kPassZ, kPassX, kPassY}));
+            const uint8_t fin = l ? uint8_t(kHome) : uint8_t(kOutput);
+            if (!win) {
+                axis_level(out, box[l], {kPassZ, kPassX, kPassY}, kHome, fin, width);
+                continue;
+            }
+            const bool direct = l || strip_output_fits(sh, width);
+            out.push_back(column_pass(kHome, kTmp0, box[l], 1));
+            out.push_back(strip_pass(sh, kTmp0, 0, 0, direct ? fin : uint8_t(kHome), 0, box[l], width, jobs));
+            if (!direct) out.push_back(make_pass(kPassCopy, kHome, kOutput, sh.d, width));
         }
+        return out;
+    }
+    const std::vector<Dims> xy = boxes_of(sh.d, sh.lx, true, false), zs = boxes_of(sh.d, sh.lz, false, true);
+    if (!win) {
+        for (int l = int(sh.lx) - 1; l >= 0; --l)
+            axis_level(out, xy[l], {kPassX, kPassY}, kHome, sh.lz || l ? uint8_t(kHome) : uint8_t(kOutput), width);
+        for (int l = int(sh.lz) - 1; l >= 0; --l)
+            axis_level(out, zs[l], {kPassZ}, kHome, l ? uint8_t(kHome) : uint8_t(kOutput), width);
+        return out;
+    }
+    uint8_t at = kHome;  // where the whole volume is
+    for (int l = int(sh.lx) - 1; l >= 0; --l) {
+        const uint8_t low = l + 1 == int(sh.lx) ? 0 : uint8_t(l + 1);
+        if (l) {
+            out.push_back(strip_pass(sh, kHome, 0, low, kTmp0, uint8_t(l), xy[l], width, jobs));
+        } else {
+            at = !sh.lz && strip_output_fits(sh, width) ? uint8_t(kOutput) : uint8_t(kTmp1);
+            out.push_back(strip_pass(sh, kHome, 0, low, at, 0, xy[0], width, jobs));
+        }
+    }
+    if (sh.lz && zcol_fits(sh.d.nz, width)) {
+        const uint8_t dst = column_output_fits(sh, width) ? uint8_t(kOutput) : at == kHome ? uint8_t(kTmp1) : uint8_t(kHome);
+        out.push_back(column_pass(at, dst, sh.d, sh.lz));
+        at = dst;
     } else {
-        Dims xy[5], zs[5], act = sh.d;
-        for (unsigned l = 0; l < sh.lx; ++l) {
-            xy[l] = act;
-            act = halve(act, true, false);
+        for (int l = int(sh.lz) - 1; l >= 0; --l) {
+            out.push_back(column_pass(at, kTmp0, zs[l], 1));
+            out.push_back(make_pass(kPassCopy, kTmp0, l ? at : uint8_t(kOutput), zs[l], width));
         }
-        act = sh.d;
-        for (unsigned l = 0; l < sh.lz; ++l) {
-            zs[l] = act;
-            act = halve(act, false, true);
-        }
-        if (sh.lx && plane_fits(sh.d, width)) levels.push_back({{kPassXYPlane, sh.d, sh.lx}});
-        else
-            for (int l = int(sh.lx) - 1; l >= 0; --l) levels.push_back(axes(xy[l], {kPassX, kPassY}));
-        if (sh.lz && zcol_fits(sh.d, width)) levels.push_back({{kPassZCol, sh.d, sh.lz}});
-        else
-            for (int l = int(sh.lz) - 1; l >= 0; --l) levels.push_back(axes(zs[l], {kPassZ}));
+        if (sh.lz) at = kOutput;
     }
-    for (size_t k = 0; k < levels.size(); ++k) {
-        const bool last = k + 1 == levels.size();
-        const uint8_t fin = last ? uint8_t(kOutput) : uint8_t(kHome);
-        uint8_t src = kHome;
-        const std::vector<Op>& L = levels[k];
-        for (size_t a = 0; a < L.size(); ++a) {
-            const Op& op = L[a];
-            const bool lds = op.kind == kPassXYPlane || op.kind == kPassZCol;
-            uint8_t dst;
-            if (a + 1 == L.size()) dst = fin;
-            else dst = src == kTmp0 ? uint8_t(kTmp1) : uint8_t(kTmp0);
-            if (dst == src && !lds) dst = src == kTmp0 ? uint8_t(kTmp1) : uint8_t(kTmp0);
-            out.push_back(lds ? lds_pass(op.kind, src, dst, op.act, op.levels) : make_pass(op.kind, src, dst, op.act, width));
-            src = dst;
-        }
-        if (src != fin) out.push_back(make_pass(kPassCopy, src, fin, L.back().act, width));
-    }
+    if (at != kOutput) out.push_back(make_pass(kPassCopy, at, kOutput, sh.d, width));
     return out;
 }
 
 // The forward schedule of transform_forward (cpu/src/transform.cpp:425-456):
-// the first pass reads the job's input, every level ends in the home bank.
-// A dyadic level is one XY-plane pass (Y then X) and its Z pass; the plane
-// schedule is one Z-column pass and one XY-plane pass, when they fit LDS.
-// Forward tiles do not change a bit.
-std::vector<Pass> forward_schedule(const JobShape& sh, unsigned width) {
+// the first pass reads the job's input, the coefficients end in the home bank.
+// Mirrors inverse_schedule; forward tiles do not change a bit.
+std::vector<Pass> forward_schedule(const JobShape& sh, unsigned width, uint32_t jobs) {
     std::vector<Pass> out;
     if (sh.lx == 0 && sh.lz == 0) {
         out.push_back(make_pass(kPassCopy, kInput, kHome, sh.d, width));
         return out;
     }
-    struct Op {
-        uint8_t kind;
-        Dims act;
-        uint32_t levels;
-    };
-    std::vector<std::vector<Op>> levels;
-    if (sh.dyadic) {
-        Dims act = sh.d;
-        for (unsigned l = 0; l < sh.lx; ++l) {
-            if (plane_fits(act, width)) levels.push_back({{kPassXYPlane, act, 1}, {kPassZ, act, 1}});
-            else levels.push_back({{kPassY, act, 1}, {kPassX, act, 1}, {kPassZ, act, 1}});
-            act = halve(act, true, true);
-        }
-    } else {
-        if (sh.lz && zcol_fits(sh.d, width)) {
-            levels.push_back({{kPassZCol, sh.d, sh.lz}});
-        } else {
-            Dims act = sh.d;
-            for (unsigned l = 0; l < sh.lz; ++l) {
-                levels.push_back({{kPassZ, act, 1}});
-                act = halve(act, false, true);
-            }
-        }
-        if (sh.lx && plane_fits(sh.d, width)) {
-            levels.push_back({{kPassXYPlane, sh.d, sh.lx}});
-        } else {
-            Dims act = sh.d;
-            for (unsigned l = 0; l < sh.lx; ++l) {
-                levels.push_back({{kPassY, act, 1}, {kPassX, act, 1}});
-                act = halve(act, true, false);
-            }
-        }
-    }
+    const bool win = windows_fit(sh, width);
     uint8_t src = kInput;
-    for (const std::vector<Op>& L : levels) {
-        for (size_t a = 0; a < L.size(); ++a) {
-            const Op& op = L[a];
-            const bool lds = op.kind == kPassXYPlane || op.kind == kPassZCol;
-            uint8_t dst;
-            if (a + 1 == L.size()) dst = kHome;
-            else dst = src == kTmp0 ? uint8_t(kTmp1) : uint8_t(kTmp0);
-            if (dst == src && !lds) dst = src == kTmp0 ? uint8_t(kTmp1) : uint8_t(kTmp0);
-            out.push_back(lds ? lds_pass(op.kind, src, dst, op.act, op.levels) : make_pass(op.kind, src, dst, op.act, width));
-            src = dst;
-        }
-        if (src != kHome) {
-            out.push_back(make_pass(kPassCopy, src, kHome, L.back().act, width));
+    if (sh.dyadic) {
+        for (const Dims& act : boxes_of(sh.d, sh.lx, true, true)) {
+            if (!win) {
+                axis_level(out, act, {kPassY, kPassX, kPassZ}, src, kHome, width);
+            } else {
+                out.push_back(strip_pass(sh, src, 0, 0, kTmp0, 0, act, width, jobs));
+                out.push_back(column_pass(kTmp0, kHome, act, 1));
+            }
             src = kHome;
         }
+        return out;
     }
+    const std::vector<Dims> xy = boxes_of(sh.d, sh.lx, true, false), zs = boxes_of(sh.d, sh.lz, false, true);
+    if (!win) {
+        for (const Dims& act : zs) {
+            axis_level(out, act, {kPassZ}, src, kHome, width);
+            src = kHome;
+        }
+        for (const Dims& act : xy) {
+            axis_level(out, act, {kPassY, kPassX}, src, kHome, width);
+            src = kHome;
+        }
+        return out;
+    }
+    const uint8_t zdst = sh.lx ? uint8_t(kTmp1) : uint8_t(kHome);
+    if (sh.lz && zcol_fits(sh.d.nz, width)) {
+        out.push_back(column_pass(src, zdst, sh.d, sh.lz));
+        src = zdst;
+    } else {
+        for (unsigned l = 0; l < sh.lz; ++l) {
+            out.push_back(column_pass(src, l ? uint8_t(kTmp0) : zdst, zs[l], 1));
+            if (l) out.push_back(make_pass(kPassCopy, kTmp0, zdst, zs[l], width));
+            src = zdst;
+        }
+    }
+    for (unsigned l = 0; l < sh.lx; ++l)
+        out.push_back(strip_pass(sh, l ? uint8_t(kTmp0) : src, uint8_t(l), l + 1 == sh.lx ? 0 : uint8_t(l + 1), kHome, 0,
+                                 xy[l], width, jobs));
     return out;
 }
 
-// Per-step launch tables: every job's pass at step st, the block prefixes of
-// the per-axis kernel (256-thread blocks of work items) and of the LDS kernel
-// (one workgroup per plane / column row), and whether that step's LDS pieces
-// need the large LDS variant.
-void build_steps(const std::vector<std::vector<Pass>>& sched, uint32_t J, unsigned width,
-                 std::vector<std::vector<Pass>>& step, std::vector<std::vector<uint32_t>>& pfx,
-                 std::vector<std::vector<uint32_t>>& lpfx, std::vector<uint8_t>& large) {
+// One step's launches: every job's pass at that step, and the block prefixes
+// of the per-axis kernel (256-thread blocks of work items), the strip kernel
+// and the column kernel (with its LDS).
+struct StepTables {
+    std::vector<std::vector<Pass>> pass;                  // [step][job]
+    std::vector<std::vector<uint32_t>> pfx, spfx, zpfx;   // [step][job + 1]
+    std::vector<uint32_t> zlds;                           // [step]
+};
+StepTables build_steps(const std::vector<std::vector<Pass>>& sched, uint32_t J, unsigned width) {
     size_t steps = 0;
     for (const auto& v : sched) steps = std::max(steps, v.size());
-    step.assign(steps, std::vector<Pass>(J));
-    pfx.assign(steps, std::vector<uint32_t>(J + 1, 0));
-    lpfx.assign(steps, std::vector<uint32_t>(J + 1, 0));
-    large.assign(steps, 0);
-    const uint64_t small = width == 4 ? PlaneCap<float, false>::value : PlaneCap<double, false>::value;
+    StepTables t;
+    t.pass.assign(steps, std::vector<Pass>(J));
+    for (auto* p : {&t.pfx, &t.spfx, &t.zpfx}) p->assign(steps, std::vector<uint32_t>(J + 1, 0));
+    t.zlds.assign(steps, 0);
     for (size_t st = 0; st < steps; ++st) {
-        uint64_t blocks = 0, lblocks = 0;
+        uint64_t blocks = 0, sblocks = 0, zblocks = 0;
         for (uint32_t j = 0; j < J; ++j) {
             Pass ps{};
             ps.kind = kPassNone;
             if (st < sched[j].size()) ps = sched[j][st];
-            step[st][j] = ps;
-            pfx[st][j] = uint32_t(blocks);
-            lpfx[st][j] = uint32_t(lblocks);
-            if (ps.kind == kPassXYPlane || ps.kind == kPassZCol) {
-                lblocks += ps.work;
-                const uint64_t piece = ps.kind == kPassXYPlane ? uint64_t(ps.act.nx | 1u) * ps.act.ny
-                                                               : uint64_t(ps.act.nz) * kColumns;
-                if (piece > small) large[st] = 1;
+            t.pass[st][j] = ps;
+            t.pfx[st][j] = uint32_t(blocks);
+            t.spfx[st][j] = uint32_t(sblocks);
+            t.zpfx[st][j] = uint32_t(zblocks);
+            if (ps.kind == kPassStrip) {
+                sblocks += ps.work;
+            } else if (ps.kind == kPassZCol) {
+                zblocks += ps.work;
+                t.zlds[st] = std::max(t.zlds[st], uint32_t(zcol_lds_bytes(ps.act.nz, ps.levels, width)));
             } else if (ps.kind != kPassNone) {
                 blocks += (uint64_t(ps.work) + 255) / 256;
             }
         }
-        if (blocks > 0x7FFFFFFFull || lblocks > 0x7FFFFFFFull) throw std::invalid_argument("batch launch limit");
-        pfx[st][J] = uint32_t(blocks);
-        lpfx[st][J] = uint32_t(lblocks);
+        if (std::max({blocks, sblocks, zblocks}) > 0x7FFFFFF0ull) throw std::invalid_argument("batch launch limit");
+        t.pfx[st][J] = uint32_t(blocks);
+        t.spfx[st][J] = uint32_t(sblocks);
+        t.zpfx[st][J] = uint32_t(zblocks);
     }
+    return t;
 }
 
 // Byte offsets of one batched compress call's workspace (all 256-byte aligned).
@@ -1228,15 +1229,10 @@ struct HostPlan {
     std::vector<uint32_t> chunk_pfx, brick_pfx;
     // chunks of the brick-pair jobs and of the others (WZP coder launches)
     std::vector<uint32_t> pair_pfx, rank_pfx, mag_pfx;
-    std::vector<std::vector<Pass>> step;      // step[s][job]
-    std::vector<std::vector<uint32_t>> pfx;   // block prefixes per step (per-axis kernel)
-    std::vector<std::vector<uint32_t>> lpfx;  // block prefixes per step (LDS kernel)
-    std::vector<uint8_t> large;               // step needs the large LDS variant
+    StepTables inv;                           // inverse passes
     uint64_t bank_elems = 0, mag_elems = 0, sign_words = 0, out_elems = 0;
     // compress
-    std::vector<std::vector<Pass>> fstep;     // forward passes, fstep[s][job]
-    std::vector<std::vector<uint32_t>> fpfx, flpfx;
-    std::vector<uint8_t> flarge;
+    StepTables fwd;                           // forward passes
     std::vector<JobComp> comp;
     std::vector<uint32_t> group_pfx, tile_pfx, pblock_pfx, place_pfx;
     uint64_t archive_bytes = 0;               // archive slots of all jobs
@@ -1272,7 +1268,6 @@ void finish_compress_plan(HostPlan& p) {
     const uint32_t J = p.jobs;
     const unsigned w = p.width;
     std::vector<std::vector<Pass>> sched(J);
-    size_t steps = 0;
     p.comp.assign(J, JobComp{});
     p.group_pfx.assign(J + 1, 0);
     p.tile_pfx.assign(J + 1, 0);
@@ -1310,8 +1305,7 @@ void finish_compress_plan(HostPlan& p) {
         tiles += c.tiles;
         pblocks += c.pblocks;
         places += uint64_t(c.tiles) + c.qblocks;
-        sched[j] = forward_schedule(s, w);
-        steps = std::max(steps, sched[j].size());
+        sched[j] = forward_schedule(s, w, J);
     }
     if (groups > 0x7FFFFFFFull || tiles > 0x7FFFFFFFull || 2 * pblocks > 0x7FFFFFFFull || places > 0x7FFFFFFFull)
         throw std::invalid_argument("batch launch limit");
@@ -1320,8 +1314,7 @@ void finish_compress_plan(HostPlan& p) {
     p.pblock_pfx[J] = uint32_t(pblocks);
     p.place_pfx[J] = uint32_t(places);
     p.archive_bytes = arc;
-    (void)steps;
-    build_steps(sched, J, w, p.fstep, p.fpfx, p.flpfx, p.flarge);
+    p.fwd = build_steps(sched, J, w);
     CompressLayout& L = p.cl;
     uint64_t at = 0;
     auto take = [&](uint64_t bytes) {
@@ -1363,7 +1356,6 @@ void finish_plan(HostPlan& p) {
     p.rank_pfx.assign(J + 1, 0);
     p.mag_pfx.assign(J + 1, 0);
     std::vector<std::vector<Pass>> sched(J);
-    size_t steps = 0;
     uint64_t bank = 0, mag = 0, sign = 0, chunks = 0, bricks = 0, pchunks = 0, rchunks = 0, mchunks = 0;
     p.rank_geo.clear();
     for (uint32_t j = 0; j < J; ++j) {
@@ -1400,8 +1392,7 @@ void finish_plan(HostPlan& p) {
             mchunks += s.chunks;
             bricks += (uint64_t(s.nbx) * s.nby * s.nbz + kBricksPerBlock - 1) / kBricksPerBlock;  // brick blocks
         }
-        sched[j] = inverse_schedule(s, p.width);
-        steps = std::max(steps, sched[j].size());
+        sched[j] = inverse_schedule(s, p.width, J);
     }
     if (chunks > 0x7FFFFFFFull || bricks > 0x7FFFFFFFull) throw std::invalid_argument("batch launch limit");
     p.chunk_pfx[J] = uint32_t(chunks);
@@ -1412,8 +1403,7 @@ void finish_plan(HostPlan& p) {
     p.bank_elems = bank;
     p.mag_elems = mag;
     p.sign_words = sign;
-    (void)steps;
-    build_steps(sched, J, p.width, p.step, p.pfx, p.lpfx, p.large);
+    p.inv = build_steps(sched, J, p.width);
     finish_compress_plan(p);
 }
 
@@ -1425,16 +1415,14 @@ struct DevicePlan {
     JobRun* run = nullptr;
     uint32_t *chunk_pfx = nullptr, *brick_pfx = nullptr, *np_pfx = nullptr, *nq_pfx = nullptr, *status = nullptr;
     uint32_t *pair_pfx = nullptr, *rank_pfx = nullptr, *mag_pfx = nullptr;
-    Pass* pass = nullptr;        // steps x jobs
-    uint32_t* pass_pfx = nullptr;  // steps x (jobs + 1)
+    struct DeviceSteps {
+        Pass* pass;                     // steps x jobs
+        uint32_t *pfx, *spfx, *zpfx;    // steps x (jobs + 1)
+    } inv{}, fwd{};
     uint32_t* host_status = nullptr;  // pinned
     // compress tables
     JobComp* comp = nullptr;
     uint32_t *group_pfx = nullptr, *tile_pfx = nullptr, *pblock_pfx = nullptr, *place_pfx = nullptr;
-    Pass* fpass = nullptr;          // forward steps x jobs
-    uint32_t* fpass_pfx = nullptr;  // forward steps x (jobs + 1)
-    uint32_t* lds_pfx = nullptr;    // inverse steps x (jobs + 1), LDS kernel
-    uint32_t* flds_pfx = nullptr;   // forward steps x (jobs + 1), LDS kernel
     EncodeResult* last_res = nullptr;  // results of the last compress (device, in its workspace)
     uint16_t* ranks = nullptr;         // kRankSet entries per distinct geometry
     // compress: the WZP group pass runs on `side` (default priority) beside
@@ -1456,7 +1444,6 @@ struct DevicePlan {
     void upload(hipStream_t s) {
         const HostPlan& p = host;
         const uint32_t J = p.jobs;
-        const size_t S = p.step.size();
         size_t used = 0;
         auto carve = [&](size_t bytes) {
             const size_t at = used;
@@ -1466,12 +1453,16 @@ struct DevicePlan {
         const size_t o_shape = carve(sizeof(JobShape) * J), o_run = carve(sizeof(JobRun) * J);
         const size_t o_pair = carve(4 * (J + 1)), o_rankp = carve(4 * (J + 1)), o_magp = carve(4 * (J + 1));
         const size_t o_cp = carve(4 * (J + 1)), o_bp = carve(4 * (J + 1)), o_np = carve(4 * (J + 1)),
-                     o_nq = carve(4 * (J + 1)), o_st = carve(4), o_pass = carve(sizeof(Pass) * J * S),
-                     o_pp = carve(4 * (J + 1) * S);
-        const size_t FS = p.fstep.size();
+                     o_nq = carve(4 * (J + 1)), o_st = carve(4);
         const size_t o_comp = carve(sizeof(JobComp) * J), o_gp = carve(4 * (J + 1)), o_tp = carve(4 * (J + 1)),
-                     o_pbp = carve(4 * (J + 1)), o_plp = carve(4 * (J + 1)), o_fpass = carve(sizeof(Pass) * J * FS),
-                     o_fpp = carve(4 * (J + 1) * FS), o_lp = carve(4 * (J + 1) * S), o_flp = carve(4 * (J + 1) * FS);
+                     o_pbp = carve(4 * (J + 1)), o_plp = carve(4 * (J + 1));
+        const StepTables* tables[2] = {&p.inv, &p.fwd};
+        size_t o_pass[2], o_pfx[2][3];
+        for (int k = 0; k < 2; ++k) {
+            const size_t S = tables[k]->pass.size();
+            o_pass[k] = carve(sizeof(Pass) * J * S);
+            for (size_t& o : o_pfx[k]) o = carve(4 * (J + 1) * S);
+        }
         hip_check(hipMalloc(reinterpret_cast<void**>(&mem), used), "batch plan allocation");
         hip_check(hipHostMalloc(reinterpret_cast<void**>(&host_status), 4), "batch status");
         hip_check(hipStreamCreateWithFlags(&side, hipStreamNonBlocking), "batch side stream");
@@ -1487,23 +1478,32 @@ struct DevicePlan {
         np_pfx = reinterpret_cast<uint32_t*>(mem + o_np);
         nq_pfx = reinterpret_cast<uint32_t*>(mem + o_nq);
         status = reinterpret_cast<uint32_t*>(mem + o_st);
-        pass = reinterpret_cast<Pass*>(mem + o_pass);
-        pass_pfx = reinterpret_cast<uint32_t*>(mem + o_pp);
         comp = reinterpret_cast<JobComp*>(mem + o_comp);
         group_pfx = reinterpret_cast<uint32_t*>(mem + o_gp);
         tile_pfx = reinterpret_cast<uint32_t*>(mem + o_tp);
         pblock_pfx = reinterpret_cast<uint32_t*>(mem + o_pbp);
         place_pfx = reinterpret_cast<uint32_t*>(mem + o_plp);
-        fpass = reinterpret_cast<Pass*>(mem + o_fpass);
-        fpass_pfx = reinterpret_cast<uint32_t*>(mem + o_fpp);
-        lds_pfx = reinterpret_cast<uint32_t*>(mem + o_lp);
-        flds_pfx = reinterpret_cast<uint32_t*>(mem + o_flp);
-        std::vector<Pass> flat;
-        std::vector<uint32_t> flat_pfx, flat_lpfx;
-        for (size_t st = 0; st < S; ++st) {
-            flat.insert(flat.end(), p.step[st].begin(), p.step[st].end());
-            flat_pfx.insert(flat_pfx.end(), p.pfx[st].begin(), p.pfx[st].end());
-            flat_lpfx.insert(flat_lpfx.end(), p.lpfx[st].begin(), p.lpfx[st].end());
+        // the steps' tables, flattened (kept until the copies are done, below)
+        std::vector<Pass> flat[2];
+        std::vector<uint32_t> prefixes[2][3];
+        for (int k = 0; k < 2; ++k) {
+            DeviceSteps& d = k ? fwd : inv;
+            d.pass = reinterpret_cast<Pass*>(mem + o_pass[k]);
+            uint32_t** place[3] = {&d.pfx, &d.spfx, &d.zpfx};
+            const std::vector<std::vector<uint32_t>>* from[3] = {&tables[k]->pfx, &tables[k]->spfx, &tables[k]->zpfx};
+            for (const auto& v : tables[k]->pass) flat[k].insert(flat[k].end(), v.begin(), v.end());
+            if (!flat[k].empty())
+                hip_check(hipMemcpyAsync(d.pass, flat[k].data(), sizeof(Pass) * flat[k].size(), hipMemcpyHostToDevice,
+                                         s),
+                          "plan");
+            for (int q = 0; q < 3; ++q) {
+                *place[q] = reinterpret_cast<uint32_t*>(mem + o_pfx[k][q]);
+                for (const auto& v : *from[q]) prefixes[k][q].insert(prefixes[k][q].end(), v.begin(), v.end());
+                if (!prefixes[k][q].empty())
+                    hip_check(hipMemcpyAsync(*place[q], prefixes[k][q].data(), 4 * prefixes[k][q].size(),
+                                             hipMemcpyHostToDevice, s),
+                              "plan");
+            }
         }
         hip_check(hipMemcpyAsync(shape, p.shape.data(), sizeof(JobShape) * J, hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(chunk_pfx, p.chunk_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
@@ -1511,33 +1511,11 @@ struct DevicePlan {
         hip_check(hipMemcpyAsync(pair_pfx, p.pair_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(rank_pfx, p.rank_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(mag_pfx, p.mag_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
-        if (S) {
-            hip_check(hipMemcpyAsync(pass, flat.data(), sizeof(Pass) * flat.size(), hipMemcpyHostToDevice, s), "plan");
-            hip_check(hipMemcpyAsync(pass_pfx, flat_pfx.data(), 4 * flat_pfx.size(), hipMemcpyHostToDevice, s),
-                      "plan");
-            hip_check(hipMemcpyAsync(lds_pfx, flat_lpfx.data(), 4 * flat_lpfx.size(), hipMemcpyHostToDevice, s),
-                      "plan");
-        }
-        std::vector<Pass> fflat;
-        std::vector<uint32_t> fflat_pfx, fflat_lpfx;
-        for (size_t st = 0; st < FS; ++st) {
-            fflat.insert(fflat.end(), p.fstep[st].begin(), p.fstep[st].end());
-            fflat_pfx.insert(fflat_pfx.end(), p.fpfx[st].begin(), p.fpfx[st].end());
-            fflat_lpfx.insert(fflat_lpfx.end(), p.flpfx[st].begin(), p.flpfx[st].end());
-        }
         hip_check(hipMemcpyAsync(comp, p.comp.data(), sizeof(JobComp) * J, hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(group_pfx, p.group_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(tile_pfx, p.tile_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(pblock_pfx, p.pblock_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(place_pfx, p.place_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
-        if (FS) {
-            hip_check(hipMemcpyAsync(fpass, fflat.data(), sizeof(Pass) * fflat.size(), hipMemcpyHostToDevice, s),
-                      "plan");
-            hip_check(hipMemcpyAsync(fpass_pfx, fflat_pfx.data(), 4 * fflat_pfx.size(), hipMemcpyHostToDevice, s),
-                      "plan");
-            hip_check(hipMemcpyAsync(flds_pfx, fflat_lpfx.data(), 4 * fflat_lpfx.size(), hipMemcpyHostToDevice, s),
-                      "plan");
-        }
         hip_check(hipMalloc(reinterpret_cast<void**>(&ranks), std::max<size_t>(1, p.rank_geo.size()) * kRankSet * 2),
                   "batch rank tables");
         for (size_t k = 0; k < p.rank_geo.size(); ++k)
@@ -1546,17 +1524,20 @@ struct DevicePlan {
         hip_check(hipStreamSynchronize(s), "plan upload");
     }
 
-    // The LDS-staged passes of one step (blocks workgroups), small or large variant.
+    // The strip and column passes of one step.
     template <class T, bool Inverse>
-    void launch_lds(uint32_t blocks, bool large_lds, const JobRun* r, const Pass* ps, const uint32_t* pf,
-                    const StageBanks& sb, T fill, uint32_t* st, hipStream_t s) const {
-        if (!blocks) return;
-        if (large_lds)
-            hipLaunchKernelGGL((batch_lds_kernel<T, true, Inverse>), dim3(blocks), dim3(kLdsThreads), 0, s, shape, r,
-                               ps, pf, host.jobs, sb, fill, st);
-        else
-            hipLaunchKernelGGL((batch_lds_kernel<T, false, Inverse>), dim3(blocks), dim3(kLdsThreads), 0, s, shape,
-                               r, ps, pf, host.jobs, sb, fill, st);
+    void launch_step(size_t st, const JobRun* r, const StageBanks& sb, T fill, uint32_t* status_word,
+                     hipStream_t s) const {
+        const StepTables& t = Inverse ? host.inv : host.fwd;
+        const DeviceSteps& d = Inverse ? inv : fwd;
+        const uint32_t J = host.jobs, strips = t.spfx[st][J], columns = t.zpfx[st][J];
+        if (strips)
+            hipLaunchKernelGGL((batch_strip_kernel<T, Inverse>), dim3(8 * ((strips + 7) / 8)), dim3(kStripThreads), 0,
+                               s, shape, r, d.pass + st * J, d.spfx + st * (J + 1), J, sb, fill, status_word);
+        if (columns)
+            hipLaunchKernelGGL((batch_zcol_kernel<T, Inverse>), dim3(8 * ((columns + 7) / 8)), dim3(kZThreads),
+                               t.zlds[st], s, shape, r, d.pass + st * J, d.zpfx + st * (J + 1), J, sb, fill,
+                               status_word);
     }
 
     // Enqueues the batched compress on `s`: no synchronisation, allocation or
@@ -1594,13 +1575,12 @@ struct DevicePlan {
         zero_words(ws + L.zero0, (L.zero_end - L.zero0) / 4, s);
         zero_words(run, uint64_t(J) * sizeof(JobRun) / 4, s);  // every job decodable for the inverse passes
         const StageBanks fsb{input, b.home, b.tmp0, b.tmp1, nullptr, b.res};
-        for (size_t st = 0; st < p.fstep.size(); ++st) {
-            const uint32_t blocks = p.fpfx[st][J];
+        for (size_t st = 0; st < p.fwd.pass.size(); ++st) {
+            const uint32_t blocks = p.fwd.pfx[st][J];
             if (blocks)
                 hipLaunchKernelGGL((batch_fwd_pass_kernel<T>), dim3(blocks), dim3(256), 0, s, shape,
-                                   fpass + st * J, fpass_pfx + st * (J + 1), J, b);
-            launch_lds<T, false>(p.flpfx[st][J], p.flarge[st], nullptr, fpass + st * J, flds_pfx + st * (J + 1), fsb,
-                                 T(0), nullptr, s);
+                                   fwd.pass + st * J, fwd.pfx + st * (J + 1), J, b);
+            launch_step<T, false>(st, nullptr, fsb, T(0), nullptr, s);
         }
         zero_words(b.tmp1, p.sign_words, s);  // sign words: bricks OR their edge words
         if (p.brick_pfx[J])
@@ -1627,13 +1607,12 @@ struct DevicePlan {
         }
         const Banks bk{b.home, b.tmp0, b.tmp1, b.recon};
         const StageBanks isb{nullptr, b.home, b.tmp0, b.tmp1, b.recon, nullptr};
-        for (size_t st = 0; st < p.step.size(); ++st) {
-            const uint32_t blocks = p.pfx[st][J];
+        for (size_t st = 0; st < p.inv.pass.size(); ++st) {
+            const uint32_t blocks = p.inv.pfx[st][J];
             if (blocks)
-                hipLaunchKernelGGL((batch_pass_kernel<T>), dim3(blocks), dim3(256), 0, s, shape, run, pass + st * J,
-                                   pass_pfx + st * (J + 1), J, bk, T(0), status);
-            launch_lds<T, true>(p.lpfx[st][J], p.large[st], run, pass + st * J, lds_pfx + st * (J + 1), isb, T(0),
-                                status, s);
+                hipLaunchKernelGGL((batch_pass_kernel<T>), dim3(blocks), dim3(256), 0, s, shape, run,
+                                   inv.pass + st * J, inv.pfx + st * (J + 1), J, bk, T(0), status);
+            launch_step<T, true>(st, run, isb, T(0), status, s);
         }
         if (p.tile_pfx[J])
             hipLaunchKernelGGL((batch_repair_kernel<T>), dim3(p.tile_pfx[J]), dim3(256), 0, s, shape, comp, tile_pfx,
@@ -1683,13 +1662,12 @@ struct DevicePlan {
         hipLaunchKernelGGL((batch_qpatch_kernel<T>), dim3(256), dim3(256), 0, s, packed, shape, run, nq_pfx, J,
                            static_cast<T*>(bk.home), status);
         const StageBanks sb{nullptr, bk.home, bk.tmp0, bk.tmp1, bk.out, nullptr};
-        for (size_t st = 0; st < p.step.size(); ++st) {
-            const uint32_t blocks = p.pfx[st][J];
+        for (size_t st = 0; st < p.inv.pass.size(); ++st) {
+            const uint32_t blocks = p.inv.pfx[st][J];
             if (blocks)
                 hipLaunchKernelGGL((batch_pass_kernel<T>), dim3(blocks), dim3(256), 0, s, shape, run,
-                                   pass + st * J, pass_pfx + st * (J + 1), J, bk, T(fill), status);
-            launch_lds<T, true>(p.lpfx[st][J], p.large[st], run, pass + st * J, lds_pfx + st * (J + 1), sb, T(fill),
-                                status, s);
+                                   inv.pass + st * J, inv.pfx + st * (J + 1), J, bk, T(fill), status);
+            launch_step<T, true>(st, run, sb, T(fill), status, s);
         }
         hipLaunchKernelGGL((batch_rpatch_kernel<T>), dim3(kRpatchBlocks), dim3(256), 0, s, packed, shape, run, np_pfx, J,
                            static_cast<T*>(bk.out), status);

@@ -40,8 +40,9 @@ struct StripPlan {
 constexpr uint32_t kStripThreads = 256;
 
 // The plan of an nx x ny box of nz planes; `pack`: lines may share a wave
-// (false: the planes of a group would not fit one 32-bit window).
-WZ_HD StripPlan strip_plan(Dims n, bool pack) {
+// (false: the planes of a group would not fit one 32-bit window); `want`: the
+// waves this box should come to, where it has the rows for them.
+WZ_HD StripPlan strip_plan(Dims n, bool pack, uint32_t want = 4096) {
     StripPlan p;
     const uint32_t np = half_len(n.nx);
     auto fits = [&](uint32_t w) { return np + 2 <= w || (np == w && !(n.nx & 1u)); };
@@ -54,8 +55,8 @@ WZ_HD StripPlan strip_plan(Dims n, bool pack) {
     // keep memory busy
     p.sy = 128;
     auto waves = [&] { return uint64_t(p.strips) * p.zgroups * ((n.ny + p.sy - 1) / p.sy); };
-    while (p.sy > 32 && waves() < 4096) p.sy >>= 1;
-    if (waves() < 1024) p.sy = 16;
+    while (p.sy > 32 && waves() < want) p.sy >>= 1;
+    if (waves() < want / 4) p.sy = 16;
     p.segs = (n.ny + p.sy - 1) / p.sy;
     return p;
 }
@@ -160,6 +161,29 @@ WZ_D StripItem strip_item(const StripPlan& p, Dims n, uint32_t item) {
     return it;
 }
 
+// What becomes of an inverse's samples besides the store: clipping to an output
+// frame, a hole's fill value instead of them, a non-finite screen.
+struct StripStore {  // none of these
+    WZ_D Dims clip(Dims n) const { return n; }
+    template <class T>
+    WZ_D T value(T v, bool) {
+        return v;
+    }
+};
+template <class T>
+struct StripOutput {
+    Dims box;  // extents that are stored
+    bool hole;
+    T fill;
+    bool finite = true;
+    WZ_D Dims clip(Dims) const { return box; }
+    WZ_D T value(T v, bool put) {
+        if (hole) return fill;
+        finite = finite && (finite_value(v) || !put);
+        return v;
+    }
+};
+
 template <class T>
 struct XYInverse {
     const T* hi;  // the level's coefficients outside its low box
@@ -180,8 +204,8 @@ struct XYInverse {
 // g + 2 and emits rows 2 (g - 2) and 2 (g - 2) + 1; the segment's first four
 // steps only warm the Y pipeline up. Four steps are one block (the fold phases
 // of the Y tile of 8 rows are then fixed).
-template <class T, bool Requant>
-WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item) {
+template <class T, bool Requant, class Output>
+WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item, Output&& out) {
     using C = Lift<T>;
     constexpr uint32_t S = sizeof(T);
     const Dims n = a.n;
@@ -198,7 +222,9 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
                              uint32_t((uint64_t(min(64u >> p.lw, n.nz - it.z0) - 1u) * a.opz +
                                        uint64_t(n.ny - 1u) * a.opy + n.nx) * S));
     const uint32_t ov = (it.zl * uint32_t(a.opz) + 2 * it.kp) * S;
-    const bool both = it.own && 2 * it.kp + 1 < n.nx, half = it.own && !both;
+    const Dims c = out.clip(n);
+    const bool here = it.own && it.z0 + (threadIdx.x & 63u) / (1u << p.lw) < c.nz;
+    const bool both = here && 2 * it.kp + 1 < c.nx, half = here && 2 * it.kp + 1 == c.nx;
     auto load = [&](int32_t g, T (&v)[4]) {  // pair g of rows: (low, high) of its even and of its odd row
         const uint32_t se = uint32_t(pair_even(g, ny)), so = hy + uint32_t(pair_odd(g, ny));
         v[0] = buf_load_at(T(0), wl, lv, se * lrow);
@@ -229,7 +255,7 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
             const int phase = (u + 2) & 3;
             T re[2], ro[2];
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
+            for (int c = 0; c < 2; ++c) {  // the pair's columns
                 const T oraw = v[2 + c];
                 const T es = v[c] * C::ik, os = oraw * (-C::k);
                 const T eA = fmadd(-C::d, OS[c] + os, es);
@@ -259,11 +285,16 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
             }
             if constexpr (emit) {
                 const uint32_t y = 2 * uint32_t(g - 2);
-                buf_store_pair(re[0], re[1], wo, both && y < n.ny ? ov + y * orow : kOutside);
-                buf_store_pair(ro[0], ro[1], wo, both && y + 1 < n.ny ? ov + (y + 1) * orow : kOutside);
-                if (n.nx & 1u) {  // the last sample of an odd line
-                    buf_store(re[0], wo, half && y < n.ny ? ov + y * orow : kOutside);
-                    buf_store(ro[0], wo, half && y + 1 < n.ny ? ov + (y + 1) * orow : kOutside);
+                const bool in0 = y < c.ny, in1 = y + 1 < c.ny;
+                re[0] = out.value(re[0], (both || half) && in0);
+                re[1] = out.value(re[1], both && in0);
+                ro[0] = out.value(ro[0], (both || half) && in1);
+                ro[1] = out.value(ro[1], both && in1);
+                buf_store_pair(re[0], re[1], wo, both && in0 ? ov + y * orow : kOutside);
+                buf_store_pair(ro[0], ro[1], wo, both && in1 ? ov + (y + 1) * orow : kOutside);
+                if (c.nx & 1u) {  // the last sample of an odd line
+                    buf_store(re[0], wo, half && in0 ? ov + y * orow : kOutside);
+                    buf_store(ro[0], wo, half && in1 ? ov + (y + 1) * orow : kOutside);
                 }
             }
         }
