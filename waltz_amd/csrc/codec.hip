@@ -54,9 +54,9 @@ struct DeviceWorkspace {
     uint16_t* rank = nullptr;  // 8*8192 forward + 8*8192 inverse
     Dims rank_dims{0, 0, 0};
     uint32_t rank_bz = 0;
-    EncodeResult* result = nullptr;      // device
-    EncodeResult* host_result = nullptr;  // pinned
-    SideStream side{};                    // the WZP group pass beside the inverse levels (default priority)
+    DecodeRecord* record = nullptr;  // device
+    void* host_result = nullptr;     // pinned: EncodeResult or DecodeRecord
+    SideStream side{};               // work beside the caller's stream (default priority)
 
     ~DeviceWorkspace() = default;  // process-lifetime cache
 
@@ -72,9 +72,8 @@ struct DeviceWorkspace {
     void init() {
         if (!rank) {
             hip_check(hipMalloc(reinterpret_cast<void**>(&rank), 2 * 8 * 8192 * sizeof(uint16_t)), "rank tables");
-            // one record for compress (EncodeResult) or decode (DecodeRecord)
-            hip_check(hipMalloc(reinterpret_cast<void**>(&result), kRecordBytes), "result");
-            hip_check(hipHostMalloc(reinterpret_cast<void**>(&host_result), kRecordBytes), "pinned result");
+            hip_check(hipMalloc(reinterpret_cast<void**>(&record), kRecordBytes), "record");
+            hip_check(hipHostMalloc(&host_result, kRecordBytes), "pinned result");
             hip_check(hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking), "side stream");
             hip_check(hipEventCreateWithFlags(&side.ready, hipEventDisableTiming), "event");
             hip_check(hipEventCreateWithFlags(&side.done, hipEventDisableTiming), "event");
@@ -151,6 +150,11 @@ Geometry geometry(Dims d, unsigned width) {
 
 uint32_t qcap(uint32_t n) { return n <= (1u << 20) ? n : (1u << 20); }
 
+// Work runs on the side stream only for fields of at least this many samples:
+// handing it over and back costs two event packets on each stream, more than
+// running it in order while its kernels are short.
+constexpr uint32_t kSideMin = 1u << 22;
+
 // An early exit (exception) must not leave side-stream work of this call
 // running into the next one.
 struct SideJoin {
@@ -219,6 +223,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
             T* rerr;
             unsigned long long* desc;
             uint32_t *size, *counters;
+            EncodeResult* res;
         } p;
         p.coeff = c.take<T>(n);
         p.t0 = c.take<T>(n);
@@ -251,6 +256,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         if (shared_words) p.rbm = c.take<uint32_t>(words);
         p.desc = c.take<unsigned long long>(ws.chunks);
         p.counters = c.take<uint32_t>(4);  // ticket, q count, repair total
+        p.res = c.take<EncodeResult>(1);
         p.zeroed = reinterpret_cast<uint32_t*>(c.base + z0);
         return std::make_pair(p, c.used - z0);
     };
@@ -259,9 +265,9 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     Carve carve{static_cast<uint8_t*>(w.reserve(probe.used))};
     auto [p, zero_bytes] = plan(carve);
 
-    EncodeResult* res = w.result;
+    EncodeResult* res = p.res;
+    EncodeResult* const host = static_cast<EncodeResult*>(w.host_result);
     uint32_t* status = &res->status;
-    zero_words(res, sizeof(EncodeResult) / 4, s);
     zero_words(p.zeroed, zero_bytes / 4, s);
 
     transform_forward<T>(input, p.coeff, p.t0, p.t1, g.d, g.lx, g.lz, g.dyadic, status, s);
@@ -274,7 +280,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     // The group pass runs on the side stream beside the inverse levels (the
     // staging slots it reads are never written by them); the archive sections
     // wait for it.
-    const SideStream* side = &w.side;
+    const SideStream* side = n >= kSideMin ? &w.side : nullptr;
     const SideJoin join{side};
     // When the coarser inverse levels requantize what they load as well (the
     // two leading levels fused), the encoder writes nothing back. They run
@@ -324,13 +330,12 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     {
         StageClock c("sections", s);
         finish_archive<T>(archive, capacity, n, rp, qo, p.seg, flags, uint8_t(g.lx), uint8_t(g.lz), uint8_t(g.bz),
-                          quantum, res, s);
+                          quantum, res, host, s);
     }
-    hip_check(hipMemcpyAsync(w.host_result, res, sizeof(EncodeResult), hipMemcpyDeviceToHost, s), "result copy");
     hip_check(hipStreamSynchronize(s), "compress");
     hip_check(hipGetLastError(), "compress launch");
     profile_collect();
-    const EncodeResult r = *w.host_result;
+    const EncodeResult r = *host;
     if (r.status) raise_status(r.status);
     return r.end;
 }
@@ -392,6 +397,15 @@ struct DecodeSource {
         build_rank_tables(d, bz, rank, rank + 8 * 8192, s);
         return rank;
     }
+    const SideStream* side(uint32_t n) const { return cache && n >= kSideMin ? &cache->side : nullptr; }
+    // The record to the host, and the wait for it.
+    uint32_t finish(hipStream_t s) const {
+        if (cache) record_out(result, host, s);  // `host` is pinned
+        else hip_check(hipMemcpyAsync(host, result, sizeof(DecodeRecord), hipMemcpyDeviceToHost, s), "status copy");
+        hip_check(hipStreamSynchronize(s), "decompress");
+        hip_check(hipGetLastError(), "decompress launch");
+        return host->status;
+    }
 };
 
 // One decode of a validated archive into `output`; returns the device status.
@@ -443,7 +457,7 @@ uint32_t decode_pass(const uint8_t* archive, const uint8_t* hdr, const Geometry&
         screen.ptable = reinterpret_cast<uint32_t*>(mag);
     }
     // the WZP directory check runs on the side stream beside the chunk decoders
-    const SideStream* side = m.cache ? &m.cache->side : nullptr;
+    const SideStream* side = m.side(n);
     const SideJoin join{side};
     const bool pairs = pair_bricks_fit(g.d.nx, g.d.ny, g.d.nz, bz);
     const uint16_t* rank = pairs ? nullptr : m.ranks(g.d, bz, s);
@@ -482,10 +496,7 @@ uint32_t decode_pass(const uint8_t* archive, const uint8_t* hdr, const Geometry&
         if (!screened) check_finite<T>(output, n, status, s);
     }
     if (side) hip_check(hipStreamWaitEvent(s, side->done, 0), "stream wait");
-    hip_check(hipMemcpyAsync(m.host, m.result, sizeof(DecodeRecord), hipMemcpyDeviceToHost, s), "status copy");
-    hip_check(hipStreamSynchronize(s), "decompress");
-    hip_check(hipGetLastError(), "decompress launch");
-    return m.host->status;
+    return m.finish(s);
 }
 
 // A decode planned on the device: a kernel checks the header into the
@@ -494,14 +505,13 @@ uint32_t decode_pass(const uint8_t* archive, const uint8_t* hdr, const Geometry&
 // first waiting for the header. It assumes the canonical archive of the
 // geometry (the one compress writes); any other header leaves every planned
 // kernel idle (record not ok) and the caller decodes on the host-header path.
-// Applies to dyadic fields whose finest inverse level runs fused (it applies
-// the repairs, so every count the launch needs comes from the record), and to
-// plane-schedule fields whose inverse runs as fused XY levels and one Z phase
-// (which screens the output; the repairs follow in a pass of their own).
-bool planned_decode_fits(const Geometry& g, uint64_t archive_bytes, unsigned width) {
-    if (archive_bytes == ~uint64_t(0) || archive_bytes < 32) return false;
-    if (!g.dyadic) return plane_fused_fits(g.d, g.lx, g.lz, width);
-    return g.lx >= 1 && tuning_for(g.d, g.lx, width, true).fused >= 1 && patch_table_words(g.d, g.n, width) != 0;
+// Repairs are folded into the finest level where it runs fused (dyadic fields:
+// every count the launch needs comes from the record); else they follow in a
+// pass of their own.
+bool planned_decode_fits(uint64_t archive_bytes) { return archive_bytes != ~uint64_t(0) && archive_bytes >= 32; }
+bool repairs_fold(const Geometry& g, unsigned width) {
+    return g.dyadic && g.lx >= 1 && tuning_for(g.d, g.lx, width, true).fused >= 1 &&
+           patch_table_words(g.d, g.n, width) != 0;
 }
 
 template <class T>
@@ -518,8 +528,10 @@ uint32_t decode_planned(const uint8_t* archive, uint64_t archive_bytes, const Ge
     DecodeRecord* rec = m.result;
     uint32_t* status = &rec->status;
     const uint8_t flags = uint8_t((g.dyadic ? 1u : 0u) | (sizeof(T) == 8 ? 4u : 0u) | (3u << 3));
+    const bool fold = repairs_fold(g, sizeof(T));
     {
-        StageClock ck("decode_plan", s);
+        // (a stage name of its own for dyadic fields without a fused finest level)
+        StageClock ck(fold || !g.dyadic ? "decode_plan" : "header_check", s);
         decode_plan(archive, archive_bytes,
                     PlanExpect{n, uint32_t(sizeof(T)), flags, uint8_t(g.lx), uint8_t(g.lz), uint8_t(g.bz)}, rec, s);
     }
@@ -528,12 +540,11 @@ uint32_t decode_planned(const uint8_t* archive, uint64_t archive_bytes, const Ge
     // only the archive), then checks the WZP directory; the caller's stream
     // waits for the table only before the finest level, after the coarse
     // levels.
-    const SideStream* side = m.cache ? &m.cache->side : nullptr;
+    const SideStream* side = m.side(n);
     const SideJoin join{side};
     const bool pairs = pair_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz);
     const uint16_t* rank = pairs ? nullptr : m.ranks(g.d, g.bz, s);
     const bool ranks = rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz) && reinterpret_cast<uintptr_t>(rank) % 8 == 0;
-    const bool fold = g.dyadic;  // repairs folded into the finest fused level (else a pass of their own)
     const bool keys_on_side = fold && (pairs || ranks) && side;
     if (side) hip_check(hipEventRecord(side->ready, s), "event record");
     if (pairs || ranks) {
@@ -558,8 +569,6 @@ uint32_t decode_planned(const uint8_t* archive, uint64_t archive_bytes, const Ge
         hip_check(hipEventRecord(side->mid, ss), "event record");
         wzp_directory_planned(archive + 32, rec, n, status, ss);
         hip_check(hipEventRecord(side->done, ss), "event record");
-    } else {
-        wzp_directory_planned(archive + 32, rec, n, status, s);
     }
     if (fold && !keys_on_side) {
         StageClock ck("patch_keys", s);
@@ -567,21 +576,19 @@ uint32_t decode_planned(const uint8_t* archive, uint64_t archive_bytes, const Ge
     }
     {
         StageClock ck("qoutliers", s);
-        apply_qoutliers_planned<T>(coeff, archive, rec, n, status, s);
+        if (side) apply_qoutliers_planned<T>(coeff, archive, rec, n, status, s);
+        else directory_qoutliers_planned<T>(coeff, archive, rec, n, status, s);
     }
     if (!fold) {
         Level0Emit<T> screen{kEmitStoreScreen, status, nullptr, 0.0, SegList{}, 0.0};
-        const bool screened = transform_inverse<T>(coeff, output, t0, t1, g.d, g.lx, g.lz, false, s, &screen);
+        const bool screened = transform_inverse<T>(coeff, output, t0, t1, g.d, g.lx, g.lz, g.dyadic, s, &screen);
         {
             StageClock ck("patches", s);
             apply_repairs_planned<T>(output, archive, rec, n, status, s);
         }
         if (!screened) check_finite<T>(output, n, status, s);
         if (side) hip_check(hipStreamWaitEvent(s, side->done, 0), "stream wait");
-        hip_check(hipMemcpyAsync(m.host, rec, sizeof(DecodeRecord), hipMemcpyDeviceToHost, s), "status copy");
-        hip_check(hipStreamSynchronize(s), "decompress");
-        hip_check(hipGetLastError(), "decompress launch");
-        return m.host->status;
+        return m.finish(s);
     }
     Level0Emit<T> screen{kEmitStoreScreen, status, nullptr, 0.0, SegList{}, 0.0};
     screen.np = n;  // an upper bound: the count comes from the record
@@ -593,10 +600,7 @@ uint32_t decode_planned(const uint8_t* archive, uint64_t archive_bytes, const Ge
     if (keys_on_side) hip_check(hipStreamWaitEvent(s, side->mid, 0), "stream wait");
     inverse_finest_level<T>(coeff, low, output, g.d, g.lx, screen, s);
     if (side) hip_check(hipStreamWaitEvent(s, side->done, 0), "stream wait");
-    hip_check(hipMemcpyAsync(m.host, rec, sizeof(DecodeRecord), hipMemcpyDeviceToHost, s), "status copy");
-    hip_check(hipStreamSynchronize(s), "decompress");
-    hip_check(hipGetLastError(), "decompress launch");
-    return m.host->status;
+    return m.finish(s);
 }
 
 // Header read and checks, then the decode (with the duplicate-checking pass
@@ -609,7 +613,7 @@ void decompress_with(const uint8_t* archive, uint64_t archive_bytes, Dims d, T* 
     uint8_t hdr[32];
     uint32_t st = 0;
     bool decoded = false;  // by the planned decode (its header was valid and canonical)
-    if (planned_decode_fits(g, archive_bytes, sizeof(T))) {
+    if (planned_decode_fits(archive_bytes)) {
         check_disjoint(archive, archive_bytes, output, uint64_t(g.n) * sizeof(T));
         st = decode_planned<T>(archive, archive_bytes, g, output, m, s);
         std::memcpy(hdr, m.host->header, 32);
@@ -657,8 +661,7 @@ void decompress(const uint8_t* archive, uint64_t archive_bytes, Dims d, T* outpu
     std::lock_guard<std::mutex> guard(w.lock);
     w.init();
     const DecodeSource m{static_cast<uint8_t*>(w.reserve(decode_scratch_bytes(g.n, sizeof(T)))),
-                         reinterpret_cast<DecodeRecord*>(w.result), reinterpret_cast<DecodeRecord*>(w.host_result), &w,
-                         nullptr};
+                         w.record, static_cast<DecodeRecord*>(w.host_result), &w, nullptr};
     decompress_with<T>(archive, archive_bytes, d, output, s, canonical_chunk, m);
 }
 

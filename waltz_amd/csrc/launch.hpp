@@ -232,6 +232,11 @@ void decode_dequantize_pairs_planned(const uint8_t* in, const DecodeRecord* rec,
 void wzp_decode_planned(const uint8_t* in, const DecodeRecord* rec, uint32_t n, uint16_t* mag, uint32_t* sign,
                         uint32_t* status, hipStream_t s);
 void wzp_directory_planned(const uint8_t* in, const DecodeRecord* rec, uint32_t n, uint32_t* status, hipStream_t s);
+// The directory check and the q-outlier patch (apply_qoutliers_planned) in one
+// launch, for fields too small to be worth a side stream.
+template <class T>
+void directory_qoutliers_planned(T* coeff, const uint8_t* archive, const DecodeRecord* rec, uint32_t n,
+                                 uint32_t* status, hipStream_t s);
 // The same fusions for the other fields of full bricks (rank_bricks_fit, z
 // band bz): `rank` is the full brick's rank table (build_rank_tables, shape
 // 0), 8-byte aligned.
@@ -260,12 +265,13 @@ struct EncodeResult {
     uint32_t np, nq, status, pad;
 };
 // Orders both side lists by index into the archive sections and writes the
-// 32-byte header and all padding. `scratch` needs finish_scratch_words(n) u32.
+// 32-byte header and all padding; the result goes to `host` (pinned) as well.
+// `scratch` needs finish_scratch_words(n) u32.
 uint64_t finish_scratch_words(uint32_t n);
 template <class T>
 void finish_archive(uint8_t* archive, uint64_t capacity, uint32_t n, SegList repairs, SideList qout,
                     uint32_t* scratch, uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz, double quantum,
-                    EncodeResult* result, hipStream_t s);
+                    EncodeResult* result, EncodeResult* host, hipStream_t s);
 template <class T>
 void apply_qoutliers(T* coeff, const uint8_t* idx, const uint8_t* val, uint32_t count, uint32_t n, double quantum,
                      uint32_t* status, hipStream_t s);
@@ -283,6 +289,7 @@ void repair_keys(const uint32_t* idx, const T* err, uint32_t count, Dims d, uint
 // cleared), and the list kernels reading counts and places from it.
 void decode_plan(const uint8_t* archive, uint64_t archive_bytes, const PlanExpect& e, DecodeRecord* rec,
                  hipStream_t s);
+void record_out(const DecodeRecord* rec, DecodeRecord* host, hipStream_t s);  // host: pinned memory
 template <class T>
 void apply_qoutliers_planned(T* coeff, const uint8_t* archive, const DecodeRecord* rec, uint32_t n, uint32_t* status,
                              hipStream_t s);

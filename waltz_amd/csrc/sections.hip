@@ -13,6 +13,8 @@
 //    popcounts). O(n), no sort, same bytes as a comparison sort.
 #include "sections.hpp"
 
+#include <algorithm>
+
 namespace wz {
 
 template <class T>
@@ -50,8 +52,78 @@ __global__ void __launch_bounds__(1024) scan_layout_kernel(uint8_t* __restrict__
                                                            uint32_t n, uint32_t* rbsum, uint32_t* qbsum,
                                                            uint32_t blocks, uint32_t* np_dev, SideList qo,
                                                            uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz,
-                                                           double quantum, EncodeResult* __restrict__ res) {
-    scan_layout<T>(archive, capacity, n, rbsum, qbsum, blocks, np_dev, qo, flags, lx, lz, bz, quantum, res);
+                                                           double quantum, EncodeResult* __restrict__ res,
+                                                           EncodeResult* host) {
+    scan_layout<T>(archive, capacity, n, rbsum, qbsum, blocks, np_dev, qo, flags, lx, lz, bz, quantum, res, host);
+}
+
+// The whole of it for a small field (at most kFinishSmall samples) by one
+// workgroup of 1024 threads: ranks of both bitmaps in LDS, layout, placement.
+// Three launches cost a field of 2^15 samples more than the work they spread;
+// from about 2^17 samples on one workgroup's gathers take longer.
+constexpr uint32_t kFinishSmall = 1u << 17;
+template <class T>
+__global__ void __launch_bounds__(1024) finish_small_kernel(uint8_t* __restrict__ archive, uint64_t capacity,
+                                                            uint32_t n, SegList rp, SideList qo, uint8_t flags,
+                                                            uint8_t lx, uint8_t lz, uint8_t bz, double quantum,
+                                                            EncodeResult* __restrict__ res, EncodeResult* host) {
+    __shared__ uint32_t pre[2][kFinishSmall / 32];
+    __shared__ uint32_t wsum[16];
+    __shared__ EncodeResult out;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6, words = (n + 31) / 32;
+    // counts of the flags before each word; returns their total
+    auto ranks = [&](const uint32_t* bm, uint32_t* p) -> uint32_t {
+        constexpr uint32_t K = kFinishSmall / 32 / 1024;
+        uint32_t c[K], sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < K; ++k) {
+            c[k] = K * t + k < words ? uint32_t(__builtin_popcount(bm[K * t + k])) : 0u;
+            sum += c[k];
+        }
+        const uint32_t inc = sec::wave_inclusive(sum);
+        if (lane == 63) wsum[wv] = inc;
+        __syncthreads();
+        uint32_t run = inc - sum, total = 0;
+        for (uint32_t k = 0; k < 16; ++k) {
+            run += k < wv ? wsum[k] : 0u;
+            total += wsum[k];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < K; ++k) {
+            p[K * t + k] = run;
+            run += c[k];
+        }
+        __syncthreads();
+        return total;
+    };
+    auto rank = [](const uint32_t* bm, const uint32_t* p, uint32_t i) {
+        return p[i >> 5] + uint32_t(__builtin_popcount(bm[i >> 5] & ((1u << (i & 31u)) - 1u)));
+    };
+    const uint32_t np = ranks(rp.bitmap, pre[0]), nq = *qo.count;
+    if (nq) ranks(qo.bitmap, pre[1]);
+    if (t == 0) {
+        write_layout<T>(archive, capacity, n, np, nq, qo.capacity, flags, lx, lz, bz, quantum, res);
+        out = *res;
+        *host = out;
+    }
+    __syncthreads();
+    if (out.status) return;
+    const Layout L = archive_layout(out.wzp_bytes, np, uint64_t(np) * sizeof(T), nq);
+    for (uint32_t k = wv; k < rp.segments; k += 16) {
+        const uint32_t c = rp.count[k];
+        const uint32_t* idx = rp.index + uint64_t(k) * rp.cap;
+        const T* val = static_cast<const T*>(rp.payload) + uint64_t(k) * rp.cap;
+        for (uint32_t j = lane; j < c; j += 64) {
+            const uint32_t i = idx[j], pos = rank(rp.bitmap, pre[0], i);
+            reinterpret_cast<uint32_t*>(archive + L.pi)[pos] = i;
+            reinterpret_cast<T*>(archive + L.pv)[pos] = val[j];
+        }
+    }
+    for (uint32_t j = t; j < nq; j += 1024) {
+        const uint32_t i = qo.index[j], pos = rank(qo.bitmap, pre[1], i);
+        reinterpret_cast<uint32_t*>(archive + L.qi)[pos] = i;
+        reinterpret_cast<uint32_t*>(archive + L.qv)[pos] = static_cast<const uint32_t*>(qo.payload)[j];
+    }
 }
 
 // Both side channels to their index-order slots in one launch: item
@@ -87,7 +159,12 @@ uint64_t finish_scratch_words(uint32_t n) {
 template <class T>
 void finish_archive(uint8_t* archive, uint64_t capacity, uint32_t n, SegList repairs, SideList qout, uint32_t* scratch,
                     uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz, double quantum, EncodeResult* result,
-                    hipStream_t s) {
+                    EncodeResult* host, hipStream_t s) {
+    if (n <= kFinishSmall) {
+        hipLaunchKernelGGL((finish_small_kernel<T>), dim3(1), dim3(1024), 0, s, archive, capacity, n, repairs, qout,
+                           flags, lx, lz, bz, quantum, result, host);
+        return;
+    }
     const uint32_t words = (n + 31) / 32, blocks = (words + kPrefixWords - 1) / kPrefixWords;
     const uint64_t half = pad64(words) + pad64(blocks);
     const Ranks rr{repairs.bitmap, scratch, scratch + pad64(words)};
@@ -98,27 +175,13 @@ void finish_archive(uint8_t* archive, uint64_t capacity, uint32_t n, SegList rep
                        const_cast<uint32_t*>(qr.bsum), static_cast<const uint32_t*>(qout.count), words, blocks);
     hipLaunchKernelGGL((scan_layout_kernel<T>), dim3(1), dim3(1024), 0, s, archive, capacity, n,
                        const_cast<uint32_t*>(rr.bsum), const_cast<uint32_t*>(qr.bsum), blocks, np_total, qout, flags,
-                       lx, lz, bz, quantum, result);
+                       lx, lz, bz, quantum, result, host);
     const uint32_t items = repairs.segments * kPlaceSlices + kPlaceQBlocks;
     hipLaunchKernelGGL((place_kernel<T>), dim3(8 * ((items + 7) / 8)), dim3(256), 0, s,
                        archive, repairs, rr, qout, qr, result);
 }
 
 // ------------------------------------------------------------------ decode patches
-// q-outlier record j: the coefficient's magnitude replaced (sign kept).
-template <class T>
-WZ_D void qpatch_one(T* __restrict__ c, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ val,
-                     uint32_t j, uint32_t n, T q, uint32_t* __restrict__ status) {
-    const uint32_t i = idx[j], v = val[j];
-    if (i >= n || v <= 65535u || v > 0x7FFFFFFFu) {
-        atomicOr(status, uint32_t(kCorrupt));
-        return;
-    }
-    if (j && idx[j - 1] >= i) atomicOr(status, uint32_t(kUnordered));  // duplicates are checked apart
-    const T x = T(v) * q;  // cpu/src/codec.cpp:299-302
-    c[i] = c[i] < T(0) ? -x : x;
-}
-
 template <class T>
 __global__ void qpatch_kernel(T* __restrict__ c, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ val,
                               uint32_t count, uint32_t n, T q, uint32_t* __restrict__ status) {
@@ -184,8 +247,20 @@ __global__ void decode_plan_kernel(const uint8_t* __restrict__ archive, uint64_t
     if (threadIdx.x == 0) plan_decode(archive, bytes, e, rec);
 }
 
+// The record to pinned host memory: a decode's last work, once every stage has
+// reported into it.
+__global__ void record_out_kernel(const DecodeRecord* __restrict__ rec, DecodeRecord* host) {
+    static_assert(sizeof(DecodeRecord) % 4 == 0 && sizeof(DecodeRecord) <= 256, "one word per lane");
+    if (threadIdx.x < sizeof(DecodeRecord) / 4)
+        reinterpret_cast<uint32_t*>(host)[threadIdx.x] = reinterpret_cast<const uint32_t*>(rec)[threadIdx.x];
+}
+void record_out(const DecodeRecord* rec, DecodeRecord* host, hipStream_t s) {
+    hipLaunchKernelGGL(record_out_kernel, dim3(1), dim3(64), 0, s, rec, host);
+}
+
 // The list kernels of a planned decode: a fixed grid walks the record's counts.
 constexpr uint32_t kPlannedBlocks = 512;
+uint32_t planned_blocks(uint32_t n) { return std::min(kPlannedBlocks, (n + 255) / 256); }
 
 template <class T>
 __global__ void __launch_bounds__(256) qpatch_planned_kernel(T* __restrict__ c, const uint8_t* __restrict__ archive,
@@ -267,7 +342,7 @@ void apply_repairs(T* out, const uint8_t* idx, const uint8_t* err, uint32_t coun
 template <class T>
 void apply_repairs_planned(T* out, const uint8_t* archive, const DecodeRecord* rec, uint32_t n, uint32_t* status,
                            hipStream_t s) {
-    hipLaunchKernelGGL((rpatch_planned_kernel<T>), dim3(kPlannedBlocks), dim3(256), 0, s, out, archive, rec, n,
+    hipLaunchKernelGGL((rpatch_planned_kernel<T>), dim3(planned_blocks(n)), dim3(256), 0, s, out, archive, rec, n,
                        status);
 }
 
@@ -288,7 +363,7 @@ void decode_plan(const uint8_t* archive, uint64_t archive_bytes, const PlanExpec
 template <class T>
 void apply_qoutliers_planned(T* coeff, const uint8_t* archive, const DecodeRecord* rec, uint32_t n, uint32_t* status,
                              hipStream_t s) {
-    hipLaunchKernelGGL((qpatch_planned_kernel<T>), dim3(kPlannedBlocks), dim3(256), 0, s, coeff, archive, rec, n,
+    hipLaunchKernelGGL((qpatch_planned_kernel<T>), dim3(planned_blocks(n)), dim3(256), 0, s, coeff, archive, rec, n,
                        status);
 }
 
@@ -325,7 +400,7 @@ void check_finite(const T* out, uint32_t n, uint32_t* status, hipStream_t s) {
 #define WZ_INST(T)                                                                                                \
     template void detect_repairs<T>(const T*, const T*, uint32_t, double, SegList, uint32_t*, hipStream_t);         \
     template void finish_archive<T>(uint8_t*, uint64_t, uint32_t, SegList, SideList, uint32_t*, uint8_t, uint8_t,  \
-                                    uint8_t, uint8_t, double, EncodeResult*, hipStream_t);                         \
+                                    uint8_t, uint8_t, double, EncodeResult*, EncodeResult*, hipStream_t);          \
     template void apply_qoutliers<T>(T*, const uint8_t*, const uint8_t*, uint32_t, uint32_t, double, uint32_t*,    \
                                      hipStream_t);                                                                \
     template void apply_repairs<T>(T*, const uint8_t*, const uint8_t*, uint32_t, uint32_t, uint32_t*, hipStream_t); \

@@ -177,18 +177,14 @@ WZ_D void exclusive_scan_block(uint32_t* a, uint32_t len, uint32_t* total) {
     __syncthreads();
 }
 
-// One 1024-thread workgroup: scans both block sums (the repair total lands in
-// *np_dev), then thread 0 lays out the archive sections and writes the header.
+// Lays out the archive sections and writes the header and the sections'
+// padding (one thread).
 template <class T>
-WZ_D void scan_layout(uint8_t* __restrict__ archive, uint64_t capacity, uint32_t n, uint32_t* rbsum, uint32_t* qbsum,
-                      uint32_t blocks, uint32_t* np_dev, const SideList& qo, uint8_t flags, uint8_t lx, uint8_t lz,
-                      uint8_t bz, double quantum, EncodeResult* __restrict__ res) {
-    exclusive_scan_block(rbsum, blocks, np_dev);
-    if (*qo.count != 0) exclusive_scan_block(qbsum, blocks, nullptr);
-    if (threadIdx.x != 0) return;
-    const uint32_t np = *np_dev, nq = *qo.count;
+WZ_D void write_layout(uint8_t* __restrict__ archive, uint64_t capacity, uint32_t n, uint32_t np, uint32_t nq,
+                       uint32_t qcapacity, uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz, double quantum,
+                       EncodeResult* __restrict__ res) {
     uint32_t st = res->status;
-    if (nq > qo.capacity || (n > (1u << 20) && nq >= (1u << 20)) || (n > (1u << 22) && np >= (1u << 22)))
+    if (nq > qcapacity || (n > (1u << 20) && nq >= (1u << 20)) || (n > (1u << 22) && np >= (1u << 22)))
         st |= kSideCapacity;
     const uint64_t wb = res->wzp_bytes;
     const Layout L = archive_layout(wb, np, uint64_t(np) * sizeof(T), nq);
@@ -217,6 +213,20 @@ WZ_D void scan_layout(uint8_t* __restrict__ archive, uint64_t capacity, uint32_t
     for (uint64_t p = L.pv + uint64_t(np) * sizeof(T); p < L.qi; ++p) archive[p] = 0;
     for (uint64_t p = L.qi + 4ull * nq; p < L.qv; ++p) archive[p] = 0;
     for (uint64_t p = L.qv + 4ull * nq; p < L.end; ++p) archive[p] = 0;
+}
+
+// One 1024-thread workgroup: scans both block sums (the repair total lands in
+// *np_dev), then thread 0 writes the layout, and the result also to `host`
+// (pinned host memory) when given.
+template <class T>
+WZ_D void scan_layout(uint8_t* __restrict__ archive, uint64_t capacity, uint32_t n, uint32_t* rbsum, uint32_t* qbsum,
+                      uint32_t blocks, uint32_t* np_dev, const SideList& qo, uint8_t flags, uint8_t lx, uint8_t lz,
+                      uint8_t bz, double quantum, EncodeResult* __restrict__ res, EncodeResult* host = nullptr) {
+    exclusive_scan_block(rbsum, blocks, np_dev);
+    if (*qo.count != 0) exclusive_scan_block(qbsum, blocks, nullptr);
+    if (threadIdx.x != 0) return;
+    write_layout<T>(archive, capacity, n, *np_dev, *qo.count, qo.capacity, flags, lx, lz, bz, quantum, res);
+    if (host) *host = *res;
 }
 
 struct Ranks {
@@ -267,5 +277,18 @@ WZ_D void place_qoutliers(uint8_t* __restrict__ archive, SideList qo, Ranks rank
     }
 }
 
+// Decode: q-outlier record j, the coefficient's magnitude replaced (sign kept).
+template <class T>
+WZ_D void qpatch_one(T* __restrict__ c, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ val,
+                     uint32_t j, uint32_t n, T q, uint32_t* __restrict__ status) {
+    const uint32_t i = idx[j], v = val[j];
+    if (i >= n || v <= 65535u || v > 0x7FFFFFFFu) {
+        atomicOr(status, uint32_t(kCorrupt));
+        return;
+    }
+    if (j && idx[j - 1] >= i) atomicOr(status, uint32_t(kUnordered));  // duplicates are checked apart
+    const T x = T(v) * q;  // cpu/src/codec.cpp:299-302
+    c[i] = c[i] < T(0) ? -x : x;
+}
 
 }  // namespace wz

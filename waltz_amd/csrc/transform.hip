@@ -158,16 +158,18 @@ void axis(const T* src, T* dst, Dims full, Dims act, int axis, const uint32_t* t
 }
 
 template <class T, bool Inverse>
-bool xy_pair(const T* src, T* dst, Dims full, Dims act, int a0, hipStream_t s);
+bool xy_pair(const T* src, T* dst, Dims full, Dims act, int a0, uint32_t* status, hipStream_t s);
 
 // X and Y passes of a box in one launch: planes up to `limit` samples (tuned:
 // 1024 or 4096, 0 = none) staged whole in LDS by one workgroup, larger ones
-// (forward Y then X, inverse X then Y) as 64 x 32 tiles with their halos.
+// and screened ones (status: the forward's input or the inverse's output) as
+// strips.
 template <class T, bool Inverse>
-bool plane_pair(const T* src, T* dst, Dims full, Dims act, int a0, int a1, uint32_t limit, hipStream_t s) {
+bool plane_pair(const T* src, T* dst, Dims full, Dims act, int a0, int a1, uint32_t limit, uint32_t* status,
+                hipStream_t s) {
     const uint64_t cells = uint64_t(act.nx) * act.ny;
     if (act.nz == 0 || a0 + a1 != 1) return false;
-    if (cells > limit) return xy_pair<T, Inverse>(src, dst, full, act, a0, s);
+    if (cells > limit || status) return xy_pair<T, Inverse>(src, dst, full, act, a0, status, s);
     if (cells <= 1024) {
         if (a0 == 0)
             hipLaunchKernelGGL((plane_pair_pass<T, Inverse, 0, 1, 1024>), dim3(act.nz), dim3(256), 0, s, src, dst,
@@ -248,10 +250,17 @@ WZ_D bool strip_of_wave(const StripPlan& p, uint32_t& item) {
     item = 4 * id + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     return id < groups && item < total;
 }
-template <class T, bool Requant>
-__global__ void __launch_bounds__(kStripThreads) xy_inverse_kernel(XYInverse<T> a, StripPlan p) {
+template <class T, bool Requant, bool Screen>
+__global__ void __launch_bounds__(kStripThreads) xy_inverse_kernel(XYInverse<T> a, StripPlan p, uint32_t* status) {
     uint32_t item;
-    if (strip_of_wave(p, item)) strip_inverse<T, Requant>(a, p, item, StripStore{});
+    if (!strip_of_wave(p, item)) return;
+    if constexpr (Screen) {
+        StripOutput<T> out{a.n, false, T(0)};
+        strip_inverse<T, Requant>(a, p, item, out);
+        if (__ballot(!out.finite) && (threadIdx.x & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteOutput));
+    } else {
+        strip_inverse<T, Requant>(a, p, item, StripStore{});
+    }
 }
 template <class T>
 __global__ void __launch_bounds__(kStripThreads) xy_forward_kernel(XYForward<T> a, StripPlan p) {
@@ -276,13 +285,15 @@ bool strips_fit(Dims n, uint64_t pitch, uint64_t rows, unsigned levels, unsigned
 // window.
 bool strips_pack(uint64_t plane, unsigned width) { return fused_plane_fits(8 * plane, 1, width); }
 
+// screen: flag non-finite results
 template <class T>
-void xy_inverse(const XYInverse<T>& a, hipStream_t s) {
+void xy_inverse(const XYInverse<T>& a, hipStream_t s, uint32_t* screen = nullptr) {
     const StripPlan p = strip_plan(a.n, strips_pack(std::max({a.hpz, a.lpz, a.opz}), sizeof(T)));
-    if (a.q > T(0))
-        hipLaunchKernelGGL((xy_inverse_kernel<T, true>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s, a, p);
-    else
-        hipLaunchKernelGGL((xy_inverse_kernel<T, false>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s, a, p);
+    const dim3 grid(strip_blocks(p)), block(kStripThreads);
+    if (a.q > T(0) && screen) throw std::logic_error("requantizing levels are not screened");
+    if (a.q > T(0)) hipLaunchKernelGGL((xy_inverse_kernel<T, true, false>), grid, block, 0, s, a, p, screen);
+    else if (screen) hipLaunchKernelGGL((xy_inverse_kernel<T, false, true>), grid, block, 0, s, a, p, screen);
+    else hipLaunchKernelGGL((xy_inverse_kernel<T, false, false>), grid, block, 0, s, a, p, screen);
 }
 template <class T>
 void xy_forward(const XYForward<T>& a, hipStream_t s) {
@@ -294,15 +305,15 @@ void xy_forward(const XYForward<T>& a, hipStream_t s) {
 // launch, in the order the strips lift (forward Y then X, inverse X then Y);
 // false for the other order and for boxes that strips do not take.
 template <class T, bool Inverse>
-bool xy_pair(const T* src, T* dst, Dims full, Dims act, int a0, hipStream_t s) {
+bool xy_pair(const T* src, T* dst, Dims full, Dims act, int a0, uint32_t* status, hipStream_t s) {
     const uint64_t py = full.nx, pz = uint64_t(full.nx) * full.ny;
     if (!strips_fit(act, full.nx, full.ny, 1, sizeof(T))) return false;
     if constexpr (Inverse) {
         if (a0 != 0) return false;
-        xy_inverse<T>(XYInverse<T>{src, py, pz, src, py, pz, dst, py, pz, act, T(0), T(0), 0u}, s);
+        xy_inverse<T>(XYInverse<T>{src, py, pz, src, py, pz, dst, py, pz, act, T(0), T(0), 0u}, s, status);
     } else {
         if (a0 != 1) return false;
-        xy_forward<T>(XYForward<T>{src, py, pz, dst, py, pz, dst, py, pz, act, nullptr}, s);
+        xy_forward<T>(XYForward<T>{src, py, pz, dst, py, pz, dst, py, pz, act, status}, s);
     }
     return true;
 }
@@ -339,6 +350,10 @@ struct Passes {
     Tuning tune;  // tiles and LDS pair limit of the per-axis passes
     bool first = true;
     unsigned base = 0;  // level number of the box's level 0 (stage names)
+    // inverse: where non-finite samples of the last level's result are flagged
+    // (null: not asked); `screened` when its last launch did
+    uint32_t* out_status = nullptr;
+    bool screened = false;
 
     // Passes: src -> tmp0 -> tmp1 -> ... -> final. A single pass whose source
     // is already `home` goes through tmp0 and is copied back.
@@ -349,17 +364,20 @@ struct Passes {
         const T* src = first ? first_src : home;
         T* final_dst = last_level && last_dst ? last_dst : home;
         for (int k = 0; k < count; ++k) {
-            const bool screen = first && k == 0 && status;
-            // two in-plane passes of a small box: one launch
-            const bool pair = !screen && k + 1 < count && axes[k] != 2 && axes[k + 1] != 2;
+            uint32_t* const screen = first && k == 0 ? status : nullptr;
+            // two in-plane passes: one launch
+            const bool pair = k + 1 < count && axes[k] != 2 && axes[k + 1] != 2;
             const int last = pair ? k + 1 : k;
             T* const other = src == tmp[0] ? tmp[1] : tmp[0];  // never the source
             T* dst = last == count - 1 ? final_dst : other;
             if (dst == src) dst = other;  // in place at the end: through scratch, copied back below
-            if (pair && plane_pair<T, Inverse>(src, dst, full, act, axes[k], axes[k + 1], tune.pair_max, s)) {
+            uint32_t* const out = Inverse && last_level && last == count - 1 ? out_status : nullptr;
+            if (pair && plane_pair<T, Inverse>(src, dst, full, act, axes[k], axes[k + 1], tune.pair_max,
+                                               Inverse ? out : screen, s)) {
                 ++k;
+                screened = out != nullptr;
             } else {
-                axis<T, Inverse>(src, dst, full, act, axes[k], tune.tile, screen ? status : nullptr, s);
+                axis<T, Inverse>(src, dst, full, act, axes[k], tune.tile, screen, s);
             }
             src = dst;
         }
@@ -732,9 +750,10 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         for (unsigned l = 0; l < lxy; ++l) { sizes[l] = act; act = shrink(act, true, true); }
         static const int zxy[3] = {2, 0, 1};
         // coarse levels as passes in coeff; then the fused levels (coarse LLL read from coeff)
+        if (!fused && emit && emit->mode == kEmitStoreScreen && !emit->np) p.out_status = emit->status;
         for (int l = int(lxy) - 1; l >= int(fused); --l)
             p.level(full, sizes[l], zxy, 3, !fused && l == 0, unsigned(l));
-        if (!fused) return false;
+        if (!fused) return p.screened;
         if (output == coeff) {  // the level-0 kernel must not overwrite what it reads
             fused_inverse<T>(coeff, tmp1, tmp0, full, fused, tu, emit, s, base);
             if (!emit || emit->mode != kEmitRepair) copy_box<T>(tmp1, coeff, full, full, s);

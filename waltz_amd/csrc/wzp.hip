@@ -21,7 +21,10 @@
 // undone top-down with popcount prefix ranks, then BIT_2, then signs are
 // expanded under the nonzero mask. Every read is bounds-checked against the
 // stream; inconsistencies raise kCorrupt.
+#include <algorithm>
+
 #include "profile.hpp"
+#include "sections.hpp"
 #include "wzp_encode.hpp"
 
 namespace wz {
@@ -147,6 +150,31 @@ __global__ void __launch_bounds__(kDirThreads) wzp_directory_planned_kernel(cons
     check_directory(in, rec->wzp, n, chunks, groups, len, sh, status);
 }
 
+// The same beside the q-outlier patch (workgroups from 1 on), which follows the
+// chunk decoders.
+constexpr uint32_t kQpatchBlocks = 32;
+template <class T>
+__global__ void __launch_bounds__(kDirThreads) directory_qpatch_planned_kernel(T* __restrict__ coeff,
+                                                                               const uint8_t* __restrict__ archive,
+                                                                               const DecodeRecord* __restrict__ rec,
+                                                                               uint32_t n, uint32_t chunks,
+                                                                               uint32_t groups,
+                                                                               uint32_t* __restrict__ status) {
+    __shared__ uint32_t len[kMaxGroups];
+    __shared__ uint32_t sh[kDirThreads / 64];
+    if (!rec->ok) return;
+    if (blockIdx.x == 0) {
+        check_directory(archive + 32, rec->wzp, n, chunks, groups, len, sh, status);
+        return;
+    }
+    const uint32_t count = rec->nq;
+    const auto* idx = reinterpret_cast<const uint32_t*>(archive + rec->qi);
+    const auto* val = reinterpret_cast<const uint32_t*>(archive + rec->qv);
+    const T q = T(rec->quantum);
+    for (uint32_t j = (blockIdx.x - 1) * kDirThreads + threadIdx.x; j < count; j += (gridDim.x - 1) * kDirThreads)
+        qpatch_one(coeff, idx, val, j, n, q, status);
+}
+
 template <class T>
 __global__ void __launch_bounds__(256) wzp_decode_pairs_planned_kernel(const uint8_t* __restrict__ in,
                                                                       const DecodeRecord* __restrict__ rec,
@@ -228,6 +256,20 @@ void wzp_directory_planned(const uint8_t* in, const DecodeRecord* rec, uint32_t 
     hipLaunchKernelGGL(wzp_directory_planned_kernel, dim3(1), dim3(kDirThreads), 0, s, in, rec, n, ws.chunks,
                        ws.groups, status);
 }
+
+template <class T>
+void directory_qoutliers_planned(T* coeff, const uint8_t* archive, const DecodeRecord* rec, uint32_t n,
+                                 uint32_t* status, hipStream_t s) {
+    const WzpShape ws = wzp_shape(n);
+    if (!ws.chunks) return;
+    const uint32_t blocks = 1 + std::min(kQpatchBlocks, (n + kDirThreads - 1) / kDirThreads);
+    hipLaunchKernelGGL((directory_qpatch_planned_kernel<T>), dim3(blocks), dim3(kDirThreads), 0, s, coeff, archive, rec,
+                       n, ws.chunks, ws.groups, status);
+}
+template void directory_qoutliers_planned<float>(float*, const uint8_t*, const DecodeRecord*, uint32_t, uint32_t*,
+                                                 hipStream_t);
+template void directory_qoutliers_planned<double>(double*, const uint8_t*, const DecodeRecord*, uint32_t, uint32_t*,
+                                                  hipStream_t);
 
 void wzp_decode(const uint8_t* in, uint64_t bytes, uint32_t n, uint16_t* mag, uint32_t* sign, uint32_t* status,
                 hipStream_t s, const SideStream* side) {
