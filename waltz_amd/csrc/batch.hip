@@ -964,7 +964,7 @@ __global__ void __launch_bounds__(kZThreads) batch_zcol_kernel(const JobShape* _
         ZColumnsOf<T>{src.p, uint32_t(src.py), uint32_t(src.pz), dst.p, uint32_t(dst.py), uint32_t(dst.pz), act,
                       ps.levels},
         y, (item - y * xb) * kZColumns, box0, box1, screen,
-        ZOutput<T>{last ? sh.clip : act, screen, state == kJobHole, fill}, ZRepair<T>{}, 0u, nullptr);
+        ZOutput<T>{last ? sh.clip : act, screen, state == kJobHole, fill}, WaveRepair<T>{}, 0u, nullptr);
     if (screen && __ballot(!fin) && (threadIdx.x & 63u) == 0) {
         if constexpr (Inverse) atomicOr(status, uint32_t(kNonFiniteOutput));
         else atomicOr(&b.res[j].status, uint32_t(kNonFiniteInput));

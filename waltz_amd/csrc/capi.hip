@@ -462,7 +462,8 @@ int waltz_amd_wzp_encode(const void* mag, const void* sign, uint32_t n, void* ou
         unsigned long long* total = reinterpret_cast<unsigned long long*>(scratch + ((ws.chunks * 16ull + 16 + 7) & ~7ull));
         wz::WzpScratch w{desc, staging, size, tail};
         wz::wzp_encode(static_cast<const uint16_t*>(mag), static_cast<const uint32_t*>(sign), n,
-                       static_cast<uint8_t*>(out), capacity, w, total, tail + 1, s);
+                       static_cast<uint8_t*>(out), capacity, w, tail + 1, s);
+        wz::wzp_pack(n, static_cast<uint8_t*>(out), capacity, w, total, tail + 1, s);
         uint32_t st = 0;
         unsigned long long tot = 0;
         wz::hip_check(hipMemcpyAsync(&st, tail + 1, 4, hipMemcpyDeviceToHost, s), "status");

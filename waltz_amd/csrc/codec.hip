@@ -198,8 +198,9 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     const WzpShape ws = wzp_shape(n);
     const uint32_t nq = qcap(n);
     const uint32_t rtiles = (n + kRepairTile - 1) / kRepairTile;
-    uint32_t fsegs = 0, fcap = 0;  // repair segments of the last inverse pass, when it detects them
-    level0_repair_segments(g.d, g.lx, g.lz, g.dyadic, sizeof(T), &fsegs, &fcap);
+    // repair segments of the last inverse pass, when it detects them
+    const RepairSegments rsegments = level0_repair_segments(g.d, g.lx, g.lz, g.dyadic, sizeof(T));
+    const uint32_t fsegs = rsegments.segments, fcap = rsegments.cap;
     const uint64_t rslots = std::max<uint64_t>(uint64_t(rtiles) * kRepairTile, uint64_t(fsegs) * fcap);
     const uint32_t rsegs = std::max(rtiles, fsegs);
 
@@ -212,8 +213,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     // other fields of full bricks quantize inside the encoder too
     const bool ranks = rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz);
     const bool fusedq = pairs || ranks;
-    // rows that share flag words: set by atomics, cleared beforehand
-    const bool shared_words = fsegs && (g.d.nx & 31u);
+    const bool shared_words = fsegs && rsegments.cleared;  // flag words set by atomics, cleared beforehand
     auto plan = [&](Carve& c) {
         struct P {
             T *coeff, *t0, *t1, *rec;
@@ -276,7 +276,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     // with the fused repair emitter and a quantizing encoder the finest
     // level's high bands stay unquantized in coeff; that kernel requantizes
     // them on load
-    const bool requant = g.dyadic && fsegs && fusedq;
+    const bool requant = g.dyadic && fsegs && fusedq && tuning_for(g.d, g.lx, sizeof(T), true).fused;
     // The group pass runs on the side stream beside the inverse levels (the
     // staging slots it reads are never written by them); the archive sections
     // wait for it.
@@ -294,13 +294,12 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     const WriteBack wb = split || plane_requant ? kWriteNone : requant ? kWriteCoarseBox : kWriteAll;
     if (pairs) {
         StageClock c("quantize_encode", s);
-        quantize_encode_pairs<T>(p.coeff, g.d, quantum, qo, archive + 32, capacity - 32, wsc, &res->wzp_bytes,
-                                 status, s, wb, side);
+        quantize_encode_pairs<T>(p.coeff, g.d, quantum, qo, archive + 32, capacity - 32, wsc, status, s, wb);
     } else if (ranks) {
         const uint16_t* rank = w.ranks(g.d, g.bz, s);
         StageClock c("quantize_encode", s);
-        quantize_encode_ranks<T>(p.coeff, g.d, g.bz, rank, quantum, qo, archive + 32, capacity - 32, wsc,
-                                 &res->wzp_bytes, status, s, wb, side);
+        quantize_encode_ranks<T>(p.coeff, g.d, g.bz, rank, quantum, qo, archive + 32, capacity - 32, wsc, status, s,
+                                 wb);
     } else {
         const BrickGeometry bg = brick_geometry(g.d, g.bz);
         const uint16_t* rank = w.ranks(g.d, g.bz, s);
@@ -309,8 +308,11 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
             quantize_bricks<T>(p.coeff, bg, quantum, rank, p.mag, p.sign, qo, status, s);
         }
         StageClock c("wzp_encode", s);
-        wzp_encode(p.mag, p.sign, n, archive + 32, capacity - 32, wsc, &res->wzp_bytes, status, s, side);
+        wzp_encode(p.mag, p.sign, n, archive + 32, capacity - 32, wsc, status, s);
     }
+    // (small fields: with the archive sections, in one launch)
+    const bool pack_last = n <= kFinishSmall;
+    if (!pack_last) wzp_pack(n, archive + 32, capacity - 32, wsc, &res->wzp_bytes, status, s, side);
     // the last inverse pass detects the native repairs where it can (fsegs);
     // otherwise reconstruct, then a repair pass
     Level0Emit<T> emit{kEmitRepair, status, input, abs_bound, SegList{p.rbm, p.ridx, p.rerr, p.rcount, fsegs, fcap},
@@ -330,7 +332,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     {
         StageClock c("sections", s);
         finish_archive<T>(archive, capacity, n, rp, qo, p.seg, flags, uint8_t(g.lx), uint8_t(g.lz), uint8_t(g.bz),
-                          quantum, res, host, s);
+                          quantum, res, host, s, pack_last ? &wsc : nullptr);
     }
     hip_check(hipStreamSynchronize(s), "compress");
     hip_check(hipGetLastError(), "compress launch");

@@ -22,8 +22,8 @@ inline void check_launch_size(uint64_t total) {
 template <class T>
 void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz,
                        bool dyadic, uint32_t* status, hipStream_t s);
-// What the last inverse pass (the fused finest level of a dyadic field, the Z
-// phase of a plane-schedule one) does with its reconstruction: store it
+// What the last inverse pass (the finest level of a dyadic field, the Z phase
+// of a plane-schedule one) does with its reconstruction: store it
 // (optionally screening for non-finite samples) or, without storing, derive
 // native repairs against `orig`.
 template <class T>
@@ -32,8 +32,7 @@ struct Level0Emit {
     uint32_t* status;
     const T* orig;
     double bound;
-    SegList rep;       // segments/cap per level0_repair_segments(); its bitmap
-                       // cleared by the caller unless rows are whole words (nx % 32 == 0)
+    SegList rep;       // as level0_repair_segments() says
     double quantum;    // kEmitRepair: > 0 when the finest level's high bands hold the
                        // unquantized coefficients (quantized and dequantized on load)
     // kEmitStoreScreen: a repair list (strictly increasing indices, np > 0
@@ -106,10 +105,14 @@ void inverse_coarse_requant(const T* coeff, T* t0, T* t1, Dims full, unsigned lx
 template <class T>
 void inverse_finest_requant(const T* coeff, const T* t0, Dims full, unsigned lxy, const Level0Emit<T>& emit,
                             hipStream_t s);
-// Segments and per-segment capacity the last inverse pass uses for repairs
-// (0 segments when it does not detect them for this geometry).
-void level0_repair_segments(Dims full, unsigned lxy, unsigned lz, bool dyadic, unsigned width, uint32_t* segments,
-                            uint32_t* cap);
+// Record segments (and their capacity) the last inverse pass uses for repairs
+// (none when it does not detect them for this geometry), and whether it sets
+// the flag bits by atomics in a bitmap cleared beforehand.
+struct RepairSegments {
+    uint32_t segments = 0, cap = 0;
+    bool cleared = false;
+};
+RepairSegments level0_repair_segments(Dims full, unsigned lxy, unsigned lz, bool dyadic, unsigned width);
 
 
 // Bit-neutral launch choices of the dyadic schedule for one geometry, type
@@ -198,11 +201,15 @@ struct SideStream {
 };
 // Staging of the encoder: kChunkSlot bytes per chunk plus read-ahead padding.
 inline uint64_t wzp_staging_bytes(uint32_t chunks) { return uint64_t(chunks) * kChunkSlot + 64; }
-// Encodes mag/sign into out (WZP stream at out[0..]); payload capacity bound
-// `capacity` (bytes available from out). Total bytes -> *total (device u64).
+// Encodes mag/sign into the WZP stream at out[0..] (payload capacity bound
+// `capacity`: bytes available from out): chunk metas, and payloads and sizes
+// into the scratch.
 void wzp_encode(const uint16_t* mag, const uint32_t* sign, uint32_t n, uint8_t* out, uint64_t capacity,
-                WzpScratch w, unsigned long long* total, uint32_t* status, hipStream_t s,
-                const SideStream* pack = nullptr);
+                WzpScratch w, uint32_t* status, hipStream_t s);
+// The group pass after an encoder (directory, payloads in place, total bytes
+// -> *total, a device u64), on `s` or on the side stream.
+void wzp_pack(uint32_t n, uint8_t* out, uint64_t capacity, const WzpScratch& w, unsigned long long* total,
+              uint32_t* status, hipStream_t s, const SideStream* side = nullptr);
 // Decodes a WZP stream of `bytes` bytes into packed mag/sign arrays. The
 // decoders and the decode_* calls below also check the group directory
 // (spans inside the payload and tiling it exactly, else kCorrupt), on `side`
@@ -218,8 +225,7 @@ void wzp_decode(const uint8_t* in, uint64_t bytes, uint32_t n, uint16_t* mag, ui
 enum WriteBack { kWriteAll, kWriteCoarseBox, kWriteNone };
 template <class T>
 void quantize_encode_pairs(T* coeff, Dims d, double quantum, SideList qo, uint8_t* out, uint64_t capacity,
-                           WzpScratch w, unsigned long long* total, uint32_t* status, hipStream_t s,
-                           WriteBack wb = kWriteAll, const SideStream* pack = nullptr);
+                           WzpScratch w, uint32_t* status, hipStream_t s, WriteBack wb = kWriteAll);
 template <class T>
 void decode_dequantize_pairs(const uint8_t* in, uint64_t bytes, Dims d, double quantum, T* coeff, uint32_t* status,
                              hipStream_t s, const SideStream* side = nullptr);
@@ -242,9 +248,8 @@ void directory_qoutliers_planned(T* coeff, const uint8_t* archive, const DecodeR
 // 0), 8-byte aligned.
 template <class T>
 void quantize_encode_ranks(T* coeff, Dims d, uint32_t bz, const uint16_t* rank, double quantum, SideList qo,
-                           uint8_t* out, uint64_t capacity, WzpScratch w, unsigned long long* total,
-                           uint32_t* status, hipStream_t s, WriteBack wb = kWriteAll,
-                           const SideStream* pack = nullptr);
+                           uint8_t* out, uint64_t capacity, WzpScratch w, uint32_t* status, hipStream_t s,
+                           WriteBack wb = kWriteAll);
 template <class T>
 void decode_dequantize_ranks(const uint8_t* in, uint64_t bytes, Dims d, uint32_t bz, const uint16_t* rank,
                              double quantum, T* coeff, uint32_t* status, hipStream_t s,
@@ -266,12 +271,14 @@ struct EncodeResult {
 };
 // Orders both side lists by index into the archive sections and writes the
 // 32-byte header and all padding; the result goes to `host` (pinned) as well.
-// `scratch` needs finish_scratch_words(n) u32.
+// `scratch` needs finish_scratch_words(n) u32. `pack` (n <= kFinishSmall only):
+// the encoder's group pass has not run and comes first, in the same launch.
+constexpr uint32_t kFinishSmall = 1u << 17;  // 16 chunks: one group
 uint64_t finish_scratch_words(uint32_t n);
 template <class T>
 void finish_archive(uint8_t* archive, uint64_t capacity, uint32_t n, SegList repairs, SideList qout,
                     uint32_t* scratch, uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz, double quantum,
-                    EncodeResult* result, EncodeResult* host, hipStream_t s);
+                    EncodeResult* result, EncodeResult* host, hipStream_t s, const WzpScratch* pack = nullptr);
 template <class T>
 void apply_qoutliers(T* coeff, const uint8_t* idx, const uint8_t* val, uint32_t count, uint32_t n, double quantum,
                      uint32_t* status, hipStream_t s);

@@ -12,6 +12,7 @@
 //    below it (per-1024-bit segment popcounts + one exclusive scan + in-segment
 //    popcounts). O(n), no sort, same bytes as a comparison sort.
 #include "sections.hpp"
+#include "wzp_encode.hpp"
 
 #include <algorithm>
 
@@ -58,15 +59,21 @@ __global__ void __launch_bounds__(1024) scan_layout_kernel(uint8_t* __restrict__
 }
 
 // The whole of it for a small field (at most kFinishSmall samples) by one
-// workgroup of 1024 threads: ranks of both bitmaps in LDS, layout, placement.
-// Three launches cost a field of 2^15 samples more than the work they spread;
-// from about 2^17 samples on one workgroup's gathers take longer.
-constexpr uint32_t kFinishSmall = 1u << 17;
+// workgroup of 1024 threads: the WZP group pass (one group; with scratch),
+// ranks of both bitmaps in LDS, layout, placement. Four launches cost a field
+// of 2^15 samples more than the work they spread; from about 2^17 samples on
+// one workgroup's gathers take longer.
 template <class T>
 __global__ void __launch_bounds__(1024) finish_small_kernel(uint8_t* __restrict__ archive, uint64_t capacity,
                                                             uint32_t n, SegList rp, SideList qo, uint8_t flags,
                                                             uint8_t lx, uint8_t lz, uint8_t bz, double quantum,
-                                                            EncodeResult* __restrict__ res, EncodeResult* host) {
+                                                            EncodeResult* res, EncodeResult* host, WzpScratch w) {
+    static_assert(kPackThreads == 1024 && kFinishSmall <= kGroup * kChunk, "one group");
+    if (w.staging) {
+        const uint32_t chunks = (n + kChunk - 1) / kChunk;
+        pack_group(0, archive + 32, capacity - 32, chunks, 1, w, &res->wzp_bytes, &res->status);
+        __syncthreads();
+    }
     __shared__ uint32_t pre[2][kFinishSmall / 32];
     __shared__ uint32_t wsum[16];
     __shared__ EncodeResult out;
@@ -159,10 +166,11 @@ uint64_t finish_scratch_words(uint32_t n) {
 template <class T>
 void finish_archive(uint8_t* archive, uint64_t capacity, uint32_t n, SegList repairs, SideList qout, uint32_t* scratch,
                     uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz, double quantum, EncodeResult* result,
-                    EncodeResult* host, hipStream_t s) {
+                    EncodeResult* host, hipStream_t s, const WzpScratch* pack) {
+    if (pack && n > kFinishSmall) throw std::logic_error("group pass deferred for a large field");
     if (n <= kFinishSmall) {
         hipLaunchKernelGGL((finish_small_kernel<T>), dim3(1), dim3(1024), 0, s, archive, capacity, n, repairs, qout,
-                           flags, lx, lz, bz, quantum, result, host);
+                           flags, lx, lz, bz, quantum, result, host, pack ? *pack : WzpScratch{});
         return;
     }
     const uint32_t words = (n + 31) / 32, blocks = (words + kPrefixWords - 1) / kPrefixWords;
@@ -400,7 +408,8 @@ void check_finite(const T* out, uint32_t n, uint32_t* status, hipStream_t s) {
 #define WZ_INST(T)                                                                                                \
     template void detect_repairs<T>(const T*, const T*, uint32_t, double, SegList, uint32_t*, hipStream_t);         \
     template void finish_archive<T>(uint8_t*, uint64_t, uint32_t, SegList, SideList, uint32_t*, uint8_t, uint8_t,  \
-                                    uint8_t, uint8_t, double, EncodeResult*, EncodeResult*, hipStream_t);          \
+                                    uint8_t, uint8_t, double, EncodeResult*, EncodeResult*, hipStream_t,           \
+                                    const WzpScratch*);                                                           \
     template void apply_qoutliers<T>(T*, const uint8_t*, const uint8_t*, uint32_t, uint32_t, double, uint32_t*,    \
                                      hipStream_t);                                                                \
     template void apply_repairs<T>(T*, const uint8_t*, const uint8_t*, uint32_t, uint32_t, uint32_t*, hipStream_t); \

@@ -190,7 +190,7 @@ bool plane_pair(const T* src, T* dst, Dims full, Dims act, int a0, int a1, uint3
 
 template <class T, bool Inverse, bool Repair>
 __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a, uint32_t* __restrict__ status,
-                                                                ZRepair<T> rp) {
+                                                                WaveRepair<T> rp) {
     static_assert(Inverse || !Repair, "repairs follow the inverse");
     __shared__ uint32_t seg_fill;  // repair entries of this workgroup
     extern __shared__ __attribute__((aligned(16))) uint8_t zlds[];
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a,
 
 template <class T, bool Inverse>
 void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* status, hipStream_t s,
-                 const ZRepair<T>* repair = nullptr) {
+                 const WaveRepair<T>* repair = nullptr) {
     if (!zcol_fits(full.nz, sizeof(T)) || levels < 1 || levels > 5 || src == dst)
         throw std::logic_error("Z phase does not fit LDS");
     const uint64_t total = uint64_t(full.ny) * ((full.nx + kZColumns - 1) / kZColumns);
@@ -237,7 +237,7 @@ void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* sta
         }
     }
     hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse, false>), grid, dim3(kZThreads), lds, s, a, status,
-                       ZRepair<T>{});
+                       WaveRepair<T>{});
 }
 
 // One XY level (of the plane schedule, or of a dyadic level that runs as
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(kStripThreads) xy_inverse_kernel(XYInverse<T> 
         strip_inverse<T, Requant>(a, p, item, out);
         if (__ballot(!out.finite) && (threadIdx.x & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteOutput));
     } else {
-        strip_inverse<T, Requant>(a, p, item, StripStore{});
+        strip_inverse<T, Requant>(a, p, item, StripStore<T>{});
     }
 }
 template <class T>
@@ -301,6 +301,209 @@ void xy_forward(const XYForward<T>& a, hipStream_t s) {
     hipLaunchKernelGGL((xy_forward_kernel<T>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s, a, p);
 }
 
+// The finest level of a dyadic field (its Z pass done, in `src`) with the
+// native repairs detected instead of the reconstruction stored.
+template <class T>
+__global__ void __launch_bounds__(kStripThreads) xy_repair_kernel(XYInverse<T> a, StripPlan p, WaveRepair<T> r,
+                                                                  uint32_t* status) {
+    uint32_t item;
+    if (!strip_of_wave(p, item)) return;
+    StripRepair<T> out{r};
+    strip_inverse<T, false>(a, p, item, out);
+    if (__ballot(!out.ok) && (threadIdx.x & 63u) == 0) atomicOr(status, uint32_t(kRepairBound));
+}
+template <class T>
+XYInverse<T> repair_level(const T* src, Dims full, const WaveRepair<T>& r) {
+    const uint64_t py = full.nx, pz = uint64_t(full.nx) * full.ny;
+    return XYInverse<T>{src, py, pz, src, py, pz, const_cast<T*>(r.orig), py, pz, full, T(0), T(0), 0u};
+}
+template <class T>
+StripPlan repair_plan(Dims full) {
+    return strip_plan(full, strips_pack(uint64_t(full.nx) * full.ny, sizeof(T)));
+}
+template <class T>
+void xy_repair(const T* src, Dims full, const WaveRepair<T>& r, uint32_t* status, hipStream_t s) {
+    const StripPlan p = repair_plan<T>(full);
+    if (r.rep.segments != p.items() || r.rep.cap < strip_repair_cap(p))
+        throw std::logic_error("repair segments do not match the finest level's launch");
+    StageClock clock("inverse_L0_repairs", s);
+    hipLaunchKernelGGL((xy_repair_kernel<T>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s,
+                       repair_level(src, full, r), p, r, status);
+}
+
+// The coarsest dyadic levels in one launch: boxes of at most kTailSamples are
+// too small to be worth a launch per pass (about 5 us each; a level of 12x16x24
+// takes 7 us here instead of 10). A box of 32^3 would take one CU 11 us per
+// level, more than its two launches. One workgroup of 16 waves runs every
+// pass of these levels, Z tiles and strips dealt to its waves, with a barrier
+// between passes; the box goes through the scratch volume and L2 as before.
+constexpr uint32_t kTailSamples = 8192, kTailWaves = 16;
+template <class T>
+struct Tail {
+    T* home;  // coefficient volume and scratch, both at the field's pitches
+    T* tmp;
+    uint64_t py, pz;
+    const T* first;  // forward: where the finest box lies (home, or the input)
+    T* last;         // inverse: where the finest box goes (home, or the output)
+    uint32_t levels;
+    Dims n[5];          // finest first
+    StripPlan plan[5];
+    uint32_t* status;   // screen for non-finite samples, or unmet bounds
+};
+template <class T>
+__global__ void __launch_bounds__(64 * kTailWaves) tail_forward_kernel(Tail<T> a) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint32_t l = 0; l < a.levels; ++l) {
+        const XYForward<T> xy{l ? a.home : a.first, a.py, a.pz, a.tmp, a.py, a.pz, a.tmp, a.py, a.pz, a.n[l],
+                              l ? nullptr : a.status};
+        for (uint32_t i = wave; i < a.plan[l].items(); i += kTailWaves) strip_forward<T>(xy, a.plan[l], i);
+        __syncthreads();
+        for (uint32_t i = wave; i < z_items<T>(a.n[l]); i += kTailWaves)
+            z_tile<T, false>(a.tmp, a.home, uint32_t(a.py), uint32_t(a.pz), a.n[l], i);
+        __syncthreads();
+    }
+}
+enum TailOut : int { kTailStore = 0, kTailScreen = 1, kTailRepair = 2 };
+template <class T, int Out>
+__global__ void __launch_bounds__(64 * kTailWaves) tail_inverse_kernel(Tail<T> a, WaveRepair<T> r) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int l = int(a.levels) - 1; l >= 0; --l) {
+        for (uint32_t i = wave; i < z_items<T>(a.n[l]); i += kTailWaves)
+            z_tile<T, true>(a.home, a.tmp, uint32_t(a.py), uint32_t(a.pz), a.n[l], i);
+        __syncthreads();
+        XYInverse<T> xy{a.tmp, a.py, a.pz, a.tmp, a.py, a.pz, l ? a.home : a.last, a.py, a.pz, a.n[l], T(0), T(0), 0u};
+        if (Out != kTailStore && l == 0) {
+            for (uint32_t i = wave; i < a.plan[0].items(); i += kTailWaves) {
+                if constexpr (Out == kTailScreen) {
+                    StripOutput<T> out{a.n[0], false, T(0)};
+                    strip_inverse<T, false>(xy, a.plan[0], i, out);
+                    if (__ballot(!out.finite) && (threadIdx.x & 63u) == 0)
+                        atomicOr(a.status, uint32_t(kNonFiniteOutput));
+                } else {
+                    xy.out = const_cast<T*>(r.orig);
+                    StripRepair<T> out{r};
+                    strip_inverse<T, false>(xy, a.plan[0], i, out);
+                    if (__ballot(!out.ok) && (threadIdx.x & 63u) == 0) atomicOr(a.status, uint32_t(kRepairBound));
+                }
+            }
+        } else {
+            for (uint32_t i = wave; i < a.plan[l].items(); i += kTailWaves)
+                strip_inverse<T, false>(xy, a.plan[l], i, StripStore<T>{});
+        }
+        __syncthreads();
+    }
+}
+
+// First level of the tail of a dyadic field whose levels below `from` run
+// otherwise (lxy: none).
+unsigned tail_level(Dims full, unsigned lxy, unsigned from, unsigned width) {
+    Dims n = full;
+    for (unsigned l = 0; l < lxy; ++l) {
+        if (l >= from && uint64_t(n.nx) * n.ny * n.nz <= kTailSamples &&
+            strips_fit(n, full.nx, full.ny, lxy - l, width))
+            return l;
+        n = shrink(n, true, true);
+    }
+    return lxy;
+}
+template <class T>
+Tail<T> make_tail(T* home, T* tmp, Dims full, unsigned level, unsigned lxy) {
+    Tail<T> t{};
+    t.home = home;
+    t.tmp = tmp;
+    t.py = full.nx;
+    t.pz = uint64_t(full.nx) * full.ny;
+    t.first = home;
+    t.last = home;
+    t.levels = lxy - level;
+    Dims n = full;
+    for (unsigned l = 0; l < lxy; ++l) {
+        if (l >= level) {
+            t.n[l - level] = n;
+            t.plan[l - level] = strip_plan(n, strips_pack(t.pz, sizeof(T)), kTailWaves, 16);
+        }
+        n = shrink(n, true, true);
+    }
+    return t;
+}
+template <class T>
+void tail_forward(const Tail<T>& t, hipStream_t s) {
+    StageClock clock("forward_tail", s);
+    hipLaunchKernelGGL((tail_forward_kernel<T>), dim3(1), dim3(64 * kTailWaves), 0, s, t);
+}
+// `repair` (the finest box is the field): records instead of the store; the
+// field's plan, whose items are the record segments.
+template <class T>
+void tail_inverse(Tail<T> t, Dims full, const WaveRepair<T>* repair, hipStream_t s) {
+    StageClock clock("inverse_tail", s);
+    const dim3 block(64 * kTailWaves);
+    if (repair) {
+        t.plan[0] = repair_plan<T>(full);
+        if (repair->rep.segments != t.plan[0].items() || repair->rep.cap < strip_repair_cap(t.plan[0]))
+            throw std::logic_error("repair segments do not match the finest level's launch");
+        hipLaunchKernelGGL((tail_inverse_kernel<T, kTailRepair>), dim3(1), block, 0, s, t, *repair);
+    } else if (t.status) {
+        hipLaunchKernelGGL((tail_inverse_kernel<T, kTailScreen>), dim3(1), block, 0, s, t, WaveRepair<T>{});
+    } else {
+        hipLaunchKernelGGL((tail_inverse_kernel<T, kTailStore>), dim3(1), block, 0, s, t, WaveRepair<T>{});
+    }
+}
+
+// The coarsest XY levels of the plane schedule in one launch: a plane's levels
+// depend on nothing else, so a workgroup takes a plane through all levels
+// whose boxes are at most kPlaneTailSamples, with a barrier between them
+// (planes of 128 x 128 still fill the device better as launches of their own).
+constexpr uint32_t kPlaneTailSamples = 4096, kPlaneTailWaves = 8;
+template <class T, class Level>
+struct PlaneTail {
+    uint32_t levels;
+    Level level[5];  // in launch order
+    StripPlan plan[5];  // of one plane
+};
+template <class T>
+__global__ void __launch_bounds__(64 * kPlaneTailWaves) plane_tail_forward_kernel(PlaneTail<T, XYForward<T>> a) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), z = blockIdx.x;
+    for (uint32_t l = 0; l < a.levels; ++l) {
+        XYForward<T> xy = a.level[l];
+        xy.src += uint64_t(z) * xy.spz;
+        xy.hi += uint64_t(z) * xy.hpz;
+        xy.lo += uint64_t(z) * xy.lpz;
+        xy.n.nz = 1;
+        for (uint32_t i = wave; i < a.plan[l].items(); i += kPlaneTailWaves) strip_forward<T>(xy, a.plan[l], i);
+        __syncthreads();
+    }
+}
+template <class T, bool Requant>
+__global__ void __launch_bounds__(64 * kPlaneTailWaves) plane_tail_inverse_kernel(PlaneTail<T, XYInverse<T>> a) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), z = blockIdx.x;
+    for (uint32_t l = 0; l < a.levels; ++l) {
+        XYInverse<T> xy = a.level[l];
+        xy.hi += uint64_t(z) * xy.hpz;
+        xy.lo += uint64_t(z) * xy.lpz;
+        xy.out += uint64_t(z) * xy.opz;
+        xy.n.nz = 1;
+        for (uint32_t i = wave; i < a.plan[l].items(); i += kPlaneTailWaves)
+            strip_inverse<T, Requant>(xy, a.plan[l], i, StripStore<T>{});
+        __syncthreads();
+    }
+}
+// First level of that tail (lxy: none; one level alone is launched as usual).
+unsigned plane_tail_level(Dims full, unsigned lxy) {
+    Dims n = full;
+    for (unsigned l = 0; l + 1 < lxy; ++l) {
+        if (uint64_t(n.nx) * n.ny <= kPlaneTailSamples) return l;
+        n = shrink(n, true, false);
+    }
+    return lxy;
+}
+template <class T, class Level>
+void add_plane(PlaneTail<T, Level>& t, const Level& a) {
+    Dims n = a.n;
+    n.nz = 1;
+    t.plan[t.levels] = strip_plan(n, false, kPlaneTailWaves, 16);
+    t.level[t.levels++] = a;
+}
+
 // The X and Y passes of box `act` (in full-pitched arrays, src != dst) as one
 // launch, in the order the strips lift (forward Y then X, inverse X then Y);
 // false for the other order and for boxes that strips do not take.
@@ -318,13 +521,19 @@ bool xy_pair(const T* src, T* dst, Dims full, Dims act, int a0, uint32_t* status
     return true;
 }
 
-// Compact XY boxes of the plane schedule's levels >= 1 (every plane) in
-// `scratch`: level l's box at offset 0 for odd l and after the largest
-// level-1 box for even l (the two never alias).
+// Compact XY boxes of the plane schedule's levels >= 1 (every plane), one after
+// the other in `scratch`: a launch that takes a plane through several levels
+// must not write one level's box where another plane still reads a finer or
+// coarser one. Their sum stays below the field (each is at most 4/9 of the one
+// before, for extents of at least 2).
 template <class T>
 T* xy_box(T* scratch, Dims full, unsigned l) {
-    const uint64_t first = uint64_t(half_len(full.nx)) * half_len(full.ny) * full.nz;
-    return (l & 1u) ? scratch : scratch + ((first + 63) & ~uint64_t(63));
+    Dims n = full;
+    for (unsigned k = 1; k < l; ++k) {
+        n = shrink(n, true, false);
+        scratch += uint64_t(n.nx) * n.ny * n.nz;
+    }
+    return scratch;
 }
 
 template <class T>
@@ -353,6 +562,9 @@ struct Passes {
     // inverse: where non-finite samples of the last level's result are flagged
     // (null: not asked); `screened` when its last launch did
     uint32_t* out_status = nullptr;
+    // inverse: the last level's result is compared with originals instead of
+    // stored (out_status takes unmet bounds)
+    const WaveRepair<T>* repair = nullptr;
     bool screened = false;
 
     // Passes: src -> tmp0 -> tmp1 -> ... -> final. A single pass whose source
@@ -372,6 +584,11 @@ struct Passes {
             T* dst = last == count - 1 ? final_dst : other;
             if (dst == src) dst = other;  // in place at the end: through scratch, copied back below
             uint32_t* const out = Inverse && last_level && last == count - 1 ? out_status : nullptr;
+            if (Inverse && pair && out && repair) {
+                xy_repair<T>(src, full, *repair, out, s);
+                screened = true;
+                return;
+            }
             if (pair && plane_pair<T, Inverse>(src, dst, full, act, axes[k], axes[k + 1], tune.pair_max,
                                                Inverse ? out : screen, s)) {
                 ++k;
@@ -629,21 +846,20 @@ void fused_inverse(T* coeff, T* output, T* tmp0, Dims full, unsigned levels, con
     launch_finest<T>(coeff, low.p, low.py, low.pz, output, full, tu.sz[0], emit, s, names[base]);
 }
 
-void level0_repair_segments(Dims full, unsigned lxy, unsigned lz, bool dyadic, unsigned width, uint32_t* segments,
-                            uint32_t* cap) {
-    *segments = 0;
-    *cap = 0;
-    if (!dyadic && plane_fused_fits(full, lxy, lz, width)) {  // the Z phase detects them, by rows of columns
-        *segments = full.ny * ((full.nx + kZColumns - 1) / kZColumns);
-        *cap = std::min(full.nx, kZColumns) * full.nz;
-        return;
-    }
-    if (!dyadic || !lxy) return;
+RepairSegments level0_repair_segments(Dims full, unsigned lxy, unsigned lz, bool dyadic, unsigned width) {
+    if (!dyadic && plane_fused_fits(full, lxy, lz, width))  // the Z phase detects them, by rows of columns
+        return {full.ny * ((full.nx + kZColumns - 1) / kZColumns), std::min(full.nx, kZColumns) * full.nz,
+                (full.nx & 31u) != 0};
+    if (!dyadic || !lxy) return {};
     const Tuning tu = tuning_for(full, lxy, width, true);
-    if (!tu.fused) return;
-    const uint32_t sz = width == 4 ? repair_z_segment<float>(full, tu.sz[0]) : repair_z_segment<double>(full, tu.sz[0]);
-    *segments = uint32_t(inv_segments(full, sz));
-    *cap = 64u * 32u * sz;
+    if (tu.fused) {
+        const uint32_t sz =
+            width == 4 ? repair_z_segment<float>(full, tu.sz[0]) : repair_z_segment<double>(full, tu.sz[0]);
+        return {uint32_t(inv_segments(full, sz)), 64u * 32u * sz, (full.nx & 31u) != 0};
+    }
+    if (!strips_fit(full, full.nx, full.ny, 1, width)) return {};
+    const StripPlan p = width == 4 ? repair_plan<float>(full) : repair_plan<double>(full);
+    return {uint32_t(p.items()), strip_repair_cap(p), true};
 }
 
 // Full multi-level transform (cpu/src/transform.cpp:409-456).
@@ -672,9 +888,18 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
             for (unsigned l = 0; l < fused; ++l) act = shrink(act, true, true);
         }
         static const int yxz[3] = {1, 0, 2};
-        for (unsigned l = fused; l < lxy; ++l) {
+        const unsigned tail = tail_level(full, lxy, fused, sizeof(T));
+        for (unsigned l = fused; l < tail; ++l) {
             p.level(full, act, yxz, 3, false, l);
             act = shrink(act, true, true);
+        }
+        if (tail < lxy) {
+            Tail<T> t = make_tail<T>(coeff, tmp0, full, tail, lxy);
+            if (p.first) {  // the whole field: reads the input
+                t.first = input;
+                t.status = status;
+            }
+            tail_forward<T>(t, s);
         }
         return;
     }
@@ -695,6 +920,8 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
         }
         Dims n = full;
         static const char* names[] = {"forward_L0", "forward_L1", "forward_L2", "forward_L3", "forward_L4"};
+        const unsigned tail = plane_tail_level(full, lxy);
+        PlaneTail<T, XYForward<T>> pt{};
         for (unsigned l = 0; l < lxy; ++l) {
             StageClock clock(names[l], s);
             const Dims h{half_len(n.nx), half_len(n.ny), n.nz};
@@ -704,11 +931,16 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
             a.lo = last ? coeff : xy_box(tmp0, full, l + 1);
             a.lpy = last ? full.nx : h.nx;
             a.lpz = last ? uint64_t(full.nx) * full.ny : uint64_t(h.nx) * h.ny;
-            xy_forward<T>(a, s);
+            if (l < tail) xy_forward<T>(a, s);
+            else add_plane(pt, a);
             src = a.lo;
             spy = a.lpy;
             spz = a.lpz;
             n = h;
+        }
+        if (pt.levels) {
+            StageClock clock("forward_tail", s);
+            hipLaunchKernelGGL((plane_tail_forward_kernel<T>), dim3(full.nz), dim3(64 * kPlaneTailWaves), 0, s, pt);
         }
         return;
     }
@@ -731,6 +963,32 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
 }
 
 namespace {
+template <class T>
+WaveRepair<T> wave_repair(const Level0Emit<T>& e) {
+    T lo = T(e.bound);
+    if (double(lo) > e.bound) lo = std::nextafter(lo, T(0));
+    return WaveRepair<T>{e.orig, e.bound, lo, e.rep};
+}
+
+// The dyadic levels lxy - 1 .. fused: the tail, then as passes; level 0 (none
+// fused) ends as `p` says (its destination, screen or repairs).
+template <class T>
+void coarse_passes(Passes<T, true>& p, Dims full, unsigned lxy, unsigned fused, const Dims* sizes) {
+    static const int zxy[3] = {2, 0, 1};
+    const unsigned tail = tail_level(full, lxy, fused, sizeof(T));
+    if (tail < lxy) {
+        Tail<T> t = make_tail<T>(p.home, p.tmp[0], full, tail, lxy);
+        if (tail == 0) {
+            if (p.last_dst) t.last = p.last_dst;
+            t.status = p.out_status;
+            p.screened = p.out_status != nullptr;
+        }
+        tail_inverse<T>(t, full, tail == 0 ? p.repair : nullptr, p.s);
+        p.first = false;
+    }
+    for (int l = int(tail) - 1; l >= int(fused); --l) p.level(full, sizes[l], zxy, 3, !fused && l == 0, unsigned(l));
+}
+
 // The inverse with launch choices `tu`; `base`: the level number of this
 // field's level 0 (a coarse box run as a field of its own), for stage names.
 template <class T>
@@ -748,11 +1006,15 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         const unsigned fused = tu.fused;
         Dims sizes[5], act = full;
         for (unsigned l = 0; l < lxy; ++l) { sizes[l] = act; act = shrink(act, true, true); }
-        static const int zxy[3] = {2, 0, 1};
         // coarse levels as passes in coeff; then the fused levels (coarse LLL read from coeff)
+        WaveRepair<T> repair{};
         if (!fused && emit && emit->mode == kEmitStoreScreen && !emit->np) p.out_status = emit->status;
-        for (int l = int(lxy) - 1; l >= int(fused); --l)
-            p.level(full, sizes[l], zxy, 3, !fused && l == 0, unsigned(l));
+        if (!fused && emit && emit->mode == kEmitRepair) {
+            p.out_status = emit->status;
+            repair = wave_repair(*emit);
+            p.repair = &repair;
+        }
+        coarse_passes(p, full, lxy, fused, sizes);
         if (!fused) return p.screened;
         if (output == coeff) {  // the level-0 kernel must not overwrite what it reads
             fused_inverse<T>(coeff, tmp1, tmp0, full, fused, tu, emit, s, base);
@@ -780,6 +1042,8 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         static const char* names[] = {"inverse_L0", "inverse_L1", "inverse_L2", "inverse_L3", "inverse_L4"};
         const T* lo = coeff;
         uint64_t lpy = full.nx, lpz = uint64_t(full.nx) * full.ny;
+        const int tail = int(plane_tail_level(full, lxy));
+        PlaneTail<T, XYInverse<T>> pt{};
         for (int l = int(lxy) - 1; l >= 0; --l) {
             StageClock clock(names[l + base], s);
             XYInverse<T> a{coeff, full.nx, uint64_t(full.nx) * full.ny, lo, lpy, lpz, nullptr, 0, 0, xy[l],
@@ -793,7 +1057,18 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
                 a.opy = xy[l].nx;
                 a.opz = uint64_t(xy[l].nx) * xy[l].ny;
             }
-            xy_inverse<T>(a, s);
+            if (l >= tail) {
+                add_plane(pt, a);
+                if (l == tail) {
+                    const dim3 grid(full.nz), block(64 * kPlaneTailWaves);
+                    if (requant > 0)
+                        hipLaunchKernelGGL((plane_tail_inverse_kernel<T, true>), grid, block, 0, s, pt);
+                    else
+                        hipLaunchKernelGGL((plane_tail_inverse_kernel<T, false>), grid, block, 0, s, pt);
+                }
+            } else {
+                xy_inverse<T>(a, s);
+            }
             lo = a.out;
             lpy = a.opy;
             lpz = a.opz;
@@ -801,9 +1076,7 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         if (lz) {
             StageClock clock("inverse_Z", s);
             if (repair) {
-                T lo = T(emit->bound);
-                if (double(lo) > emit->bound) lo = std::nextafter(lo, T(0));
-                const ZRepair<T> z{emit->orig, emit->bound, lo, emit->rep};
+                const WaveRepair<T> z = wave_repair(*emit);
                 zcol_levels<T, true>(tmp1, output, full, lz, emit->status, s, &z);
             } else {
                 zcol_levels<T, true>(tmp1, output, full, lz, screen, s);
@@ -839,8 +1112,7 @@ LowBox<T> inverse_coarse_levels(T* coeff, T* tmp0, T* tmp1, Dims full, unsigned 
     Passes<T, true> p{coeff, {tmp0, tmp1}, coeff, nullptr, nullptr, s, tu};
     Dims sizes[5], act = full;
     for (unsigned l = 0; l < lxy; ++l) { sizes[l] = act; act = shrink(act, true, true); }
-    static const int zxy[3] = {2, 0, 1};
-    for (int l = int(lxy) - 1; l >= int(tu.fused); --l) p.level(full, sizes[l], zxy, 3, false, unsigned(l));
+    coarse_passes(p, full, lxy, tu.fused, sizes);
     return fused_coarse<T>(coeff, tmp0, full, tu.fused, tu, s, 0);
 }
 

@@ -46,16 +46,16 @@ __global__ void __launch_bounds__(kPackThreads) wzp_pack_kernel(uint8_t* __restr
     pack_group(g_sh, out, capacity, chunks, groups, w, total, status);
 }
 
-// The group pass after the encoder, on `s` or on the side stream.
-void launch_pack(uint8_t* out, uint64_t capacity, const WzpShape& ws, const WzpScratch& w, unsigned long long* total,
-                 uint32_t* status, hipStream_t s, const SideStream* side) {
+void wzp_pack(uint32_t n, uint8_t* out, uint64_t capacity, const WzpScratch& w, unsigned long long* total,
+              uint32_t* status, hipStream_t s, const SideStream* side) {
+    const WzpShape ws = wzp_shape(n);
     hipStream_t ps = s;
     if (side) {
         hip_check(hipEventRecord(side->ready, s), "event record");
         hip_check(hipStreamWaitEvent(side->stream, side->ready, 0), "stream wait");
         ps = side->stream;
     }
-    {
+    if (ws.chunks) {
         StageClock c("wzp_pack", ps);
         hipLaunchKernelGGL(wzp_pack_kernel, dim3(ws.groups), dim3(kPackThreads), 0, ps, out, capacity, ws.chunks,
                            ws.groups, w, total, status);
@@ -64,21 +64,16 @@ void launch_pack(uint8_t* out, uint64_t capacity, const WzpShape& ws, const WzpS
 }
 
 void wzp_encode(const uint16_t* mag, const uint32_t* sign, uint32_t n, uint8_t* out, uint64_t capacity, WzpScratch w,
-                unsigned long long* total, uint32_t* status, hipStream_t s, const SideStream* pack) {
+                uint32_t* status, hipStream_t s) {
     const WzpShape ws = wzp_shape(n);
-    if (ws.chunks == 0) {
-        if (pack) hip_check(hipEventRecord(pack->done, s), "event record");
-        return;
-    }
+    if (ws.chunks == 0) return;
     hipLaunchKernelGGL(wzp_encode_kernel<MagSource>, dim3(ws.chunks), dim3(kThreads), 0, s, MagSource{mag, sign}, n,
                        ws.groups, out, capacity, w, status);
-    launch_pack(out, capacity, ws, w, total, status, s, pack);
 }
 
 template <class T>
 void quantize_encode_pairs(T* coeff, Dims d, double quantum, SideList qo, uint8_t* out, uint64_t capacity,
-                           WzpScratch w, unsigned long long* total, uint32_t* status, hipStream_t s,
-                           WriteBack wb, const SideStream* pack) {
+                           WzpScratch w, uint32_t* status, hipStream_t s, WriteBack wb) {
     if (!pair_bricks_fit(d.nx, d.ny, d.nz, 16)) throw std::invalid_argument("field does not tile into brick pairs");
     const uint32_t n = d.nx * d.ny * d.nz;
     const WzpShape ws = wzp_shape(n);
@@ -93,7 +88,6 @@ void quantize_encode_pairs(T* coeff, Dims d, double quantum, SideList qo, uint8_
                              wb == kWriteNone ? 0u : wb == kWriteCoarseBox ? half_len(d.nz) : d.nz};
     hipLaunchKernelGGL(wzp_encode_kernel<BrickSource<T>>, dim3(ws.chunks), dim3(kThreads), 0, s, src, n, ws.groups,
                        out, capacity, w, status);
-    launch_pack(out, capacity, ws, w, total, status, s, pack);
 }
 
 // The write-back box of a fused quantizing encoder.
@@ -110,8 +104,8 @@ void check_rank_bricks(Dims d, uint32_t bz, const uint16_t* rank) {
 
 template <class T>
 void quantize_encode_ranks(T* coeff, Dims d, uint32_t bz, const uint16_t* rank, double quantum, SideList qo,
-                           uint8_t* out, uint64_t capacity, WzpScratch w, unsigned long long* total,
-                           uint32_t* status, hipStream_t s, WriteBack wb, const SideStream* pack) {
+                           uint8_t* out, uint64_t capacity, WzpScratch w, uint32_t* status, hipStream_t s,
+                           WriteBack wb) {
     check_rank_bricks(d, bz, rank);
     const uint32_t n = d.nx * d.ny * d.nz;
     const WzpShape ws = wzp_shape(n);
@@ -120,7 +114,6 @@ void quantize_encode_ranks(T* coeff, Dims d, uint32_t bz, const uint16_t* rank, 
                             h.nz};
     hipLaunchKernelGGL(wzp_encode_kernel<RankSource<T>>, dim3(ws.chunks), dim3(kThreads), 0, s, src, n, ws.groups,
                        out, capacity, w, status);
-    launch_pack(out, capacity, ws, w, total, status, s, pack);
 }
 
 template <class Sink>
@@ -325,8 +318,7 @@ void decode_dequantize_ranks(const uint8_t* in, uint64_t bytes, Dims d, uint32_t
 
 #define WZ_RANKS(T)                                                                                               \
     template void quantize_encode_ranks<T>(T*, Dims, uint32_t, const uint16_t*, double, SideList, uint8_t*,      \
-                                           uint64_t, WzpScratch, unsigned long long*, uint32_t*, hipStream_t,    \
-                                           WriteBack, const SideStream*);                                          \
+                                           uint64_t, WzpScratch, uint32_t*, hipStream_t, WriteBack);             \
     template void decode_dequantize_ranks<T>(const uint8_t*, uint64_t, Dims, uint32_t, const uint16_t*, double,  \
                                              T*, uint32_t*, hipStream_t, const SideStream*);                       \
     template void decode_dequantize_ranks_planned<T>(const uint8_t*, const DecodeRecord*, Dims, uint32_t,        \
@@ -335,11 +327,10 @@ WZ_RANKS(float)
 WZ_RANKS(double)
 #undef WZ_RANKS
 
-template void quantize_encode_pairs<float>(float*, Dims, double, SideList, uint8_t*, uint64_t, WzpScratch,
-                                           unsigned long long*, uint32_t*, hipStream_t, WriteBack, const SideStream*);
+template void quantize_encode_pairs<float>(float*, Dims, double, SideList, uint8_t*, uint64_t, WzpScratch, uint32_t*,
+                                           hipStream_t, WriteBack);
 template void quantize_encode_pairs<double>(double*, Dims, double, SideList, uint8_t*, uint64_t, WzpScratch,
-                                            unsigned long long*, uint32_t*, hipStream_t, WriteBack,
-                                            const SideStream*);
+                                            uint32_t*, hipStream_t, WriteBack);
 template void decode_dequantize_pairs<float>(const uint8_t*, uint64_t, Dims, double, float*, uint32_t*,
                                              hipStream_t, const SideStream*);
 template void decode_dequantize_pairs<double>(const uint8_t*, uint64_t, Dims, double, double*, uint32_t*,

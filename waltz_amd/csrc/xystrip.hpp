@@ -26,6 +26,7 @@
 #include "buffer.hpp"
 #include "common.hpp"
 #include "lifting.hpp"
+#include "repair.hpp"
 
 namespace wz {
 
@@ -41,8 +42,9 @@ constexpr uint32_t kStripThreads = 256;
 
 // The plan of an nx x ny box of nz planes; `pack`: lines may share a wave
 // (false: the planes of a group would not fit one 32-bit window); `want`: the
-// waves this box should come to, where it has the rows for them.
-WZ_HD StripPlan strip_plan(Dims n, bool pack, uint32_t want = 4096) {
+// waves this box should come to, where it has the rows for them; `least`: the
+// shortest segment it is cut to for that.
+WZ_HD StripPlan strip_plan(Dims n, bool pack, uint32_t want = 4096, uint32_t least = 32) {
     StripPlan p;
     const uint32_t np = half_len(n.nx);
     auto fits = [&](uint32_t w) { return np + 2 <= w || (np == w && !(n.nx & 1u)); };
@@ -55,7 +57,7 @@ WZ_HD StripPlan strip_plan(Dims n, bool pack, uint32_t want = 4096) {
     // keep memory busy
     p.sy = 128;
     auto waves = [&] { return uint64_t(p.strips) * p.zgroups * ((n.ny + p.sy - 1) / p.sy); };
-    while (p.sy > 32 && waves() < want) p.sy >>= 1;
+    while (p.sy > least && waves() < want) p.sy >>= 1;
     if (waves() < want / 4) p.sy = 16;
     p.segs = (n.ny + p.sy - 1) / p.sy;
     return p;
@@ -161,26 +163,100 @@ WZ_D StripItem strip_item(const StripPlan& p, Dims n, uint32_t item) {
     return it;
 }
 
-// What becomes of an inverse's samples besides the store: clipping to an output
-// frame, a hole's fill value instead of them, a non-finite screen.
-struct StripStore {  // none of these
-    WZ_D Dims clip(Dims n) const { return n; }
-    template <class T>
-    WZ_D T value(T v, bool) {
-        return v;
+// What becomes of an inverse strip's samples. box(): extents that are kept;
+// fetch(y): what rows y and y + 1 need is loaded ahead; put(): rows y, y + 1 of
+// the lane's two columns, `both` / `half`: the lane keeps its two samples, or
+// the first only; in0, in1: the rows are kept (wave-uniform); `wo`, `ov`,
+// `orow`: the destination's window, the lane's offset and the row pitch.
+template <class T>
+struct StripStore {
+    WZ_D Dims box(Dims n) const { return n; }
+    WZ_D void fetch(uint32_t) {}
+    WZ_D void put(uint32_t y, const T (&r0)[2], const T (&r1)[2], bool both, bool half, bool in0, bool in1, bool odd,
+                  __amdgpu_buffer_rsrc_t wo, uint32_t ov, uint32_t orow) {
+        // lanes and rows outside go past the window's range (dropped)
+        const uint32_t at = ov + y * orow;
+        buf_store_pair(r0[0], r0[1], wo, both && in0 ? at : kOutside);
+        buf_store_pair(r1[0], r1[1], wo, both && in1 ? at + orow : kOutside);
+        if (odd) {  // the last sample of an odd line
+            buf_store(r0[0], wo, half && in0 ? at : kOutside);
+            buf_store(r1[0], wo, half && in1 ? at + orow : kOutside);
+        }
     }
 };
+// The same with a non-finite screen, clipped to an output frame, or a hole's
+// fill value instead of the samples.
 template <class T>
 struct StripOutput {
-    Dims box;  // extents that are stored
+    Dims frame;
     bool hole;
     T fill;
     bool finite = true;
-    WZ_D Dims clip(Dims) const { return box; }
-    WZ_D T value(T v, bool put) {
-        if (hole) return fill;
-        finite = finite && (finite_value(v) || !put);
-        return v;
+    WZ_D Dims box(Dims) const { return frame; }
+    WZ_D void fetch(uint32_t) {}
+    WZ_D void put(uint32_t y, T (&r0)[2], T (&r1)[2], bool both, bool half, bool in0, bool in1, bool odd,
+                  __amdgpu_buffer_rsrc_t wo, uint32_t ov, uint32_t orow) {
+        auto value = [&](T& v, bool kept) {
+            if (hole) v = fill;
+            else finite = finite && (finite_value(v) || !kept);
+        };
+        value(r0[0], (both || half) && in0);
+        value(r0[1], both && in0);
+        value(r1[0], (both || half) && in1);
+        value(r1[1], both && in1);
+        StripStore<T>{}.put(y, r0, r1, both, half, in0, in1, odd, wo, ov, orow);
+    }
+};
+// Compared with the originals (the destination's window and pitches are
+// theirs) instead of stored: flag bits (of a cleared bitmap: rows share words)
+// and records in the wave's own segment of `cap` entries, counted in a scalar.
+template <class T>
+struct StripRepair {
+    WaveRepair<T> r;
+    uint32_t segment;     // the wave's item
+    uint32_t row0, nx;    // sample index of the lane's pair in row 0; samples per row
+    __amdgpu_buffer_rsrc_t wo;
+    uint32_t ov, orow;
+    T ref[2][2] = {};
+    uint32_t fill = 0;
+    bool ok = true;
+    WZ_D Dims box(Dims n) const { return n; }
+    WZ_D void fetch(uint32_t y) {
+        buf_load_pair(wo, ov + y * orow, 0u, ref[0][0], ref[0][1]);
+        buf_load_pair(wo, ov + (y + 1) * orow, 0u, ref[1][0], ref[1][1]);
+    }
+    WZ_D void put(uint32_t y, const T (&r0)[2], const T (&r1)[2], bool both, bool half, bool in0, bool in1, bool,
+                  __amdgpu_buffer_rsrc_t, uint32_t, uint32_t) {
+        const bool kept[2] = {both || half, both};
+        const unsigned long long km[2] = {__ballot(kept[0]), __ballot(kept[1])};
+        uint32_t* const index = r.rep.index + uint64_t(segment) * r.rep.cap;
+        T* const payload = static_cast<T*>(r.rep.payload) + uint64_t(segment) * r.rep.cap;
+        const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+        for (int row = 0; row < 2; ++row) {
+            if (!(row ? in1 : in0)) continue;  // (wave-uniform)
+            const T(&v)[2] = row ? r1 : r0;
+            const uint32_t at = row0 + (y + uint32_t(row)) * nx;
+            unsigned long long m[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) m[c] = repair_mask<T>(v[c], ref[row][c], kept[c], km[c], r, &ok);
+            const bool p0 = (m[0] >> lane) & 1ull, p1 = (m[1] >> lane) & 1ull;
+            if (p0 || p1) {
+                const uint32_t s = at & 31u, bits = uint32_t(p0) | uint32_t(p1) << 1;
+                atomicOr(&r.rep.bitmap[at >> 5], bits << s);
+                if (s == 31 && p1) atomicOr(&r.rep.bitmap[(at >> 5) + 1], 1u);
+            }
+            const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                if (c ? p1 : p0) {
+                    const uint32_t k = fill + uint32_t(__popcll(m[c] & below));
+                    index[k] = at + uint32_t(c);
+                    payload[k] = v[c] - ref[row][c];
+                }
+                fill += uint32_t(__popcll(m[c]));
+            }
+        }
     }
 };
 
@@ -217,14 +293,21 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
     const uint32_t hrow = uint32_t(a.hpy) * S, lrow = uint32_t(a.lpy) * S, orow = uint32_t(a.opy) * S;
     const uint32_t lv = (it.zl * uint32_t(a.lpz) + ce) * S, hv = it.zl * uint32_t(a.hpz) * S;
     const uint32_t he = hv + ce * S, ho = hv + co * S;
-    // stores: lanes and rows outside go past the window's range (dropped)
     const auto wo = window_n(a.out + uint64_t(it.z0) * a.opz,
                              uint32_t((uint64_t(min(64u >> p.lw, n.nz - it.z0) - 1u) * a.opz +
                                        uint64_t(n.ny - 1u) * a.opy + n.nx) * S));
     const uint32_t ov = (it.zl * uint32_t(a.opz) + 2 * it.kp) * S;
-    const Dims c = out.clip(n);
+    const Dims c = out.box(n);
     const bool here = it.own && it.z0 + (threadIdx.x & 63u) / (1u << p.lw) < c.nz;
     const bool both = here && 2 * it.kp + 1 < c.nx, half = here && 2 * it.kp + 1 == c.nx;
+    if constexpr (std::is_same_v<std::decay_t<Output>, StripRepair<T>>) {
+        out.segment = item;
+        out.nx = n.nx;
+        out.row0 = (it.z0 + it.zl) * n.nx * n.ny + 2 * it.kp;
+        out.wo = wo;
+        out.ov = ov;
+        out.orow = orow;
+    }
     auto load = [&](int32_t g, T (&v)[4]) {  // pair g of rows: (low, high) of its even and of its odd row
         const uint32_t se = uint32_t(pair_even(g, ny)), so = hy + uint32_t(pair_odd(g, ny));
         v[0] = buf_load_at(T(0), wl, lv, se * lrow);
@@ -244,6 +327,7 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
 #pragma unroll
         for (int u = 0; u < 4; ++u, ++g) {
             load(g + 2, buf[(u + 2) & 3]);
+            if constexpr (emit) out.fetch(2 * uint32_t(g - 2));
             T(&v)[4] = buf[u];
             if constexpr (Requant) {
                 if (a.lo_coeff) v[0] = requantize<T>(v[0], a.q, a.inv);
@@ -285,23 +369,18 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
             }
             if constexpr (emit) {
                 const uint32_t y = 2 * uint32_t(g - 2);
-                const bool in0 = y < c.ny, in1 = y + 1 < c.ny;
-                re[0] = out.value(re[0], (both || half) && in0);
-                re[1] = out.value(re[1], both && in0);
-                ro[0] = out.value(ro[0], (both || half) && in1);
-                ro[1] = out.value(ro[1], both && in1);
-                buf_store_pair(re[0], re[1], wo, both && in0 ? ov + y * orow : kOutside);
-                buf_store_pair(ro[0], ro[1], wo, both && in1 ? ov + (y + 1) * orow : kOutside);
-                if (c.nx & 1u) {  // the last sample of an odd line
-                    buf_store(re[0], wo, half && in0 ? ov + y * orow : kOutside);
-                    buf_store(ro[0], wo, half && in1 ? ov + (y + 1) * orow : kOutside);
-                }
+                out.put(y, re, ro, both, half, y < c.ny, y + 1 < c.ny, (c.nx & 1u) != 0, wo, ov, orow);
             }
         }
     };
     block(std::false_type{});
     for (uint32_t b = 0; b < it.blocks; ++b) block(std::true_type{});
+    if constexpr (std::is_same_v<std::decay_t<Output>, StripRepair<T>>) {
+        if ((threadIdx.x & 63u) == 0) out.r.rep.count[item] = out.fill;
+    }
 }
+// Record slots of one item of the repair form.
+WZ_HD uint32_t strip_repair_cap(const StripPlan& p) { return p.sy * 128u; }
 
 template <class T>
 struct XYForward {

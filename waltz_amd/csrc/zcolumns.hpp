@@ -6,6 +6,7 @@
 #include "buffer.hpp"
 #include "common.hpp"
 #include "lifting.hpp"
+#include "repair.hpp"
 
 namespace wz {
 
@@ -39,24 +40,16 @@ inline bool zcol_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5
 // records and flag bits go out (one segment per workgroup, columns x nz slots).
 // That drops a write and a read of the field and one launch: 384x384x96
 // double, inverse and repair passes 67 + 47 us before.
-template <class T>
-struct ZRepair {
-    const T* orig;
-    double bound;
-    T bound_lo;  // the largest T <= bound
-    SegList rep;
-};
 // Decides the samples v[j] (rows z + j of column x, row y) of a wave's tile
 // against their originals, sets their flag bits and appends their records to
 // segment `id`; false when a lane's sample cannot meet the bound. Wave masks
 // as in the fused finest level: the rounded difference of the final value and
 // the original settles the strict bound unless it is not below it.
 template <class T, int Tile>
-WZ_D bool zcol_repairs(const T (&v)[Tile], const T (&ref)[Tile], const ZRepair<T>& rp, Dims full, uint32_t x,
+WZ_D bool zcol_repairs(const T (&v)[Tile], const T (&ref)[Tile], const WaveRepair<T>& rp, Dims full, uint32_t x,
                        uint32_t y, uint32_t z, bool in, uint32_t id, uint32_t* seg_fill) {
     const uint32_t lane = threadIdx.x & 63u;
     const unsigned long long in_m = __ballot(in);
-    const T nb = T(rp.bound);
     bool ok = true;
     unsigned long long masks[Tile];
     T err[Tile];
@@ -66,18 +59,7 @@ WZ_D bool zcol_repairs(const T (&v)[Tile], const T (&ref)[Tile], const ZRepair<T
         masks[j] = 0;
         err[j] = v[j] - ref[j];
         if (z + uint32_t(j) >= full.nz) continue;  // (wave-uniform)
-        const T e = err[j];
-        const bool p = abs_t(e) > nb;
-        const T d = p ? (v[j] - e) - ref[j] : e;
-        const bool fast = abs_t(d) < rp.bound_lo;
-        masks[j] = __ballot(p) & in_m;
-        if (in_m & ~__ballot(fast)) {  // a tie at the bound or a non-finite sample: the full test
-            bool okj = true;
-            T ej;
-            const bool pj = repair_decision<T>(v[j], ref[j], nb, rp.bound, &ej, &okj);
-            masks[j] = __ballot(pj) & in_m;
-            ok = ok && (!in || okj);
-        }
+        masks[j] = repair_mask<T>(v[j], ref[j], in, in_m, rp, &ok);
         total += uint32_t(__popcll(masks[j]));
     }
     uint32_t base = 0;
@@ -141,7 +123,7 @@ struct ZColumnsOf {
 // (a non-finite sample of a screened pass, or an unmet bound).
 template <class T, bool Inverse, bool Repair>
 WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0, T* box1, bool screen,
-                       const ZOutput<T>& out, const ZRepair<T>& rp, uint32_t id, uint32_t* seg_fill) {
+                       const ZOutput<T>& out, const WaveRepair<T>& rp, uint32_t id, uint32_t* seg_fill) {
     constexpr int Tile = sizeof(T) == 4 ? 16 : 8, P = Tile / 2 + 4;  // (the inverse's is part of the format)
     constexpr uint32_t W = kZThreads / 64, S = sizeof(T);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
@@ -286,6 +268,43 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
         __syncthreads();
     }
     return fin;
+}
+
+// One Z level of a box, one wave per item: a tile of 64 columns, columns
+// counted row by row so that narrow boxes fill the lanes. Items: z_items().
+template <class T>
+WZ_HD uint32_t z_items(Dims n) {
+    constexpr uint32_t Tile = sizeof(T) == 4 ? 16 : 8;
+    return ((n.nx * n.ny + 63) / 64) * ((n.nz + Tile - 1) / Tile);
+}
+template <class T, bool Inverse>
+WZ_D void z_tile(const T* src, T* dst, uint32_t py, uint32_t pz, Dims box, uint32_t item) {
+    constexpr int Tile = sizeof(T) == 4 ? 16 : 8, P = Tile / 2 + 4;
+    constexpr uint32_t S = sizeof(T);
+    const int32_t n = int32_t(box.nz), h = int32_t(half_len(box.nz));
+    const uint32_t columns = box.nx * box.ny, blocks = (columns + 63) / 64;
+    const uint32_t tile = item / blocks, c = (item - tile * blocks) * 64u + (threadIdx.x & 63u);
+    const bool in = c < columns;
+    const uint32_t cc = in ? c : 0u, y = cc / box.nx;
+    const uint32_t col = (y * py + (cc - y * box.nx)) * S, plane = pz * S;
+    const auto ws = window(src), wd = window(dst);
+    const int32_t k0 = int32_t(tile) * (Tile / 2) - 2;
+    T e[P], o[P];
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const uint32_t ie = uint32_t(pair_even(k0 + j, n)), io = uint32_t(pair_odd(k0 + j, n));
+        e[j] = buf_load_at(T(0), ws, col, (Inverse ? ie : 2 * ie) * plane);
+        o[j] = buf_load_at(T(0), ws, col, (Inverse ? uint32_t(h) + io : 2 * io + 1) * plane);
+    }
+    if constexpr (Inverse) lift_inverse<T, P, true>(e, o);
+    else lift_forward<T, P>(e, o);
+    if (!in) return;
+#pragma unroll
+    for (int j = 2; j < P - 2; ++j) {
+        const uint32_t k = uint32_t(k0 + j);
+        if (2 * int32_t(k) < n) buf_store_at(e[j], wd, col, (Inverse ? 2 * k : k) * plane);
+        if (2 * int32_t(k) + 1 < n) buf_store_at(o[j], wd, col, (Inverse ? 2 * k + 1 : uint32_t(h) + k) * plane);
+    }
 }
 
 }  // namespace wz
