@@ -54,9 +54,9 @@ enum PassKind : uint8_t { kPassX = 0, kPassY = 1, kPassZ = 2, kPassCopy = 3, kPa
 enum BankId : uint8_t { kHome = 0, kTmp0 = 1, kTmp1 = 2, kOutput = 3 };
 enum JobState : uint32_t { kJobOk = 0, kJobHole = 1, kJobBad = 2 };
 // (De)quantization of a job: separate brick passes around the WZP coders, or
-// inside them for full 16^3 brick pairs (pair_bricks_fit) and for the other
-// fields of full bricks (rank_bricks_fit).
-enum JobCoder : uint32_t { kCoderSeparate = 0, kCoderPairs = 1, kCoderRanks = 2 };
+// inside them for fields of full bricks, with a z band of a power of two
+// (direct_bricks_fit; kCoderCubes: 16) or another (rank_bricks_fit).
+enum JobCoder : uint32_t { kCoderSeparate = 0, kCoderCubes = 1, kCoderRanks = 2, kCoderDirect = 3 };
 
 struct JobShape {
     Dims d;
@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(1024) batch_plan_kernel(const uint8_t* __restr
     }
 }
 
-// Chunks of the jobs that are not brick pairs (mag_pfx counts only theirs):
+// Chunks of the jobs with edge bricks (mag_pfx counts only theirs):
 // magnitudes and signs, dequantized by batch_dequant_kernel.
 __global__ void __launch_bounds__(256) batch_wzp_kernel(const uint8_t* __restrict__ packed,
                                                         const JobShape* __restrict__ shape,
@@ -245,20 +245,21 @@ __global__ void __launch_bounds__(256) batch_wzp_kernel(const uint8_t* __restric
                  MagSink{mag + sh.mag, sign + sh.sign}, status);
 }
 
-// Chunks of the brick-pair jobs (pair_pfx): decoded straight into dequantized
-// coefficients, as the single-field decoder's BrickSink does.
-template <class T>
-__global__ void __launch_bounds__(256) batch_wzp_pairs_kernel(const uint8_t* __restrict__ packed,
-                                                              const JobShape* __restrict__ shape,
-                                                              const JobRun* __restrict__ run,
-                                                              const uint32_t* __restrict__ pair_pfx, uint32_t jobs,
-                                                              T* __restrict__ home, uint32_t* status) {
-    const uint32_t j = job_of_wave(pair_pfx, jobs, blockIdx.x);
+// Chunks of the direct-brick jobs (`pfx`: those of z band 16 for Cube, of the
+// other powers of two else): decoded straight into dequantized coefficients,
+// as the single-field decoder's BrickSink does.
+template <class T, bool Cube>
+__global__ void __launch_bounds__(256) batch_wzp_direct_kernel(const uint8_t* __restrict__ packed,
+                                                               const JobShape* __restrict__ shape,
+                                                               const JobRun* __restrict__ run,
+                                                               const uint32_t* __restrict__ pfx, uint32_t jobs,
+                                                               T* __restrict__ home, uint32_t* status) {
+    const uint32_t j = job_of_wave(pfx, jobs, blockIdx.x);
     const JobRun& r = run[j];
     if (r.state != kJobOk) return;
     const JobShape& sh = shape[j];
-    decode_chunk(packed + r.arc + 32, r.wzp, sh.n, sh.chunks, sh.groups, blockIdx.x - pair_pfx[j],
-                 BrickSink<T>{home + sh.bank, sh.d.nx, sh.d.ny, T(r.quantum)}, status);
+    decode_chunk(packed + r.arc + 32, r.wzp, sh.n, sh.chunks, sh.groups, blockIdx.x - pfx[j],
+                 BrickSink<T, Cube>{home + sh.bank, DirectBricks::of(sh.d, sh.bz), T(r.quantum)}, status);
 }
 
 // Rank table sets of a plan: per distinct (geometry, z band) the packed rank
@@ -688,7 +689,7 @@ WZ_D WzpScratch job_wzp(const CompBufs& b, const JobComp& jc) {
     return WzpScratch{b.desc + jc.group0, b.staging + jc.staging, b.sizes + jc.chunk0, nullptr};
 }
 
-// Chunks of the jobs that are not brick pairs (mag_pfx counts only theirs):
+// Chunks of the jobs with edge bricks (mag_pfx counts only theirs):
 // the magnitudes and signs of batch_quantize_kernel.
 __global__ void __launch_bounds__(256) batch_encode_kernel(const JobShape* __restrict__ shape,
                                                            const JobComp* __restrict__ comp,
@@ -702,21 +703,22 @@ __global__ void __launch_bounds__(256) batch_encode_kernel(const JobShape* __res
                  &b.res[j].status);
 }
 
-// Chunks of the brick-pair jobs (pair_pfx): quantized inside the encoder, as
-// the single-field BrickSource does, with the dequantized coefficients
-// written back over the whole job for the inverse passes.
-template <class T>
-__global__ void __launch_bounds__(256) batch_encode_pairs_kernel(const JobShape* __restrict__ shape,
-                                                                 const JobComp* __restrict__ comp,
-                                                                 const uint32_t* __restrict__ pair_pfx,
-                                                                 uint32_t jobs, double quantum, CompBufs b) {
-    const uint32_t j = job_of_wave(pair_pfx, jobs, blockIdx.x);
+// Chunks of the direct-brick jobs (`pfx` as in batch_wzp_direct_kernel):
+// quantized inside the encoder, as the single-field BrickSource does, with the
+// dequantized coefficients written back over the whole job for the inverse
+// passes.
+template <class T, bool Cube>
+__global__ void __launch_bounds__(256) batch_encode_direct_kernel(const JobShape* __restrict__ shape,
+                                                                  const JobComp* __restrict__ comp,
+                                                                  const uint32_t* __restrict__ pfx, uint32_t jobs,
+                                                                  double quantum, CompBufs b) {
+    const uint32_t j = job_of_wave(pfx, jobs, blockIdx.x);
     const JobShape& sh = shape[j];
     const JobComp& jc = comp[j];
     const SideList qo{b.qbm + jc.words, b.qidx + jc.qlist, b.qval + jc.qlist, b.qcount + j, jc.qcap};
-    const BrickSource<T> src{static_cast<T*>(b.home) + sh.bank, sh.d.nx, sh.d.ny, T(quantum), T(1.0 / quantum), qo,
-                             sh.d.nx, sh.d.ny, sh.d.nz};
-    encode_chunk(src, blockIdx.x - pair_pfx[j], sh.n, sh.groups, b.out + jc.arc + 32, jc.cap - 32, job_wzp(b, jc),
+    const BrickSource<T, Cube> src{static_cast<T*>(b.home) + sh.bank, DirectBricks::of(sh.d, sh.bz), T(quantum),
+                                   T(1.0 / quantum), qo, sh.d.nx, sh.d.ny, sh.d.nz};
+    encode_chunk(src, blockIdx.x - pfx[j], sh.n, sh.groups, b.out + jc.arc + 32, jc.cap - 32, job_wzp(b, jc),
                  &b.res[j].status);
 }
 
@@ -1227,8 +1229,8 @@ struct HostPlan {
     uint32_t jobs = 0;
     std::vector<JobShape> shape;
     std::vector<uint32_t> chunk_pfx, brick_pfx;
-    // chunks of the brick-pair jobs and of the others (WZP coder launches)
-    std::vector<uint32_t> pair_pfx, rank_pfx, mag_pfx;
+    // chunks of each kind of coder's jobs (one WZP launch each)
+    std::vector<uint32_t> cube_pfx, direct_pfx, rank_pfx, mag_pfx;
     StepTables inv;                           // inverse passes
     uint64_t bank_elems = 0, mag_elems = 0, sign_words = 0, out_elems = 0;
     // compress
@@ -1352,11 +1354,12 @@ void finish_plan(HostPlan& p) {
     const uint32_t J = p.jobs;
     p.chunk_pfx.assign(J + 1, 0);
     p.brick_pfx.assign(J + 1, 0);
-    p.pair_pfx.assign(J + 1, 0);
+    p.cube_pfx.assign(J + 1, 0);
+    p.direct_pfx.assign(J + 1, 0);
     p.rank_pfx.assign(J + 1, 0);
     p.mag_pfx.assign(J + 1, 0);
     std::vector<std::vector<Pass>> sched(J);
-    uint64_t bank = 0, mag = 0, sign = 0, chunks = 0, bricks = 0, pchunks = 0, rchunks = 0, mchunks = 0;
+    uint64_t bank = 0, mag = 0, sign = 0, chunks = 0, bricks = 0, cubes = 0, dchunks = 0, rchunks = 0, mchunks = 0;
     p.rank_geo.clear();
     for (uint32_t j = 0; j < J; ++j) {
         JobShape& s = p.shape[j];
@@ -1375,17 +1378,20 @@ void finish_plan(HostPlan& p) {
         sign += (uint64_t(s.n) + 31) / 32;
         p.chunk_pfx[j] = uint32_t(chunks);
         p.brick_pfx[j] = uint32_t(bricks);
-        p.pair_pfx[j] = uint32_t(pchunks);
+        p.cube_pfx[j] = uint32_t(cubes);
+        p.direct_pfx[j] = uint32_t(dchunks);
         p.rank_pfx[j] = uint32_t(rchunks);
         p.mag_pfx[j] = uint32_t(mchunks);
         chunks += s.chunks;
         // full-brick jobs (de)quantize inside the WZP coder: no bricks in the
         // separate passes
-        s.coder = pair_bricks_fit(s.d.nx, s.d.ny, s.d.nz, s.bz)   ? kCoderPairs
+        s.coder = direct_bricks_fit(s.d.nx, s.d.ny, s.d.nz, s.bz, p.width) ? (s.bz == 16 ? kCoderCubes : kCoderDirect)
                   : rank_bricks_fit(s.d.nx, s.d.ny, s.d.nz, s.bz) ? kCoderRanks
                                                                   : kCoderSeparate;
-        if (s.coder == kCoderPairs) {
-            pchunks += s.chunks;
+        if (s.coder == kCoderCubes) {
+            cubes += s.chunks;
+        } else if (s.coder == kCoderDirect) {
+            dchunks += s.chunks;
         } else if (s.coder == kCoderRanks) {
             rchunks += s.chunks;
         } else {
@@ -1397,7 +1403,8 @@ void finish_plan(HostPlan& p) {
     if (chunks > 0x7FFFFFFFull || bricks > 0x7FFFFFFFull) throw std::invalid_argument("batch launch limit");
     p.chunk_pfx[J] = uint32_t(chunks);
     p.brick_pfx[J] = uint32_t(bricks);
-    p.pair_pfx[J] = uint32_t(pchunks);
+    p.cube_pfx[J] = uint32_t(cubes);
+    p.direct_pfx[J] = uint32_t(dchunks);
     p.rank_pfx[J] = uint32_t(rchunks);
     p.mag_pfx[J] = uint32_t(mchunks);
     p.bank_elems = bank;
@@ -1414,7 +1421,7 @@ struct DevicePlan {
     JobShape* shape = nullptr;
     JobRun* run = nullptr;
     uint32_t *chunk_pfx = nullptr, *brick_pfx = nullptr, *np_pfx = nullptr, *nq_pfx = nullptr, *status = nullptr;
-    uint32_t *pair_pfx = nullptr, *rank_pfx = nullptr, *mag_pfx = nullptr;
+    uint32_t *cube_pfx = nullptr, *direct_pfx = nullptr, *rank_pfx = nullptr, *mag_pfx = nullptr;
     struct DeviceSteps {
         Pass* pass;                     // steps x jobs
         uint32_t *pfx, *spfx, *zpfx;    // steps x (jobs + 1)
@@ -1451,7 +1458,7 @@ struct DevicePlan {
             return at;
         };
         const size_t o_shape = carve(sizeof(JobShape) * J), o_run = carve(sizeof(JobRun) * J);
-        const size_t o_pair = carve(4 * (J + 1)), o_rankp = carve(4 * (J + 1)), o_magp = carve(4 * (J + 1));
+        const size_t o_cube = carve(4 * (J + 1)), o_direct = carve(4 * (J + 1)), o_rankp = carve(4 * (J + 1)), o_magp = carve(4 * (J + 1));
         const size_t o_cp = carve(4 * (J + 1)), o_bp = carve(4 * (J + 1)), o_np = carve(4 * (J + 1)),
                      o_nq = carve(4 * (J + 1)), o_st = carve(4);
         const size_t o_comp = carve(sizeof(JobComp) * J), o_gp = carve(4 * (J + 1)), o_tp = carve(4 * (J + 1)),
@@ -1472,7 +1479,8 @@ struct DevicePlan {
         run = reinterpret_cast<JobRun*>(mem + o_run);
         chunk_pfx = reinterpret_cast<uint32_t*>(mem + o_cp);
         brick_pfx = reinterpret_cast<uint32_t*>(mem + o_bp);
-        pair_pfx = reinterpret_cast<uint32_t*>(mem + o_pair);
+        cube_pfx = reinterpret_cast<uint32_t*>(mem + o_cube);
+        direct_pfx = reinterpret_cast<uint32_t*>(mem + o_direct);
         rank_pfx = reinterpret_cast<uint32_t*>(mem + o_rankp);
         mag_pfx = reinterpret_cast<uint32_t*>(mem + o_magp);
         np_pfx = reinterpret_cast<uint32_t*>(mem + o_np);
@@ -1508,7 +1516,8 @@ struct DevicePlan {
         hip_check(hipMemcpyAsync(shape, p.shape.data(), sizeof(JobShape) * J, hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(chunk_pfx, p.chunk_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(brick_pfx, p.brick_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
-        hip_check(hipMemcpyAsync(pair_pfx, p.pair_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
+        hip_check(hipMemcpyAsync(cube_pfx, p.cube_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
+        hip_check(hipMemcpyAsync(direct_pfx, p.direct_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(rank_pfx, p.rank_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(mag_pfx, p.mag_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(comp, p.comp.data(), sizeof(JobComp) * J, hipMemcpyHostToDevice, s), "plan");
@@ -1582,15 +1591,20 @@ struct DevicePlan {
                                    fwd.pass + st * J, fwd.pfx + st * (J + 1), J, b);
             launch_step<T, false>(st, nullptr, fsb, T(0), nullptr, s);
         }
-        zero_words(b.tmp1, p.sign_words, s);  // sign words: bricks OR their edge words
-        if (p.brick_pfx[J])
+        if (p.brick_pfx[J]) {
+            zero_words(b.tmp1, p.sign_words, s);  // sign words: bricks OR their edge words
             hipLaunchKernelGGL((batch_quantize_kernel<T>), dim3(p.brick_pfx[J]), dim3(256), 0, s, shape, comp,
                                brick_pfx, J, ranks, quantum, b);
+        }
         if (p.mag_pfx[J])
             hipLaunchKernelGGL(batch_encode_kernel, dim3(p.mag_pfx[J]), dim3(256), 0, s, shape, comp, mag_pfx, J, b);
-        if (p.pair_pfx[J])
-            hipLaunchKernelGGL((batch_encode_pairs_kernel<T>), dim3(p.pair_pfx[J]), dim3(256), 0, s, shape, comp,
-                               pair_pfx, J, quantum, b);
+        if (p.cube_pfx[J])
+            hipLaunchKernelGGL((batch_encode_direct_kernel<T, true>), dim3(p.cube_pfx[J]), dim3(256), 0, s, shape,
+                               comp, cube_pfx, J, quantum, b);
+        if constexpr (sizeof(T) == 4)
+            if (p.direct_pfx[J])
+                hipLaunchKernelGGL((batch_encode_direct_kernel<T, false>), dim3(p.direct_pfx[J]), dim3(256), 0, s,
+                                   shape, comp, direct_pfx, J, quantum, b);
         if (p.rank_pfx[J])
             hipLaunchKernelGGL((batch_encode_ranks_kernel<T>), dim3(p.rank_pfx[J]), dim3(256), 0, s, shape, comp,
                                rank_pfx, J, ranks, quantum, b);
@@ -1649,9 +1663,13 @@ struct DevicePlan {
         if (p.mag_pfx[J])
             hipLaunchKernelGGL(batch_wzp_kernel, dim3(p.mag_pfx[J]), dim3(256), 0, s, packed, shape, run, mag_pfx, J,
                                static_cast<uint16_t*>(bk.tmp0), static_cast<uint32_t*>(bk.tmp1), status);
-        if (p.pair_pfx[J])
-            hipLaunchKernelGGL((batch_wzp_pairs_kernel<T>), dim3(p.pair_pfx[J]), dim3(256), 0, s, packed, shape, run,
-                               pair_pfx, J, static_cast<T*>(bk.home), status);
+        if (p.cube_pfx[J])
+            hipLaunchKernelGGL((batch_wzp_direct_kernel<T, true>), dim3(p.cube_pfx[J]), dim3(256), 0, s, packed, shape,
+                               run, cube_pfx, J, static_cast<T*>(bk.home), status);
+        if constexpr (sizeof(T) == 4)
+            if (p.direct_pfx[J])
+                hipLaunchKernelGGL((batch_wzp_direct_kernel<T, false>), dim3(p.direct_pfx[J]), dim3(256), 0, s,
+                                   packed, shape, run, direct_pfx, J, static_cast<T*>(bk.home), status);
         if (p.rank_pfx[J])
             hipLaunchKernelGGL((batch_wzp_ranks_kernel<T>), dim3(p.rank_pfx[J]), dim3(256), 0, s, packed, shape, run,
                                rank_pfx, J, ranks, static_cast<T*>(bk.home), status);

@@ -63,7 +63,7 @@ WZ_D void quantize_brick(T* __restrict__ coeff, const BrickGeometry& g, T q, T i
     constexpr uint32_t kBurst = 8;
     for (uint32_t i0 = 0; i0 < vol; i0 += kBurst * 256u) {
       T cv[kBurst];
-      uint32_t rv[kBurst];
+      uint32_t rv[kBurst], mv[kBurst], over = 0;
       uint64_t av[kBurst];
 #pragma unroll
       for (uint32_t u = 0; u < kBurst; ++u) {
@@ -78,7 +78,6 @@ WZ_D void quantize_brick(T* __restrict__ coeff, const BrickGeometry& g, T q, T i
 #pragma unroll
       for (uint32_t u = 0; u < kBurst; ++u) {
         if (i0 + u * 256u + threadIdx.x >= vol) continue;
-        const uint64_t at = av[u];
         const uint32_t r = rv[u];
         const T scaled = cv[u] * inv;
         // cpu/src/quantize_avx2.cpp:45-62: finite, |scaled| < 2^63, llrint, INT32 saturation.
@@ -87,11 +86,13 @@ WZ_D void quantize_brick(T* __restrict__ coeff, const BrickGeometry& g, T q, T i
         const bool negative = rounded < T(0);
         const T am = abs_t(rounded);
         const int32_t m = am >= T(2147483648.0) ? INT32_MAX : int32_t(am);
-        coeff[at] = m ? T(negative ? -m : m) * q : T(0);
+        coeff[av[u]] = m ? T(negative ? -m : m) * q : T(0);
         mag[k.base + r] = uint16_t(m > 65535 ? 65535 : m);
         if (negative && m) atomicOr(&bits[(r + shift) >> 5], 1u << ((r + shift) & 31u));
-        append_qoutlier(qo, m > 65535, uint32_t(at), uint32_t(m));
+        over |= uint32_t(m > 65535) << u;
+        mv[u] = uint32_t(m);
       }
+      append_qoutliers<kBurst>(qo, over, [&](int u) { return uint32_t(av[u]); }, [&](int u) { return mv[u]; });
     }
     if (bad) atomicOr(status, uint32_t(kQuantDomain));
     __syncthreads();

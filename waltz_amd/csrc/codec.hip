@@ -208,11 +208,10 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     std::lock_guard<std::mutex> guard(w.lock);
     w.init();
     // layout of the per-call scratch
-    // brick-pair fields quantize inside the encoder: no sign words to clear
-    const bool pairs = pair_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz);
-    // other fields of full bricks quantize inside the encoder too
-    const bool ranks = rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz);
-    const bool fusedq = pairs || ranks;
+    // fields of full bricks quantize inside the encoder: no sign words to clear
+    const bool direct = direct_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz, sizeof(T));
+    const bool ranks = !direct && rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz);
+    const bool fusedq = direct || ranks;
     const bool shared_words = fsegs && rsegments.cleared;  // flag words set by atomics, cleared beforehand
     auto plan = [&](Carve& c) {
         struct P {
@@ -292,9 +291,9 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     // and dequantizes the coefficients as they load: nothing written back
     const bool plane_requant = !g.dyadic && fusedq && plane_fused_fits(g.d, g.lx, g.lz, sizeof(T));
     const WriteBack wb = split || plane_requant ? kWriteNone : requant ? kWriteCoarseBox : kWriteAll;
-    if (pairs) {
+    if (direct) {
         StageClock c("quantize_encode", s);
-        quantize_encode_pairs<T>(p.coeff, g.d, quantum, qo, archive + 32, capacity - 32, wsc, status, s, wb);
+        quantize_encode_direct<T>(p.coeff, g.d, g.bz, quantum, qo, archive + 32, capacity - 32, wsc, status, s, wb);
     } else if (ranks) {
         const uint16_t* rank = w.ranks(g.d, g.bz, s);
         StageClock c("quantize_encode", s);
@@ -461,12 +460,12 @@ uint32_t decode_pass(const uint8_t* archive, const uint8_t* hdr, const Geometry&
     // the WZP directory check runs on the side stream beside the chunk decoders
     const SideStream* side = m.side(n);
     const SideJoin join{side};
-    const bool pairs = pair_bricks_fit(g.d.nx, g.d.ny, g.d.nz, bz);
-    const uint16_t* rank = pairs ? nullptr : m.ranks(g.d, bz, s);
-    const bool ranks = rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, bz) && reinterpret_cast<uintptr_t>(rank) % 8 == 0;
-    if (pairs || ranks) {
+    const bool direct = direct_bricks_fit(g.d.nx, g.d.ny, g.d.nz, bz, sizeof(T));
+    const uint16_t* rank = direct ? nullptr : m.ranks(g.d, bz, s);
+    const bool ranks = !direct && rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, bz) && reinterpret_cast<uintptr_t>(rank) % 8 == 0;
+    if (direct || ranks) {
         StageClock ck("decode_dequantize", s);
-        if (pairs) decode_dequantize_pairs<T>(archive + 32, wzp, g.d, quantum, coeff, status, s, side);
+        if (direct) decode_dequantize_direct<T>(archive + 32, wzp, g.d, bz, quantum, coeff, status, s, side);
         else decode_dequantize_ranks<T>(archive + 32, wzp, g.d, bz, rank, quantum, coeff, status, s, side);
         if (keys && side) {
             // the key table reads only the archive, and the dequantizing
@@ -544,14 +543,14 @@ uint32_t decode_planned(const uint8_t* archive, uint64_t archive_bytes, const Ge
     // levels.
     const SideStream* side = m.side(n);
     const SideJoin join{side};
-    const bool pairs = pair_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz);
-    const uint16_t* rank = pairs ? nullptr : m.ranks(g.d, g.bz, s);
-    const bool ranks = rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz) && reinterpret_cast<uintptr_t>(rank) % 8 == 0;
-    const bool keys_on_side = fold && (pairs || ranks) && side;
+    const bool direct = direct_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz, sizeof(T));
+    const uint16_t* rank = direct ? nullptr : m.ranks(g.d, g.bz, s);
+    const bool ranks = !direct && rank_bricks_fit(g.d.nx, g.d.ny, g.d.nz, g.bz) && reinterpret_cast<uintptr_t>(rank) % 8 == 0;
+    const bool keys_on_side = fold && (direct || ranks) && side;
     if (side) hip_check(hipEventRecord(side->ready, s), "event record");
-    if (pairs || ranks) {
+    if (direct || ranks) {
         StageClock ck("decode_dequantize", s);
-        if (pairs) decode_dequantize_pairs_planned<T>(archive + 32, rec, g.d, coeff, status, s);
+        if (direct) decode_dequantize_direct_planned<T>(archive + 32, rec, g.d, g.bz, coeff, status, s);
         else decode_dequantize_ranks_planned<T>(archive + 32, rec, g.d, g.bz, rank, coeff, status, s);
     } else {
         {

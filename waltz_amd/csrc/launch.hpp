@@ -88,7 +88,7 @@ void inverse_finest_level(const T* coeff, const LowBox<T>& low, T* output, Dims 
 template <class T>
 void transform_adjoint(T* data, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz, bool dyadic,
                        bool of_inverse, hipStream_t s, const T* src = nullptr);
-// The compress inverse of a brick-pair field whose coefficients stay
+// The compress inverse of a full-brick field whose coefficients stay
 // unquantized (the encoder writes nothing back), in two halves: levels >= 2
 // on a quantized and dequantized compact copy of their box (in t1), level 1
 // as a fused kernel that requantizes the high bands it loads, its
@@ -155,23 +155,37 @@ struct SideList {          // unsorted (index, payload) list + row-major flag bi
     uint32_t capacity;
 };
 
-// Appends this lane's q-outlier (row-major index g, magnitude m) when `over`,
-// with one counter atomic per wave for all of the wave's entries (thousands
-// of entries on one counter otherwise serialise); the list's order is free,
-// the archive orders it by the flag bitmap. Called by every active lane.
-WZ_D void append_qoutlier(const SideList& qo, bool over, uint32_t g, uint32_t m) {
-    const unsigned long long mask = __ballot(over);
-    if (!mask) return;
-    const uint32_t lane = __lane_id(), leader = uint32_t(__ffsll((long long)mask)) - 1u;
+// Appends this lane's q-outliers: bit i < N of `over` is one, place(i) gives its
+// row-major index and value(i) its magnitude. One counter atomic per wave for
+// all of its entries: atomics on one word from every XCD serialise, and a
+// field with many outliers (384x384x96 double fronts at REL 1e-6) spent most of
+// the quantizing encoder's 139 us on one per sample position of a wave. The
+// list's order is free, the archive orders it by the flag bitmap. Called by
+// every lane of the wave.
+template <int N, class Place, class Value>
+WZ_D void append_qoutliers(const SideList& qo, uint32_t over, Place&& place, Value&& value) {
+    if (!__ballot(over != 0)) return;
+    const uint32_t lane = __lane_id(), count = uint32_t(__builtin_popcount(over));
+    uint32_t inc = count;  // inclusive prefix over the wave
+#pragma unroll
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += t;
+    }
+    const uint32_t total = uint32_t(__builtin_amdgcn_readlane(int(inc), 63));
     uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(qo.count, uint32_t(__popcll(mask)));
-    base = uint32_t(__builtin_amdgcn_readlane(int(base), int(leader)));  // leader: wave-uniform
-    if (!over) return;
-    atomicOr(&qo.bitmap[g >> 5], 1u << (g & 31u));
-    const uint32_t slot = base + uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
-    if (slot < qo.capacity) {
-        qo.index[slot] = g;
-        static_cast<uint32_t*>(qo.payload)[slot] = m;
+    if (lane == 0) base = atomicAdd(qo.count, total);
+    uint32_t slot = uint32_t(__builtin_amdgcn_readfirstlane(int(base))) + inc - count;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if (!((over >> i) & 1u)) continue;
+        const uint32_t g = place(i);
+        atomicOr(&qo.bitmap[g >> 5], 1u << (g & 31u));
+        if (slot < qo.capacity) {
+            qo.index[slot] = g;
+            static_cast<uint32_t*>(qo.payload)[slot] = value(i);
+        }
+        ++slot;
     }
 }
 
@@ -217,24 +231,24 @@ void wzp_pack(uint32_t n, uint8_t* out, uint64_t capacity, const WzpScratch& w, 
 // caller's stream must wait for side->done before it reads the status.
 void wzp_decode(const uint8_t* in, uint64_t bytes, uint32_t n, uint16_t* mag, uint32_t* sign, uint32_t* status,
                 hipStream_t s, const SideStream* side = nullptr);
-// Paired-brick geometry only (pair_bricks_fit): quantization fused into the
-// encoder (q-outliers appended to `qo`; the dequantized coefficients written
-// back in place over the whole volume, over the coarser levels' box only, or
-// nowhere), and dequantization fused into the decoder (writes the
-// coefficient volume).
+// Fields that direct_bricks_fit takes: quantization fused into the encoder
+// (q-outliers appended to `qo`; the dequantized coefficients written back in
+// place over the whole volume, over the coarser levels' box only, or nowhere),
+// and dequantization fused into the decoder (writes the coefficient volume).
 enum WriteBack { kWriteAll, kWriteCoarseBox, kWriteNone };
 template <class T>
-void quantize_encode_pairs(T* coeff, Dims d, double quantum, SideList qo, uint8_t* out, uint64_t capacity,
-                           WzpScratch w, uint32_t* status, hipStream_t s, WriteBack wb = kWriteAll);
+void quantize_encode_direct(T* coeff, Dims d, uint32_t bz, double quantum, SideList qo, uint8_t* out,
+                            uint64_t capacity, WzpScratch w, uint32_t* status, hipStream_t s,
+                            WriteBack wb = kWriteAll);
 template <class T>
-void decode_dequantize_pairs(const uint8_t* in, uint64_t bytes, Dims d, double quantum, T* coeff, uint32_t* status,
-                             hipStream_t s, const SideStream* side = nullptr);
+void decode_dequantize_direct(const uint8_t* in, uint64_t bytes, Dims d, uint32_t bz, double quantum, T* coeff,
+                              uint32_t* status, hipStream_t s, const SideStream* side = nullptr);
 // The same two, planned on the device: stream size and quantum from `rec`
 // (nothing happens unless rec->ok); the directory check is a launch of its
 // own (wzp_directory_planned), on whichever stream the caller picks.
 template <class T>
-void decode_dequantize_pairs_planned(const uint8_t* in, const DecodeRecord* rec, Dims d, T* coeff, uint32_t* status,
-                                     hipStream_t s);
+void decode_dequantize_direct_planned(const uint8_t* in, const DecodeRecord* rec, Dims d, uint32_t bz, T* coeff,
+                                      uint32_t* status, hipStream_t s);
 void wzp_decode_planned(const uint8_t* in, const DecodeRecord* rec, uint32_t n, uint16_t* mag, uint32_t* sign,
                         uint32_t* status, hipStream_t s);
 void wzp_directory_planned(const uint8_t* in, const DecodeRecord* rec, uint32_t n, uint32_t* status, hipStream_t s);

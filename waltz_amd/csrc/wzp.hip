@@ -22,6 +22,7 @@
 // expanded under the nonzero mask. Every read is bounds-checked against the
 // stream; inconsistencies raise kCorrupt.
 #include <algorithm>
+#include <type_traits>
 
 #include "profile.hpp"
 #include "sections.hpp"
@@ -71,30 +72,41 @@ void wzp_encode(const uint16_t* mag, const uint32_t* sign, uint32_t n, uint8_t* 
                        ws.groups, out, capacity, w, status);
 }
 
-template <class T>
-void quantize_encode_pairs(T* coeff, Dims d, double quantum, SideList qo, uint8_t* out, uint64_t capacity,
-                           WzpScratch w, uint32_t* status, hipStream_t s, WriteBack wb) {
-    if (!pair_bricks_fit(d.nx, d.ny, d.nz, 16)) throw std::invalid_argument("field does not tile into brick pairs");
-    const uint32_t n = d.nx * d.ny * d.nz;
-    const WzpShape ws = wzp_shape(n);
-    const BrickSource<T> src{coeff,
-                             d.nx,
-                             d.ny,
-                             T(quantum),
-                             T(1.0 / quantum),
-                             qo,
-                             wb == kWriteNone ? 0u : wb == kWriteCoarseBox ? half_len(d.nx) : d.nx,
-                             wb == kWriteNone ? 0u : wb == kWriteCoarseBox ? half_len(d.ny) : d.ny,
-                             wb == kWriteNone ? 0u : wb == kWriteCoarseBox ? half_len(d.nz) : d.nz};
-    hipLaunchKernelGGL(wzp_encode_kernel<BrickSource<T>>, dim3(ws.chunks), dim3(kThreads), 0, s, src, n, ws.groups,
-                       out, capacity, w, status);
-}
-
 // The write-back box of a fused quantizing encoder.
 Dims writeback_box(Dims d, WriteBack wb) {
     if (wb == kWriteNone) return Dims{0, 0, 0};
     if (wb == kWriteCoarseBox) return Dims{half_len(d.nx), half_len(d.ny), half_len(d.nz)};
     return d;
+}
+
+template <class T>
+void check_direct_bricks(Dims d, uint32_t bz) {
+    if (!direct_bricks_fit(d.nx, d.ny, d.nz, bz, sizeof(T)))
+        throw std::invalid_argument("field does not tile into direct bricks");
+}
+// f(true_type) for cubes, f(false_type) for the flatter bands (float only)
+template <class T, class F>
+void of_band(uint32_t bz, F&& f) {
+    if constexpr (sizeof(T) == 4) {
+        if (bz != 16) return f(std::false_type{});
+    }
+    f(std::true_type{});
+}
+
+template <class T>
+void quantize_encode_direct(T* coeff, Dims d, uint32_t bz, double quantum, SideList qo, uint8_t* out,
+                            uint64_t capacity, WzpScratch w, uint32_t* status, hipStream_t s, WriteBack wb) {
+    check_direct_bricks<T>(d, bz);
+    const uint32_t n = d.nx * d.ny * d.nz;
+    const WzpShape ws = wzp_shape(n);
+    const Dims h = writeback_box(d, wb);
+    const DirectBricks g = DirectBricks::of(d, bz);
+    const T q = T(quantum), inv = T(1.0 / quantum);
+    of_band<T>(bz, [&](auto cube) {
+        using Source = BrickSource<T, decltype(cube)::value>;
+        hipLaunchKernelGGL((wzp_encode_kernel<Source>), dim3(ws.chunks), dim3(kThreads), 0, s,
+                           Source{coeff, g, q, inv, qo, h.nx, h.ny, h.nz}, n, ws.groups, out, capacity, w, status);
+    });
 }
 
 void check_rank_bricks(Dims d, uint32_t bz, const uint16_t* rank) {
@@ -168,14 +180,14 @@ __global__ void __launch_bounds__(kDirThreads) directory_qpatch_planned_kernel(T
         qpatch_one(coeff, idx, val, j, n, q, status);
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) wzp_decode_pairs_planned_kernel(const uint8_t* __restrict__ in,
-                                                                      const DecodeRecord* __restrict__ rec,
-                                                                      uint32_t n, uint32_t chunks, uint32_t groups,
-                                                                      T* __restrict__ coeff, uint32_t nx, uint32_t ny,
-                                                                      uint32_t* __restrict__ status) {
+template <class T, bool Cube>
+__global__ void __launch_bounds__(256) wzp_decode_direct_planned_kernel(const uint8_t* __restrict__ in,
+                                                                       const DecodeRecord* __restrict__ rec,
+                                                                       uint32_t n, uint32_t chunks, uint32_t groups,
+                                                                       T* __restrict__ coeff, DirectBricks g,
+                                                                       uint32_t* __restrict__ status) {
     if (!rec->ok) return;
-    decode_chunk(in, rec->wzp, n, chunks, groups, blockIdx.x, BrickSink<T>{coeff, nx, ny, T(rec->quantum)}, status);
+    decode_chunk(in, rec->wzp, n, chunks, groups, blockIdx.x, BrickSink<T, Cube>{coeff, g, T(rec->quantum)}, status);
 }
 
 template <class T>
@@ -214,14 +226,17 @@ void stream_decode(uint32_t n, hipStream_t s, const SideStream* side, Decoders d
 }
 
 template <class T>
-void decode_dequantize_pairs_planned(const uint8_t* in, const DecodeRecord* rec, Dims d, T* coeff, uint32_t* status,
-                                     hipStream_t s) {
-    if (!pair_bricks_fit(d.nx, d.ny, d.nz, 16)) throw std::invalid_argument("field does not tile into brick pairs");
+void decode_dequantize_direct_planned(const uint8_t* in, const DecodeRecord* rec, Dims d, uint32_t bz, T* coeff,
+                                      uint32_t* status, hipStream_t s) {
+    check_direct_bricks<T>(d, bz);
     const uint32_t n = d.nx * d.ny * d.nz;
     const WzpShape ws = wzp_shape(n);
     if (!ws.chunks) return;
-    hipLaunchKernelGGL(wzp_decode_pairs_planned_kernel<T>, dim3(ws.chunks), dim3(kThreads), 0, s, in, rec, n,
-                       ws.chunks, ws.groups, coeff, d.nx, d.ny, status);
+    const DirectBricks g = DirectBricks::of(d, bz);
+    of_band<T>(bz, [&](auto cube) {
+        hipLaunchKernelGGL((wzp_decode_direct_planned_kernel<T, decltype(cube)::value>), dim3(ws.chunks),
+                           dim3(kThreads), 0, s, in, rec, n, ws.chunks, ws.groups, coeff, g, status);
+    });
 }
 
 template <class T>
@@ -280,16 +295,20 @@ void wzp_decode(const uint8_t* in, uint64_t bytes, uint32_t n, uint16_t* mag, ui
 }
 
 template <class T>
-void decode_dequantize_pairs(const uint8_t* in, uint64_t bytes, Dims d, double quantum, T* coeff, uint32_t* status,
-                             hipStream_t s, const SideStream* side) {
-    if (!pair_bricks_fit(d.nx, d.ny, d.nz, 16)) throw std::invalid_argument("field does not tile into brick pairs");
+void decode_dequantize_direct(const uint8_t* in, uint64_t bytes, Dims d, uint32_t bz, double quantum, T* coeff,
+                              uint32_t* status, hipStream_t s, const SideStream* side) {
+    check_direct_bricks<T>(d, bz);
     const uint32_t n = d.nx * d.ny * d.nz;
     if (bytes < wzp_shape(n).header) throw std::runtime_error("WZP archive size is outside its valid bounds");
+    const DirectBricks g = DirectBricks::of(d, bz);
     stream_decode(
         n, s, side,
         [&](const WzpShape& ws) {
-            hipLaunchKernelGGL(wzp_decode_kernel<BrickSink<T>>, dim3(ws.chunks), dim3(kThreads), 0, s, in, bytes, n,
-                               ws.chunks, ws.groups, BrickSink<T>{coeff, d.nx, d.ny, T(quantum)}, status);
+            of_band<T>(bz, [&](auto cube) {
+                using Sink = BrickSink<T, decltype(cube)::value>;
+                hipLaunchKernelGGL((wzp_decode_kernel<Sink>), dim3(ws.chunks), dim3(kThreads), 0, s, in, bytes, n,
+                                   ws.chunks, ws.groups, Sink{coeff, g, T(quantum)}, status);
+            });
         },
         [&](const WzpShape& ws, hipStream_t ds) {
             hipLaunchKernelGGL(wzp_directory_kernel, dim3(1), dim3(kDirThreads), 0, ds, in, bytes, n, ws.chunks,
@@ -327,17 +346,15 @@ WZ_RANKS(float)
 WZ_RANKS(double)
 #undef WZ_RANKS
 
-template void quantize_encode_pairs<float>(float*, Dims, double, SideList, uint8_t*, uint64_t, WzpScratch, uint32_t*,
-                                           hipStream_t, WriteBack);
-template void quantize_encode_pairs<double>(double*, Dims, double, SideList, uint8_t*, uint64_t, WzpScratch,
-                                            uint32_t*, hipStream_t, WriteBack);
-template void decode_dequantize_pairs<float>(const uint8_t*, uint64_t, Dims, double, float*, uint32_t*,
-                                             hipStream_t, const SideStream*);
-template void decode_dequantize_pairs<double>(const uint8_t*, uint64_t, Dims, double, double*, uint32_t*,
-                                              hipStream_t, const SideStream*);
-template void decode_dequantize_pairs_planned<float>(const uint8_t*, const DecodeRecord*, Dims, float*, uint32_t*,
-                                                     hipStream_t);
-template void decode_dequantize_pairs_planned<double>(const uint8_t*, const DecodeRecord*, Dims, double*, uint32_t*,
-                                                      hipStream_t);
+#define WZ_DIRECT(T)                                                                                              \
+    template void quantize_encode_direct<T>(T*, Dims, uint32_t, double, SideList, uint8_t*, uint64_t, WzpScratch, \
+                                            uint32_t*, hipStream_t, WriteBack);                                   \
+    template void decode_dequantize_direct<T>(const uint8_t*, uint64_t, Dims, uint32_t, double, T*, uint32_t*,     \
+                                              hipStream_t, const SideStream*);                                    \
+    template void decode_dequantize_direct_planned<T>(const uint8_t*, const DecodeRecord*, Dims, uint32_t, T*,     \
+                                                      uint32_t*, hipStream_t);
+WZ_DIRECT(float)
+WZ_DIRECT(double)
+#undef WZ_DIRECT
 
 }  // namespace wz

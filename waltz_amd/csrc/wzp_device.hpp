@@ -103,28 +103,41 @@ struct MagSink {  // packed magnitude / sign arrays
     }
 };
 
-// Dequantizes straight into the coefficient volume (paired-brick geometry),
-// as dequantize_kernel does per sample (cpu/src/codec.cpp:146-147).
-template <class T>
+// Where the runs of a thread's sub-block lie (direct_bricks_fit geometry): the
+// four of a plane a row apart, the other four `up` samples further.
+struct DirectBricks {
+    uint32_t nx, ny, lbz, up;
+    WZ_HD static DirectBricks of(Dims d, uint32_t bz) {
+        const uint32_t l = log2_band(bz);
+        return {d.nx, d.ny, l, l >= 3 ? d.nx * d.ny : 4u};
+    }
+    WZ_D uint32_t run(uint32_t r) const { return (r & 3u) * nx + (r >> 2) * up; }
+};
+
+// Dequantizes straight into the coefficient volume (direct_bricks_fit
+// geometry; Cube: bz = 16), as dequantize_kernel does per sample
+// (cpu/src/codec.cpp:146-147).
+template <class T, bool Cube>
 struct BrickSink {
     static constexpr bool kCollective = false;
     T* coeff;
-    uint32_t nx, ny;
+    DirectBricks g;
     T q;
-    WZ_D void store(uint32_t c, uint32_t t, uint32_t, const uint32_t (&m)[32], uint32_t sw, uint32_t*) const {
+    WZ_D void store(uint32_t c, uint32_t t, uint32_t E, const uint32_t (&m)[32], uint32_t sw, uint32_t*) const {
+        if (32 * t >= E) return;  // (whole bricks: E is a multiple of 32)
         uint32_t X, Y, Z;
-        pair_subblock(nx, ny, c, t, X, Y, Z);
+        direct_subblock(g.nx, g.ny, g.lbz, c, t, X, Y, Z);
+        T* const p = coeff + (uint64_t(Z) * g.ny + Y) * g.nx + X;
 #pragma unroll
         for (uint32_t r = 0; r < 8; ++r) {
-            const uint32_t dy = r & 3u, dz = r >> 2;
             T d[4];
 #pragma unroll
             for (uint32_t dx = 0; dx < 4; ++dx) {
-                const uint32_t i = subblock_rank(dx, dy, dz);
+                const uint32_t i = direct_rank<Cube>(dx, r);
                 const T v = T(m[i]) * q;
                 d[dx] = ((sw >> i) & 1u) ? -v : v;
             }
-            store4(coeff + (uint64_t(Z + dz) * ny + (Y + dy)) * nx + X, d);
+            store4(p + g.run(r), d);
         }
     }
 };

@@ -53,37 +53,39 @@ struct MagSource {  // packed magnitude / sign arrays
     }
 };
 
-// Quantizes the coefficient volume on the fly (paired-brick geometry): reads
-// the thread's 4x4x2 sub-block, writes the dequantized coefficients back in
-// place and appends q-outliers, exactly as quantize_kernel does per sample.
-template <class T>
+// Quantizes the coefficient volume on the fly (direct_bricks_fit geometry;
+// Cube: bz = 16): reads the thread's sub-block, writes the dequantized
+// coefficients back in place and appends q-outliers, exactly as
+// quantize_kernel does per sample.
+template <class T, bool Cube>
 struct BrickSource {
     static constexpr bool kCollective = false;
     T* coeff;
-    uint32_t nx, ny;
+    DirectBricks g;
     T q, inv;
     SideList qo;
     // dequantized coefficients are written back inside [0,hx) x [0,hy) x
     // [0,hz) only: the whole volume, or the coarser levels' box when the
     // finest inverse level requantizes its high bands on load
     uint32_t hx, hy, hz;
-    WZ_D uint32_t load(uint32_t c, uint32_t t, uint32_t, uint32_t (&m)[32], uint32_t* status, uint32_t*) const {
-        uint32_t X, Y, Z;
-        pair_subblock(nx, ny, c, t, X, Y, Z);
-        uint32_t sw = 0;
+    WZ_D uint32_t load(uint32_t c, uint32_t t, uint32_t E, uint32_t (&m)[32], uint32_t* status, uint32_t*) const {
+        uint32_t sw = 0, overs = 0;
         bool bad = false;
-        // all eight rows in flight at once (the write-backs and q-outlier
+        // past the last brick (whole bricks: E is a multiple of 32): zeros
+        const bool live = 32 * t < E;
+        uint32_t X, Y, Z;
+        direct_subblock(g.nx, g.ny, g.lbz, c, live ? t : 0u, X, Y, Z);
+        const uint64_t at0 = (uint64_t(Z) * g.ny + Y) * g.nx + X;
+        // all eight runs in flight at once (the write-backs and q-outlier
         // atomics below would otherwise hold each load until the previous
-        // row is done)
+        // run is done)
         T v[8][4];
 #pragma unroll
-        for (uint32_t r = 0; r < 8; ++r)
-            load4(coeff + (uint64_t(Z + (r >> 2)) * ny + (Y + (r & 3u))) * nx + X, v[r]);
+        for (uint32_t r = 0; r < 8; ++r) load4(coeff + at0 + g.run(r), v[r]);
+        const uint32_t dz = g.lbz >= 3 ? 1u : 0u, ux = g.lbz >= 3 ? 0u : 4u;  // what `up` adds
 #pragma unroll
         for (uint32_t r = 0; r < 8; ++r) {
-            const uint32_t dy = r & 3u, dz = r >> 2;
-            const uint64_t at = (uint64_t(Z + dz) * ny + (Y + dy)) * nx + X;
-            uint32_t mv[4], over = 0;
+            const uint64_t at = at0 + g.run(r);
 #pragma unroll
             for (uint32_t dx = 0; dx < 4; ++dx) {
                 // cpu/src/quantize_avx2.cpp:45-62: finite and |scaled| < 2^63
@@ -92,32 +94,35 @@ struct BrickSource {
                 const T scaled = v[r][dx] * inv;
                 bad = bad || !(abs_t(scaled) < T(9223372036854775808.0));
                 const T rounded = rint_t(scaled);
-                const T am = abs_t(rounded);
-                mv[dx] = am >= T(2147483648.0) ? uint32_t(INT32_MAX) : uint32_t(int32_t(am));
-                const uint32_t i = subblock_rank(dx, dy, dz);
-                m[i] = mv[dx] > 65535u ? 65535u : mv[dx];
+                const uint32_t mv = magnitude(abs_t(rounded));
+                const uint32_t i = direct_rank<Cube>(dx, r);
+                m[i] = live ? (mv > 65535u ? 65535u : mv) : 0u;
                 sw |= uint32_t(rounded < T(0)) << i;
-                over |= uint32_t(mv[dx] > 65535u) << dx;
+                overs |= uint32_t(mv > 65535u) << (4 * r + dx);
             }
-            if (__ballot(over != 0)) {  // q-outliers (rare): one wave-uniform branch per row
-#pragma unroll
-                for (uint32_t dx = 0; dx < 4; ++dx)
-                    append_qoutlier(qo, (over >> dx) & 1u, uint32_t(at + dx), mv[dx]);
-            }
-            if (X < hx && Y + dy < hy && Z + dz < hz) {  // dequantized write-back inside the box
+            // dequantized write-back inside the box (a run never straddles
+            // hx: hx is 0, nx or nx / 2, multiples of 8)
+            if (live && X + (r >> 2) * ux < hx && Y + (r & 3u) < hy && Z + (r >> 2) * dz < hz) {
                 T d[4];
 #pragma unroll
                 for (uint32_t dx = 0; dx < 4; ++dx) d[dx] = requantize<T>(v[r][dx], q, inv);
                 store4(coeff + at, d);
             }
         }
-        if (bad) atomicOr(status, uint32_t(kQuantDomain));
-        return sw;
+        append_qoutliers<32>(
+            qo, live ? overs : 0u, [&](int i) { return uint32_t(at0) + g.run(uint32_t(i) / 4) + uint32_t(i) % 4; },
+            [&](int i) { return magnitude(abs_t(rint_t(v[i / 4][i % 4] * inv))); });
+        if (bad && live) atomicOr(status, uint32_t(kQuantDomain));
+        return live ? sw : 0u;
+    }
+    // llrint of a rounded magnitude, saturated at INT32_MAX
+    WZ_D static uint32_t magnitude(T am) {
+        return am >= T(2147483648.0) ? uint32_t(INT32_MAX) : uint32_t(int32_t(am));
     }
 };
 
-// Quantizes the coefficient volume of a field of full bricks on the fly
-// (rank_bricks_fit): the workgroup reads the chunk's bricks row by row (four
+// Quantizes the coefficient volume of the other fields of full bricks on the
+// fly (rank_bricks_fit): the workgroup reads the chunk's bricks row by row (four
 // x-consecutive samples per thread and step), quantizes them as
 // quantize_kernel does (write-back inside [0,hx) x [0,hy) x [0,hz) as in
 // BrickSource, q-outliers appended) and places magnitudes and sign bits at
@@ -152,13 +157,13 @@ struct RankSource {
                 rq[u] = rank_quad(g, rc, by_q, kb, f < nq ? f : 0u);
                 load4(coeff + rq[u].at, v[u]);
             }
+            uint32_t overs = 0;
 #pragma unroll
             for (uint32_t u = 0; u < kBurst; ++u) {
                 if (f0 + u * kThreads + t >= nq) continue;
                 const RankQuad& r = rq[u];
                 T d[4];
                 bool all = true;
-                uint32_t mvs[4], over = 0;
 #pragma unroll
                 for (uint32_t k = 0; k < 4; ++k) {
                     const bool in = r.j[k] < E;
@@ -168,19 +173,13 @@ struct RankSource {
                     // INT32 saturation
                     const T scaled = v[u][k] * inv;
                     const T rounded = rint_t(scaled);
-                    const T am = abs_t(rounded);
-                    const uint32_t mv = am >= T(2147483648.0) ? uint32_t(INT32_MAX) : uint32_t(int32_t(am));
-                    mvs[k] = mv;
+                    const uint32_t mv = magnitude(abs_t(rounded));
                     d[k] = requantize<T>(v[u][k], q, inv);
                     if (!in) continue;
-                    over |= uint32_t(mv > 65535u) << k;
+                    overs |= uint32_t(mv > 65535u) << (4 * u + k);
                     bad = bad || !(abs_t(scaled) < T(9223372036854775808.0));
                     mg[r.j[k]] = uint16_t(mv > 65535u ? 65535u : mv);
                     if (rounded < T(0)) atomicOr(&sg[r.j[k] >> 5], 1u << (r.j[k] & 31u));
-                }
-                if (__ballot(over != 0)) {  // q-outliers (rare): one wave-uniform branch per quad
-#pragma unroll
-                    for (uint32_t k = 0; k < 4; ++k) append_qoutlier(qo, (over >> k) & 1u, r.at + k, mvs[k]);
                 }
                 // dequantized write-back inside the box (a quad never
                 // straddles hx: hx is 0, nx or nx / 2, multiples of 8)
@@ -196,6 +195,9 @@ struct RankSource {
                     }
                 }
             }
+            append_qoutliers<4 * kBurst>(
+                qo, overs, [&](int i) { return rq[i / 4].at + uint32_t(i) % 4; },
+                [&](int i) { return magnitude(abs_t(rint_t(v[i / 4][i % 4] * inv))); });
         }
         __syncthreads();
         const uint32_t first = 32u * t;
@@ -214,6 +216,10 @@ struct RankSource {
         __syncthreads();  // the buffer is free again for the caller
         if (bad) atomicOr(status, uint32_t(kQuantDomain));
         return sw;
+    }
+    // llrint of a rounded magnitude, saturated at INT32_MAX
+    WZ_D static uint32_t magnitude(T am) {
+        return am >= T(2147483648.0) ? uint32_t(INT32_MAX) : uint32_t(int32_t(am));
     }
 };
 
