@@ -128,13 +128,12 @@ void autotune(Dims full, hipStream_t s) {
         hip_check(hipStreamSynchronize(s), "autotune");
         return;
     }
-    const Tuning base = heuristic_tuning(full, lxy);
     DeviceBuffer in(n * sizeof(T)), coeff(n * sizeof(T)), low(n * sizeof(T));
     hipLaunchKernelGGL((tune_fill<T>), dim3(uint32_t((n + 255) / 256)), dim3(256), 0, s, static_cast<T*>(in.p), n);
     hipLaunchKernelGGL((tune_fill<T>), dim3(uint32_t((n + 255) / 256)), dim3(256), 0, s, static_cast<T*>(coeff.p), n);
     hipLaunchKernelGGL((tune_fill<T>), dim3(uint32_t((n + 255) / 256)), dim3(256), 0, s, static_cast<T*>(low.p), n);
     Timer timer;
-    Tuning fw = base, iv = base;
+    Tuning fw = heuristic_tuning(full, lxy, sizeof(T), false), iv = heuristic_tuning(full, lxy, sizeof(T), true);
     Dims box = full;
     for (unsigned l = 0; l < lxy; ++l) {
         const Dims h{half_len(box.nx), half_len(box.ny), half_len(box.nz)};
@@ -186,7 +185,7 @@ void autotune(Dims full, hipStream_t s) {
     T* const t0 = static_cast<T*>(low.p);
     T* const t1 = static_cast<T*>(spare.p);
     float best_f = 1e30f, best_i = 1e30f;
-    unsigned fuse_f = base.fused, fuse_i = base.fused;
+    unsigned fuse_f = fw.fused, fuse_i = iv.fused;
     for (unsigned f = 0; f <= lxy; ++f) {
         Tuning tf = fw, ti = iv;
         tf.fused = ti.fused = f;

@@ -846,15 +846,8 @@ uint32_t repair_z_segment(Dims n, uint32_t tuned) {
     int dev = 0, cus = 0;
     hip_check(hipGetDevice(&dev), "device");
     hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "CU count");
-    const uint64_t resident = uint64_t(cus) * per_cu;
-    const uint32_t top = (n.nz + 15) & ~15u;
-    uint32_t sz = tuned;
-    auto tiles = [&](uint32_t z) {
-        const Dims g = tile_grid(n, z);
-        return uint64_t(g.nx) * g.ny * g.nz;
-    };
-    while (sz < top && tiles(sz) > resident) sz = sz * 2 < top ? sz * 2 : top;
-    return sz;
+    if (inv_segments(n, tuned) <= uint64_t(cus) * per_cu) return tuned;
+    return best_z_segment(n, uint32_t(cus), per_cu, per_cu);
 }
 
 template uint32_t repair_z_segment<float>(Dims, uint32_t);

@@ -67,9 +67,33 @@ template <class T>
 void launch_fwd_level(const FwdLevel<T>& a, hipStream_t s);
 template <class T>
 void launch_inv_level(const InvLevel<T>& a, hipStream_t s);
+// z segment (a multiple of 16) of the least estimated time over up to `most`
+// workgroups per CU, of which `per_cu` run at once. A workgroup streams sz
+// planes and 8 of halo, and the level lasts as long as its busiest CU: about
+// (sz + 8) times its workgroups, one that runs alone counting 1.2 (nothing
+// hides its waits). Against "about 1024 workgroups", the finest level (us):
+// forward 512^3 f32 337 -> 275 (1024 workgroups are three at once and then
+// one, 512 are two at once), 320^3 f32 107 -> 80, 448x384x400 f32 282 -> 240,
+// 320x256x384 f64 181 -> 150.
+inline uint32_t best_z_segment(Dims n, uint32_t cus, uint32_t per_cu, uint32_t most) {
+    const uint64_t tiles = uint64_t((n.nx + 63) / 64) * ((n.ny + 31) / 32);
+    uint32_t best = 0;
+    double least = 0;
+    for (uint32_t c = most; c; --c) {  // ties: more workgroups
+        const uint64_t segs = std::max<uint64_t>(uint64_t(c) * cus / tiles, 1);
+        const uint32_t sz = uint32_t(((n.nz + segs - 1) / segs + 15) & ~uint64_t(15));
+        const uint64_t per = (tiles * ((n.nz + sz - 1) / sz) + cus - 1) / cus;
+        const double cost = (double(sz) + 8) * (double(per) + (per_cu > 1 && per % per_cu == 1 ? 0.2 : 0.0));
+        if (!best || cost < least) {
+            best = sz;
+            least = cost;
+        }
+    }
+    return best;
+}
 // z segment of the finest level's repair emitter for box n: the tuned segment,
-// doubled while the tiles outnumber the workgroups the device holds at once
-// (a multiple of 16 either way)
+// or, where its tiles outnumber the workgroups the device holds at once, the
+// best of those whose tiles do not
 template <class T>
 uint32_t repair_z_segment(Dims n, uint32_t tuned);
 

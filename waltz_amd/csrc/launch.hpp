@@ -130,7 +130,7 @@ struct Tuning {
     uint32_t pair_max;
 };
 Tuning tuning_for(Dims full, unsigned lxy, unsigned width, bool inverse);
-Tuning heuristic_tuning(Dims full, unsigned lxy);
+Tuning heuristic_tuning(Dims full, unsigned lxy, unsigned width, bool inverse);
 void set_tuning(Dims full, unsigned width, bool inverse, const Tuning& t);
 void clear_tuning();
 std::string tuning_report();

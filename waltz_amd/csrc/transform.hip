@@ -606,17 +606,6 @@ struct Passes {
 
 // ------------------------------------------------------------------ fused dyadic schedule
 namespace {
-// z segment per workgroup: enough segments for ~1024 workgroups, a multiple of
-// 16 (the canonical f32 inverse Z tile, and twice the f64 one). Bit-neutral.
-uint32_t z_segment(Dims n) {
-    const uint64_t tiles = uint64_t((n.nx + 63) / 64) * ((n.ny + 31) / 32);
-    uint64_t segs = (1024 + tiles - 1) / tiles;
-    if (segs < 1) segs = 1;
-    uint64_t sz = (n.nz + segs - 1) / segs;
-    sz = (sz + 15) & ~uint64_t(15);
-    return uint32_t(sz < 16 ? 16 : sz);
-}
-
 // Leading levels whose box fills the GPU with fused workgroups (>= 512 of
 // them at the smallest z segment); coarser boxes are cheaper as axis passes.
 unsigned fused_levels(Dims n, unsigned levels) {
@@ -643,14 +632,19 @@ struct TuneKey {
 std::mutex g_tune_mu;
 std::map<TuneKey, Tuning> g_tune;
 
-Tuning heuristic_impl(Dims full, unsigned lxy) {
+// Workgroups of a fused level that share a CU (LDS: 42 KiB forward, 44-61 KiB
+// inverse in float, twice that in double); constants, so that the choice needs
+// no device.
+Tuning heuristic_impl(Dims full, unsigned lxy, unsigned width, bool inverse) {
+    constexpr uint32_t kCus = 256;
+    const uint32_t per_cu = width == 8 ? 1 : inverse ? 2 : 3;
     Tuning t{};
     t.fused = fused_levels(full, lxy);
     t.tile[0] = t.tile[1] = t.tile[2] = 8;
     t.pair_max = 1024;
     Dims n = full;
     for (unsigned l = 0; l < 5; ++l) {
-        t.sz[l] = z_segment(n);
+        t.sz[l] = best_z_segment(n, kCus, per_cu, 8);
         n = shrink(n, true, true);
     }
     return t;
@@ -669,13 +663,15 @@ T* low_box(T* scratch, Dims full, unsigned l) {
 Tuning tuning_for(Dims full, unsigned lxy, unsigned width, bool inverse) {
     std::lock_guard<std::mutex> g(g_tune_mu);
     const auto it = g_tune.find(TuneKey{full.nx, full.ny, full.nz, width, inverse ? 1u : 0u});
-    Tuning t = it != g_tune.end() ? it->second : heuristic_impl(full, lxy);
+    Tuning t = it != g_tune.end() ? it->second : heuristic_impl(full, lxy, width, inverse);
     if (t.fused > lxy) t.fused = lxy;
     if (!fused_plane_fits(full.nx, full.ny, width)) t.fused = 0;  // planes of 4 GiB and more: axis passes
     return t;
 }
 
-Tuning heuristic_tuning(Dims full, unsigned lxy) { return heuristic_impl(full, lxy); }
+Tuning heuristic_tuning(Dims full, unsigned lxy, unsigned width, bool inverse) {
+    return heuristic_impl(full, lxy, width, inverse);
+}
 
 void clear_tuning() {
     std::lock_guard<std::mutex> g(g_tune_mu);
