@@ -138,16 +138,24 @@ WZ_D uint32_t bitmap_words(const unsigned long long (&m)[8], std::integer_sequen
     return v;
 }
 
-// Four consecutive staged values to a 16-byte aligned destination.
-// (non-temporal, see buf_store_nt)
-WZ_D void store_vec4(float* dst, const float* v) {
+// Four consecutive staged values to a 16-byte aligned destination,
+// non-temporal (see buf_store_nt) or not.
+WZ_D void store_vec4(float* dst, const float* v, bool nt) {
     using F4 = float __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(*reinterpret_cast<const F4*>(v), reinterpret_cast<F4*>(dst));
+    const F4 x = *reinterpret_cast<const F4*>(v);
+    if (nt) __builtin_nontemporal_store(x, reinterpret_cast<F4*>(dst));
+    else *reinterpret_cast<F4*>(dst) = x;
 }
-WZ_D void store_vec4(double* dst, const double* v) {
+WZ_D void store_vec4(double* dst, const double* v, bool nt) {
     using D2 = double __attribute__((ext_vector_type(2)));
-    __builtin_nontemporal_store(reinterpret_cast<const D2*>(v)[0], reinterpret_cast<D2*>(dst));
-    __builtin_nontemporal_store(reinterpret_cast<const D2*>(v)[1], reinterpret_cast<D2*>(dst) + 1);
+    const D2 x = reinterpret_cast<const D2*>(v)[0], y = reinterpret_cast<const D2*>(v)[1];
+    if (nt) {
+        __builtin_nontemporal_store(x, reinterpret_cast<D2*>(dst));
+        __builtin_nontemporal_store(y, reinterpret_cast<D2*>(dst) + 1);
+    } else {
+        reinterpret_cast<D2*>(dst)[0] = x;
+        reinterpret_cast<D2*>(dst)[1] = y;
+    }
 }
 
 }  // namespace
@@ -162,12 +170,14 @@ WZ_D void store_vec4(double* dst, const double* v) {
 //   4. Z: 512 threads each stream 4 columns of a row through the Z lifting
 //      pipeline (five registers per column) and stage the two z bands of the
 //      finished pair in C (aliasing B);
-//   5. the staged rows are written with 16-byte stores: the LLL band to the
-//      next level's box, the seven other bands to the coefficient volume.
+//   5. the staged rows are written (16-byte stores, or one sample a thread
+//      where rows are not 16-byte aligned): the LLL band to the next level's
+//      box, the seven other bands to the coefficient volume.
 constexpr int CP = TX + 4;             // row pitch of the X and C stages (16-byte rows)
 
 template <class T>
-__global__ void __launch_bounds__(FT) fwd_level_kernel(FwdLevel<T> a) {
+// (seven waves per SIMD in float: three workgroups per CU)
+__global__ void __launch_bounds__(FT, sizeof(T) == 4 ? 7 : 1) fwd_level_kernel(FwdLevel<T> a) {
     constexpr int ASZ = 2 * FH * PA, BSZ = 2 * TY * PA;
     static_assert(2 * TY * CP <= ASZ && 2 * TY * CP <= BSZ, "stage aliasing");
     __shared__ __attribute__((aligned(16))) T A[ASZ];  // two input planes; then X results [plane][row][CP]
@@ -197,9 +207,12 @@ __global__ void __launch_bounds__(FT) fwd_level_kernel(FwdLevel<T> a) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) E[k] = O[k] = O1[k] = E2[k] = O3[k] = T(0);
 
-    // 16-byte stores need 4-aligned rows and band offsets in both destinations
-    const bool vec_hi = (a.hpy & 3u) == 0 && (a.hpz & 3u) == 0 && (hx & 3u) == 0;
-    const bool vec_lo = (a.lpy & 3u) == 0 && (a.lpz & 3u) == 0;
+    // 16-byte stores need 4-aligned rows and band offsets in both destinations,
+    // else a wave stores two 32-sample runs a time; non-temporal ones pay where
+    // the runs are whole lines, elsewhere L2 merges neighbouring tiles' pieces
+    // (f32: 448x384x400 234 -> 178 us, 311x405x287 393 -> 147)
+    const uint32_t rows = uint32_t(a.hpy | a.hpz | a.lpy | a.lpz) | hx;
+    const bool quads = (rows & 3u) == 0, lines = (rows & 31u) == 0;
 
     const int npairs = int(a.sz / 2) + 4;
     // the two planes of the next step are in flight while this step runs
@@ -298,8 +311,24 @@ __global__ void __launch_bounds__(FT) fwd_level_kernel(FwdLevel<T> a) {
         }
         __syncthreads();  // X (in A) consumed; C (in B) complete
         if (i < 4) continue;
-        // 5. rows of the finished pair: 64 rows (z band, y row) x 16 groups of 4
         const uint32_t iz = z0 / 2 + uint32_t(i - 4);
+        if (!quads) {  // 5a. 64 rows (z band, y row) x 64 samples, one per thread
+            for (uint32_t w = t; w < 2 * TY * TX; w += FT) {
+                const uint32_t row = w / TX, c = w % TX;
+                const uint32_t zb = row / TY, rr = row % TY, yb = rr >> 4, iy = y0 / 2 + (rr & 15u);
+                const uint32_t xb = c >> 5, ix = x0 / 2 + (c & 31u);
+                if (!(zb ? 2 * iz + 1 < n.nz : 2 * iz < n.nz) || !(yb ? 2 * iy + 1 < n.ny : 2 * iy < n.ny) ||
+                    2 * ix + xb >= n.nx)
+                    continue;
+                const T v = Cs[row * CP + c];
+                if (xb | yb | zb)
+                    a.hi[uint64_t(zb ? hz + iz : iz) * a.hpz + uint64_t(yb ? hy + iy : iy) * a.hpy + (xb ? hx + ix : ix)] = v;
+                else
+                    a.lo[uint64_t(iz) * a.lpz + uint64_t(iy) * a.lpy + ix] = v;
+            }
+            continue;
+        }
+        // 5b. 64 rows x 16 groups of 4
         for (uint32_t w = t; w < 2 * TY * 16; w += FT) {
             const uint32_t row = w >> 4, q = w & 15u;
             const uint32_t zb = row / TY, rr = row % TY, yb = rr >> 4, iy = y0 / 2 + (rr & 15u);
@@ -316,12 +345,12 @@ __global__ void __launch_bounds__(FT) fwd_level_kernel(FwdLevel<T> a) {
             }
             // samples 2*ix+xb .. of the level box exist up to nx
             const bool full = 2 * (ix + 3) + xb < n.nx;
-            if (full && (low ? vec_lo : vec_hi)) {
-                store_vec4(dst, v);
+            if (full) {
+                store_vec4(dst, v, lines);
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    if (2 * (ix + k) + xb < n.nx) __builtin_nontemporal_store(v[k], dst + k);
+                    if (2 * (ix + k) + xb < n.nx) dst[k] = v[k];
             }
         }
     }
