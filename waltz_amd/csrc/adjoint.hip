@@ -19,9 +19,22 @@
 // tile's 16-sample neighbourhood), with no barrier between the updates.
 //
 // The adjoint of a multi-level transform runs the transposed passes in the
-// reverse order of the transform's schedule.
+// reverse order of the transform's schedule. Each level is one XY launch (the
+// strips of the transforms, Adjoint) and one Z launch, each reading and
+// writing its box once; low boxes move on in compact copies, so no level is
+// copied back. Against a pass per axis through LDS (and, on small planes, one
+// for X and Y with a halo of 2.4 times its outputs), IDWT^T / DWT^T:
+// 256^3 float 199 -> 112 / 234 -> 132 us, double 439 -> 186 / 508 -> 208;
+// 203x150x61 double 142 -> 62 / 159 -> 69. Memory bounds the finest level,
+// launches the coarse ones. The passes per axis (adjoint_pass) are left for
+// lines of one sample and planes past a 32-bit window.
+#include <algorithm>
+
 #include "common.hpp"
+#include "fused.hpp"
 #include "launch.hpp"
+#include "lifting.hpp"
+#include "xystrip.hpp"
 
 namespace wz {
 namespace {
@@ -164,91 +177,6 @@ __global__ void __launch_bounds__(256) adjoint_pass(const T* __restrict__ src, T
     }
 }
 
-// The transposes of the inverse's X and Y passes (Y^T, then X^T) of one z
-// plane in one launch: a workgroup owns 64 x 32 outputs (natural positions
-// [x0, x0 + 64) x [y0, y0 + 32)) and stages the zero-extended input window
-// [x0 - 12, x0 + 76) x [y0 - 12, y0 + 44) in LDS. Y^T runs as 8-sample
-// register tiles on all 88 columns of rows [y0 - 8, y0 + 40), its fold gives
-// rows [y0, y0 + 32) (columns outside the box stay zero, as X^T's
-// zero extension needs), X^T then runs on those rows over [x0 - 8, x0 + 72),
-// and its fold writes the outputs at their split positions in both axes.
-// Each value is the same sequence of operations as in the two separate
-// passes. Lines of at least 9 samples (the fold of adjoint_pass's long-line
-// case).
-constexpr int kXYOx = 64, kXYOy = 32;                 // outputs per tile
-constexpr int kXYWx = kXYOx + 24, kXYWy = kXYOy + 24;  // input window
-template <class T>
-__global__ void __launch_bounds__(256) adjoint_xy_kernel(const T* __restrict__ src, T* __restrict__ dst, Dims full,
-                                                         Dims act, uint32_t tx, uint32_t ty) {
-    __shared__ T A[kXYWy][kXYWx + 1];      // window; then the Y-folded rows (rows 0..31)
-    __shared__ T B[kXYOy + 16][kXYWx + 1];  // Y^T results of rows [y0 - 8, y0 + 40); then X^T results
-    using C = Lift<T>;
-    const uint32_t bx = blockIdx.x % tx, rest = blockIdx.x / tx, by = rest % ty, z = rest / ty;
-    const int32_t x0 = int32_t(bx) * kXYOx, y0 = int32_t(by) * kXYOy;
-    const int32_t nx = int32_t(act.nx), ny = int32_t(act.ny);
-    const uint64_t plane = uint64_t(full.nx) * full.ny;
-    const T* sp = src + uint64_t(z) * plane;
-    const uint32_t t = threadIdx.x;
-    for (uint32_t w = t; w < uint32_t(kXYWy * kXYWx); w += 256) {
-        const int32_t i = int32_t(w / kXYWx), j = int32_t(w % kXYWx), y = y0 - 12 + i, x = x0 - 12 + j;
-        A[i][j] = y >= 0 && y < ny && x >= 0 && x < nx ? sp[uint64_t(y) * full.nx + uint32_t(x)] : T(0);
-    }
-    __syncthreads();
-    // Y^T: column j, tile k -> rows [y0 - 8 + 8k, +8) from rows [y0 - 12 + 8k, +16)
-    for (uint32_t w = t; w < uint32_t(6 * kXYWx); w += 256) {
-        const uint32_t j = w % kXYWx, k = w / kXYWx;
-        tile_transposed<T, true>(&A[8 * k][j], &B[8 * k][j], kXYWx + 1, kXYWx + 1);
-    }
-    __syncthreads();
-    for (uint32_t w = t; w < uint32_t(kXYOy * kXYWx); w += 256) {
-        const int32_t i = int32_t(w / kXYWx), j = int32_t(w % kXYWx), p = y0 + i;
-        T v = T(0);
-        if (p < ny) {
-            auto u = [&](int32_t q) { return B[q - y0 + 8][j]; };
-            v = u(p);
-            if (p >= 1 && p <= 4) v += u(-p);
-            const int32_t m = 2 * ny - 2 - p;
-            if (m != p && m < ny + 4) v += u(m);
-            v = (p & 1) ? v * (-C::k) : v * C::ik;
-        }
-        A[i][j] = v;
-    }
-    __syncthreads();
-    // X^T: row i, tile k -> columns [x0 - 8 + 8k, +8) from [x0 - 12 + 8k, +16)
-    for (uint32_t w = t; w < uint32_t(10 * kXYOy); w += 256) {
-        const uint32_t i = w % kXYOy, k = w / kXYOy;
-        tile_transposed<T, true>(&A[i][8 * k], &B[i][8 * k]);
-    }
-    __syncthreads();
-    T* dp = dst + uint64_t(z) * plane;
-    for (uint32_t w = t; w < uint32_t(kXYOy * kXYOx); w += 256) {
-        const int32_t i = int32_t(w / kXYOx), x = x0 + int32_t(w % kXYOx), p = y0 + i;
-        if (x >= nx || p >= ny) continue;
-        auto u = [&](int32_t q) { return B[i][q - x0 + 8]; };
-        T v = u(x);
-        if (x >= 1 && x <= 4) v += u(-x);
-        const int32_t m = 2 * nx - 2 - x;
-        if (m != x && m < nx + 4) v += u(m);
-        v = (x & 1) ? v * (-C::k) : v * C::ik;
-        dp[uint64_t(split_index(uint32_t(p), act.ny)) * full.nx + split_index(uint32_t(x), act.nx)] = v;
-    }
-}
-
-// Only for planes up to 128 x 128: there the launch saved beats the halo
-// (each workgroup stages 2.4x its outputs); on a 256 x 256 plane the two
-// passes took 82 µs and the joint launch 100 µs.
-bool adjoint_xy_fits(Dims act) {
-    return act.nx >= 9 && act.ny >= 9 && act.nz && uint64_t(act.nx) * act.ny <= 128u * 128u;
-}
-
-template <class T>
-void launch_adjoint_xy(const T* src, T* dst, Dims full, Dims act, hipStream_t s) {
-    const uint32_t tx = (act.nx + kXYOx - 1) / kXYOx, ty = (act.ny + kXYOy - 1) / kXYOy;
-    const uint64_t blocks = uint64_t(tx) * ty * act.nz;
-    check_launch_size(blocks * 256);
-    hipLaunchKernelGGL((adjoint_xy_kernel<T>), dim3(uint32_t(blocks)), dim3(256), 0, s, src, dst, full, act, tx, ty);
-}
-
 Dims shrink_box(Dims d, bool xy, bool z) {
     if (xy) {
         d.nx = half_len(d.nx);
@@ -290,6 +218,258 @@ __global__ void __launch_bounds__(256) adjoint_copy(const T* __restrict__ src, T
     dst[at] = src[at];
 }
 
+// ------------------------------------------------------------------ levels in registers
+// OfInverse: the transpose of the inverse's level (natural -> split), else of
+// the forward's (split -> natural).
+template <class T, bool OfInverse>
+__global__ void __launch_bounds__(kStripThreads) adjoint_xy_kernel(std::conditional_t<OfInverse, XYForward<T>,
+                                                                                      XYInverse<T>> a, StripPlan p) {
+    uint32_t item;
+    if (!strip_of_wave(p, item)) return;
+    if constexpr (OfInverse) strip_forward<T, true>(a, p, item);
+    else strip_inverse<T, false, true>(a, p, item, StripStore<T>{});
+}
+
+// One Z level of a box. `nat`: its samples along z; `lo`: the low planes of
+// the columns x < lx, y < ly; `hi`: everything else of the split.
+template <class T>
+struct ZLevel {
+    T* nat;  // read by OfInverse, else written; the other two the other way round
+    uint64_t npy, npz;
+    T* hi;
+    uint64_t hpy, hpz;
+    T* lo;
+    uint64_t lpy, lpz;
+    Dims n;
+    uint32_t lx, ly;
+    uint32_t sz, groups, items;  // planes of a segment, waves per segment, waves
+};
+
+// A lane streams one column of the box (columns counted row by row), two
+// planes a step, as the strips stream rows; ends weighted as there.
+template <class T, bool OfInverse>
+__global__ void __launch_bounds__(256) adjoint_z_kernel(ZLevel<T> a) {
+    using C = Lift<T>;
+    constexpr uint32_t S = sizeof(T);
+    const uint32_t per = ((a.items + 3) / 4 + 7) / 8;
+    const uint32_t item = 4 * ((blockIdx.x & 7u) * per + (blockIdx.x >> 3)) +
+                          __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (item >= a.items || (blockIdx.x >> 3) >= per) return;
+    const uint32_t seg = item / a.groups, c = (item - seg * a.groups) * 64u + (threadIdx.x & 63u);
+    const Dims n = a.n;
+    const int32_t nz = int32_t(n.nz);
+    const uint32_t hz = half_len(n.nz);
+    const bool live = c < n.nx * n.ny;
+    const uint32_t y = live ? c / n.nx : 0u, x = live ? c - y * n.nx : 0u;
+    const bool low = x < a.lx && y < a.ly;
+    // one plane's windows; lanes outside go past their range (loads 0, stores
+    // dropped)
+    const uint32_t nr = ((n.ny - 1u) * uint32_t(a.npy) + n.nx) * S, hr = ((n.ny - 1u) * uint32_t(a.hpy) + n.nx) * S;
+    const uint32_t lr = ((a.ly - 1u) * uint32_t(a.lpy) + a.lx) * S;
+    auto natural = [&](T* p, uint32_t z) { return window_n(p + uint64_t(z) * a.npz, nr); };
+    auto high = [&](T* p, uint32_t z) { return window_n(p + uint64_t(z) * a.hpz, hr); };
+    auto lower = [&](T* p, uint32_t z) { return window_n(p + uint64_t(z) * a.lpz, lr); };
+    const uint32_t nv = live ? (y * uint32_t(a.npy) + x) * S : kOutside;
+    const uint32_t hv = live ? (y * uint32_t(a.hpy) + x) * S : kOutside;
+    const uint32_t lv = live && low ? (y * uint32_t(a.lpy) + x) * S : kOutside;
+    const uint32_t hl = low ? kOutside : hv;  // this column's low planes in `hi`
+    const bool some = __ballot(live && !low) != 0;
+    const uint32_t zs = seg * a.sz, blocks = (min(a.sz, n.nz - zs) + 7) / 8;
+    auto load = [&](int32_t g, T (&v)[2]) {
+        const uint32_t pe = uint32_t(pair_even(g, nz)), po = uint32_t(pair_odd(g, nz));
+        if constexpr (OfInverse) {
+            v[0] = buf_load<T>(natural(a.nat, 2 * pe), nv);
+            v[1] = buf_load<T>(natural(a.nat, 2 * po + 1), nv);
+        } else {
+            v[0] = buf_load<T>(lower(a.lo, pe), lv);
+            if (some) {
+                const T h = buf_load<T>(high(a.hi, pe), hl);
+                v[0] = low ? v[0] : h;
+            }
+            v[1] = buf_load<T>(high(a.hi, hz + po), hv);
+        }
+    };
+    T s0 = T(0), s1 = T(0), s2 = T(0), s3 = T(0), s4 = T(0);  // the pipeline's states
+    T buf[4][2];
+    int32_t g = int32_t(zs / 2) - 2;
+    load(g, buf[0]);
+    load(g + 1, buf[1]);
+    load(g + 2, buf[2]);
+    auto block = [&](bool emit) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u, ++g) {
+            load(g + 3, buf[(u + 3) & 3]);
+            const T we = end_load<T>(2 * uint32_t(pair_even(g, nz)), n.nz);
+            const T wo = end_load<T>(2 * uint32_t(pair_odd(g, nz)) + 1u, n.nz);
+            const uint32_t k = uint32_t(g - 2);
+            const T ve = end_store<T>(2 * k, n.nz), vo = end_store<T>(2 * k + 1u, n.nz);
+            const T e = buf[u][0] * we, o = buf[u][1] * wo;
+            T r0, r1;  // pair g - 2
+            if constexpr (OfInverse) {
+                const T e1 = fmadd(-C::a, s0 + o, e);
+                const T o1 = fmadd(-C::b, s1 + e1, s0);
+                const T e2 = fmadd(-C::g, s2 + o1, s1);
+                r0 = s3 * (C::ik * ve);
+                r1 = fmadd(-C::d, s3 + e2, s2) * (-C::k * vo);
+                s0 = o;
+                s1 = e1;
+                s2 = o1;
+                s3 = e2;
+            } else {
+                const T ev = e * C::k, ov = o * (-C::ik);
+                const T o1 = fmadd(C::d, s4 + ev, s0);
+                const T e1 = fmadd(C::g, s1 + o1, s4);
+                const T o2 = fmadd(C::b, s2 + e1, s1);
+                r0 = fmadd(C::a, s3 + o2, s2) * ve;
+                r1 = o2 * vo;
+                s4 = ev;
+                s0 = ov;
+                s1 = o1;
+                s2 = e1;
+                s3 = o2;
+            }
+            if (!emit) continue;
+            if constexpr (OfInverse) {
+                if (2 * k < n.nz) {
+                    buf_store(r0, lower(a.lo, k), lv);
+                    if (some) buf_store(r0, high(a.hi, k), hl);
+                }
+                if (2 * k + 1 < n.nz) buf_store(r1, high(a.hi, hz + k), hv);
+            } else {
+                if (2 * k < n.nz) buf_store(r0, natural(a.nat, 2 * k), nv);
+                if (2 * k + 1 < n.nz) buf_store(r1, natural(a.nat, 2 * k + 1), nv);
+            }
+        }
+    };
+    block(false);
+    for (uint32_t b = 0; b < blocks; ++b) block(true);
+}
+
+// A box and where it lies.
+template <class T>
+struct Box {
+    T* p;
+    uint64_t py, pz;
+};
+template <class T>
+Box<T> volume(T* p, Dims full) { return {p, full.nx, uint64_t(full.nx) * full.ny}; }
+template <class T>
+Box<T> compact(T* p, Dims n) { return {p, n.nx, uint64_t(n.nx) * n.ny}; }
+
+// in: the samples' gradient (OfInverse) or the split one, its low box `lo`
+template <class T, bool OfInverse>
+void xy_level(Box<T> in, Box<T> lo, Box<T> out, Dims n, hipStream_t s) {
+    const StripPlan p = strip_plan(n, strips_pack(std::max({in.pz, lo.pz, out.pz}), sizeof(T)));
+    const dim3 grid(strip_blocks(p)), block(kStripThreads);
+    if constexpr (OfInverse) {
+        const XYForward<T> a{in.p, in.py, in.pz, out.p, out.py, out.pz, lo.p, lo.py, lo.pz, n, nullptr};
+        hipLaunchKernelGGL((adjoint_xy_kernel<T, true>), grid, block, 0, s, a, p);
+    } else {
+        const XYInverse<T> a{in.p, in.py, in.pz, lo.p, lo.py, lo.pz, out.p, out.py, out.pz, n, T(0), T(0), 0u};
+        hipLaunchKernelGGL((adjoint_xy_kernel<T, false>), grid, block, 0, s, a, p);
+    }
+}
+// nat: the samples along z; hi, lo: the split and its low box of lx x ly columns
+template <class T, bool OfInverse>
+void z_level(Box<T> nat, Box<T> hi, Box<T> lo, Dims n, uint32_t lx, uint32_t ly, hipStream_t s) {
+    ZLevel<T> a{nat.p, nat.py, nat.pz, hi.p, hi.py, hi.pz, lo.p, lo.py, lo.pz, n, lx, ly, 128, 0, 0};
+    a.groups = uint32_t((uint64_t(n.nx) * n.ny + 63) / 64);
+    auto waves = [&] { return uint64_t(a.groups) * ((n.nz + a.sz - 1) / a.sz); };
+    while (a.sz > 32 && waves() < 8192) a.sz >>= 1;
+    if (waves() < 1024) a.sz = 16;
+    const uint64_t blocks = 8 * (((waves() + 3) / 4 + 7) / 8);
+    check_launch_size(blocks * 256);
+    a.items = uint32_t(waves());
+    hipLaunchKernelGGL((adjoint_z_kernel<T, OfInverse>), dim3(uint32_t(blocks)), dim3(256), 0, s, a);
+}
+
+// Whether every level runs in registers: no line of one sample, planes inside
+// one 32-bit window.
+bool levels_fit(Dims full, unsigned lxy, unsigned lz, unsigned width) {
+    uint32_t z = full.nz;
+    for (unsigned l = 0; l < lz; ++l, z = half_len(z))
+        if (z < 2) return false;
+    return full.nx && full.ny && full.nz && strips_fit(full, full.nx, full.ny, lxy, width);
+}
+
+// The transforms' schedules reversed, from `src` into `data` (which may be the
+// same). The high bands of a level go to (or come from) their place in a full
+// volume, its low box to a compact one: odd levels' at the start of tmp1, even
+// ones' after the largest odd one (lines of at least 2 samples: both fit).
+template <class T, bool OfInverse>
+void adjoint_levels(T* data, const T* src, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz, bool dyadic,
+                    hipStream_t s) {
+    T* from = const_cast<T*>(src);  // (only read unless it is data)
+    auto low_of = [&](unsigned l, bool xy, bool z) {  // the compact box of level l >= 1
+        const Dims h = shrink_box(full, xy, z);
+        Dims n = full;
+        for (unsigned k = 0; k < l; ++k) n = shrink_box(n, xy, z);
+        return compact(tmp1 + ((l & 1u) ? 0u : uint64_t(h.nx) * h.ny * h.nz), n);
+    };
+    auto box_of = [&](unsigned l, bool xy, bool z) {
+        Dims n = full;
+        for (unsigned k = 0; k < l; ++k) n = shrink_box(n, xy, z);
+        return n;
+    };
+    const Box<T> home = volume(data, full);
+    if (dyadic) {
+        for (unsigned k = 0; k < lxy; ++k) {
+            const unsigned l = OfInverse ? k : lxy - 1 - k;
+            const Dims n = box_of(l, true, true);
+            const uint32_t lx = half_len(n.nx), ly = half_len(n.ny);
+            const bool last = l + 1 == lxy;
+            const Box<T> mid = compact(tmp0, n);
+            if constexpr (OfInverse) {
+                const Box<T> in = l ? low_of(l, true, true) : volume(from, full);
+                xy_level<T, true>(in, mid, mid, n, s);
+                z_level<T, true>(mid, home, last ? home : low_of(l + 1, true, true), n, lx, ly, s);
+            } else {
+                const Box<T> hi = volume(from, full);
+                z_level<T, false>(mid, hi, last ? hi : low_of(l + 1, true, true), n, lx, ly, s);
+                xy_level<T, false>(mid, mid, l ? low_of(l, true, true) : home, n, s);
+            }
+        }
+        return;
+    }
+    // one of the two phases only: it must not write the volume it reads
+    if (from == data && (!lxy || !lz)) {
+        hip_check(hipMemcpyAsync(tmp0, data, uint64_t(full.nx) * full.ny * full.nz * sizeof(T),
+                                 hipMemcpyDeviceToDevice, s),
+                  "copy");
+        from = tmp0;
+    }
+    const Box<T> mid = lxy && lz ? volume(tmp0, full) : home;  // between the two phases
+    auto z_phase = [&](Box<T> in, Box<T> out) {
+        for (unsigned k = 0; k < lz; ++k) {
+            const unsigned l = OfInverse ? k : lz - 1 - k;
+            const Dims n = box_of(l, false, true);
+            const bool last = l + 1 == lz;
+            const Box<T> split = OfInverse ? out : in;
+            const Box<T> nat = l ? low_of(l, false, true) : OfInverse ? in : out;
+            z_level<T, OfInverse>(nat, split, last ? split : low_of(l + 1, false, true), n, n.nx, n.ny, s);
+        }
+    };
+    auto xy_phase = [&](Box<T> in, Box<T> out) {
+        for (unsigned k = 0; k < lxy; ++k) {
+            const unsigned l = OfInverse ? k : lxy - 1 - k;
+            const Dims n = box_of(l, true, false);
+            const Box<T> split = OfInverse ? out : in;
+            const Box<T> nat = l ? low_of(l, true, false) : OfInverse ? in : out;
+            const Box<T> lo = l + 1 == lxy ? split : low_of(l + 1, true, false);
+            if constexpr (OfInverse) xy_level<T, true>(nat, lo, split, n, s);
+            else xy_level<T, false>(split, lo, nat, n, s);
+        }
+    };
+    const Box<T> in = volume(from, full);
+    if constexpr (OfInverse) {
+        z_phase(in, mid);
+        xy_phase(lz ? mid : in, home);
+    } else {
+        xy_phase(in, mid);
+        z_phase(lxy ? mid : in, home);
+    }
+}
+
 // One group of passes over one box, out of place through tmp0/tmp1, ending in
 // `home`; the first pass reads `first` when given (the whole volume's data).
 template <class T, bool OfInverse>
@@ -297,16 +477,6 @@ void box_passes(T* home, T* tmp0, T* tmp1, Dims full, Dims act, const int* axes,
                 const T* first = nullptr) {
     const T* src = first ? first : home;
     for (int k = 0; k < count; ++k) {
-        // the transposes of the inverse's X and Y passes, Y^T then X^T: one launch
-        if (OfInverse && k + 1 < count && axes[k] == 1 && axes[k + 1] == 0 && adjoint_xy_fits(act)) {
-            T* dst = k + 1 == count - 1 ? home : ((k + 1) & 1 ? tmp1 : tmp0);
-            if (dst != src) {
-                launch_adjoint_xy<T>(src, dst, full, act, s);
-                src = dst;
-                ++k;
-                continue;
-            }
-        }
         T* dst = k == count - 1 ? home : (k & 1 ? tmp1 : tmp0);
         if (dst == src) dst = tmp0;
         adjoint_axis<T, OfInverse>(src, dst, full, act, axes[k], s);
@@ -327,6 +497,11 @@ void box_passes(T* home, T* tmp0, T* tmp1, Dims full, Dims act, const int* axes,
 template <class T>
 void transform_adjoint(T* data, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz, bool dyadic,
                        bool of_inverse, hipStream_t s, const T* src) {
+    if ((lxy || lz) && levels_fit(full, lxy, lz, sizeof(T))) {
+        if (of_inverse) adjoint_levels<T, true>(data, src ? src : data, tmp0, tmp1, full, lxy, lz, dyadic, s);
+        else adjoint_levels<T, false>(data, src ? src : data, tmp0, tmp1, full, lxy, lz, dyadic, s);
+        return;
+    }
     // the adjoint of the inverse starts with a pass over the whole volume,
     // which reads src itself; the other schedules start inside a box
     const T* first = src != data && of_inverse && (lxy || lz) ? src : nullptr;

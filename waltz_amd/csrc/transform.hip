@@ -240,16 +240,6 @@ void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* sta
                        WaveRepair<T>{});
 }
 
-// One XY level (of the plane schedule, or of a dyadic level that runs as
-// passes) per launch, four strips of planes per workgroup. Consecutive items
-// go to one XCD (workgroups are dealt to the eight XCDs in turn), so that
-// neighbours' halos and warm-up rows meet in its L2.
-WZ_D bool strip_of_wave(const StripPlan& p, uint32_t& item) {
-    const uint32_t total = uint32_t(p.items()), groups = (total + 3) / 4, per = (groups + 7) / 8;
-    const uint32_t id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
-    item = 4 * id + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    return id < groups && item < total;
-}
 template <class T, bool Requant, bool Screen>
 __global__ void __launch_bounds__(kStripThreads) xy_inverse_kernel(XYInverse<T> a, StripPlan p, uint32_t* status) {
     uint32_t item;
@@ -267,24 +257,6 @@ __global__ void __launch_bounds__(kStripThreads) xy_forward_kernel(XYForward<T> 
     uint32_t item;
     if (strip_of_wave(p, item)) strip_forward<T>(a, p, item);
 }
-uint32_t strip_blocks(const StripPlan& p) {
-    const uint64_t groups = (p.items() + 3) / 4, blocks = 8 * ((groups + 7) / 8);
-    check_launch_size(blocks * kStripThreads);
-    return uint32_t(blocks);
-}
-// Whether every XY level of an nx x ny plane runs as strips: no line of one
-// sample, and a plane inside one 32-bit window.
-bool strips_fit(Dims n, uint64_t pitch, uint64_t rows, unsigned levels, unsigned width) {
-    for (unsigned l = 0; l < levels; ++l) {
-        if (n.nx < 2 || n.ny < 2) return false;
-        n = shrink(n, true, false);
-    }
-    return fused_plane_fits(pitch, rows, width);
-}
-// Lines share a wave only while the planes of a group (at most eight) share a
-// window.
-bool strips_pack(uint64_t plane, unsigned width) { return fused_plane_fits(8 * plane, 1, width); }
-
 // screen: flag non-finite results
 template <class T>
 void xy_inverse(const XYInverse<T>& a, hipStream_t s, uint32_t* screen = nullptr) {

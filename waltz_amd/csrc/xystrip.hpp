@@ -25,6 +25,8 @@
 
 #include "buffer.hpp"
 #include "common.hpp"
+#include "fused.hpp"
+#include "launch.hpp"
 #include "lifting.hpp"
 #include "repair.hpp"
 
@@ -108,6 +110,38 @@ WZ_D void strip_x_forward(T& e, T& o, bool first, bool last) {
     e = e4 * C::k;
     o = o3 * (-C::ik);
 }
+
+// The transposed steps of the inverse / forward X lifting (Adjoint in
+// strip_forward and strip_inverse).
+template <class T>
+WZ_D void strip_x_inverse_adjoint(T& e, T& o, bool first, bool last) {
+    using C = Lift<T>;
+    const T e1 = fmadd(-C::a, lane_prev(o, first) + o, e);
+    const T o1 = fmadd(-C::b, e1 + lane_next(e1, last), o);
+    const T e2 = fmadd(-C::g, lane_prev(o1, first) + o1, e1);
+    const T o2 = fmadd(-C::d, e2 + lane_next(e2, last), o1);
+    e = e2 * C::ik;
+    o = o2 * (-C::k);
+}
+template <class T>
+WZ_D void strip_x_forward_adjoint(T& e, T& o, bool first, bool last) {
+    using C = Lift<T>;
+    const T e0 = e * C::k, o0 = o * (-C::ik);
+    const T o1 = fmadd(C::d, e0 + lane_next(e0, last), o0);
+    const T e1 = fmadd(C::g, lane_prev(o1, first) + o1, e0);
+    o = fmadd(C::b, e1 + lane_next(e1, last), o1);
+    e = fmadd(C::a, lane_prev(o, first) + o, e1);
+}
+// Weights that turn a mirrored lifting step into the transpose of one. With
+// M the step on a mirrored line and W halving the line's two end samples,
+// M^T = W M' W^-1, M' the mirrored step with the roles of the parities
+// exchanged (an end sample is its own mirror image and is counted once where
+// the others count twice). So the ends are doubled as they load and halved as
+// they store, both exact, and everything between is ordinary lifting.
+template <class T>
+WZ_D T end_load(uint32_t p, uint32_t n) { return p == 0 || p == n - 1u ? T(2) : T(1); }
+template <class T>
+WZ_D T end_store(uint32_t p, uint32_t n) { return p == 0 || p == n - 1u ? T(0.5) : T(1); }
 
 // Two consecutive samples (dword-aligned).
 WZ_D void buf_load_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, float& a, float& b) {
@@ -279,8 +313,9 @@ struct XYInverse {
 // One item of an inverse level (nx, ny >= 2): the step of pair g loads pair
 // g + 2 and emits rows 2 (g - 2) and 2 (g - 2) + 1; the segment's first four
 // steps only warm the Y pipeline up. Four steps are one block (the fold phases
-// of the Y tile of 8 rows are then fixed).
-template <class T, bool Requant, class Output>
+// of the Y tile of 8 rows are then fixed). Adjoint: the transpose of the
+// forward level instead, whose input is the split gradient.
+template <class T, bool Requant, bool Adjoint = false, class Output>
 WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item, Output&& out) {
     using C = Lift<T>;
     constexpr uint32_t S = sizeof(T);
@@ -318,6 +353,9 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
     T OS[2], EA[2], OB[2], EC[2], SF[2];  // Y state, as the fused level's Z synthesis
 #pragma unroll
     for (int c = 0; c < 2; ++c) OS[c] = EA[c] = OB[c] = EC[c] = SF[c] = T(0);
+    [[maybe_unused]] const T cw[2] = {end_load<T>(reflect_pos(int32_t(2 * it.kp), n.nx), n.nx),
+                                      end_load<T>(reflect_pos(int32_t(2 * it.kp + 1), n.nx), n.nx)};
+    [[maybe_unused]] const T cs[2] = {end_store<T>(2 * it.kp, n.nx), end_store<T>(2 * it.kp + 1, n.nx)};
     T buf[4][4];
     int32_t g = int32_t(it.ys / 2) - 2;
     load(g, buf[0]);
@@ -334,38 +372,66 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
 #pragma unroll
                 for (int i = 1; i < 4; ++i) v[i] = requantize<T>(v[i], a.q, a.inv);
             }
-            strip_x_inverse(v[0], v[1], it.first, it.last);
-            strip_x_inverse(v[2], v[3], it.first, it.last);
-            const int phase = (u + 2) & 3;
             T re[2], ro[2];
+            if constexpr (Adjoint) {
+                const T re0 = end_load<T>(2 * uint32_t(pair_even(g, ny)), n.ny);
+                const T ro0 = end_load<T>(2 * uint32_t(pair_odd(g, ny)) + 1u, n.ny);
+                const uint32_t y = 2 * uint32_t(g - 2);
+                const T se = end_store<T>(y, n.ny), so = end_store<T>(y + 1u, n.ny);
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {  // the pair's columns
-                const T oraw = v[2 + c];
-                const T es = v[c] * C::ik, os = oraw * (-C::k);
-                const T eA = fmadd(-C::d, OS[c] + os, es);
-                const T oB = fmadd(-C::g, EA[c] + eA, OS[c]);
-                const T eC = fmadd(-C::b, OB[c] + oB, EA[c]);
-                re[c] = EC[c];
-                ro[c] = fmadd(-C::a, EC[c] + eC, OB[c]);
-                if (phase == 3) {  // g = B - 1: fold of tile B's first pair
-                    SF[c] = fmadd(-C::d, fmadd(SF[c], -C::k, os), es);
-                } else if (phase == 0) {
-                    SF[c] = fmadd(-C::g, SF[c] + eA, OS[c]);
-                } else if (phase == 1) {  // and the tile before's last sample
-                    SF[c] = fmadd(-C::b, SF[c] + oB, EA[c]);
-                    const T eAe = fmadd(-C::d, fmadd(oraw, -C::k, OS[c]), es);
-                    const T oBe = fmadd(-C::g, EA[c] + eAe, OS[c]);
-                    const T eCe = fmadd(-C::b, OB[c] + oBe, EA[c]);
-                    ro[c] = fmadd(-C::a, EC[c] + eCe, OB[c]);
-                } else {  // g = B + 2: tile B's first two samples; o_raw[B' - 2] for the next fold
-                    re[c] = SF[c];
-                    ro[c] = fmadd(-C::a, SF[c] + eC, OB[c]);
-                    SF[c] = oraw;
+                for (int c = 0; c < 2; ++c) {
+                    v[c] *= cw[c] * re0;
+                    v[2 + c] *= cw[c] * ro0;
                 }
-                OS[c] = os;
-                EA[c] = eA;
-                OB[c] = oB;
-                EC[c] = eC;
+                strip_x_forward_adjoint(v[0], v[1], it.first, it.last);
+                strip_x_forward_adjoint(v[2], v[3], it.first, it.last);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {  // (the forward pipeline's states: O, O1, E2, O3, E)
+                    const T ev = v[c] * C::k, odd = v[2 + c] * (-C::ik);
+                    const T o1 = fmadd(C::d, SF[c] + ev, OS[c]);
+                    const T e2 = fmadd(C::g, EA[c] + o1, SF[c]);
+                    const T o3 = fmadd(C::b, OB[c] + e2, EA[c]);
+                    re[c] = fmadd(C::a, EC[c] + o3, OB[c]) * (cs[c] * se);
+                    ro[c] = o3 * (cs[c] * so);
+                    SF[c] = ev;
+                    OS[c] = odd;
+                    EA[c] = o1;
+                    OB[c] = e2;
+                    EC[c] = o3;
+                }
+            } else {
+                strip_x_inverse(v[0], v[1], it.first, it.last);
+                strip_x_inverse(v[2], v[3], it.first, it.last);
+                const int phase = (u + 2) & 3;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {  // the pair's columns
+                    const T oraw = v[2 + c];
+                    const T es = v[c] * C::ik, os = oraw * (-C::k);
+                    const T eA = fmadd(-C::d, OS[c] + os, es);
+                    const T oB = fmadd(-C::g, EA[c] + eA, OS[c]);
+                    const T eC = fmadd(-C::b, OB[c] + oB, EA[c]);
+                    re[c] = EC[c];
+                    ro[c] = fmadd(-C::a, EC[c] + eC, OB[c]);
+                    if (phase == 3) {  // g = B - 1: fold of tile B's first pair
+                        SF[c] = fmadd(-C::d, fmadd(SF[c], -C::k, os), es);
+                    } else if (phase == 0) {
+                        SF[c] = fmadd(-C::g, SF[c] + eA, OS[c]);
+                    } else if (phase == 1) {  // and the tile before's last sample
+                        SF[c] = fmadd(-C::b, SF[c] + oB, EA[c]);
+                        const T eAe = fmadd(-C::d, fmadd(oraw, -C::k, OS[c]), es);
+                        const T oBe = fmadd(-C::g, EA[c] + eAe, OS[c]);
+                        const T eCe = fmadd(-C::b, OB[c] + oBe, EA[c]);
+                        ro[c] = fmadd(-C::a, EC[c] + eCe, OB[c]);
+                    } else {  // g = B + 2: tile B's first two samples; o_raw[B' - 2] for the next fold
+                        re[c] = SF[c];
+                        ro[c] = fmadd(-C::a, SF[c] + eC, OB[c]);
+                        SF[c] = oraw;
+                    }
+                    OS[c] = os;
+                    EA[c] = eA;
+                    OB[c] = oB;
+                    EC[c] = eC;
+                }
             }
             if constexpr (emit) {
                 const uint32_t y = 2 * uint32_t(g - 2);
@@ -395,8 +461,10 @@ struct XYForward {
 };
 
 // One item of a forward level (nx, ny >= 2): the step of row pair g loads pair
-// g + 2 and emits the low and high row g - 2 of the split.
-template <class T>
+// g + 2 and emits the low and high row g - 2 of the split. Adjoint: the
+// transpose of the inverse level instead, whose input is the gradient of the
+// samples.
+template <class T, bool Adjoint = false>
 WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item) {
     using C = Lift<T>;
     constexpr uint32_t S = sizeof(T);
@@ -426,6 +494,8 @@ WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item
     T E[2], O[2], O1[2], E2[2], O3[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) E[c] = O[c] = O1[c] = E2[c] = O3[c] = T(0);
+    [[maybe_unused]] const T cw[2] = {end_load<T>(xe, n.nx), end_load<T>(xo, n.nx)};
+    [[maybe_unused]] const T cs[2] = {end_store<T>(2 * it.kp, n.nx), end_store<T>(2 * it.kp + 1, n.nx)};
     T buf[4][4];
     int32_t g = int32_t(it.ys / 2) - 2;
     load(g, buf[0]);
@@ -445,6 +515,20 @@ WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item
             for (int c = 0; c < 2; ++c) {
                 const bool other = (c != 0) != swap;
                 const T ev = other ? v[1] : v[0], ov = other ? v[3] : v[2];
+                if constexpr (Adjoint) {  // (the inverse pipeline's states: OS, EA, OB, EC)
+                    const T es = ev * (cw[c] * end_load<T>(2 * uint32_t(pair_even(g, ny)), n.ny));
+                    const T os = ov * (cw[c] * end_load<T>(2 * uint32_t(pair_odd(g, ny)) + 1u, n.ny));
+                    const T eA = fmadd(-C::a, O[c] + os, es);
+                    const T oB = fmadd(-C::b, O1[c] + eA, O[c]);
+                    const T eC = fmadd(-C::g, E2[c] + oB, O1[c]);
+                    le[c] = O3[c] * C::ik;
+                    hi[c] = fmadd(-C::d, O3[c] + eC, E2[c]) * (-C::k);
+                    O[c] = os;
+                    O1[c] = eA;
+                    E2[c] = oB;
+                    O3[c] = eC;
+                    continue;
+                }
                 const T o1 = fmadd(C::a, E[c] + ev, O[c]);
                 const T e2 = fmadd(C::b, O1[c] + o1, E[c]);
                 const T o3 = fmadd(C::g, E2[c] + e2, O1[c]);
@@ -458,9 +542,20 @@ WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item
                 O3[c] = o3;
             }
             if constexpr (emit) {
-                strip_x_forward(le[0], le[1], it.first, it.last);
-                strip_x_forward(hi[0], hi[1], it.first, it.last);
                 const uint32_t iy = uint32_t(g - 2);
+                if constexpr (Adjoint) {
+                    strip_x_inverse_adjoint(le[0], le[1], it.first, it.last);
+                    strip_x_inverse_adjoint(hi[0], hi[1], it.first, it.last);
+                    const T sl = end_store<T>(2 * iy, n.ny), sh = end_store<T>(2 * iy + 1u, n.ny);
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        le[c] *= cs[c] * sl;
+                        hi[c] *= cs[c] * sh;
+                    }
+                } else {
+                    strip_x_forward(le[0], le[1], it.first, it.last);
+                    strip_x_forward(hi[0], hi[1], it.first, it.last);
+                }
                 const bool low = 2 * iy < n.ny, high = 2 * iy + 1 < n.ny;
                 const uint32_t at = hv + iy * hrow, up = hv + (hy + iy) * hrow;
                 buf_store(le[0], wl, it.own && low ? lv + iy * lrow : kOutside);
@@ -474,5 +569,33 @@ WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item
     for (uint32_t b = 0; b < it.blocks; ++b) block(std::true_type{});
     if (a.status && __ballot(!ok) && (threadIdx.x & 63u) == 0) atomicOr(a.status, uint32_t(kNonFiniteInput));
 }
+
+// One XY level (of the plane schedule, or of a dyadic level that runs as
+// passes) per launch, four strips of planes per workgroup. Consecutive items
+// go to one XCD (workgroups are dealt to the eight XCDs in turn), so that
+// neighbours' halos and warm-up rows meet in its L2.
+WZ_D bool strip_of_wave(const StripPlan& p, uint32_t& item) {
+    const uint32_t total = uint32_t(p.items()), groups = (total + 3) / 4, per = (groups + 7) / 8;
+    const uint32_t id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+    item = 4 * id + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    return id < groups && item < total;
+}
+inline uint32_t strip_blocks(const StripPlan& p) {
+    const uint64_t groups = (p.items() + 3) / 4, blocks = 8 * ((groups + 7) / 8);
+    check_launch_size(blocks * kStripThreads);
+    return uint32_t(blocks);
+}
+// Whether every XY level of an nx x ny plane runs as strips: no line of one
+// sample, and a plane inside one 32-bit window.
+inline bool strips_fit(Dims n, uint64_t pitch, uint64_t rows, unsigned levels, unsigned width) {
+    for (unsigned l = 0; l < levels; ++l) {
+        if (n.nx < 2 || n.ny < 2) return false;
+        n = Dims{half_len(n.nx), half_len(n.ny), n.nz};
+    }
+    return fused_plane_fits(pitch, rows, width);
+}
+// Lines share a wave only while the planes of a group (at most eight) share a
+// window.
+inline bool strips_pack(uint64_t plane, unsigned width) { return fused_plane_fits(8 * plane, 1, width); }
 
 }  // namespace wz
