@@ -289,13 +289,6 @@ __global__ void __launch_bounds__(256) batch_wzp_ranks_kernel(const uint8_t* __r
 // spent most of its life finding its job and brick
 constexpr uint32_t kBricksPerBlock = 8;
 
-struct SetRank {
-    const uint16_t* set;
-    WZ_D uint32_t operator()(const Brick& k, uint32_t i, uint32_t, uint32_t, uint32_t) const {
-        return set[k.shape * 8192 + i];
-    }
-};
-
 // Dequantization of one brick (quantize.hip's brick order, packed base and ranks).
 // Dequantization of up to kBricksPerBlock consecutive bricks of one job
 // (quantize.hip's brick order, packed base and ranks), their samples taken
@@ -673,15 +666,15 @@ __global__ void __launch_bounds__(256) batch_quantize_kernel(const JobShape* __r
     const JobComp& jc = comp[j];
     const BrickGeometry g{sh.d, sh.bz, sh.nbx, sh.nby, sh.nbz};
     const SideList qo{b.qbm + jc.words, b.qidx + jc.qlist, b.qval + jc.qlist, b.qcount + j, jc.qcap};
-    // up to kBricksPerBlock consecutive bricks of the job, one after another
+    // up to kBricksPerBlock consecutive bricks of the job, a group at a time
     const uint32_t b0 = (blockIdx.x - brick_pfx[j]) * kBricksPerBlock;
     const uint32_t b1 = min(b0 + kBricksPerBlock, sh.nbx * sh.nby * sh.nbz);
-    for (uint32_t k = b0; k < b1; ++k) {
-        if (k != b0) __syncthreads();  // the previous brick's sign words are out of LDS
-        quantize_brick(static_cast<T*>(b.home) + sh.bank, g, T(quantum), T(1.0 / quantum),
-                       SetRank{ranks + uint64_t(sh.rank) * kRankSet},
-                       static_cast<uint16_t*>(b.tmp0) + sh.mag, static_cast<uint32_t*>(b.tmp1) + sh.sign, qo,
-                       &b.res[j].status, k);
+    const uint32_t per = group_bricks(sh.bz);
+    for (uint32_t k = b0; k < b1; k += per) {
+        if (k != b0) __syncthreads();  // the previous group is out of LDS
+        quantize_group(static_cast<T*>(b.home) + sh.bank, g, T(quantum), T(1.0 / quantum),
+                       ranks + uint64_t(sh.rank) * kRankSet, static_cast<uint16_t*>(b.tmp0) + sh.mag,
+                       static_cast<uint32_t*>(b.tmp1) + sh.sign, qo, &b.res[j].status, k, min(per, b1 - k), sh.d);
     }
 }
 

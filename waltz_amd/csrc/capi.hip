@@ -413,6 +413,7 @@ size_t waltz_amd_tuning_report(char* buf, size_t cap) {
 int waltz_amd_quantize(int width, void* coeff, uint32_t nx, uint32_t ny, uint32_t nz, uint32_t bz, double quantum,
                        void* mag, void* sign, void* qidx, void* qval, uint32_t* nq, void* stream) {
     return guarded([&] {
+        if (!bz || bz > 32) throw std::invalid_argument("z band must be 1 to 32");
         const wz::Dims d = dims_of(nx, ny, nz);
         const uint64_t n = uint64_t(nx) * ny * nz;
         const uint64_t words = (n + 31) / 32;

@@ -272,10 +272,9 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     transform_forward<T>(input, p.coeff, p.t0, p.t1, g.d, g.lx, g.lz, g.dyadic, status, s);
     SideList qo{p.qbm, p.qidx, p.qval, p.counters + 1, nq};
     WzpScratch wsc{p.desc, p.stage, p.size, p.counters};
-    // with the fused repair emitter and a quantizing encoder the finest
-    // level's high bands stay unquantized in coeff; that kernel requantizes
-    // them on load
-    const bool requant = g.dyadic && fsegs && fusedq && tuning_for(g.d, g.lx, sizeof(T), true).fused;
+    // with the fused repair emitter the finest level's high bands stay
+    // unquantized in coeff; that kernel requantizes them on load
+    const bool requant = g.dyadic && fsegs && tuning_for(g.d, g.lx, sizeof(T), true).fused;
     // The group pass runs on the side stream beside the inverse levels (the
     // staging slots it reads are never written by them); the archive sections
     // wait for it.
@@ -289,7 +288,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     const bool split = requant && coarse_split_fits(g.d, g.lx, sizeof(T));
     // a plane-schedule field whose inverse runs as fused XY levels quantizes
     // and dequantizes the coefficients as they load: nothing written back
-    const bool plane_requant = !g.dyadic && fusedq && plane_fused_fits(g.d, g.lx, g.lz, sizeof(T));
+    const bool plane_requant = !g.dyadic && plane_fused_fits(g.d, g.lx, g.lz, sizeof(T));
     const WriteBack wb = split || plane_requant ? kWriteNone : requant ? kWriteCoarseBox : kWriteAll;
     if (direct) {
         StageClock c("quantize_encode", s);
@@ -304,7 +303,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         const uint16_t* rank = w.ranks(g.d, g.bz, s);
         {
             StageClock c("quantize", s);
-            quantize_bricks<T>(p.coeff, bg, quantum, rank, p.mag, p.sign, qo, status, s);
+            quantize_bricks<T>(p.coeff, bg, quantum, rank, p.mag, p.sign, qo, status, s, wb);
         }
         StageClock c("wzp_encode", s);
         wzp_encode(p.mag, p.sign, n, archive + 32, capacity - 32, wsc, status, s);

@@ -146,6 +146,12 @@ WZ_D T requantize(T v, T q, T inv) {
     return rounded == T(0) ? T(0) : m * q;
 }
 
+// Magnitude of a rounded |v| / quantum: saturated at INT32_MAX.
+template <class T>
+WZ_D uint32_t quantum_count(T am) {
+    return am >= T(2147483648.0) ? uint32_t(INT32_MAX) : uint32_t(int32_t(am));
+}
+
 // Segmented side list: each producer workgroup appends to its own segment of
 // `cap` entries and records the count; a complete row-major flag bitmap lets
 // the archive assembly find every entry's index-order position.

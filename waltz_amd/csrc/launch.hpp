@@ -189,9 +189,16 @@ WZ_D void append_qoutliers(const SideList& qo, uint32_t over, Place&& place, Val
     }
 }
 
+// Where a quantizing pass writes the dequantized coefficients back.
+enum WriteBack { kWriteAll, kWriteCoarseBox, kWriteNone };
+inline Dims writeback_box(Dims d, WriteBack wb) {
+    if (wb == kWriteNone) return Dims{0, 0, 0};
+    if (wb == kWriteCoarseBox) return Dims{half_len(d.nx), half_len(d.ny), half_len(d.nz)};
+    return d;
+}
 template <class T>
 void quantize_bricks(T* coeff, const BrickGeometry& g, double quantum, const uint16_t* rank, uint16_t* mag,
-                     uint32_t* sign, SideList q, uint32_t* status, hipStream_t s);
+                     uint32_t* sign, SideList q, uint32_t* status, hipStream_t s, WriteBack wb = kWriteAll);
 // plan: a planned decode's device record (quantum from it; nothing unless ok)
 template <class T>
 void dequantize_bricks(const uint16_t* mag, const uint32_t* sign, const BrickGeometry& g, double quantum,
@@ -235,7 +242,6 @@ void wzp_decode(const uint8_t* in, uint64_t bytes, uint32_t n, uint16_t* mag, ui
 // (q-outliers appended to `qo`; the dequantized coefficients written back in
 // place over the whole volume, over the coarser levels' box only, or nowhere),
 // and dequantization fused into the decoder (writes the coefficient volume).
-enum WriteBack { kWriteAll, kWriteCoarseBox, kWriteNone };
 template <class T>
 void quantize_encode_direct(T* coeff, Dims d, uint32_t bz, double quantum, SideList qo, uint8_t* out,
                             uint64_t capacity, WzpScratch w, uint32_t* status, hipStream_t s,

@@ -8,11 +8,10 @@
 // the recursive ceil-half octant rank (cpu/src/codec.cpp:96-107), tabulated
 // once per geometry for the eight edge shapes.
 //
-// One workgroup owns one brick: it reads the brick's coefficients (rows of
-// <=16 contiguous values), writes the dequantized value back in place, scatters
-// u16 magnitudes inside the brick's own packed span, and assembles the brick's
-// sign bits in LDS before writing whole 32-bit words (only the two words that a
-// brick shares with its neighbours use atomics).
+// A workgroup of the quantization owns a group of consecutive bricks
+// (quantize_group), one of the dequantization a brick.
+#include <algorithm>
+
 #include "bricks.hpp"
 
 namespace wz {
@@ -43,29 +42,26 @@ void build_rank_tables(Dims d, uint32_t bz, uint16_t* rank, uint16_t* inv, hipSt
     hipLaunchKernelGGL(rank_tables, dim3(8), dim3(256), 0, s, d, bz, rank, inv);
 }
 
-// Packed rank from the geometry's tabulated edge shapes.
-struct TableRank {
-    const uint16_t* rank;
-    WZ_D uint32_t operator()(const Brick& k, uint32_t i, uint32_t, uint32_t, uint32_t) const {
-        return rank[k.shape * 8192 + i];
-    }
-};
-
 template <class T>
 __global__ void __launch_bounds__(256) quantize_kernel(T* __restrict__ coeff, BrickGeometry g, T q, T inv,
                                                        const uint16_t* __restrict__ rank, uint16_t* __restrict__ mag,
                                                        uint32_t* __restrict__ sign, SideList qo,
-                                                       uint32_t* __restrict__ status) {
-    quantize_brick(coeff, g, q, inv, TableRank{rank}, mag, sign, qo, status, blockIdx.x);
+                                                       uint32_t* __restrict__ status, uint32_t per, Dims box) {
+    const uint32_t bricks = g.nbx * g.nby * g.nbz, first = blockIdx.x * per;
+    quantize_group(coeff, g, q, inv, rank, mag, sign, qo, status, first, min(per, bricks - first), box);
 }
 
 template <class T>
 void quantize_bricks(T* coeff, const BrickGeometry& g, double quantum, const uint16_t* rank, uint16_t* mag,
-                     uint32_t* sign, SideList q, uint32_t* status, hipStream_t s) {
+                     uint32_t* sign, SideList q, uint32_t* status, hipStream_t s, WriteBack wb) {
     const uint64_t bricks = uint64_t(g.nbx) * g.nby * g.nbz;
-    check_launch_size(bricks * 256);
-    hipLaunchKernelGGL((quantize_kernel<T>), dim3(uint32_t(bricks)), dim3(256), 0, s, coeff, g, T(quantum),
-                       T(1.0 / quantum), rank, mag, sign, q, status);
+    // fewer bricks a group while the groups are too few to fill the chip
+    const uint32_t per = uint32_t(std::min<uint64_t>(group_bricks(g.bz), std::max<uint64_t>(bricks / 1024, 1)));
+    const uint64_t groups = (bricks + per - 1) / per;
+    check_launch_size(groups * 256);
+    if (!groups) return;
+    hipLaunchKernelGGL((quantize_kernel<T>), dim3(uint32_t(groups)), dim3(256), 0, s, coeff, g, T(quantum),
+                       T(1.0 / quantum), rank, mag, sign, q, status, per, writeback_box(g.d, wb));
 }
 
 template <class T>
@@ -113,9 +109,9 @@ void dequantize_bricks(const uint16_t* mag, const uint32_t* sign, const BrickGeo
 }
 
 template void quantize_bricks<float>(float*, const BrickGeometry&, double, const uint16_t*, uint16_t*, uint32_t*,
-                                     SideList, uint32_t*, hipStream_t);
+                                     SideList, uint32_t*, hipStream_t, WriteBack);
 template void quantize_bricks<double>(double*, const BrickGeometry&, double, const uint16_t*, uint16_t*, uint32_t*,
-                                      SideList, uint32_t*, hipStream_t);
+                                      SideList, uint32_t*, hipStream_t, WriteBack);
 template void dequantize_bricks<float>(const uint16_t*, const uint32_t*, const BrickGeometry&, double,
                                        const uint16_t*, float*, hipStream_t, const DecodeRecord*);
 template void dequantize_bricks<double>(const uint16_t*, const uint32_t*, const BrickGeometry&, double,

@@ -73,12 +73,6 @@ void wzp_encode(const uint16_t* mag, const uint32_t* sign, uint32_t n, uint8_t* 
 }
 
 // The write-back box of a fused quantizing encoder.
-Dims writeback_box(Dims d, WriteBack wb) {
-    if (wb == kWriteNone) return Dims{0, 0, 0};
-    if (wb == kWriteCoarseBox) return Dims{half_len(d.nx), half_len(d.ny), half_len(d.nz)};
-    return d;
-}
-
 template <class T>
 void check_direct_bricks(Dims d, uint32_t bz) {
     if (!direct_bricks_fit(d.nx, d.ny, d.nz, bz, sizeof(T)))

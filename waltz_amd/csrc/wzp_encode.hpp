@@ -94,7 +94,7 @@ struct BrickSource {
                 const T scaled = v[r][dx] * inv;
                 bad = bad || !(abs_t(scaled) < T(9223372036854775808.0));
                 const T rounded = rint_t(scaled);
-                const uint32_t mv = magnitude(abs_t(rounded));
+                const uint32_t mv = quantum_count(abs_t(rounded));
                 const uint32_t i = direct_rank<Cube>(dx, r);
                 m[i] = live ? (mv > 65535u ? 65535u : mv) : 0u;
                 sw |= uint32_t(rounded < T(0)) << i;
@@ -111,13 +111,9 @@ struct BrickSource {
         }
         append_qoutliers<32>(
             qo, live ? overs : 0u, [&](int i) { return uint32_t(at0) + g.run(uint32_t(i) / 4) + uint32_t(i) % 4; },
-            [&](int i) { return magnitude(abs_t(rint_t(v[i / 4][i % 4] * inv))); });
+            [&](int i) { return quantum_count(abs_t(rint_t(v[i / 4][i % 4] * inv))); });
         if (bad && live) atomicOr(status, uint32_t(kQuantDomain));
         return live ? sw : 0u;
-    }
-    // llrint of a rounded magnitude, saturated at INT32_MAX
-    WZ_D static uint32_t magnitude(T am) {
-        return am >= T(2147483648.0) ? uint32_t(INT32_MAX) : uint32_t(int32_t(am));
     }
 };
 
@@ -173,7 +169,7 @@ struct RankSource {
                     // INT32 saturation
                     const T scaled = v[u][k] * inv;
                     const T rounded = rint_t(scaled);
-                    const uint32_t mv = magnitude(abs_t(rounded));
+                    const uint32_t mv = quantum_count(abs_t(rounded));
                     d[k] = requantize<T>(v[u][k], q, inv);
                     if (!in) continue;
                     overs |= uint32_t(mv > 65535u) << (4 * u + k);
@@ -197,7 +193,7 @@ struct RankSource {
             }
             append_qoutliers<4 * kBurst>(
                 qo, overs, [&](int i) { return rq[i / 4].at + uint32_t(i) % 4; },
-                [&](int i) { return magnitude(abs_t(rint_t(v[i / 4][i % 4] * inv))); });
+                [&](int i) { return quantum_count(abs_t(rint_t(v[i / 4][i % 4] * inv))); });
         }
         __syncthreads();
         const uint32_t first = 32u * t;
@@ -216,10 +212,6 @@ struct RankSource {
         __syncthreads();  // the buffer is free again for the caller
         if (bad) atomicOr(status, uint32_t(kQuantDomain));
         return sw;
-    }
-    // llrint of a rounded magnitude, saturated at INT32_MAX
-    WZ_D static uint32_t magnitude(T am) {
-        return am >= T(2147483648.0) ? uint32_t(INT32_MAX) : uint32_t(int32_t(am));
     }
 };
 
