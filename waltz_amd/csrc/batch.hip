@@ -559,8 +559,7 @@ struct CompBufs {
     uint32_t *qidx, *qval;  // q-outlier lists
     uint32_t* ridx;         // repair segments: indices
     void* rval;             // repair segments: corrections
-    uint32_t *rcount, *qcount, *prefix, *sizes, *ticket;
-    unsigned long long* desc;
+    uint32_t *rcount, *qcount, *prefix, *sizes, *glen;
     EncodeResult* res;
     uint8_t* out;           // archive slots
     uint64_t* spans;        // jobs x {offset, size}
@@ -679,7 +678,7 @@ __global__ void __launch_bounds__(256) batch_quantize_kernel(const JobShape* __r
 }
 
 WZ_D WzpScratch job_wzp(const CompBufs& b, const JobComp& jc) {
-    return WzpScratch{b.desc + jc.group0, b.staging + jc.staging, b.sizes + jc.chunk0, nullptr};
+    return WzpScratch{b.glen + jc.group0, b.staging + jc.staging, b.sizes + jc.chunk0};
 }
 
 // Chunks of the jobs with edge bricks (mag_pfx counts only theirs):
@@ -735,20 +734,16 @@ __global__ void __launch_bounds__(256) batch_encode_ranks_kernel(const JobShape*
                  &b.res[j].status);
 }
 
-// Groups of all jobs in one ticket order (job by job, group by group), so
-// every group's predecessors in its own stream are held by running workgroups.
-__global__ void __launch_bounds__(kPackThreads) batch_pack_kernel(const JobShape* __restrict__ shape,
-                                                                  const JobComp* __restrict__ comp,
-                                                                  const uint32_t* __restrict__ group_pfx,
-                                                                  uint32_t jobs, CompBufs b) {
-    __shared__ uint32_t g_sh;
-    if (threadIdx.x == 0) g_sh = atomicAdd(b.ticket, 1u);
-    __syncthreads();
-    const uint32_t j = job_of_wave(group_pfx, jobs, g_sh);
+// Payload placement, a workgroup per chunk of any job.
+__global__ void __launch_bounds__(256) batch_pack_kernel(const JobShape* __restrict__ shape,
+                                                         const JobComp* __restrict__ comp,
+                                                         const uint32_t* __restrict__ chunk_pfx, uint32_t jobs,
+                                                         CompBufs b) {
+    const uint32_t j = job_of_wave(chunk_pfx, jobs, blockIdx.x);
     const JobShape& sh = shape[j];
     const JobComp& jc = comp[j];
-    pack_group(g_sh - group_pfx[j], b.out + jc.arc + 32, jc.cap - 32, sh.chunks, sh.groups, job_wzp(b, jc),
-               &b.res[j].wzp_bytes, &b.res[j].status);
+    pack_chunks<256, 1>(blockIdx.x - chunk_pfx[j], b.out + jc.arc + 32, jc.cap - 32, sh.chunks, sh.groups,
+                        job_wzp(b, jc), &b.res[j].wzp_bytes, &b.res[j].status);
 }
 
 template <class T>
@@ -1213,8 +1208,8 @@ StepTables build_steps(const std::vector<std::vector<Pass>>& sched, uint32_t J, 
 
 // Byte offsets of one batched compress call's workspace (all 256-byte aligned).
 struct CompressLayout {
-    uint64_t home, tmp0, tmp1, recon, staging, qbm, rbm, qidx, qval, ridx, rval, rcount, prefix, sizes, desc;
-    uint64_t zero0, qcount, ticket, res, zero_end, total;
+    uint64_t home, tmp0, tmp1, recon, staging, qbm, rbm, qidx, qval, ridx, rval, rcount, prefix, sizes, glen;
+    uint64_t zero0, qcount, res, zero_end, total;
 };
 
 struct HostPlan {
@@ -1229,7 +1224,7 @@ struct HostPlan {
     // compress
     StepTables fwd;                           // forward passes
     std::vector<JobComp> comp;
-    std::vector<uint32_t> group_pfx, tile_pfx, pblock_pfx, place_pfx;
+    std::vector<uint32_t> tile_pfx, pblock_pfx, place_pfx;
     uint64_t archive_bytes = 0;               // archive slots of all jobs
     CompressLayout cl{};
     std::vector<std::pair<Dims, uint32_t>> rank_geo;  // distinct (geometry, z band) of the rank table sets
@@ -1264,7 +1259,6 @@ void finish_compress_plan(HostPlan& p) {
     const unsigned w = p.width;
     std::vector<std::vector<Pass>> sched(J);
     p.comp.assign(J, JobComp{});
-    p.group_pfx.assign(J + 1, 0);
     p.tile_pfx.assign(J + 1, 0);
     p.pblock_pfx.assign(J + 1, 0);
     p.place_pfx.assign(J + 1, 0);
@@ -1292,7 +1286,6 @@ void finish_compress_plan(HostPlan& p) {
         c.pblocks = uint32_t((wds + kPrefixWords - 1) / kPrefixWords);
         c.qblocks = std::max(1u, std::min(16u, (c.qcap + 4095) / 4096));
         c.rlist = uint64_t(c.tile0) * kRepairTile;
-        p.group_pfx[j] = c.group0;
         p.tile_pfx[j] = c.tile0;
         p.pblock_pfx[j] = uint32_t(pblocks);
         p.place_pfx[j] = uint32_t(places);
@@ -1304,7 +1297,6 @@ void finish_compress_plan(HostPlan& p) {
     }
     if (groups > 0x7FFFFFFFull || tiles > 0x7FFFFFFFull || 2 * pblocks > 0x7FFFFFFFull || places > 0x7FFFFFFFull)
         throw std::invalid_argument("batch launch limit");
-    p.group_pfx[J] = uint32_t(groups);
     p.tile_pfx[J] = uint32_t(tiles);
     p.pblock_pfx[J] = uint32_t(pblocks);
     p.place_pfx[J] = uint32_t(places);
@@ -1333,9 +1325,8 @@ void finish_compress_plan(HostPlan& p) {
     L.sizes = take(uint64_t(p.chunk_pfx[J]) * 4);
     L.zero0 = at;  // zero-initialised from here on
     L.qbm = take(words * 4);
-    L.desc = take(groups * 8);
+    L.glen = take(groups * 4);
     L.qcount = take(uint64_t(J) * 4);
-    L.ticket = take(4);
     L.res = take(uint64_t(J) * sizeof(EncodeResult));
     L.zero_end = at;
     L.total = at;
@@ -1422,10 +1413,10 @@ struct DevicePlan {
     uint32_t* host_status = nullptr;  // pinned
     // compress tables
     JobComp* comp = nullptr;
-    uint32_t *group_pfx = nullptr, *tile_pfx = nullptr, *pblock_pfx = nullptr, *place_pfx = nullptr;
+    uint32_t *tile_pfx = nullptr, *pblock_pfx = nullptr, *place_pfx = nullptr;
     EncodeResult* last_res = nullptr;  // results of the last compress (device, in its workspace)
     uint16_t* ranks = nullptr;         // kRankSet entries per distinct geometry
-    // compress: the WZP group pass runs on `side` (default priority) beside
+    // compress: the WZP payload placement runs on `side` (default priority) beside
     // the inverse passes, between the two events
     hipStream_t side = nullptr;
     hipEvent_t pack_ready = nullptr, pack_done = nullptr;
@@ -1454,7 +1445,7 @@ struct DevicePlan {
         const size_t o_cube = carve(4 * (J + 1)), o_direct = carve(4 * (J + 1)), o_rankp = carve(4 * (J + 1)), o_magp = carve(4 * (J + 1));
         const size_t o_cp = carve(4 * (J + 1)), o_bp = carve(4 * (J + 1)), o_np = carve(4 * (J + 1)),
                      o_nq = carve(4 * (J + 1)), o_st = carve(4);
-        const size_t o_comp = carve(sizeof(JobComp) * J), o_gp = carve(4 * (J + 1)), o_tp = carve(4 * (J + 1)),
+        const size_t o_comp = carve(sizeof(JobComp) * J), o_tp = carve(4 * (J + 1)),
                      o_pbp = carve(4 * (J + 1)), o_plp = carve(4 * (J + 1));
         const StepTables* tables[2] = {&p.inv, &p.fwd};
         size_t o_pass[2], o_pfx[2][3];
@@ -1480,7 +1471,6 @@ struct DevicePlan {
         nq_pfx = reinterpret_cast<uint32_t*>(mem + o_nq);
         status = reinterpret_cast<uint32_t*>(mem + o_st);
         comp = reinterpret_cast<JobComp*>(mem + o_comp);
-        group_pfx = reinterpret_cast<uint32_t*>(mem + o_gp);
         tile_pfx = reinterpret_cast<uint32_t*>(mem + o_tp);
         pblock_pfx = reinterpret_cast<uint32_t*>(mem + o_pbp);
         place_pfx = reinterpret_cast<uint32_t*>(mem + o_plp);
@@ -1514,7 +1504,6 @@ struct DevicePlan {
         hip_check(hipMemcpyAsync(rank_pfx, p.rank_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(mag_pfx, p.mag_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(comp, p.comp.data(), sizeof(JobComp) * J, hipMemcpyHostToDevice, s), "plan");
-        hip_check(hipMemcpyAsync(group_pfx, p.group_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(tile_pfx, p.tile_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(pblock_pfx, p.pblock_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
         hip_check(hipMemcpyAsync(place_pfx, p.place_pfx.data(), 4 * (J + 1), hipMemcpyHostToDevice, s), "plan");
@@ -1568,8 +1557,7 @@ struct DevicePlan {
         b.qcount = reinterpret_cast<uint32_t*>(ws + L.qcount);
         b.prefix = reinterpret_cast<uint32_t*>(ws + L.prefix);
         b.sizes = reinterpret_cast<uint32_t*>(ws + L.sizes);
-        b.ticket = reinterpret_cast<uint32_t*>(ws + L.ticket);
-        b.desc = reinterpret_cast<unsigned long long*>(ws + L.desc);
+        b.glen = reinterpret_cast<uint32_t*>(ws + L.glen);
         b.res = reinterpret_cast<EncodeResult*>(ws + L.res);
         b.out = out;
         b.spans = spans;
@@ -1601,15 +1589,15 @@ struct DevicePlan {
         if (p.rank_pfx[J])
             hipLaunchKernelGGL((batch_encode_ranks_kernel<T>), dim3(p.rank_pfx[J]), dim3(256), 0, s, shape, comp,
                                rank_pfx, J, ranks, quantum, b);
-        // the group pass beside the inverse passes and the repair pass (none of
+        // the payload placement beside the inverse passes and the repair pass (none of
         // them reads or writes its staging slots, descriptors or archive
         // payload); the layout waits for it
-        const bool pack = p.group_pfx[J] != 0;
+        const bool pack = p.chunk_pfx[J] != 0;
         if (pack) {
             hip_check(hipEventRecord(pack_ready, s), "event record");
             hip_check(hipStreamWaitEvent(side, pack_ready, 0), "stream wait");
-            hipLaunchKernelGGL(batch_pack_kernel, dim3(p.group_pfx[J]), dim3(kPackThreads), 0, side, shape, comp,
-                               group_pfx, J, b);
+            hipLaunchKernelGGL(batch_pack_kernel, dim3(p.chunk_pfx[J]), dim3(256), 0, side, shape, comp, chunk_pfx,
+                               J, b);
             hip_check(hipEventRecord(pack_done, side), "event record");
         }
         const Banks bk{b.home, b.tmp0, b.tmp1, b.recon};
@@ -1913,7 +1901,6 @@ int waltz_amd_batch_compress_check(waltz_amd_batch* b, void* stream) {
                                : (st & wz::kRepairBound)    ? "native repair cannot meet strict bound or nonfinite reconstruction"
                                : (st & wz::kSideCapacity)   ? "portable GPU side-channel capacity reached"
                                : (st & wz::kWzpCapacity)    ? "archive capacity too small"
-                               : (st & wz::kLookbackTimeout) ? "WZP lookback did not complete"
                                                             : "Waltz device status error";
             throw std::runtime_error("job " + std::to_string(j) + ": " + what);
         }

@@ -457,11 +457,11 @@ int waltz_amd_wzp_encode(const void* mag, const void* sign, uint32_t n, void* ou
             throw std::runtime_error("wzp staging allocation failed");
         }
         wz::zero_words(scratch, (bytes + 512) / 4, s);
-        unsigned long long* desc = reinterpret_cast<unsigned long long*>(scratch);
+        uint32_t* glen = reinterpret_cast<uint32_t*>(scratch);
         uint32_t* size = reinterpret_cast<uint32_t*>(scratch + ws.chunks * 8ull) + ws.chunks;
-        uint32_t* tail = size + ws.chunks;  // ticket, status, pad, total(u64)
+        uint32_t* tail = size + ws.chunks;  // pad, status, pad, total(u64)
         unsigned long long* total = reinterpret_cast<unsigned long long*>(scratch + ((ws.chunks * 16ull + 16 + 7) & ~7ull));
-        wz::WzpScratch w{desc, staging, size, tail};
+        wz::WzpScratch w{glen, staging, size};
         wz::wzp_encode(static_cast<const uint16_t*>(mag), static_cast<const uint32_t*>(sign), n,
                        static_cast<uint8_t*>(out), capacity, w, tail + 1, s);
         wz::wzp_pack(n, static_cast<uint8_t*>(out), capacity, w, total, tail + 1, s);
@@ -472,7 +472,7 @@ int waltz_amd_wzp_encode(const void* mag, const void* sign, uint32_t n, void* ou
         wz::hip_check(hipStreamSynchronize(s), "wzp encode");
         hipFree(scratch);
         hipFree(staging);
-        if (st) throw std::runtime_error("WZP encode failed (capacity or lookback)");
+        if (st) throw std::runtime_error("WZP encode failed (capacity)");
         *written = n ? size_t(tot) : 0;
     });
 }

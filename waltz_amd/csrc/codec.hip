@@ -142,7 +142,6 @@ Geometry geometry(Dims d, unsigned width) {
     if (st & kRepairBound) throw std::runtime_error("native repair cannot meet strict bound or nonfinite reconstruction");
     if (st & kSideCapacity) throw std::runtime_error("portable GPU side-channel capacity reached");
     if (st & kWzpCapacity) throw std::runtime_error("archive capacity too small");
-    if (st & kLookbackTimeout) throw std::runtime_error("WZP lookback did not complete");
     if (st & kCorrupt) throw std::runtime_error("corrupt Waltz archive");
     if (st & kNonFiniteOutput) throw std::runtime_error("nonfinite reconstruction");
     throw std::runtime_error("Waltz device status error");
@@ -220,8 +219,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
             uint16_t* mag;
             uint32_t *sign, *qbm, *rbm, *qidx, *qval, *ridx, *rcount, *seg, *zeroed;
             T* rerr;
-            unsigned long long* desc;
-            uint32_t *size, *counters;
+            uint32_t *size, *counters, *glen;
             EncodeResult* res;
         } p;
         p.coeff = c.take<T>(n);
@@ -229,7 +227,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         p.t1 = c.take<T>(n);
         // the reconstruction and the encoder's staging slots: one region when
         // the last inverse pass detects the repairs (the reconstruction is
-        // never written then), else two, so that the WZP group pass can run
+        // never written then), else two, so that the WZP payload placement can run
         // beside the inverse
         if (fsegs) {
             p.rec = reinterpret_cast<T*>(
@@ -248,12 +246,12 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         p.qval = c.take<uint32_t>(nq);
         p.seg = c.take<uint32_t>(finish_scratch_words(n));
         p.size = c.take<uint32_t>(ws.chunks);
-        // zero-initialised region: sign, bitmaps, lookback descriptors, counters
+        // zero-initialised region: sign, bitmaps, group lengths, counters
         const size_t z0 = c.used;
         p.sign = c.take<uint32_t>(fusedq ? 0 : words);
         p.qbm = c.take<uint32_t>(words);
         if (shared_words) p.rbm = c.take<uint32_t>(words);
-        p.desc = c.take<unsigned long long>(ws.chunks);
+        p.glen = c.take<uint32_t>(ws.groups);
         p.counters = c.take<uint32_t>(4);  // ticket, q count, repair total
         p.res = c.take<EncodeResult>(1);
         p.zeroed = reinterpret_cast<uint32_t*>(c.base + z0);
@@ -271,19 +269,19 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
 
     transform_forward<T>(input, p.coeff, p.t0, p.t1, g.d, g.lx, g.lz, g.dyadic, status, s);
     SideList qo{p.qbm, p.qidx, p.qval, p.counters + 1, nq};
-    WzpScratch wsc{p.desc, p.stage, p.size, p.counters};
+    WzpScratch wsc{p.glen, p.stage, p.size};
     // with the fused repair emitter the finest level's high bands stay
     // unquantized in coeff; that kernel requantizes them on load
     const bool requant = g.dyadic && fsegs && tuning_for(g.d, g.lx, sizeof(T), true).fused;
-    // The group pass runs on the side stream beside the inverse levels (the
+    // The payload placement runs on the side stream beside the inverse levels (the
     // staging slots it reads are never written by them); the archive sections
     // wait for it.
     const SideStream* side = n >= kSideMin ? &w.side : nullptr;
     const SideJoin join{side};
     // When the coarser inverse levels requantize what they load as well (the
     // two leading levels fused), the encoder writes nothing back. They run
-    // after the encoder, beside its group pass: beside the encoder they slowed
-    // it as much as they hid, and the group pass then collided with the
+    // after the encoder, beside its payload placement: beside the encoder they slowed
+    // it as much as they hid, and the payload placement then collided with the
     // finest level, which needs every CU's two workgroup slots.
     const bool split = requant && coarse_split_fits(g.d, g.lx, sizeof(T));
     // a plane-schedule field whose inverse runs as fused XY levels quantizes

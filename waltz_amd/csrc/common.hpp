@@ -274,7 +274,6 @@ enum Status : uint32_t {
     kQuantDomain = 1u << 1,
     kRepairBound = 1u << 2,
     kWzpCapacity = 1u << 3,
-    kLookbackTimeout = 1u << 4,
     kCorrupt = 1u << 5,
     kNonFiniteOutput = 1u << 6,
     kSideCapacity = 1u << 7,

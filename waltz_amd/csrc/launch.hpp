@@ -206,12 +206,11 @@ void dequantize_bricks(const uint16_t* mag, const uint32_t* sign, const BrickGeo
 
 // wzp.hip
 struct WzpScratch {
-    unsigned long long* desc;  // groups lookback descriptors (zeroed)
+    uint32_t* glen;            // payload bytes of each group (zeroed; the encoders add to it)
     uint8_t* staging;          // wzp_staging_bytes(chunks): one payload slot per chunk
     uint32_t* size;            // chunks payload sizes
-    uint32_t* ticket;          // 1 counter (zeroed)
 };
-// A second stream for the WZP group pass, so that it runs beside the work
+// A second stream for the WZP payload placement, so that it runs beside the work
 // queued after the encoder on the caller's stream: the pass waits for `ready`
 // (recorded after the encoder) and records `done`, which the caller's stream
 // must wait for before it reads the stream's bytes or total.
@@ -227,7 +226,7 @@ inline uint64_t wzp_staging_bytes(uint32_t chunks) { return uint64_t(chunks) * k
 // into the scratch.
 void wzp_encode(const uint16_t* mag, const uint32_t* sign, uint32_t n, uint8_t* out, uint64_t capacity,
                 WzpScratch w, uint32_t* status, hipStream_t s);
-// The group pass after an encoder (directory, payloads in place, total bytes
+// The payload placement after an encoder (directory, payloads in place, total bytes
 // -> *total, a device u64), on `s` or on the side stream.
 void wzp_pack(uint32_t n, uint8_t* out, uint64_t capacity, const WzpScratch& w, unsigned long long* total,
               uint32_t* status, hipStream_t s, const SideStream* side = nullptr);

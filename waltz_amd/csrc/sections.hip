@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(1024) scan_layout_kernel(uint8_t* __restrict__
 }
 
 // The whole of it for a small field (at most kFinishSmall samples) by one
-// workgroup of 1024 threads: the WZP group pass (one group; with scratch),
+// workgroup of 1024 threads: the WZP payload placement (one group; with scratch),
 // ranks of both bitmaps in LDS, layout, placement. Four launches cost a field
 // of 2^15 samples more than the work they spread; from about 2^17 samples on
 // one workgroup's gathers take longer.
@@ -68,10 +68,10 @@ __global__ void __launch_bounds__(1024) finish_small_kernel(uint8_t* __restrict_
                                                             uint32_t n, SegList rp, SideList qo, uint8_t flags,
                                                             uint8_t lx, uint8_t lz, uint8_t bz, double quantum,
                                                             EncodeResult* res, EncodeResult* host, WzpScratch w) {
-    static_assert(kPackThreads == 1024 && kFinishSmall <= kGroup * kChunk, "one group");
+    static_assert(kFinishSmall <= kGroup * kChunk, "one group");
     if (w.staging) {
         const uint32_t chunks = (n + kChunk - 1) / kChunk;
-        pack_group(0, archive + 32, capacity - 32, chunks, 1, w, &res->wzp_bytes, &res->status);
+        pack_chunks<1024, kGroup>(0, archive + 32, capacity - 32, chunks, 1, w, &res->wzp_bytes, &res->status);
         __syncthreads();
     }
     __shared__ uint32_t pre[2][kFinishSmall / 32];
@@ -167,7 +167,7 @@ template <class T>
 void finish_archive(uint8_t* archive, uint64_t capacity, uint32_t n, SegList repairs, SideList qout, uint32_t* scratch,
                     uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz, double quantum, EncodeResult* result,
                     EncodeResult* host, hipStream_t s, const WzpScratch* pack) {
-    if (pack && n > kFinishSmall) throw std::logic_error("group pass deferred for a large field");
+    if (pack && n > kFinishSmall) throw std::logic_error("payload placement deferred for a large field");
     if (n <= kFinishSmall) {
         hipLaunchKernelGGL((finish_small_kernel<T>), dim3(1), dim3(1024), 0, s, archive, capacity, n, repairs, qout,
                            flags, lx, lz, bz, quantum, result, host, pack ? *pack : WzpScratch{});

@@ -10,11 +10,9 @@
 // bitmap B0 = one byte of B1. All counts are packed two per 32-bit word into
 // block-wide scans (wave shuffles + LDS). Each chunk writes its meta, its size
 // and its payload into a 16-byte aligned staging slot and ends; no workgroup
-// waits for another. A second kernel, one workgroup per 16-chunk group taken
-// in ticket order, finds the group's payload offset by a decoupled lookback
-// over group descriptors (aggregate / inclusive flags, relaxed agent-scope
-// atomics), writes the group directory entry and moves the group's payloads
-// from their slots to their final place in logical order.
+// waits for another. A second kernel (pack_chunks) moves the payloads from
+// their slots to their final place in logical order and writes the group
+// directory; its offsets are sums of the group lengths and chunk sizes.
 //
 // Decoder: one workgroup per chunk; the chunk offset is the group offset plus
 // the sizes of the earlier chunks of its group (from their metas). RZE is
@@ -37,14 +35,12 @@ __global__ void __launch_bounds__(256) wzp_encode_kernel(Source src, uint32_t n,
     encode_chunk(src, blockIdx.x, n, groups, out, capacity, w, status);
 }
 
+constexpr uint32_t kPackThreads = 256;
 __global__ void __launch_bounds__(kPackThreads) wzp_pack_kernel(uint8_t* __restrict__ out, uint64_t capacity,
                                                                 uint32_t chunks, uint32_t groups, WzpScratch w,
                                                                 unsigned long long* __restrict__ total,
                                                                 uint32_t* __restrict__ status) {
-    __shared__ uint32_t g_sh;
-    if (threadIdx.x == 0) g_sh = atomicAdd(w.ticket, 1u);
-    __syncthreads();
-    pack_group(g_sh, out, capacity, chunks, groups, w, total, status);
+    pack_chunks<kPackThreads, 1>(blockIdx.x, out, capacity, chunks, groups, w, total, status);
 }
 
 void wzp_pack(uint32_t n, uint8_t* out, uint64_t capacity, const WzpScratch& w, unsigned long long* total,
@@ -58,7 +54,7 @@ void wzp_pack(uint32_t n, uint8_t* out, uint64_t capacity, const WzpScratch& w, 
     }
     if (ws.chunks) {
         StageClock c("wzp_pack", ps);
-        hipLaunchKernelGGL(wzp_pack_kernel, dim3(ws.groups), dim3(kPackThreads), 0, ps, out, capacity, ws.chunks,
+        hipLaunchKernelGGL(wzp_pack_kernel, dim3(ws.chunks), dim3(kPackThreads), 0, ps, out, capacity, ws.chunks,
                            ws.groups, w, total, status);
     }
     if (side) hip_check(hipEventRecord(side->done, ps), "event record");

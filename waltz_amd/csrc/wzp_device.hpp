@@ -44,11 +44,6 @@ WZ_D uint32_t block_exclusive(uint32_t v, uint32_t* sh, uint32_t& total) {
 WZ_D uint32_t load24(const uint8_t* p) { return uint32_t(p[0]) | (uint32_t(p[1]) << 8) | (uint32_t(p[2]) << 16); }
 WZ_D uint32_t load32(const uint8_t* p) { return load24(p) | (uint32_t(p[3]) << 24); }
 
-constexpr unsigned long long kFlagAggregate = 1ull << 62;
-constexpr unsigned long long kFlagInclusive = 2ull << 62;
-constexpr unsigned long long kValueMask = (1ull << 62) - 1;
-constexpr uint32_t kSpinLimit = 1u << 26;
-
 WZ_D uint32_t chunk_elements(uint32_t n, uint32_t c) {
     const uint32_t rest = n - c * kChunk;
     return rest < kChunk ? rest : kChunk;

@@ -1,7 +1,7 @@
 // WZP encoder pieces shared by the single-field and batched pipelines:
 // encoder sources (packed magnitudes, or quantization of paired bricks on
-// the fly), the per-chunk encoder and the per-group pass (payload placement
-// by decoupled lookback). See wzp.hip for the stream format.
+// the fly), the per-chunk encoder and the payload placement. See wzp.hip for
+// the stream format.
 #pragma once
 
 #include "wzp_device.hpp"
@@ -355,9 +355,10 @@ WZ_D void encode_chunk(const Source& src, uint32_t c, uint32_t n, uint32_t group
         }
     }
 
-    // 5. size and meta of the chunk (its payload offset is found by the group pass)
+    // 5. size and meta of the chunk (its payload offset is found by the placement)
     if (t == 0) {
         w.size[c] = chunk_bytes;
+        if (chunk_bytes) atomicAdd(&w.glen[c / kGroup], chunk_bytes);
         if (uint64_t(groups) * 4 + uint64_t(c) * 3 + 3 <= capacity) {
             const uint32_t sign_code = sign_bytes == kSignSlot ? 0u : sign_bytes;
             const uint32_t meta = NNZ ? ((raw ? kRawCode : stored) | (sign_code << 14)) : 0u;
@@ -449,96 +450,49 @@ WZ_D void encode_chunk(const Source& src, uint32_t c, uint32_t n, uint32_t group
     for (uint32_t q = t; q < (chunk_bytes + 15) / 16; q += kThreads) slot[q] = reinterpret_cast<const uint4*>(ob32)[q];
 }
 
-// Group pass (cpu/src/wzp_cpu.cpp:789-830 for the directory): workgroup =
-// one 16-chunk group, in ticket order. Wave 0 scans the group's chunk sizes
-// and publishes the group length; the whole workgroup looks back over the
-// earlier groups' descriptors (one per thread per round trip, nearest
-// inclusive prefix by ballots, block reduction of the aggregates up to it).
-// Descriptors are the only data passed between workgroups, so relaxed
-// agent-scope atomics suffice (the slots were written by the previous
-// kernel). Then the group's directory entry (offset of its first payload
-// byte, 0 for an empty group) and its payloads, moved
-// from the slots with 16-byte stores over funnel-shifted 16-byte loads.
-constexpr uint32_t kPackThreads = 1024, kPackUnroll = 4;
-// Group g (taken in ticket order by the caller: every earlier group of the
-// stream is held by a running workgroup) by a workgroup of kPackThreads threads.
-WZ_D void pack_group(uint32_t g, uint8_t* __restrict__ out, uint64_t capacity, uint32_t chunks, uint32_t groups,
-                     const WzpScratch& w, unsigned long long* __restrict__ total, uint32_t* __restrict__ status) {
+// Payload placement after the encoders (cpu/src/wzp_cpu.cpp:789-830 for the
+// directory): a workgroup of `Threads` threads owns up to `Per` chunks of one
+// 16-chunk group. Its offset is the sum of the earlier groups' lengths, which
+// the encoders added up, and of its group's earlier sizes; no workgroup waits
+// for another. Then the payloads move from the slots with 16-byte stores over
+// funnel-shifted 16-byte loads, the first chunk's workgroup writes the group's
+// directory entry (offset of its first payload byte, 0 for an empty group),
+// and the last chunk's the stream's size. Bound by memory latency: one round
+// trip for lengths and sizes, one for a chunk's payload. A workgroup of 1024
+// threads per group, placed by a decoupled lookback, left most of the chip
+// idle: with one of 256 per chunk 128^3 floats take 10 instead of 25 us,
+// 500x500x100 floats 19 instead of 73, 384x384x96 doubles 17 instead of 91.
+// Four chunks a workgroup cost the 512^3 compress 15 us more.
+constexpr uint32_t kPackUnroll = 4;
+template <uint32_t Threads, uint32_t Per>
+WZ_D void pack_chunks(uint32_t c0, uint8_t* __restrict__ out, uint64_t capacity, uint32_t chunks, uint32_t groups,
+                      const WzpScratch& w, unsigned long long* __restrict__ total, uint32_t* __restrict__ status) {
+    static_assert(kGroup % Per == 0, "a workgroup's chunks lie in one group");
     __shared__ uint32_t off_sh[kGroup + 1];  // chunk offsets inside the group; [kGroup] = group length
-    __shared__ uint32_t qpre[kGroup + 1];    // 16-byte destination groups before each chunk
-    __shared__ uint32_t ok_sh, wait_sh;
-    __shared__ uint32_t near_w[kPackThreads / 64];        // per wave: nearest inclusive lane (or 64)
-    __shared__ unsigned long long part_w[kPackThreads / 64];
-    __shared__ unsigned long long excl_sh;
+    __shared__ uint32_t qpre[Per + 1];       // 16-byte destination groups before each of its chunks
+    __shared__ unsigned long long part_w[Threads / 64];
     const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
-    const uint32_t first = g * kGroup, count = min(kGroup, chunks - first);
+    const uint32_t g = c0 / kGroup, first = g * kGroup, count = min(kGroup, chunks - first), in = c0 - first;
     const uint64_t header = uint64_t(groups) * 4 + uint64_t(chunks) * 3;
-    // the group's chunk offsets and length (wave 0), published at once
+    unsigned long long acc = 0;
+    for (uint32_t i = t; i < g; i += Threads) acc += w.glen[i];
     if (t < 64) {
         const uint32_t size = lane < count ? w.size[first + lane] : 0u;
         const uint32_t incl = wave_inclusive(size);
         if (lane <= kGroup) off_sh[lane] = incl - size;  // lane kGroup: the group length
-        if (lane == 63)
-            __hip_atomic_store(&w.desc[g], (g == 0 ? kFlagInclusive : kFlagAggregate) | incl, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
     }
-    __syncthreads();
-    const uint32_t glen = off_sh[kGroup];
-    // decoupled lookback with the whole workgroup: thread t reads the
-    // descriptor of group j - t, so one round trip covers kPackThreads groups;
-    // stop at the nearest inclusive prefix and sum the aggregates up to it
-    unsigned long long acc = 0;
-    if (g > 0) {
-        int64_t j = int64_t(g) - 1;
-        uint32_t spins = 0;
-        for (;;) {
-            const int64_t idx = j - int64_t(t);
-            const unsigned long long d =
-                idx >= 0 ? __hip_atomic_load(&w.desc[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                         : kFlagInclusive;  // nothing before group 0
-            const unsigned long long flag = d & ~kValueMask;
-            const unsigned long long im = __ballot(flag == kFlagInclusive);
-            if (lane == 0) near_w[wv] = im ? uint32_t(__ffsll((long long)im) - 1) : 64u;
-            if (t == 0) wait_sh = 0;
-            __syncthreads();
-            uint32_t stop = kPackThreads;  // block position of the nearest inclusive descriptor
-            for (uint32_t k = 0; k < kPackThreads / 64; ++k)
-                if (near_w[k] < 64) {
-                    stop = 64 * k + near_w[k];
-                    break;
-                }
-            if (t <= stop && flag == 0) wait_sh = 1;  // a descriptor we need is not published yet
-            unsigned long long v = t <= stop ? (d & kValueMask) : 0ull;
 #pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-            if (lane == 0) part_w[wv] = v;
-            __syncthreads();
-            const bool wait = wait_sh != 0;
-            unsigned long long sum = 0;
-            for (uint32_t k = 0; k < kPackThreads / 64; ++k) sum += part_w[k];
-            __syncthreads();  // near_w / part_w / wait_sh are rewritten by the next round
-            if (wait) {
-                if (++spins > kSpinLimit) {
-                    if (t == 0) atomicOr(status, uint32_t(kLookbackTimeout));
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-                continue;
-            }
-            acc += sum;
-            if (stop < kPackThreads) break;
-            j -= kPackThreads;
-        }
-        if (t == 0)
-            __hip_atomic_store(&w.desc[g], kFlagInclusive | (acc + glen), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if (lane == 0) part_w[wv] = acc;
+    __syncthreads();
+    acc = 0;
+    for (uint32_t k = 0; k < Threads / 64; ++k) acc += part_w[k];
+    const uint32_t glen = off_sh[kGroup];
+    const bool fits = header + acc + glen <= capacity;
     if (t == 0) {
-        excl_sh = acc;
-        const bool fits = header + acc + glen <= capacity;
-        ok_sh = fits;
         if (!fits) atomicOr(status, uint32_t(kWzpCapacity));
-        if (g == groups - 1) *total = header + acc + glen;
-        if (uint64_t(g) * 4 + 4 <= capacity) {
+        if (c0 + Per >= chunks) *total = header + acc + glen;
+        if (in == 0 && uint64_t(g) * 4 + 4 <= capacity) {
             const uint32_t off = glen ? uint32_t(acc) : 0u;
             uint8_t* p = out + uint64_t(g) * 4;
             p[0] = uint8_t(off);
@@ -547,19 +501,19 @@ WZ_D void pack_group(uint32_t g, uint8_t* __restrict__ out, uint64_t capacity, u
             p[3] = uint8_t(off >> 24);
         }
     }
+    if (!fits) return;
     if (t < 64) {  // destination 16-byte groups per chunk, then their prefix
-        const uint32_t size = lane < kGroup ? off_sh[lane + 1] - off_sh[lane] : 0u;
-        const uint64_t dst0 = reinterpret_cast<uintptr_t>(out) + header + acc + (lane < kGroup ? off_sh[lane] : 0u);
-        const uint32_t lead = uint32_t(dst0 & 15u);
+        const uint32_t c = in + min(lane, Per - 1);
+        const uint32_t size = lane < Per ? off_sh[c + 1] - off_sh[c] : 0u;
+        const uint32_t lead = uint32_t((reinterpret_cast<uintptr_t>(out) + header + acc + off_sh[c]) & 15u);
         const uint32_t nq = size ? (lead + size + 15) / 16 : 0u;
         const uint32_t qi = wave_inclusive(nq);
-        if (lane <= kGroup) qpre[lane] = qi - nq;
+        if (lane <= Per) qpre[lane] = qi - nq;
     }
     __syncthreads();
-    if (!ok_sh) return;
-    // every destination group of every chunk of the group, kPackUnroll per
-    // thread per round with all their loads issued before any store
-    const uint32_t all = qpre[kGroup];
+    // every destination group of the chunks, kPackUnroll per thread per round
+    // with all their loads issued before any store
+    const uint32_t all = qpre[Per];
     struct Unit {
         uint8_t* dst;        // 16-byte aligned destination group
         const uint8_t* src;  // the chunk's slot
@@ -569,21 +523,21 @@ WZ_D void pack_group(uint32_t g, uint8_t* __restrict__ out, uint64_t capacity, u
     auto unit = [&](uint32_t u) {
         uint32_t i = 0;
 #pragma unroll
-        for (uint32_t k = 1; k < kGroup; ++k) i += u >= qpre[k] ? 1u : 0u;
-        uint8_t* const d = out + header + excl_sh + off_sh[i];
+        for (uint32_t k = 1; k < Per; ++k) i += u >= qpre[k] ? 1u : 0u;
+        uint8_t* const d = out + header + acc + off_sh[in + i];
         const uint32_t lead = uint32_t(reinterpret_cast<uintptr_t>(d) & 15u);
         const uint32_t q = u - qpre[i];
-        return Unit{d - lead + 16 * q, w.staging + uint64_t(first + i) * kChunkSlot, int32_t(16 * q) - int32_t(lead),
-                    off_sh[i + 1] - off_sh[i]};
+        return Unit{d - lead + 16 * q, w.staging + uint64_t(c0 + i) * kChunkSlot, int32_t(16 * q) - int32_t(lead),
+                    off_sh[in + i + 1] - off_sh[in + i]};
     };
     // the archive is not read again here: non-temporal stores (staging keeps
     // ordinary loads, which neighbouring destination groups share)
     using U4 = uint32_t __attribute__((ext_vector_type(4)));
-    for (uint32_t u0 = t; u0 < all; u0 += kPackThreads * kPackUnroll) {
+    for (uint32_t u0 = t; u0 < all; u0 += Threads * kPackUnroll) {
         U4 lo[kPackUnroll], hi[kPackUnroll];
 #pragma unroll
         for (uint32_t r = 0; r < kPackUnroll; ++r) {
-            const uint32_t u = u0 + r * kPackThreads;
+            const uint32_t u = u0 + r * Threads;
             if (u >= all) break;
             const Unit x = unit(u);
             if (x.o >= 0 && uint32_t(x.o) + 16 <= x.size) {  // the 16 bytes lie in two aligned 16-byte loads
@@ -593,7 +547,7 @@ WZ_D void pack_group(uint32_t g, uint8_t* __restrict__ out, uint64_t capacity, u
         }
 #pragma unroll
         for (uint32_t r = 0; r < kPackUnroll; ++r) {
-            const uint32_t u = u0 + r * kPackThreads;
+            const uint32_t u = u0 + r * Threads;
             if (u >= all) break;
             const Unit x = unit(u);
             if (x.o >= 0 && uint32_t(x.o) + 16 <= x.size) {
