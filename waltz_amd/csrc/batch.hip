@@ -491,7 +491,7 @@ __global__ void __launch_bounds__(256) batch_pass_kernel(const JobShape* __restr
     if (__ballot(!fin) && (threadIdx.x & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteOutput));
 }
 
-constexpr uint32_t kRecords = 4;         // consecutive repair records per thread and round
+constexpr uint32_t kRecords = 8;         // repair records per thread and round
 constexpr uint32_t kRpatchBlocks = 2048;  // fixed grid (the record count is known on the device only)
 
 template <class T>
@@ -500,31 +500,57 @@ __global__ void __launch_bounds__(256) batch_rpatch_kernel(const uint8_t* __rest
                                                            const JobRun* __restrict__ run,
                                                            const uint32_t* __restrict__ np_pfx, uint32_t jobs,
                                                            T* __restrict__ out, uint32_t* status) {
-    // each thread takes kRecords consecutive records (of one job or a few)
-    // per round: one job search, then a walk to the next job
-    const uint32_t total = np_pfx[jobs];
-    for (uint32_t k0 = (blockIdx.x * 256u + threadIdx.x) * kRecords; k0 < total;
-         k0 += gridDim.x * 256u * kRecords) {
-        uint32_t j = job_of(np_pfx, jobs, k0);
-        for (uint32_t k = k0; k < min(k0 + kRecords, total); ++k) {
-            while (k >= np_pfx[j + 1]) ++j;  // jobs without repairs are skipped
-            const uint32_t e = k - np_pfx[j];
-            const JobRun& r = run[j];
-            const JobShape& sh = shape[j];
+    // a wave takes 64 * kRecords consecutive records, a lane every 64th of
+    // them: their indexes and errors, then their samples, are all in flight
+    // at once. A record is a chain of two scattered reads, so one after the
+    // other the pass was bound by their latency (256 float chunks, 96 M
+    // samples: 102 us, now 80: partial lines read and written at memory).
+    const uint32_t total = np_pfx[jobs], lane = threadIdx.x & 63u;
+    const uint32_t wave = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint64_t base = uint64_t(wave) * 64u * kRecords; base < total; base += uint64_t(gridDim.x) * 256u * kRecords) {
+        const uint32_t b0 = uint32_t(base), b1 = min(b0 + 64u * kRecords, total);
+        const uint32_t j0 = __builtin_amdgcn_readfirstlane(job_of_wave(np_pfx, jobs, b0));
+        const bool one = b1 <= np_pfx[j0 + 1];  // the usual case: scalar job data
+        uint32_t j = j0;
+        uint32_t jr[kRecords], at[kRecords];
+        T err[kRecords], v[kRecords];
+        uint64_t o[kRecords];
+        uint32_t kept = 0;  // bit u: record u changes a sample
+#pragma unroll
+        for (uint32_t u = 0; u < kRecords; ++u) {
+            const uint32_t k = min(b0 + 64u * u + lane, b1 - 1u);
+            if (!one)
+                while (k >= np_pfx[j + 1]) ++j;  // jobs without repairs are skipped
+            jr[u] = one ? j0 : j;
+            const JobRun& r = run[jr[u]];
             const uint8_t* a = packed + r.arc;
-            const uint32_t i = reinterpret_cast<const uint32_t*>(a + r.pi)[e];
-            const T err = reinterpret_cast<const T*>(a + r.pv)[e];
-            if (i >= sh.n || !__builtin_isfinite(err)) {
-                atomicOr(status, uint32_t(kCorrupt));
-                continue;
-            }
-            const uint32_t x = i % sh.d.nx, y = (i / sh.d.nx) % sh.d.ny, z = i / (sh.d.nx * sh.d.ny);
-            if (x >= sh.clip.nx || y >= sh.clip.ny || z >= sh.clip.nz) continue;
-            T* o = out + sh.out + uint64_t(z) * sh.opz + uint64_t(y) * sh.opy + x;
-            const T v = *o - err;  // cpu/src/codec.cpp:330
-            *o = v;
-            if (!__builtin_isfinite(v)) atomicOr(status, uint32_t(kNonFiniteOutput));
+            const uint32_t e = k - np_pfx[jr[u]];
+            at[u] = reinterpret_cast<const uint32_t*>(a + r.pi)[e];
+            err[u] = reinterpret_cast<const T*>(a + r.pv)[e];
         }
+        bool corrupt = false, fin = true;
+#pragma unroll
+        for (uint32_t u = 0; u < kRecords; ++u) {
+            const bool in = b0 + 64u * u + lane < b1;
+            const JobShape& sh = shape[jr[u]];
+            const uint32_t i = at[u];
+            const bool bad = i >= sh.n || !__builtin_isfinite(err[u]);
+            corrupt = corrupt || (in && bad);
+            const uint32_t x = i % sh.d.nx, y = (i / sh.d.nx) % sh.d.ny, z = i / (sh.d.nx * sh.d.ny);
+            const bool put = in && !bad && x < sh.clip.nx && y < sh.clip.ny && z < sh.clip.nz;
+            kept |= uint32_t(put) << u;
+            o[u] = sh.out + (put ? uint64_t(z) * sh.opz + uint64_t(y) * sh.opy + x : 0u);
+            v[u] = out[o[u]];  // (any sample of the tile, where none is kept)
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kRecords; ++u) {
+            if (!((kept >> u) & 1u)) continue;
+            const T w = v[u] - err[u];  // cpu/src/codec.cpp:330
+            out[o[u]] = w;
+            fin = fin && __builtin_isfinite(w);
+        }
+        if (corrupt) atomicOr(status, uint32_t(kCorrupt));
+        if (!fin) atomicOr(status, uint32_t(kNonFiniteOutput));
     }
 }
 
