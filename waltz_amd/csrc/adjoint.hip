@@ -34,7 +34,7 @@
 #include "fused.hpp"
 #include "launch.hpp"
 #include "lifting.hpp"
-#include "xystrip.hpp"
+#include "planetail.hpp"
 
 namespace wz {
 namespace {
@@ -358,16 +358,23 @@ Box<T> compact(T* p, Dims n) { return {p, n.nx, uint64_t(n.nx) * n.ny}; }
 
 // in: the samples' gradient (OfInverse) or the split one, its low box `lo`
 template <class T, bool OfInverse>
+using XYLevel = std::conditional_t<OfInverse, XYForward<T>, XYInverse<T>>;
+template <class T, bool OfInverse>
+XYLevel<T, OfInverse> level_of(Box<T> in, Box<T> lo, Box<T> out, Dims n) {
+    if constexpr (OfInverse) return {in.p, in.py, in.pz, out.p, out.py, out.pz, lo.p, lo.py, lo.pz, n, nullptr};
+    else return {in.p, in.py, in.pz, lo.p, lo.py, lo.pz, out.p, out.py, out.pz, n, T(0), T(0), 0u};
+}
+template <class T, bool OfInverse>
 void xy_level(Box<T> in, Box<T> lo, Box<T> out, Dims n, hipStream_t s) {
     const StripPlan p = strip_plan(n, strips_pack(std::max({in.pz, lo.pz, out.pz}), sizeof(T)));
-    const dim3 grid(strip_blocks(p)), block(kStripThreads);
-    if constexpr (OfInverse) {
-        const XYForward<T> a{in.p, in.py, in.pz, out.p, out.py, out.pz, lo.p, lo.py, lo.pz, n, nullptr};
-        hipLaunchKernelGGL((adjoint_xy_kernel<T, true>), grid, block, 0, s, a, p);
-    } else {
-        const XYInverse<T> a{in.p, in.py, in.pz, lo.p, lo.py, lo.pz, out.p, out.py, out.pz, n, T(0), T(0), 0u};
-        hipLaunchKernelGGL((adjoint_xy_kernel<T, false>), grid, block, 0, s, a, p);
-    }
+    hipLaunchKernelGGL((adjoint_xy_kernel<T, OfInverse>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s,
+                       (level_of<T, OfInverse>(in, lo, out, n)), p);
+}
+template <class T, bool OfInverse>
+void xy_tail(const PlaneTail<T, XYLevel<T, OfInverse>>& t, uint32_t planes, hipStream_t s) {
+    const dim3 grid(planes), block(64 * kPlaneTailWaves);
+    if constexpr (OfInverse) hipLaunchKernelGGL((plane_tail_forward_kernel<T, true>), grid, block, 0, s, t);
+    else hipLaunchKernelGGL((plane_tail_inverse_kernel<T, false, true>), grid, block, 0, s, t);
 }
 // nat: the samples along z; hi, lo: the split and its low box of lx x ly columns
 template <class T, bool OfInverse>
@@ -394,8 +401,9 @@ bool levels_fit(Dims full, unsigned lxy, unsigned lz, unsigned width) {
 
 // The transforms' schedules reversed, from `src` into `data` (which may be the
 // same). The high bands of a level go to (or come from) their place in a full
-// volume, its low box to a compact one: odd levels' at the start of tmp1, even
-// ones' after the largest odd one (lines of at least 2 samples: both fit).
+// volume, its low box to a compact one in tmp1: odd levels' at its start, even
+// ones' after the largest odd one (lines of at least 2 samples: both fit), the
+// plane schedule's XY boxes one after the other.
 template <class T, bool OfInverse>
 void adjoint_levels(T* data, const T* src, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz, bool dyadic,
                     hipStream_t s) {
@@ -449,15 +457,25 @@ void adjoint_levels(T* data, const T* src, T* tmp0, T* tmp1, Dims full, unsigned
             z_level<T, OfInverse>(nat, split, last ? split : low_of(l + 1, false, true), n, n.nx, n.ny, s);
         }
     };
+    // (the tail takes each plane through several levels: no two levels' boxes
+    // may share memory)
+    auto plane_box = [&](unsigned l) { return compact(xy_box(tmp1, full, l), box_of(l, true, false)); };
     auto xy_phase = [&](Box<T> in, Box<T> out) {
+        const unsigned tail = plane_tail_level(full, lxy);
+        PlaneTail<T, XYLevel<T, OfInverse>> pt{};
         for (unsigned k = 0; k < lxy; ++k) {
             const unsigned l = OfInverse ? k : lxy - 1 - k;
             const Dims n = box_of(l, true, false);
             const Box<T> split = OfInverse ? out : in;
-            const Box<T> nat = l ? low_of(l, true, false) : OfInverse ? in : out;
-            const Box<T> lo = l + 1 == lxy ? split : low_of(l + 1, true, false);
-            if constexpr (OfInverse) xy_level<T, true>(nat, lo, split, n, s);
-            else xy_level<T, false>(split, lo, nat, n, s);
+            const Box<T> nat = l ? plane_box(l) : OfInverse ? in : out;
+            const Box<T> lo = l + 1 == lxy ? split : plane_box(l + 1);
+            const Box<T> from_box = OfInverse ? nat : split, to_box = OfInverse ? split : nat;
+            if (l < tail) {
+                xy_level<T, OfInverse>(from_box, lo, to_box, n, s);
+            } else {
+                add_plane(pt, level_of<T, OfInverse>(from_box, lo, to_box, n));
+                if (l == (OfInverse ? lxy - 1 : tail)) xy_tail<T, OfInverse>(pt, full.nz, s);
+            }
         }
     };
     const Box<T> in = volume(from, full);

@@ -29,6 +29,7 @@
 #include "fused.hpp"
 #include "launch.hpp"
 #include "lifting.hpp"
+#include "planetail.hpp"
 #include "profile.hpp"
 #include "xystrip.hpp"
 #include "zcolumns.hpp"
@@ -421,61 +422,6 @@ void tail_inverse(Tail<T> t, Dims full, const WaveRepair<T>* repair, hipStream_t
     }
 }
 
-// The coarsest XY levels of the plane schedule in one launch: a plane's levels
-// depend on nothing else, so a workgroup takes a plane through all levels
-// whose boxes are at most kPlaneTailSamples, with a barrier between them
-// (planes of 128 x 128 still fill the device better as launches of their own).
-constexpr uint32_t kPlaneTailSamples = 4096, kPlaneTailWaves = 8;
-template <class T, class Level>
-struct PlaneTail {
-    uint32_t levels;
-    Level level[5];  // in launch order
-    StripPlan plan[5];  // of one plane
-};
-template <class T>
-__global__ void __launch_bounds__(64 * kPlaneTailWaves) plane_tail_forward_kernel(PlaneTail<T, XYForward<T>> a) {
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), z = blockIdx.x;
-    for (uint32_t l = 0; l < a.levels; ++l) {
-        XYForward<T> xy = a.level[l];
-        xy.src += uint64_t(z) * xy.spz;
-        xy.hi += uint64_t(z) * xy.hpz;
-        xy.lo += uint64_t(z) * xy.lpz;
-        xy.n.nz = 1;
-        for (uint32_t i = wave; i < a.plan[l].items(); i += kPlaneTailWaves) strip_forward<T>(xy, a.plan[l], i);
-        __syncthreads();
-    }
-}
-template <class T, bool Requant>
-__global__ void __launch_bounds__(64 * kPlaneTailWaves) plane_tail_inverse_kernel(PlaneTail<T, XYInverse<T>> a) {
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), z = blockIdx.x;
-    for (uint32_t l = 0; l < a.levels; ++l) {
-        XYInverse<T> xy = a.level[l];
-        xy.hi += uint64_t(z) * xy.hpz;
-        xy.lo += uint64_t(z) * xy.lpz;
-        xy.out += uint64_t(z) * xy.opz;
-        xy.n.nz = 1;
-        for (uint32_t i = wave; i < a.plan[l].items(); i += kPlaneTailWaves)
-            strip_inverse<T, Requant>(xy, a.plan[l], i, StripStore<T>{});
-        __syncthreads();
-    }
-}
-// First level of that tail (lxy: none; one level alone is launched as usual).
-unsigned plane_tail_level(Dims full, unsigned lxy) {
-    Dims n = full;
-    for (unsigned l = 0; l + 1 < lxy; ++l) {
-        if (uint64_t(n.nx) * n.ny <= kPlaneTailSamples) return l;
-        n = shrink(n, true, false);
-    }
-    return lxy;
-}
-template <class T, class Level>
-void add_plane(PlaneTail<T, Level>& t, const Level& a) {
-    Dims n = a.n;
-    n.nz = 1;
-    t.plan[t.levels] = strip_plan(n, false, kPlaneTailWaves, 16);
-    t.level[t.levels++] = a;
-}
-
 // The X and Y passes of box `act` (in full-pitched arrays, src != dst) as one
 // launch, in the order the strips lift (forward Y then X, inverse X then Y);
 // false for the other order and for boxes that strips do not take.
@@ -491,21 +437,6 @@ bool xy_pair(const T* src, T* dst, Dims full, Dims act, int a0, uint32_t* status
         xy_forward<T>(XYForward<T>{src, py, pz, dst, py, pz, dst, py, pz, act, status}, s);
     }
     return true;
-}
-
-// Compact XY boxes of the plane schedule's levels >= 1 (every plane), one after
-// the other in `scratch`: a launch that takes a plane through several levels
-// must not write one level's box where another plane still reads a finer or
-// coarser one. Their sum stays below the field (each is at most 4/9 of the one
-// before, for extents of at least 2).
-template <class T>
-T* xy_box(T* scratch, Dims full, unsigned l) {
-    Dims n = full;
-    for (unsigned k = 1; k < l; ++k) {
-        n = shrink(n, true, false);
-        scratch += uint64_t(n.nx) * n.ny * n.nz;
-    }
-    return scratch;
 }
 
 template <class T>
@@ -908,7 +839,7 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
         }
         if (pt.levels) {
             StageClock clock("forward_tail", s);
-            hipLaunchKernelGGL((plane_tail_forward_kernel<T>), dim3(full.nz), dim3(64 * kPlaneTailWaves), 0, s, pt);
+            hipLaunchKernelGGL((plane_tail_forward_kernel<T, false>), dim3(full.nz), dim3(64 * kPlaneTailWaves), 0, s, pt);
         }
         return;
     }
@@ -1030,9 +961,9 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
                 if (l == tail) {
                     const dim3 grid(full.nz), block(64 * kPlaneTailWaves);
                     if (requant > 0)
-                        hipLaunchKernelGGL((plane_tail_inverse_kernel<T, true>), grid, block, 0, s, pt);
+                        hipLaunchKernelGGL((plane_tail_inverse_kernel<T, true, false>), grid, block, 0, s, pt);
                     else
-                        hipLaunchKernelGGL((plane_tail_inverse_kernel<T, false>), grid, block, 0, s, pt);
+                        hipLaunchKernelGGL((plane_tail_inverse_kernel<T, false, false>), grid, block, 0, s, pt);
                 }
             } else {
                 xy_inverse<T>(a, s);
@@ -1098,12 +1029,11 @@ bool transform_inverse_preserving(const T* coeff, T* output, T* tmp0, T* tmp1, D
     const Tuning tu = tuning_for(full, lxy, sizeof(T), true);
     if (!lxy || !tu.fused || output == coeff) return false;
     const Dims h1 = shrink(full, true, true);
-    copy_box<T>(coeff, output, full, h1, s);
-    LowBox<T> low = inverse_coarse_levels<T>(output, tmp0, tmp1, full, lxy, s);
-    if (low.p == output) {  // the finest level's coarse input would be overwritten as it stores
-        copy_box<T>(output, tmp1, full, h1, s);
-        low.p = tmp1;
-    }
+    // the coarser levels work on a copy of their box, with the output as a
+    // scratch volume: the finest level reads their result as it stores
+    copy_box<T>(coeff, tmp1, full, h1, s);
+    const LowBox<T> low = inverse_coarse_levels<T>(tmp1, tmp0, output, full, lxy, s);
+    if (low.p == output) throw std::logic_error("coarse levels ended in the output");
     const Level0Emit<T> store{kEmitStore, nullptr, nullptr, 0.0, SegList{}, 0.0};
     inverse_finest_level<T>(coeff, low, output, full, lxy, store, s);
     return true;
