@@ -88,6 +88,15 @@ WZB_HD void bit2_forward_pair(const uint32_t (&m)[32], uint32_t (&planes)[16]) {
     for (int q = 0; q < 16; ++q) planes[q] = bitrev32((m[15 - q] << 16) | m[31 - q]);
     transpose16x2(planes);
 }
+// Which of the pair's 32 magnitudes are not zero (bit i: m[i]), from its planes:
+// plane bit j belongs to magnitude 15 - j of its block.
+WZB_HD uint32_t pair_nonzero(const uint32_t (&planes)[16]) {
+    uint32_t any = 0;
+#pragma unroll
+    for (int p = 0; p < 16; ++p) any |= planes[p];
+    const uint32_t r = bitrev32(any);
+    return (r >> 16) | (r << 16);
+}
 // Inverse of bit2_forward_pair.
 WZB_HD void bit2_inverse_pair(const uint32_t (&planes)[16], uint32_t (&m)[32]) {
     uint32_t a[16];

@@ -99,6 +99,18 @@ WZP_HD constexpr uint32_t direct_rank(uint32_t dx, uint32_t r) {
     return Cube ? subblock_rank(dx, r & 3u, r >> 2)
                 : (dx & 1u) | ((r & 1u) << 1) | ((dx >> 1) << 2) | (((r >> 1) & 1u) << 3) | ((r >> 2) << 4);
 }
+// The same the other way round.
+template <bool Cube>
+WZP_HD constexpr void direct_place(uint32_t rank, uint32_t& dx, uint32_t& r) {
+    auto bit = [rank](uint32_t k) { return (rank >> k) & 1u; };
+    if (Cube) {
+        dx = bit(0) | bit(3) << 1;
+        r = bit(1) | bit(4) << 1 | bit(2) << 2;
+    } else {
+        dx = bit(0) | bit(2) << 1;
+        r = bit(1) | bit(3) << 1 | bit(4) << 2;
+    }
+}
 
 // Chunk <-> brick map of the other fields of full bricks (z bands that are no
 // power of two, doubles of a band below 16): brick b of the row-major brick
