@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(1024) batch_plan_kernel(const uint8_t* __restr
 
 // Chunks of the jobs with edge bricks (mag_pfx counts only theirs):
 // magnitudes and signs, dequantized by batch_dequant_kernel.
-__global__ void __launch_bounds__(256) batch_wzp_kernel(const uint8_t* __restrict__ packed,
+__global__ void __launch_bounds__(256, 8) batch_wzp_kernel(const uint8_t* __restrict__ packed,
                                                         const JobShape* __restrict__ shape,
                                                         const JobRun* __restrict__ run,
                                                         const uint32_t* __restrict__ mag_pfx, uint32_t jobs,
@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(256) batch_wzp_kernel(const uint8_t* __restric
 // other powers of two else): decoded straight into dequantized coefficients,
 // as the single-field decoder's BrickSink does.
 template <class T, bool Cube>
-__global__ void __launch_bounds__(256) batch_wzp_direct_kernel(const uint8_t* __restrict__ packed,
+__global__ void __launch_bounds__(256, 8) batch_wzp_direct_kernel(const uint8_t* __restrict__ packed,
                                                                const JobShape* __restrict__ shape,
                                                                const JobRun* __restrict__ run,
                                                                const uint32_t* __restrict__ pfx, uint32_t jobs,
@@ -270,7 +270,7 @@ constexpr uint64_t kRankSet = 2ull * 8 * 8192;  // u16 entries per set (rank + i
 // Chunks of the other full-brick jobs (rank_pfx): decoded straight into
 // dequantized coefficients, as the single-field decoder's RankSink does.
 template <class T>
-__global__ void __launch_bounds__(256) batch_wzp_ranks_kernel(const uint8_t* __restrict__ packed,
+__global__ void __launch_bounds__(256, 8) batch_wzp_ranks_kernel(const uint8_t* __restrict__ packed,
                                                               const JobShape* __restrict__ shape,
                                                               const JobRun* __restrict__ run,
                                                               const uint32_t* __restrict__ rank_pfx, uint32_t jobs,

@@ -119,7 +119,7 @@ void quantize_encode_ranks(T* coeff, Dims d, uint32_t bz, const uint16_t* rank, 
 }
 
 template <class Sink>
-__global__ void __launch_bounds__(256) wzp_decode_kernel(const uint8_t* __restrict__ in, uint64_t bytes, uint32_t n,
+__global__ void __launch_bounds__(256, 8) wzp_decode_kernel(const uint8_t* __restrict__ in, uint64_t bytes, uint32_t n,
                                                          uint32_t chunks, uint32_t groups, Sink sink,
                                                          uint32_t* __restrict__ status) {
     decode_chunk(in, bytes, n, chunks, groups, blockIdx.x, sink, status);
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(kDirThreads) directory_qpatch_planned_kernel(T
 }
 
 template <class T, bool Cube>
-__global__ void __launch_bounds__(256) wzp_decode_direct_planned_kernel(const uint8_t* __restrict__ in,
+__global__ void __launch_bounds__(256, 8) wzp_decode_direct_planned_kernel(const uint8_t* __restrict__ in,
                                                                        const DecodeRecord* __restrict__ rec,
                                                                        uint32_t n, uint32_t chunks, uint32_t groups,
                                                                        T* __restrict__ coeff, DirectBricks g,
@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(256) wzp_decode_direct_planned_kernel(const ui
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) wzp_decode_ranks_planned_kernel(const uint8_t* __restrict__ in,
+__global__ void __launch_bounds__(256, 8) wzp_decode_ranks_planned_kernel(const uint8_t* __restrict__ in,
                                                                       const DecodeRecord* __restrict__ rec,
                                                                       uint32_t n, uint32_t chunks, uint32_t groups,
                                                                       T* __restrict__ coeff, RankBricks g,
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(256) wzp_decode_ranks_planned_kernel(const uin
     decode_chunk(in, rec->wzp, n, chunks, groups, blockIdx.x, RankSink<T>{coeff, g, T(rec->quantum)}, status);
 }
 
-__global__ void __launch_bounds__(256) wzp_decode_mag_planned_kernel(const uint8_t* __restrict__ in,
+__global__ void __launch_bounds__(256, 8) wzp_decode_mag_planned_kernel(const uint8_t* __restrict__ in,
                                                                     const DecodeRecord* __restrict__ rec, uint32_t n,
                                                                     uint32_t chunks, uint32_t groups, MagSink sink,
                                                                     uint32_t* __restrict__ status) {
