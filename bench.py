@@ -266,8 +266,8 @@ STAGE_KERNEL = {
     "inverse_L0_repairs": "wz::inv_level_kernel<float, 2, true, true, false>",
     "inverse_L0": "wz::inv_level_kernel<float, 1, false, true, true>",
     "forward_L0": "wz::fwd_level_kernel<float>",
-    "decode_dequantize": "wz::wzp_decode_pairs_planned_kernel<float>",
-    "quantize_encode": "wz::wzp_encode_kernel<wz::BrickSource<float> >",
+    "decode_dequantize": "wz::wzp_decode_direct_planned_kernel<float, true>",
+    "quantize_encode": "wz::wzp_encode_kernel<wz::BrickSource<float, true> >",
 }
 
 

@@ -9,10 +9,10 @@
 //   -> side channels ordered by index into their sections, header, padding.
 // One 48-byte status/result read back at the end decides success.
 //
-// Decompress (cpu/src/codec.cpp:276-336): 32-byte header read and validated on
-// the host, WZP decode, dequantization into row-major coefficients, q-outlier
-// patches, inverse lifting into the caller's output, repair patches, finite
-// screen.
+// Decompress (cpu/src/codec.cpp:276-336): 32-byte header validated on the device
+// (on the host for a side list out of order), WZP decode, dequantization into
+// row-major coefficients, q-outlier patches, inverse lifting into the caller's
+// output, repair patches, finite screen.
 //
 // Scratch lives in one cached, grow-only device allocation per device.
 #include <hip/hip_runtime.h>

@@ -1,5 +1,11 @@
 // CDF 9/7 lifting passes for gfx950.
 //
+// The plane schedule is one pass over all Z levels (zcolumns.hpp) and one launch
+// per XY level (xystrip.hpp), its coarse planes in one (planetail.hpp); a dyadic
+// level is one fused launch (fused.hip), or a Z axis pass and one XY launch, the
+// coarsest boxes in one workgroup. What none of these fits is left to the axis
+// passes:
+//
 // One launch lifts one axis of the active low box [0,act.nx)x[0,act.ny)x[0,act.nz)
 // of a full row-major volume (x fastest), out of place: src -> dst, both with
 // the full volume's strides. Each thread owns one canonical tile of one line:
