@@ -11,11 +11,13 @@
 //            it against the job's shape and span, and scans the side-channel
 //            counts over jobs;
 //   wzp      one workgroup per WZP chunk of every job (the single-field
-//            chunk decoder, writing into the job's magnitude/sign banks);
-//   dequant  one workgroup per Morton brick (rank computed on the fly);
+//            chunk decoder: straight into the coefficient bank for fields of
+//            full bricks, else into the job's magnitude/sign banks);
+//   dequant  bricks of the jobs with edge bricks;
 //   qpatch   q-outliers of all jobs, grid-stride;
-//   passes   the inverse lifting schedule, one launch per schedule step, each
-//            job running its own axis, box and tile size at that step; the
+//   passes   the inverse lifting schedule, a launch of XY strips, of Z columns
+//            and of what is left per schedule step, each job running its own
+//            box at that step; the
 //            job's last pass writes straight into the output with clipping
 //            (holes are filled there);
 //   rpatch   native repairs of all jobs into the output.
@@ -883,8 +885,10 @@ __global__ void __launch_bounds__(256) batch_place_kernel(const JobShape* __rest
 // Strip passes (one XY level of a job's box, xystrip.hpp) and column passes
 // (Z levels, zcolumns.hpp) over all jobs, each one launch per step. Bound by
 // memory; staging whole planes and columns in LDS was bound by vector issue:
-// 256 chunks (94 M float samples) decoded 1310 -> 862 us, 64 chunks compressed
-// 765 -> 550 us.
+// 256 chunks (96 M float samples) decoded 1310 -> 862 us, 64 chunks compressed
+// 765 -> 550 us. A workgroup per plane taking the coarse levels in one launch,
+// as the single-field path does, is slower here: there are planes enough to
+// fill a launch per level (decode 835 -> 956 us).
 enum : uint8_t { kPassStrip = 6, kPassZCol = 7 };
 
 // Banks of these passes: input (compress forward), the three work banks, the
