@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <vector>
 
+#include "../waltz_amd/csrc/bits.hpp"
 #include "../waltz_amd/csrc/pairbrick.hpp"
 
 using namespace wz;
@@ -49,8 +50,35 @@ static int check(uint32_t nx, uint32_t ny, uint32_t nz, uint32_t bz) {
     return bad;
 }
 
-int main() {
+// The sample a rank belongs to, and the nonzero mask of a pair of bit planes.
+template <bool Cube>
+static int check_places() {
     int bad = 0;
+    for (uint32_t i = 0; i < 32; ++i) {
+        uint32_t dx, r;
+        direct_place<Cube>(i, dx, r);
+        bad += dx > 3 || r > 7 || direct_rank<Cube>(dx, r) != i;
+    }
+    return bad;
+}
+static int check_nonzero() {
+    int bad = 0;
+    uint32_t x = 12345;
+    for (int it = 0; it < 20000; ++it) {
+        uint32_t m[32], planes[16], nz = 0;
+        for (int i = 0; i < 32; ++i) {
+            x = x * 1664525u + 1013904223u;
+            m[i] = it < 32 ? uint32_t(i == it) << (it & 15) : (x >> 30) ? 0u : (x >> 8 & 0xFFFFu) >> (x >> 4 & 15u);
+            nz |= uint32_t(m[i] != 0) << i;
+        }
+        bit2_forward_pair(m, planes);
+        bad += pair_nonzero(planes) != nz;
+    }
+    return bad;
+}
+
+int main() {
+    int bad = check_places<true>() + check_places<false>() + check_nonzero();
     bad += check<true>(48, 32, 32, 16) + check<true>(16, 16, 16, 16);
     for (uint32_t bz : {1u, 2u, 4u, 8u})
         bad += check<false>(48, 32, 3 * bz, bz) + check<false>(16, 16, bz, bz) + check<false>(112, 48, 5 * bz, bz);
