@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(1024) finish_small_kernel(uint8_t* __restrict_
 }
 
 // Both side channels to their index-order slots in one launch: item
-// g < segments * kPlaceSlices places repairs of segment g / kPlaceSlices,
+// g < segments * slices places repairs of segment g / slices,
 // the remaining kPlaceQBlocks place q-outliers. Items map to workgroups
 // XCD-aware: the dispatcher deals workgroups round-robin to the 8 XCDs, and
 // XCD k takes the k-th contiguous range of items instead, so the slices of
@@ -146,10 +146,10 @@ template <class T>
 __global__ void __launch_bounds__(256) place_kernel(uint8_t* __restrict__ archive, SegList rp, Ranks rr, SideList qo,
                                                     Ranks qr, const EncodeResult* __restrict__ res) {
     if (res->status) return;
-    const uint32_t rblocks = rp.segments * kPlaceSlices, per = gridDim.x / 8;
+    const uint32_t slices = place_slices(rp.segments), rblocks = rp.segments * slices, per = gridDim.x / 8;
     const uint32_t g = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
     if (g >= rblocks + kPlaceQBlocks) return;
-    if (g < rblocks) place_repairs<T>(archive, rp, rr, res, g / kPlaceSlices, g % kPlaceSlices);
+    if (g < rblocks) place_repairs<T>(archive, rp, rr, res, g / slices, g % slices, slices);
     else place_qoutliers(archive, qo, qr, uint64_t(sizeof(T)), res, g - rblocks);
 }
 
@@ -184,7 +184,7 @@ void finish_archive(uint8_t* archive, uint64_t capacity, uint32_t n, SegList rep
     hipLaunchKernelGGL((scan_layout_kernel<T>), dim3(1), dim3(1024), 0, s, archive, capacity, n,
                        const_cast<uint32_t*>(rr.bsum), const_cast<uint32_t*>(qr.bsum), blocks, np_total, qout, flags,
                        lx, lz, bz, quantum, result, host);
-    const uint32_t items = repairs.segments * kPlaceSlices + kPlaceQBlocks;
+    const uint32_t items = repairs.segments * place_slices(repairs.segments) + kPlaceQBlocks;
     hipLaunchKernelGGL((place_kernel<T>), dim3(8 * ((items + 7) / 8)), dim3(256), 0, s,
                        archive, repairs, rr, qout, qr, result);
 }

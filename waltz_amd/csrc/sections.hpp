@@ -240,12 +240,23 @@ struct Ranks {
 };
 
 // Repairs: segment k's entries go to their index-order rank (bitmap popcounts);
-// gridDim.y workgroups share a segment so that enough index -> rank -> store
-// chains are in flight.
-constexpr uint32_t kPlaceSlices = 8;
+// `slices` workgroups share a segment so that enough index -> rank -> store
+// chains are in flight: bound by that chain's latency where segments are few
+// and large, by the dispatch of workgroups that find next to nothing where
+// they are many. 500x500x100 floats have 4000 segments: with eight workgroups
+// each the list kernels (word_prefix2 to place_kernel) take 40.5 us, with one
+// 23.7; 384x384x96 doubles, 2304 segments, 32.9 and 22.6;
+// 200x210x190 doubles 22.8 and 18.3. Segments few enough keep eight (512^3
+// floats, 512 segments: the same 58.6). A target of 12288 workgroups instead
+// of 4096: 24.3, 25.4, 22.7 and the same.
+constexpr uint32_t kPlaceTarget = 4096;  // workgroups
+WZ_HD uint32_t place_slices(uint32_t segments) {
+    const uint32_t s = kPlaceTarget / (segments ? segments : 1u);
+    return s < 1 ? 1u : s > 8 ? 8u : s;
+}
 template <class T>
 WZ_D void place_repairs(uint8_t* __restrict__ archive, SegList rp, Ranks rank, const EncodeResult* __restrict__ res,
-                        uint32_t k, uint32_t slice, uint32_t slices = kPlaceSlices) {
+                        uint32_t k, uint32_t slice, uint32_t slices) {
     const uint32_t c = rp.count[k];
     if (!c) return;
     const uint32_t np = res->np;
