@@ -1130,7 +1130,7 @@ std::vector<Pass> inverse_schedule(const JobShape& sh, unsigned width, uint32_t 
             out.push_back(strip_pass(sh, kHome, 0, low, at, 0, xy[0], width, jobs));
         }
     }
-    if (sh.lz && zcol_fits(sh.d.nz, width)) {
+    if (sh.lz && zcol_lds_fits(sh.d.nz, width)) {
         const uint8_t dst = column_output_fits(sh, width) ? uint8_t(kOutput) : at == kHome ? uint8_t(kTmp1) : uint8_t(kHome);
         out.push_back(column_pass(at, dst, sh.d, sh.lz));
         at = dst;
@@ -1181,7 +1181,7 @@ std::vector<Pass> forward_schedule(const JobShape& sh, unsigned width, uint32_t 
         return out;
     }
     const uint8_t zdst = sh.lx ? uint8_t(kTmp1) : uint8_t(kHome);
-    if (sh.lz && zcol_fits(sh.d.nz, width)) {
+    if (sh.lz && zcol_lds_fits(sh.d.nz, width)) {
         out.push_back(column_pass(src, zdst, sh.d, sh.lz));
         src = zdst;
     } else {

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "windows.hpp"
 
 namespace wz {
 
@@ -17,13 +18,6 @@ struct FwdLevel {
     uint32_t sz;        // z segment length (even)
     uint32_t* status;   // non-null: screen the input for non-finite samples
 };
-
-// Whether `rows` rows of pitch `pitch` elements of `width` bytes stay below
-// 4 GiB less 1 MiB (the level kernels' 32-bit byte offsets within a plane,
-// with room above the plane for the offset that masks a lane off).
-inline bool fused_plane_fits(uint64_t pitch, uint64_t rows, uint64_t width) {
-    return pitch * rows * width <= (uint64_t(1) << 32) - (uint64_t(1) << 20);
-}
 
 enum InvEmit : int {
     kEmitStore = 0,        // write the reconstruction

@@ -1,0 +1,37 @@
+// Which volumes the kernels with 32-bit byte offsets take. Host code without
+// HIP, so that a CPU test checks the rules against the offsets.
+#pragma once
+
+#include <cstdint>
+
+namespace wz {
+
+// Whether `rows` rows of pitch `pitch` elements of `width` bytes stay below
+// 4 GiB less 1 MiB (the level kernels' 32-bit byte offsets within a plane,
+// with room above the plane for the offset that masks a lane off).
+inline bool fused_plane_fits(uint64_t pitch, uint64_t rows, uint64_t width) {
+    return pitch * rows * width <= (uint64_t(1) << 32) - (uint64_t(1) << 20);
+}
+
+// Column passes (zcolumns.hpp): LDS of the low boxes between the levels, 64
+// columns of ceil(nz/2) and ceil(nz/4) samples.
+constexpr uint32_t kZColumns = 64;
+inline uint64_t zcol_lds_bytes(uint32_t nz, unsigned levels, unsigned width) {
+    if (levels < 2) return 0;
+    const uint32_t n1 = nz - nz / 2, n2 = levels > 2 ? n1 - n1 / 2 : 0u;
+    return uint64_t(n1 + n2) * kZColumns * width;
+}
+// 64 KiB of LDS: nz up to 340 (float) or 170 (double) whatever the levels
+inline bool zcol_lds_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5, width) <= 65536; }
+// Whether the Z phase of an nx x ny x nz volume runs as columns, ...
+inline bool zcol_fits(uint32_t nx, uint32_t ny, uint32_t nz, unsigned width) {
+    return zcol_lds_fits(nz, width) && fused_plane_fits(nx, ny, width);
+}
+// ... and whether it has to address every plane through a window of its own:
+// one window (of 2^32 - 1 bytes, no lane masked off by its offset) holds every
+// field of the codec, but not every volume of the transforms.
+inline bool zcol_wide(uint32_t nx, uint32_t ny, uint32_t nz, unsigned width) {
+    return uint64_t(nx) * ny > 0xFFFFFFFFull / width / nz;
+}
+
+}  // namespace wz

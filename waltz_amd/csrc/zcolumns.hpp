@@ -7,6 +7,7 @@
 #include "common.hpp"
 #include "lifting.hpp"
 #include "repair.hpp"
+#include "windows.hpp"
 
 namespace wz {
 
@@ -25,16 +26,8 @@ namespace wz {
 // every column staged in LDS and per-lane index arithmetic it was bound by
 // vector issue: 500x500x100 float 108 -> 55 us (forward), 127 -> 61 us
 // (inverse), 384x384x96 double 70 -> 56 us, 73 -> 67 us.
-constexpr uint32_t kZColumns = 64, kZThreads = 256;
-inline uint64_t zcol_lds_bytes(uint32_t nz, unsigned levels, unsigned width) {
-    if (levels < 2) return 0;
-    const uint32_t n1 = half_len(nz), n2 = levels > 2 ? half_len(n1) : 0u;
-    return uint64_t(n1 + n2) * kZColumns * width;
-}
-// 64 KiB of LDS: nz up to 341 (float) or 170 (double) whatever the levels
-inline bool zcol_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5, width) <= 65536; }
+constexpr uint32_t kZThreads = 256;
 
-//
 // Repair (inverse, compress): the reconstruction is not written; each sample
 // is compared with the original as its tile is lifted, and the native repair
 // records and flag bits go out (one segment per workgroup, columns x nz slots).
@@ -107,7 +100,7 @@ struct ZOutput {
 };
 // The source and destination volumes of a column pass (pitches in elements;
 // nz planes of either, but only 16 of an inverse's destination, inside one
-// 32-bit byte window) and the box lifted.
+// 32-bit byte window; Wide: one plane of either) and the box lifted.
 template <class T>
 struct ZColumnsOf {
     const T* src;
@@ -120,12 +113,15 @@ struct ZColumnsOf {
 
 // Row y, columns x0 .. x0 + 63 by one workgroup of kZThreads threads; `box0`,
 // `box1`: zcol_lds_bytes of LDS. Returns whether this lane met nothing to flag
-// (a non-finite sample of a screened pass, or an unmet bound).
-template <class T, bool Inverse, bool Repair>
+// (a non-finite sample of a screened pass, or an unmet bound). Wide: volumes
+// past one window, every plane through its own (3370x3300x99 float, 4.4 GB:
+// forward 2.2 ms, 4.0 TB/s).
+template <class T, bool Inverse, bool Repair, bool Wide = false>
 WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0, T* box1, bool screen,
                        const ZOutput<T>& out, const WaveRepair<T>& rp, uint32_t id, uint32_t* seg_fill) {
     constexpr int Tile = sizeof(T) == 4 ? 16 : 8, P = Tile / 2 + 4;  // (the inverse's is part of the format)
     constexpr uint32_t W = kZThreads / 64, S = sizeof(T);
+    static_assert(!(Repair && Wide), "the codec's fields fit one window");
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const uint32_t x = x0 + lane;
     const bool in = x < a.n.nx;
@@ -133,6 +129,16 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
     const uint32_t xc = in ? x : a.n.nx - 1u;
     const uint32_t scol = (y * a.spy + xc) * S, dcol = (y * a.dpy + xc) * S;
     const auto ws = window(a.src), wd = window(Repair ? rp.orig : a.dst);
+    // plane z of the source / destination, `at`: its offset inside one window
+    auto load = [&](uint32_t z, uint32_t at) {
+        if constexpr (Wide) return buf_load<T>(window(a.src + uint64_t(z) * a.spz), scol);
+        else return buf_load_at(T(0), ws, scol, at);
+    };
+    auto row = [&](uint32_t z) { return load(z, z * splane); };
+    auto store = [&](T v, uint32_t z, uint32_t at) {
+        if constexpr (Wide) buf_store(v, window(a.dst + uint64_t(z) * a.dpz), dcol);
+        else buf_store_at(v, wd, dcol, at);
+    };
     // the finest inverse store's lanes and rows
     const bool put = Inverse ? x < out.clip.nx && y < out.clip.ny : in;
     const int32_t rows = int32_t(Inverse ? out.clip.nz : a.n.nz);
@@ -156,15 +162,15 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
                         uint32_t at = uint32_t(2 * k0) * splane;
 #pragma unroll
                         for (int j = 0; j < P; ++j) {
-                            e[j] = buf_load_at(T(0), ws, scol, at);
-                            o[j] = buf_load_at(T(0), ws, scol, at + splane);
+                            e[j] = load(uint32_t(2 * (k0 + j)), at);
+                            o[j] = load(uint32_t(2 * (k0 + j) + 1), at + splane);
                             at += 2 * splane;
                         }
                     } else {
 #pragma unroll
                         for (int j = 0; j < P; ++j) {
-                            e[j] = buf_load_at(T(0), ws, scol, uint32_t(2 * pair_even(k0 + j, n)) * splane);
-                            o[j] = buf_load_at(T(0), ws, scol, uint32_t(2 * pair_odd(k0 + j, n) + 1) * splane);
+                            e[j] = row(uint32_t(2 * pair_even(k0 + j, n)));
+                            o[j] = row(uint32_t(2 * pair_odd(k0 + j, n) + 1));
                         }
                     }
                     if (screen) {
@@ -186,9 +192,9 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
                 for (int j = 2; j < P - 2; ++j) {
                     if (2 * (k0 + j) < n) {
                         if (!coarsest) b[uint32_t(j - 2) * kZColumns] = e[j];
-                        else if (in) buf_store_at(e[j], wd, dcol, at);
+                        else if (in) store(e[j], uint32_t(k0 + j), at);
                     }
-                    if (2 * (k0 + j) + 1 < n && in) buf_store_at(o[j], wd, dcol, up);
+                    if (2 * (k0 + j) + 1 < n && in) store(o[j], uint32_t(k0 + j + h), up);
                     at += dplane;
                     up += dplane;
                 }
@@ -197,16 +203,16 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
                     uint32_t at = uint32_t(k0) * splane, up = uint32_t(k0 + h) * splane;
 #pragma unroll
                     for (int j = 0; j < P; ++j) {
-                        if (coarsest) e[j] = buf_load_at(T(0), ws, scol, at);
-                        o[j] = buf_load_at(T(0), ws, scol, up);
+                        if (coarsest) e[j] = load(uint32_t(k0 + j), at);
+                        o[j] = load(uint32_t(k0 + j + h), up);
                         at += splane;
                         up += splane;
                     }
                 } else {
 #pragma unroll
                     for (int j = 0; j < P; ++j) {
-                        if (coarsest) e[j] = buf_load_at(T(0), ws, scol, uint32_t(pair_even(k0 + j, n)) * splane);
-                        o[j] = buf_load_at(T(0), ws, scol, uint32_t(h + pair_odd(k0 + j, n)) * splane);
+                        if (coarsest) e[j] = row(uint32_t(pair_even(k0 + j, n)));
+                        o[j] = row(uint32_t(h + pair_odd(k0 + j, n)));
                     }
                 }
                 T ref[Repair ? Tile : 1];  // the tile's originals, in flight with its coefficients
@@ -249,7 +255,8 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
                     continue;
                 }
                 // (a tile's rows only inside one window: frames may be large)
-                const auto wt = window(a.dst + uint64_t(tile * uint32_t(Tile)) * a.dpz);
+                const uint32_t z0 = tile * uint32_t(Tile);
+                const auto wt = window(a.dst + uint64_t(z0) * a.dpz);
                 uint32_t at = 0;
 #pragma unroll
                 for (int j = 2; j < P - 2; ++j) {
@@ -257,7 +264,10 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
                     for (int b = 0; b < 2; ++b) {
                         if (2 * (k0 + j) + b < rows) {
                             const T v = out.hole ? out.fill : b ? o[j] : e[j];
-                            if (put) buf_store_at(v, wt, dcol, at);
+                            if (put) {
+                                if constexpr (Wide) store(v, uint32_t(2 * (k0 + j) + b), 0u);
+                                else buf_store_at(v, wt, dcol, at);
+                            }
                             if (out.screen) fin = fin && (finite_value(v) || !put || out.hole);
                         }
                         at += dplane;
