@@ -246,7 +246,7 @@ struct ZLevel {
 };
 
 // A lane streams one column of the box (columns counted row by row), two
-// planes a step, as the strips stream rows; ends weighted as there.
+// planes a step, as the strips stream rows; ends as there (mirror_lift).
 template <class T, bool OfInverse>
 __global__ void __launch_bounds__(256) adjoint_z_kernel(ZLevel<T> a) {
     using C = Lift<T>;
@@ -295,39 +295,40 @@ __global__ void __launch_bounds__(256) adjoint_z_kernel(ZLevel<T> a) {
     load(g, buf[0]);
     load(g + 1, buf[1]);
     load(g + 2, buf[2]);
+    const uint32_t images = line_images(nz);
     auto block = [&](bool emit) {
 #pragma unroll
         for (int u = 0; u < 4; ++u, ++g) {
             load(g + 3, buf[(u + 3) & 3]);
-            const T we = end_load<T>(2 * uint32_t(pair_even(g, nz)), n.nz);
-            const T wo = end_load<T>(2 * uint32_t(pair_odd(g, nz)) + 1u, n.nz);
             const uint32_t k = uint32_t(g - 2);
-            const T ve = end_store<T>(2 * k, n.nz), vo = end_store<T>(2 * k + 1u, n.nz);
-            const T e = buf[u][0] * we, o = buf[u][1] * wo;
+            const T e = buf[u][0], o = buf[u][1];
             T r0, r1;  // pair g - 2
-            if constexpr (OfInverse) {
-                const T e1 = fmadd(-C::a, s0 + o, e);
-                const T o1 = fmadd(-C::b, s1 + e1, s0);
-                const T e2 = fmadd(-C::g, s2 + o1, s1);
-                r0 = s3 * (C::ik * ve);
-                r1 = fmadd(-C::d, s3 + e2, s2) * (-C::k * vo);
-                s0 = o;
-                s1 = e1;
-                s2 = o1;
-                s3 = e2;
-            } else {
-                const T ev = e * C::k, ov = o * (-C::ik);
-                const T o1 = fmadd(C::d, s4 + ev, s0);
-                const T e1 = fmadd(C::g, s1 + o1, s4);
-                const T o2 = fmadd(C::b, s2 + e1, s1);
-                r0 = fmadd(C::a, s3 + o2, s2) * ve;
-                r1 = o2 * vo;
-                s4 = ev;
-                s0 = ov;
-                s1 = o1;
-                s2 = e1;
-                s3 = o2;
-            }
+            mirror_stream(g, nz, images, [&](const MirrorSteps& m, auto ends_c) {
+                constexpr bool ends = decltype(ends_c)::value;
+                if constexpr (OfInverse) {
+                    const T e1 = mirror_lift<ends>(-C::a, s0, o, e, m, 5);
+                    const T o1 = mirror_lift<ends>(-C::b, s1, e1, s0, m, 4);
+                    const T e2 = mirror_lift<ends>(-C::g, s2, o1, s1, m, 3);
+                    r0 = s3 * C::ik;
+                    r1 = mirror_lift<ends>(-C::d, s3, e2, s2, m, 2) * (-C::k);
+                    s0 = o;
+                    s1 = e1;
+                    s2 = o1;
+                    s3 = e2;
+                } else {
+                    const T ev = e * C::k, ov = o * (-C::ik);
+                    const T o1 = mirror_lift<ends>(C::d, s4, ev, s0, m, 4);
+                    const T e1 = mirror_lift<ends>(C::g, s1, o1, s4, m, 3);
+                    const T o2 = mirror_lift<ends>(C::b, s2, e1, s1, m, 2);
+                    r0 = mirror_lift<ends>(C::a, s3, o2, s2, m, 1);
+                    r1 = o2;
+                    s4 = ev;
+                    s0 = ov;
+                    s1 = o1;
+                    s2 = e1;
+                    s3 = o2;
+                }
+            });
             if (!emit) continue;
             if constexpr (OfInverse) {
                 if (2 * k < n.nz) {

@@ -111,37 +111,108 @@ WZ_D void strip_x_forward(T& e, T& o, bool first, bool last) {
     o = o3 * (-C::ik);
 }
 
+// A lifting step on a mirrored line adds c (l + r) of a sample's neighbours to
+// it. Its transpose adds c (u l + v r): a sample next to an end of the line
+// counts the end twice (the end's own step read that sample twice), and an end,
+// whose two neighbours are mirror images of each other, counts them once. In
+// terms of t += scale c (l' + r'), l' and r' halved or not, so that nothing is
+// doubled before it is multiplied: what fits the type before a step and after
+// it fits inside it too, as it does without mirroring.
+struct MirrorSteps {
+    uint32_t two, left, right;  // bit k, for position q0 + k: scale of 2; l, r halved
+};
+// Bit k: position q0 + k is an end of a line of n >= 2 samples or the mirror
+// image of one (up to four samples outside the line, more on shorter lines).
+// `images`: line_images(n).
+WZ_HD uint32_t line_images(int32_t n) {  // of lines below 9 samples, bit q + 16
+    uint32_t m = 0;
+    if (n < 9)
+        for (int32_t q = -16; q < 16; ++q) m |= uint32_t(q % (n - 1) == 0) << (q + 16);
+    return m;
+}
+WZ_HD uint32_t line_ends(int32_t q0, int32_t n, uint32_t images) {
+    if (images) return images >> min(uint32_t(q0 + 16), 31u);
+    const uint32_t a = uint32_t(-q0), b = uint32_t(n - 1 - q0);
+    return (a < 32u ? 1u << a : 0u) | (b < 32u ? 1u << b : 0u);
+}
+WZ_HD MirrorSteps mirror_steps(uint32_t ends) {
+    const uint32_t l = ends << 1, r = ends >> 1;
+    return {l | r, ends | (r & ~l), ends | (l & ~r)};
+}
+// f(steps, true_type) when the stream's step of pair g touches an end, else
+// f(steps, false_type); position 2g - 5 is bit 0.
+template <class F>
+WZ_D void mirror_stream(int32_t g, int32_t n, uint32_t images, F&& f) {
+    const uint32_t ends = line_ends(2 * g - 5, n, images) & 0x7Fu;
+    if (ends) f(mirror_steps(ends), std::true_type{});
+    else f(MirrorSteps{0, 0, 0}, std::false_type{});
+}
+// v 2^e (neither zero nor near the ends of the range), on the exponent: scalar
+// arithmetic where both are wave-uniform.
+WZ_D float times_power(float v, uint32_t e) {
+    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) + (e << 23));
+}
+WZ_D double times_power(double v, uint32_t e) {
+    return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, v) + (uint64_t(e << 20) << 32));
+}
+// The step into position k of wave-uniform `m`; Ends: not known to be empty.
+template <bool Ends, class T>
+WZ_D T mirror_lift(T c, T l, T r, T t, const MirrorSteps& m, int k) {
+    if constexpr (!Ends) return fmadd(c, l + r, t);
+    auto bit = [k](uint32_t w) { return (w >> k) & 1u; };
+    const T fl = times_power(T(1), 0u - bit(m.left)), fr = times_power(T(1), 0u - bit(m.right));
+    return fmadd(times_power(c, bit(m.two)), fmadd(l, fl, r * fr), t);
+}
+// The same of the four steps of a pair's two samples (even: steps into the even
+// one) with per-lane positions, kept in registers.
+template <class T, bool OfInverse>
+struct MirrorLine {
+    T l[2], r[2];    // factors of a neighbour, into the even / odd sample
+    T c[4];          // coefficients of the steps in their order
+    WZ_D static MirrorLine of(int32_t q, int32_t n) {
+        using C = Lift<T>;
+        MirrorLine a;
+        const MirrorSteps m = mirror_steps(line_ends(q - 1, n, line_images(n)));  // (q: bit 1)
+        const T plain[4] = {OfInverse ? -C::a : C::d, OfInverse ? -C::b : C::g, OfInverse ? -C::g : C::b,
+                            OfInverse ? -C::d : C::a};
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            a.l[p] = (m.left >> (p + 1)) & 1u ? T(0.5) : T(1);
+            a.r[p] = (m.right >> (p + 1)) & 1u ? T(0.5) : T(1);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int p = OfInverse ? k & 1 : 1 - (k & 1);  // of the inverse: into the even sample first
+            a.c[k] = (m.two >> (p + 1)) & 1u ? T(2) * plain[k] : plain[k];
+        }
+        return a;
+    }
+    WZ_D T lift(int k, T left, T right, T t) const {
+        const int p = OfInverse ? k & 1 : 1 - (k & 1);
+        return fmadd(c[k], fmadd(left, l[p], right * r[p]), t);
+    }
+};
 // The transposed steps of the inverse / forward X lifting (Adjoint in
 // strip_forward and strip_inverse).
 template <class T>
-WZ_D void strip_x_inverse_adjoint(T& e, T& o, bool first, bool last) {
+WZ_D void strip_x_inverse_adjoint(T& e, T& o, bool first, bool last, const MirrorLine<T, true>& m) {
     using C = Lift<T>;
-    const T e1 = fmadd(-C::a, lane_prev(o, first) + o, e);
-    const T o1 = fmadd(-C::b, e1 + lane_next(e1, last), o);
-    const T e2 = fmadd(-C::g, lane_prev(o1, first) + o1, e1);
-    const T o2 = fmadd(-C::d, e2 + lane_next(e2, last), o1);
+    const T e1 = m.lift(0, lane_prev(o, first), o, e);
+    const T o1 = m.lift(1, e1, lane_next(e1, last), o);
+    const T e2 = m.lift(2, lane_prev(o1, first), o1, e1);
+    const T o2 = m.lift(3, e2, lane_next(e2, last), o1);
     e = e2 * C::ik;
     o = o2 * (-C::k);
 }
 template <class T>
-WZ_D void strip_x_forward_adjoint(T& e, T& o, bool first, bool last) {
+WZ_D void strip_x_forward_adjoint(T& e, T& o, bool first, bool last, const MirrorLine<T, false>& m) {
     using C = Lift<T>;
     const T e0 = e * C::k, o0 = o * (-C::ik);
-    const T o1 = fmadd(C::d, e0 + lane_next(e0, last), o0);
-    const T e1 = fmadd(C::g, lane_prev(o1, first) + o1, e0);
-    o = fmadd(C::b, e1 + lane_next(e1, last), o1);
-    e = fmadd(C::a, lane_prev(o, first) + o, e1);
+    const T o1 = m.lift(0, e0, lane_next(e0, last), o0);
+    const T e1 = m.lift(1, lane_prev(o1, first), o1, e0);
+    o = m.lift(2, e1, lane_next(e1, last), o1);
+    e = m.lift(3, lane_prev(o, first), o, e1);
 }
-// Weights that turn a mirrored lifting step into the transpose of one. With
-// M the step on a mirrored line and W halving the line's two end samples,
-// M^T = W M' W^-1, M' the mirrored step with the roles of the parities
-// exchanged (an end sample is its own mirror image and is counted once where
-// the others count twice). So the ends are doubled as they load and halved as
-// they store, both exact, and everything between is ordinary lifting.
-template <class T>
-WZ_D T end_load(uint32_t p, uint32_t n) { return p == 0 || p == n - 1u ? T(2) : T(1); }
-template <class T>
-WZ_D T end_store(uint32_t p, uint32_t n) { return p == 0 || p == n - 1u ? T(0.5) : T(1); }
 
 // Two consecutive samples (dword-aligned).
 WZ_D void buf_load_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, float& a, float& b) {
@@ -353,9 +424,9 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
     T OS[2], EA[2], OB[2], EC[2], SF[2];  // Y state, as the fused level's Z synthesis
 #pragma unroll
     for (int c = 0; c < 2; ++c) OS[c] = EA[c] = OB[c] = EC[c] = SF[c] = T(0);
-    [[maybe_unused]] const T cw[2] = {end_load<T>(reflect_pos(int32_t(2 * it.kp), n.nx), n.nx),
-                                      end_load<T>(reflect_pos(int32_t(2 * it.kp + 1), n.nx), n.nx)};
-    [[maybe_unused]] const T cs[2] = {end_store<T>(2 * it.kp, n.nx), end_store<T>(2 * it.kp + 1, n.nx)};
+    std::conditional_t<Adjoint, MirrorLine<T, false>, int> line{};
+    if constexpr (Adjoint) line = MirrorLine<T, false>::of(int32_t(2 * it.kp), int32_t(n.nx));
+    [[maybe_unused]] const uint32_t images = Adjoint ? line_images(ny) : 0u;
     T buf[4][4];
     int32_t g = int32_t(it.ys / 2) - 2;
     load(g, buf[0]);
@@ -374,31 +445,25 @@ WZ_D void strip_inverse(const XYInverse<T>& a, const StripPlan& p, uint32_t item
             }
             T re[2], ro[2];
             if constexpr (Adjoint) {
-                const T re0 = end_load<T>(2 * uint32_t(pair_even(g, ny)), n.ny);
-                const T ro0 = end_load<T>(2 * uint32_t(pair_odd(g, ny)) + 1u, n.ny);
-                const uint32_t y = 2 * uint32_t(g - 2);
-                const T se = end_store<T>(y, n.ny), so = end_store<T>(y + 1u, n.ny);
+                strip_x_forward_adjoint(v[0], v[1], it.first, it.last, line);
+                strip_x_forward_adjoint(v[2], v[3], it.first, it.last, line);
+                mirror_stream(g, ny, images, [&](const MirrorSteps& m, auto ends_c) {
+                    constexpr bool ends = decltype(ends_c)::value;
 #pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    v[c] *= cw[c] * re0;
-                    v[2 + c] *= cw[c] * ro0;
-                }
-                strip_x_forward_adjoint(v[0], v[1], it.first, it.last);
-                strip_x_forward_adjoint(v[2], v[3], it.first, it.last);
-#pragma unroll
-                for (int c = 0; c < 2; ++c) {  // (the forward pipeline's states: O, O1, E2, O3, E)
-                    const T ev = v[c] * C::k, odd = v[2 + c] * (-C::ik);
-                    const T o1 = fmadd(C::d, SF[c] + ev, OS[c]);
-                    const T e2 = fmadd(C::g, EA[c] + o1, SF[c]);
-                    const T o3 = fmadd(C::b, OB[c] + e2, EA[c]);
-                    re[c] = fmadd(C::a, EC[c] + o3, OB[c]) * (cs[c] * se);
-                    ro[c] = o3 * (cs[c] * so);
-                    SF[c] = ev;
-                    OS[c] = odd;
-                    EA[c] = o1;
-                    OB[c] = e2;
-                    EC[c] = o3;
-                }
+                    for (int c = 0; c < 2; ++c) {  // (the forward pipeline's states: O, O1, E2, O3, E)
+                        const T ev = v[c] * C::k, odd = v[2 + c] * (-C::ik);
+                        const T o1 = mirror_lift<ends>(C::d, SF[c], ev, OS[c], m, 4);
+                        const T e2 = mirror_lift<ends>(C::g, EA[c], o1, SF[c], m, 3);
+                        const T o3 = mirror_lift<ends>(C::b, OB[c], e2, EA[c], m, 2);
+                        re[c] = mirror_lift<ends>(C::a, EC[c], o3, OB[c], m, 1);
+                        ro[c] = o3;
+                        SF[c] = ev;
+                        OS[c] = odd;
+                        EA[c] = o1;
+                        OB[c] = e2;
+                        EC[c] = o3;
+                    }
+                });
             } else {
                 strip_x_inverse(v[0], v[1], it.first, it.last);
                 strip_x_inverse(v[2], v[3], it.first, it.last);
@@ -494,8 +559,9 @@ WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item
     T E[2], O[2], O1[2], E2[2], O3[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) E[c] = O[c] = O1[c] = E2[c] = O3[c] = T(0);
-    [[maybe_unused]] const T cw[2] = {end_load<T>(xe, n.nx), end_load<T>(xo, n.nx)};
-    [[maybe_unused]] const T cs[2] = {end_store<T>(2 * it.kp, n.nx), end_store<T>(2 * it.kp + 1, n.nx)};
+    std::conditional_t<Adjoint, MirrorLine<T, true>, int> line{};
+    if constexpr (Adjoint) line = MirrorLine<T, true>::of(int32_t(2 * it.kp), int32_t(n.nx));
+    [[maybe_unused]] const uint32_t images = Adjoint ? line_images(ny) : 0u;
     T buf[4][4];
     int32_t g = int32_t(it.ys / 2) - 2;
     load(g, buf[0]);
@@ -511,47 +577,47 @@ WZ_D void strip_forward(const XYForward<T>& a, const StripPlan& p, uint32_t item
                 for (int i = 0; i < 4; ++i) ok = ok && finite_value(v[i]);
             }
             T le[2], hi[2];  // the two columns of the low and of the high row
+            if constexpr (Adjoint) {
+                mirror_stream(g, ny, images, [&](const MirrorSteps& m, auto ends_c) {
+                    constexpr bool ends = decltype(ends_c)::value;
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                const bool other = (c != 0) != swap;
-                const T ev = other ? v[1] : v[0], ov = other ? v[3] : v[2];
-                if constexpr (Adjoint) {  // (the inverse pipeline's states: OS, EA, OB, EC)
-                    const T es = ev * (cw[c] * end_load<T>(2 * uint32_t(pair_even(g, ny)), n.ny));
-                    const T os = ov * (cw[c] * end_load<T>(2 * uint32_t(pair_odd(g, ny)) + 1u, n.ny));
-                    const T eA = fmadd(-C::a, O[c] + os, es);
-                    const T oB = fmadd(-C::b, O1[c] + eA, O[c]);
-                    const T eC = fmadd(-C::g, E2[c] + oB, O1[c]);
-                    le[c] = O3[c] * C::ik;
-                    hi[c] = fmadd(-C::d, O3[c] + eC, E2[c]) * (-C::k);
-                    O[c] = os;
-                    O1[c] = eA;
-                    E2[c] = oB;
-                    O3[c] = eC;
-                    continue;
+                    for (int c = 0; c < 2; ++c) {  // (the inverse pipeline's states: OS, EA, OB, EC)
+                        const bool other = (c != 0) != swap;
+                        const T ev = other ? v[1] : v[0], ov = other ? v[3] : v[2];
+                        const T eA = mirror_lift<ends>(-C::a, O[c], ov, ev, m, 5);
+                        const T oB = mirror_lift<ends>(-C::b, O1[c], eA, O[c], m, 4);
+                        const T eC = mirror_lift<ends>(-C::g, E2[c], oB, O1[c], m, 3);
+                        le[c] = O3[c] * C::ik;
+                        hi[c] = mirror_lift<ends>(-C::d, O3[c], eC, E2[c], m, 2) * (-C::k);
+                        O[c] = ov;
+                        O1[c] = eA;
+                        E2[c] = oB;
+                        O3[c] = eC;
+                    }
+                });
+            } else {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const bool other = (c != 0) != swap;
+                    const T ev = other ? v[1] : v[0], ov = other ? v[3] : v[2];
+                    const T o1 = fmadd(C::a, E[c] + ev, O[c]);
+                    const T e2 = fmadd(C::b, O1[c] + o1, E[c]);
+                    const T o3 = fmadd(C::g, E2[c] + e2, O1[c]);
+                    const T e4 = fmadd(C::d, O3[c] + o3, E2[c]);
+                    le[c] = e4 * C::k;
+                    hi[c] = o3 * (-C::ik);
+                    E[c] = ev;
+                    O[c] = ov;
+                    O1[c] = o1;
+                    E2[c] = e2;
+                    O3[c] = o3;
                 }
-                const T o1 = fmadd(C::a, E[c] + ev, O[c]);
-                const T e2 = fmadd(C::b, O1[c] + o1, E[c]);
-                const T o3 = fmadd(C::g, E2[c] + e2, O1[c]);
-                const T e4 = fmadd(C::d, O3[c] + o3, E2[c]);
-                le[c] = e4 * C::k;
-                hi[c] = o3 * (-C::ik);
-                E[c] = ev;
-                O[c] = ov;
-                O1[c] = o1;
-                E2[c] = e2;
-                O3[c] = o3;
             }
             if constexpr (emit) {
                 const uint32_t iy = uint32_t(g - 2);
                 if constexpr (Adjoint) {
-                    strip_x_inverse_adjoint(le[0], le[1], it.first, it.last);
-                    strip_x_inverse_adjoint(hi[0], hi[1], it.first, it.last);
-                    const T sl = end_store<T>(2 * iy, n.ny), sh = end_store<T>(2 * iy + 1u, n.ny);
-#pragma unroll
-                    for (int c = 0; c < 2; ++c) {
-                        le[c] *= cs[c] * sl;
-                        hi[c] *= cs[c] * sh;
-                    }
+                    strip_x_inverse_adjoint(le[0], le[1], it.first, it.last, line);
+                    strip_x_inverse_adjoint(hi[0], hi[1], it.first, it.last, line);
                 } else {
                     strip_x_forward(le[0], le[1], it.first, it.last);
                     strip_x_forward(hi[0], hi[1], it.first, it.last);
