@@ -14,7 +14,7 @@ static int failures = 0;
 static void check(uint32_t nx, uint32_t ny, uint32_t nz, unsigned width, bool fits, bool wide) {
     const uint64_t plane = uint64_t(nx) * ny * width, volume = plane * nz;
     const bool one = volume <= 0xFFFFFFFFull;  // the end of the last sample
-    bool ok = zcol_fits(nx, ny, nz, width) == fits;
+    bool ok = zcol_fits(nx, ny, nz, 0, width) == fits;
     if (fits) {
         ok = ok && zcol_wide(nx, ny, nz, width) == wide && wide == !one;
         ok = ok && plane <= 0xFFFFFFFFull;
@@ -22,7 +22,7 @@ static void check(uint32_t nx, uint32_t ny, uint32_t nz, unsigned width, bool fi
         if (!wide) ok = ok && uint64_t(uint32_t(volume - width)) == volume - width;
     }
     if (!ok) {
-        std::printf("%ux%ux%u width %u: fits %d wide %d\n", nz, ny, nx, width, zcol_fits(nx, ny, nz, width),
+        std::printf("%ux%ux%u width %u: fits %d wide %d\n", nz, ny, nx, width, zcol_fits(nx, ny, nz, 0, width),
                     zcol_wide(nx, ny, nz, width));
         ++failures;
     }
@@ -56,6 +56,20 @@ int main() {
         check(64, 64, top + 1, width, false, false);
         if (zcol_lds_bytes(top, 5, width) > 65536 || zcol_lds_bytes(top + 1, 5, width) <= 65536) {
             std::printf("LDS limit, width %u\n", width);
+            ++failures;
+        }
+    }
+    // lines of one sample, at the first level and later
+    const struct { uint32_t n; unsigned levels; bool fit; } lines[] = {
+        {1, 0, true}, {1, 1, false}, {2, 1, true}, {2, 2, false}, {3, 2, true}, {3, 3, false}, {9, 4, true}, {9, 5, false},
+        {16, 4, true}, {16, 5, false}, {17, 5, true}, {340, 5, true}};
+    for (const auto& k : lines) {
+        bool ok = lines_fit(k.n, k.levels) == k.fit && zcol_fits(64, 64, k.n, k.levels, 4) == k.fit;
+        // what a pass addresses: the halves of a line of m samples start at 0 and ceil(m / 2), both inside it
+        uint32_t m = k.n;
+        for (unsigned l = 0; k.fit && l < k.levels; ++l, m -= m / 2) ok = ok && m - m / 2 < m;
+        if (!ok) {
+            std::printf("lines of %u, %u levels\n", k.n, k.levels);
             ++failures;
         }
     }

@@ -195,7 +195,7 @@ bool plane_pair(const T* src, T* dst, Dims full, Dims act, int a0, int a1, uint3
     return true;
 }
 
-bool zcol_fits(Dims n, unsigned width) { return wz::zcol_fits(n.nx, n.ny, n.nz, width); }
+bool zcol_fits(Dims n, unsigned levels, unsigned width) { return wz::zcol_fits(n.nx, n.ny, n.nz, levels, width); }
 
 template <class T, bool Inverse, bool Repair, bool Wide = false>
 __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a, uint32_t* __restrict__ status,
@@ -229,7 +229,7 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a,
 template <class T, bool Inverse>
 void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* status, hipStream_t s,
                  const WaveRepair<T>* repair = nullptr) {
-    if (!zcol_fits(full, sizeof(T)) || levels < 1 || levels > 5 || src == dst)
+    if (!zcol_fits(full, levels, sizeof(T)) || levels < 1 || levels > 5 || src == dst)
         throw std::logic_error("Z phase does not fit LDS");
     const bool wide = zcol_wide(full.nx, full.ny, full.nz, sizeof(T));
     const uint64_t total = uint64_t(full.ny) * ((full.nx + kZColumns - 1) / kZColumns);
@@ -386,7 +386,7 @@ unsigned tail_level(Dims full, unsigned lxy, unsigned from, unsigned width) {
     Dims n = full;
     for (unsigned l = 0; l < lxy; ++l) {
         if (l >= from && uint64_t(n.nx) * n.ny * n.nz <= kTailSamples &&
-            strips_fit(n, full.nx, full.ny, lxy - l, width))
+            strips_fit(n, full.nx, full.ny, lxy - l, width) && lines_fit(n.nz, lxy - l))
             return l;
         n = shrink(n, true, true);
     }
@@ -822,7 +822,7 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
     // tmp0) and writes its high bands into coeff and its low band into the
     // next box (coeff for the last level)
     if (strips_fit(full, full.nx, full.ny, lxy, sizeof(T)) && lxy &&
-        (lz ? zcol_fits(full, sizeof(T)) : input != coeff)) {
+        (lz ? zcol_fits(full, lz, sizeof(T)) : input != coeff)) {
         const T* src = input;
         uint64_t spy = full.nx, spz = uint64_t(full.nx) * full.ny;
         if (lz) {
@@ -857,7 +857,7 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
         return;
     }
     Dims act = full;
-    if (lz && zcol_fits(full, sizeof(T)) && p.first_src != coeff) {  // the Z phase in one pass
+    if (lz && zcol_fits(full, lz, sizeof(T)) && p.first_src != coeff) {  // the Z phase in one pass
         StageClock clock("forward_Z", s);
         zcol_levels<T, false>(p.first_src, coeff, full, lz, status, s);
         p.first = false;
@@ -947,7 +947,7 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
     // then the compact boxes in tmp0) and writes its box to tmp0, the finest
     // into tmp1, from which the Z phase (one pass) writes output
     if (strips_fit(full, full.nx, full.ny, lxy, sizeof(T)) && lxy &&
-        (lz ? zcol_fits(full, sizeof(T)) : output != coeff)) {
+        (lz ? zcol_fits(full, lz, sizeof(T)) : output != coeff)) {
         // the Z phase screens the output when asked (no repairs to fold here)
         uint32_t* screen = emit && emit->mode == kEmitStoreScreen && !emit->np && lz ? emit->status : nullptr;
         const bool repair = emit && emit->mode == kEmitRepair && lz;
@@ -997,7 +997,7 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         return screen != nullptr || repair;
     }
     for (int l = int(lxy) - 1; l >= 0; --l) p.level(full, xy[l], xyo, 2, lz == 0 && l == 0, unsigned(l));
-    if (lz && zcol_fits(full, sizeof(T)) && (p.first ? p.first_src : p.home) != output) {  // in one pass
+    if (lz && zcol_fits(full, lz, sizeof(T)) && (p.first ? p.first_src : p.home) != output) {  // in one pass
         StageClock clock("inverse_Z", s);
         zcol_levels<T, true>(p.first ? p.first_src : p.home, output, full, lz, nullptr, s);
     } else {
@@ -1053,7 +1053,7 @@ bool transform_inverse_preserving(const T* coeff, T* output, T* tmp0, T* tmp1, D
 }
 
 bool plane_fused_fits(Dims full, unsigned lxy, unsigned lz, unsigned width) {
-    return lxy && lz && zcol_fits(full, width) && strips_fit(full, full.nx, full.ny, lxy, width);
+    return lxy && lz && zcol_fits(full, lz, width) && strips_fit(full, full.nx, full.ny, lxy, width);
 }
 
 bool coarse_split_fits(Dims full, unsigned lxy, unsigned width) {

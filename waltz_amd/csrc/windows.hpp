@@ -23,9 +23,17 @@ inline uint64_t zcol_lds_bytes(uint32_t nz, unsigned levels, unsigned width) {
 }
 // 64 KiB of LDS: nz up to 340 (float) or 170 (double) whatever the levels
 inline bool zcol_lds_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5, width) <= 65536; }
+// Whether every one of `levels` levels lifts lines of at least two samples. One
+// sample is its own even and odd neighbour: kernels that address the two halves
+// of a line apart would read past it.
+inline bool lines_fit(uint32_t n, unsigned levels) {
+    for (unsigned l = 0; l < levels; ++l, n -= n / 2)
+        if (n < 2) return false;
+    return true;
+}
 // Whether the Z phase of an nx x ny x nz volume runs as columns, ...
-inline bool zcol_fits(uint32_t nx, uint32_t ny, uint32_t nz, unsigned width) {
-    return zcol_lds_fits(nz, width) && fused_plane_fits(nx, ny, width);
+inline bool zcol_fits(uint32_t nx, uint32_t ny, uint32_t nz, unsigned levels, unsigned width) {
+    return zcol_lds_fits(nz, width) && lines_fit(nz, levels) && fused_plane_fits(nx, ny, width);
 }
 // ... and whether it has to address every plane through a window of its own:
 // one window (of 2^32 - 1 bytes, no lane masked off by its offset) holds every
