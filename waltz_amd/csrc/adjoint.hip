@@ -172,7 +172,16 @@ __global__ void __launch_bounds__(256) adjoint_pass(const T* __restrict__ src, T
             for (int32_t q = lo; q < hi; ++q)
                 if (q != int32_t(p) && reflect_pos(q, n) == p) s += u(q);
         }
-        if (OfInverse) s = (p & 1u) ? s * (-C::k) : s * C::ik;
+        if (OfInverse && n == 1) {  // its one sample is every even and every odd one
+            T even = T(0), odd = T(0);
+            for (int32_t q = lo; q < hi; ++q) {
+                if (q & 1) odd += u(q);
+                else even += u(q);
+            }
+            s = even * C::ik + odd * (-C::k);
+        } else if (OfInverse) {
+            s = (p & 1u) ? s * (-C::k) : s * C::ik;
+        }
         dst[base + uint64_t(OfInverse ? split_index(p, n) : p) * stride] = s;
     }
 }
