@@ -323,10 +323,10 @@ int waltz_amd_transform_async(int width, int inverse, const void* input, void* o
             T* t0 = static_cast<T*>(tmp0);
             T* t1 = static_cast<T*>(tmp1);
             if (inverse) {
-                // a fused finest level reads the input's high bands in place
-                // and writes the output once
-                if (dyadic && input != output &&
-                    wz::transform_inverse_preserving<T>(static_cast<const T*>(input), out, t0, t1, d, lxy, s))
+                // a fused finest level or a Z phase by itself reads the input in
+                // place and writes the output once
+                if (wz::transform_inverse_preserving<T>(static_cast<const T*>(input), out, t0, t1, d, lxy, lz,
+                                                        dyadic != 0, s))
                     return;
                 if (input != output)
                     wz::hip_check(hipMemcpyAsync(out, input, n * sizeof(T), hipMemcpyDeviceToDevice, s), "copy");

@@ -72,13 +72,14 @@ struct LowBox {
 };
 template <class T>
 LowBox<T> inverse_coarse_levels(T* coeff, T* tmp0, T* tmp1, Dims full, unsigned lxy, hipStream_t s);
-// transform_inverse of a dyadic field whose finest level runs fused, leaving
-// `coeff` intact: the level-1 box is copied into `output` and the coarse
-// levels run there, the finest level reads the high bands from coeff. False
-// (nothing done) when the geometry has no fused finest level.
+// transform_inverse that leaves `coeff` intact, where the geometry has such a
+// form, else false (nothing done). A dyadic field whose finest level runs fused:
+// the level-1 box is copied into tmp1 and the coarse levels run there, with
+// `output` as a scratch volume, then the finest level reads the high bands from
+// coeff. A plane schedule of Z levels only: one pass.
 template <class T>
-bool transform_inverse_preserving(const T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy,
-                                  hipStream_t s);
+bool transform_inverse_preserving(const T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz,
+                                  bool dyadic, hipStream_t s);
 template <class T>
 void inverse_finest_level(const T* coeff, const LowBox<T>& low, T* output, Dims full, unsigned lxy,
                           const Level0Emit<T>& emit, hipStream_t s);

@@ -197,7 +197,7 @@ bool plane_pair(const T* src, T* dst, Dims full, Dims act, int a0, int a1, uint3
 
 bool zcol_fits(Dims n, unsigned levels, unsigned width) { return wz::zcol_fits(n.nx, n.ny, n.nz, levels, width); }
 
-template <class T, bool Inverse, bool Repair, bool Wide = false>
+template <class T, bool Inverse, bool Repair, bool Wide = false, bool InPlace = false>
 __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a, uint32_t* __restrict__ status,
                                                                 WaveRepair<T> rp) {
     static_assert(Inverse || !Repair, "repairs follow the inverse");
@@ -217,8 +217,10 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a,
         __syncthreads();
     }
     const bool screen = status && !Repair;
-    const bool fin = zcol_columns<T, Inverse, Repair, Wide>(a, id / xb, (id % xb) * kZColumns, box0, box1, screen,
-                                                            ZOutput<T>{a.n, screen, false, T(0)}, rp, id, &seg_fill);
+    T* const held = InPlace ? box0 + zcol_lds_rows(a.n.nz, a.levels) * kZColumns : nullptr;
+    const bool fin = zcol_columns<T, Inverse, Repair, Wide, InPlace>(
+        a, id / xb, (id % xb) * kZColumns, box0, box1, screen, ZOutput<T>{a.n, screen, false, T(0)}, rp, id, &seg_fill,
+        held);
     if (status && __ballot(!fin) && (threadIdx.x & 63u) == 0)
         atomicOr(status, uint32_t(Repair ? kRepairBound : Inverse ? kNonFiniteOutput : kNonFiniteInput));
     if constexpr (Repair) {
@@ -229,14 +231,16 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a,
 template <class T, bool Inverse>
 void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* status, hipStream_t s,
                  const WaveRepair<T>* repair = nullptr) {
-    if (!zcol_fits(full, levels, sizeof(T)) || levels < 1 || levels > 5 || src == dst)
+    const bool place = src == dst;
+    if (!zcol_fits(full, levels, sizeof(T)) || levels < 1 || levels > 5 ||
+        (place && (repair || !zcol_place_fits(full.nz, levels, sizeof(T)))))
         throw std::logic_error("Z phase does not fit LDS");
     const bool wide = zcol_wide(full.nx, full.ny, full.nz, sizeof(T));
     const uint64_t total = uint64_t(full.ny) * ((full.nx + kZColumns - 1) / kZColumns);
     const uint64_t blocks = 8 * ((total + 7) / 8);
     check_launch_size(blocks * kZThreads);
     const dim3 grid{uint32_t(blocks)};
-    const uint32_t lds = uint32_t(zcol_lds_bytes(full.nz, levels, sizeof(T)));
+    const uint32_t lds = uint32_t(zcol_lds_bytes(full.nz, levels, sizeof(T), place));
     const ZColumnsOf<T> a{src, full.nx, full.nx * full.ny, dst, full.nx, full.nx * full.ny, full, uint32_t(levels)};
     if constexpr (Inverse) {
         if (repair) {
@@ -246,12 +250,14 @@ void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* sta
             return;
         }
     }
-    if (wide)
-        hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse, false, true>), grid, dim3(kZThreads), lds, s, a, status,
-                           WaveRepair<T>{});
-    else
-        hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse, false>), grid, dim3(kZThreads), lds, s, a, status,
-                           WaveRepair<T>{});
+    auto launch = [&](auto wide_c, auto place_c) {
+        hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse, false, decltype(wide_c)::value, decltype(place_c)::value>),
+                           grid, dim3(kZThreads), lds, s, a, status, WaveRepair<T>{});
+    };
+    if (wide && place) launch(std::true_type{}, std::true_type{});
+    else if (wide) launch(std::true_type{}, std::false_type{});
+    else if (place) launch(std::false_type{}, std::true_type{});
+    else launch(std::false_type{}, std::false_type{});
 }
 
 template <class T, bool Requant, bool Screen>
@@ -459,6 +465,18 @@ void copy_box(const T* src, T* dst, Dims full, Dims act, hipStream_t s) {
     check_launch_size(total);
     hipLaunchKernelGGL((box_copy<T>), dim3(uint32_t((total + 255) / 256)), dim3(256), 0, s, src, dst, full, act,
                        uint32_t(total));
+}
+
+// The source of the Z phase: `src`, or a copy of it in `scratch` where the
+// phase ends in `src` itself and does not fit in place (one more pass over the
+// volume, against two per level for axis passes).
+template <class T>
+const T* z_source(const T* src, const T* dst, T* scratch, Dims full, unsigned levels, hipStream_t s) {
+    if (src != dst || zcol_place_fits(full.nz, levels, sizeof(T))) return src;
+    hip_check(hipMemcpyAsync(scratch, src, uint64_t(full.nx) * full.ny * full.nz * sizeof(T), hipMemcpyDeviceToDevice,
+                             s),
+              "copy");
+    return scratch;
 }
 
 // Runs a sequence of axis passes on one box: data starts in `home` (or in
@@ -857,9 +875,10 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
         return;
     }
     Dims act = full;
-    if (lz && zcol_fits(full, lz, sizeof(T)) && p.first_src != coeff) {  // the Z phase in one pass
+    if (lz && zcol_fits(full, lz, sizeof(T))) {  // the Z phase in one pass
         StageClock clock("forward_Z", s);
-        zcol_levels<T, false>(p.first_src, coeff, full, lz, status, s);
+        const T* src = z_source<T>(p.first_src, coeff, tmp0, full, lz, s);
+        zcol_levels<T, false>(src, coeff, full, lz, status, s);
         p.first = false;
     } else {
         for (unsigned l = 0; l < lz; ++l) {
@@ -997,9 +1016,10 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
         return screen != nullptr || repair;
     }
     for (int l = int(lxy) - 1; l >= 0; --l) p.level(full, xy[l], xyo, 2, lz == 0 && l == 0, unsigned(l));
-    if (lz && zcol_fits(full, lz, sizeof(T)) && (p.first ? p.first_src : p.home) != output) {  // in one pass
+    if (lz && zcol_fits(full, lz, sizeof(T))) {  // the Z phase in one pass
         StageClock clock("inverse_Z", s);
-        zcol_levels<T, true>(p.first ? p.first_src : p.home, output, full, lz, nullptr, s);
+        const T* src = z_source<T>(p.first ? p.first_src : p.home, output, tmp0, full, lz, s);
+        zcol_levels<T, true>(src, output, full, lz, nullptr, s);
     } else {
         for (int l = int(lz) - 1; l >= 0; --l) p.level(full, zs[l], zonly, 1, l == 0, unsigned(l));
     }
@@ -1037,10 +1057,17 @@ void inverse_finest_level(const T* coeff, const LowBox<T>& low, T* output, Dims 
 }
 
 template <class T>
-bool transform_inverse_preserving(const T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy,
-                                  hipStream_t s) {
+bool transform_inverse_preserving(const T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz,
+                                  bool dyadic, hipStream_t s) {
+    if (output == coeff) return false;
+    if (!dyadic) {
+        if (lxy || !lz || !zcol_fits(full, lz, sizeof(T))) return false;
+        StageClock clock("inverse_Z", s);
+        zcol_levels<T, true>(coeff, output, full, lz, nullptr, s);
+        return true;
+    }
     const Tuning tu = tuning_for(full, lxy, sizeof(T), true);
-    if (!lxy || !tu.fused || output == coeff) return false;
+    if (!lxy || !tu.fused) return false;
     const Dims h1 = shrink(full, true, true);
     // the coarser levels work on a copy of their box, with the output as a
     // scratch volume: the finest level reads their result as it stores
@@ -1112,9 +1139,10 @@ void inverse_finest_requant(const T* coeff, const T* t0, Dims full, unsigned lxy
     launch_finest<T>(coeff, t0, h1.nx, h1.nx * h1.ny, nullptr, full, tu.sz[0], &emit, s, "inverse_L0");
 }
 
-template bool transform_inverse_preserving<float>(const float*, float*, float*, float*, Dims, unsigned, hipStream_t);
-template bool transform_inverse_preserving<double>(const double*, double*, double*, double*, Dims, unsigned,
-                                                   hipStream_t);
+template bool transform_inverse_preserving<float>(const float*, float*, float*, float*, Dims, unsigned, unsigned, bool,
+                                                  hipStream_t);
+template bool transform_inverse_preserving<double>(const double*, double*, double*, double*, Dims, unsigned, unsigned,
+                                                   bool, hipStream_t);
 template LowBox<float> inverse_coarse_levels<float>(float*, float*, float*, Dims, unsigned, hipStream_t);
 template LowBox<double> inverse_coarse_levels<double>(double*, double*, double*, Dims, unsigned, hipStream_t);
 template void inverse_finest_level<float>(const float*, const LowBox<float>&, float*, Dims, unsigned,

@@ -13,16 +13,25 @@ inline bool fused_plane_fits(uint64_t pitch, uint64_t rows, uint64_t width) {
     return pitch * rows * width <= (uint64_t(1) << 32) - (uint64_t(1) << 20);
 }
 
-// Column passes (zcolumns.hpp): LDS of the low boxes between the levels, 64
-// columns of ceil(nz/2) and ceil(nz/4) samples.
+// Column passes (zcolumns.hpp): LDS rows of 64 columns for the low boxes between
+// the levels, ceil(nz/2) and ceil(nz/4) of them.
 constexpr uint32_t kZColumns = 64;
-inline uint64_t zcol_lds_bytes(uint32_t nz, unsigned levels, unsigned width) {
-    if (levels < 2) return 0;
-    const uint32_t n1 = nz - nz / 2, n2 = levels > 2 ? n1 - n1 / 2 : 0u;
-    return uint64_t(n1 + n2) * kZColumns * width;
+constexpr uint32_t zcol_lds_rows(uint32_t nz, unsigned levels) {
+    const uint32_t n1 = nz - nz / 2;
+    return levels < 2 ? 0u : levels > 2 ? n1 + (n1 - n1 / 2) : n1;
 }
-// 64 KiB of LDS: nz up to 340 (float) or 170 (double) whatever the levels
-inline bool zcol_lds_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5, width) <= 65536; }
+// In place: the finest level's results that would overwrite rows it still reads
+// (the high half, of a single level both) wait in LDS behind those.
+constexpr uint32_t zcol_held_rows(uint32_t nz, unsigned levels) { return levels > 1 ? nz / 2 : nz; }
+constexpr uint64_t zcol_lds_bytes(uint32_t nz, unsigned levels, unsigned width, bool in_place = false) {
+    return (uint64_t(zcol_lds_rows(nz, levels)) + (in_place ? zcol_held_rows(nz, levels) : 0u)) * kZColumns * width;
+}
+// 64 KiB of LDS: nz up to 340 (float) or 170 (double) whatever the levels, in
+// place up to 204 or 102
+constexpr bool zcol_lds_fits(uint32_t nz, unsigned width) { return zcol_lds_bytes(nz, 5, width) <= 65536; }
+constexpr bool zcol_place_fits(uint32_t nz, unsigned levels, unsigned width) {
+    return zcol_lds_bytes(nz, levels, width, true) <= 65536;
+}
 // Whether every one of `levels` levels lifts lines of at least two samples. One
 // sample is its own even and odd neighbour: kernels that address the two halves
 // of a line apart would read past it.

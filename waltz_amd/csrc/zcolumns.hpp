@@ -115,10 +115,12 @@ struct ZColumnsOf {
 // `box1`: zcol_lds_bytes of LDS. Returns whether this lane met nothing to flag
 // (a non-finite sample of a screened pass, or an unmet bound). Wide: volumes
 // past one window, every plane through its own (3370x3300x99 float, 4.4 GB:
-// forward 2.2 ms, 4.0 TB/s).
-template <class T, bool Inverse, bool Repair, bool Wide = false>
+// forward 2.2 ms, 4.0 TB/s). InPlace: src may be dst; the finest level's rows
+// from `from` on wait in `held` (zcol_held_rows of LDS) until all are read.
+template <class T, bool Inverse, bool Repair, bool Wide = false, bool InPlace = false>
 WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0, T* box1, bool screen,
-                       const ZOutput<T>& out, const WaveRepair<T>& rp, uint32_t id, uint32_t* seg_fill) {
+                       const ZOutput<T>& out, const WaveRepair<T>& rp, uint32_t id, uint32_t* seg_fill,
+                       T* held = nullptr) {
     constexpr int Tile = sizeof(T) == 4 ? 16 : 8, P = Tile / 2 + 4;  // (the inverse's is part of the format)
     constexpr uint32_t W = kZThreads / 64, S = sizeof(T);
     static_assert(!(Repair && Wide), "the codec's fields fit one window");
@@ -139,6 +141,8 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
         if constexpr (Wide) buf_store(v, window(a.dst + uint64_t(z) * a.dpz), dcol);
         else buf_store_at(v, wd, dcol, at);
     };
+    [[maybe_unused]] const uint32_t from = a.n.nz - zcol_held_rows(a.n.nz, a.levels);
+    auto hold = [&](T v, uint32_t z) { held[(z - from) * kZColumns + lane] = v; };
     // the finest inverse store's lanes and rows
     const bool put = Inverse ? x < out.clip.nx && y < out.clip.ny : in;
     const int32_t rows = int32_t(Inverse ? out.clip.nz : a.n.nz);
@@ -192,9 +196,14 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
                 for (int j = 2; j < P - 2; ++j) {
                     if (2 * (k0 + j) < n) {
                         if (!coarsest) b[uint32_t(j - 2) * kZColumns] = e[j];
+                        else if (InPlace && finest) hold(e[j], uint32_t(k0 + j));
                         else if (in) store(e[j], uint32_t(k0 + j), at);
                     }
-                    if (2 * (k0 + j) + 1 < n && in) store(o[j], uint32_t(k0 + j + h), up);
+                    if (InPlace && finest) {
+                        if (2 * (k0 + j) + 1 < n) hold(o[j], uint32_t(k0 + j + h));
+                    } else if (2 * (k0 + j) + 1 < n && in) {
+                        store(o[j], uint32_t(k0 + j + h), up);
+                    }
                     at += dplane;
                     up += dplane;
                 }
@@ -264,8 +273,11 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
                     for (int b = 0; b < 2; ++b) {
                         if (2 * (k0 + j) + b < rows) {
                             const T v = out.hole ? out.fill : b ? o[j] : e[j];
-                            if (put) {
-                                if constexpr (Wide) store(v, uint32_t(2 * (k0 + j) + b), 0u);
+                            const uint32_t z = uint32_t(2 * (k0 + j) + b);
+                            if (InPlace && z >= from) {
+                                hold(v, z);
+                            } else if (put) {
+                                if constexpr (Wide) store(v, z, 0u);
                                 else buf_store_at(v, wt, dcol, at);
                             }
                             if (out.screen) fin = fin && (finite_value(v) || !put || out.hole);
@@ -276,6 +288,11 @@ WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0,
             }
         }
         __syncthreads();
+        if constexpr (InPlace) {
+            if (finest)
+                for (uint32_t z = from + wave; z < a.n.nz; z += W)
+                    if (in) store(held[(z - from) * kZColumns + lane], z, z * dplane);
+        }
     }
     return fin;
 }
