@@ -1,7 +1,9 @@
 """Transforms of Z levels only (planes of at most 8 rows or columns, or custom
 levels): the whole phase is one column pass, also in place and from an input
 that is kept, with the results of the oracle. 102 (double) and 204 (float)
-planes are the most that fit LDS in place; above, the pass works on a copy."""
+planes are the most that fit LDS in place; above, the pass works on a copy. Up to
+256 rows of columns take workgroups of 16 waves, more of 4, in place with over
+48 KiB of 8."""
 import numpy as np
 import pytest
 
@@ -12,7 +14,8 @@ torch = pytest.importorskip("torch")
 
 
 @pytest.mark.parametrize("shape,lz", [((100, 8, 300), 4), ((64, 70, 8), 3), ((17, 40, 50), 2), ((20, 3, 130), 1),
-                                      ((102, 8, 66), 5), ((103, 8, 66), 5), ((204, 8, 66), 5), ((205, 8, 66), 5)],
+                                      ((102, 8, 66), 5), ((103, 8, 66), 5), ((204, 8, 66), 5), ((205, 8, 66), 5),
+                                      ((20, 256, 9), 2), ((40, 257, 9), 3), ((102, 129, 65), 5), ((160, 257, 9), 5)],
                          ids=str)
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 def test_one_pass(oracle, shape, lz, dtype):

@@ -197,8 +197,8 @@ bool plane_pair(const T* src, T* dst, Dims full, Dims act, int a0, int a1, uint3
 
 bool zcol_fits(Dims n, unsigned levels, unsigned width) { return wz::zcol_fits(n.nx, n.ny, n.nz, levels, width); }
 
-template <class T, bool Inverse, bool Repair, bool Wide = false, bool InPlace = false>
-__global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a, uint32_t* __restrict__ status,
+template <class T, bool Inverse, bool Repair, bool Wide, bool InPlace, uint32_t Threads>
+__global__ void __launch_bounds__(Threads) zcol_levels_kernel(ZColumnsOf<T> a, uint32_t* __restrict__ status,
                                                                 WaveRepair<T> rp) {
     static_assert(Inverse || !Repair, "repairs follow the inverse");
     __shared__ uint32_t seg_fill;  // repair entries of this workgroup
@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(kZThreads) zcol_levels_kernel(ZColumnsOf<T> a,
     }
     const bool screen = status && !Repair;
     T* const held = InPlace ? box0 + zcol_lds_rows(a.n.nz, a.levels) * kZColumns : nullptr;
-    const bool fin = zcol_columns<T, Inverse, Repair, Wide, InPlace>(
+    const bool fin = zcol_columns<T, Inverse, Repair, Wide, InPlace, Threads>(
         a, id / xb, (id % xb) * kZColumns, box0, box1, screen, ZOutput<T>{a.n, screen, false, T(0)}, rp, id, &seg_fill,
         held);
     if (status && __ballot(!fin) && (threadIdx.x & 63u) == 0)
@@ -238,26 +238,38 @@ void zcol_levels(const T* src, T* dst, Dims full, unsigned levels, uint32_t* sta
     const bool wide = zcol_wide(full.nx, full.ny, full.nz, sizeof(T));
     const uint64_t total = uint64_t(full.ny) * ((full.nx + kZColumns - 1) / kZColumns);
     const uint64_t blocks = 8 * ((total + 7) / 8);
-    check_launch_size(blocks * kZThreads);
     const dim3 grid{uint32_t(blocks)};
     const uint32_t lds = uint32_t(zcol_lds_bytes(full.nz, levels, sizeof(T), place));
     const ZColumnsOf<T> a{src, full.nx, full.nx * full.ny, dst, full.nx, full.nx * full.ny, full, uint32_t(levels)};
-    if constexpr (Inverse) {
-        if (repair) {
-            if (wide || repair->rep.segments != total || repair->rep.cap < uint64_t(std::min(full.nx, kZColumns)) * full.nz)
-                throw std::logic_error("repair segments do not match the Z phase's launch");
-            hipLaunchKernelGGL((zcol_levels_kernel<T, true, true>), grid, dim3(kZThreads), lds, s, a, status, *repair);
-            return;
+    if (repair && (wide || repair->rep.segments != total ||
+                   repair->rep.cap < uint64_t(std::min(full.nx, kZColumns)) * full.nz))
+        throw std::logic_error("repair segments do not match the Z phase's launch");
+    const uint32_t threads = zcol_threads(total, place, lds);
+    check_launch_size(blocks * threads);
+    auto launch = [&](auto repair_c, auto wide_c, auto place_c) {
+        constexpr bool R = decltype(repair_c)::value, W = decltype(wide_c)::value, P = decltype(place_c)::value;
+        const WaveRepair<T> rp = R ? *repair : WaveRepair<T>{};
+        auto run = [&](auto threads_c) {
+            constexpr uint32_t N = decltype(threads_c)::value;
+            hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse, R, W, P, N>), grid, dim3(N), lds, s, a, status, rp);
+        };
+        if constexpr (!W) {  // (volumes past a window have more workgroups)
+            if (threads == kZThreadsMost) return run(std::integral_constant<uint32_t, kZThreadsMost>{});
         }
-    }
-    auto launch = [&](auto wide_c, auto place_c) {
-        hipLaunchKernelGGL((zcol_levels_kernel<T, Inverse, false, decltype(wide_c)::value, decltype(place_c)::value>),
-                           grid, dim3(kZThreads), lds, s, a, status, WaveRepair<T>{});
+        if constexpr (P) {
+            if (threads == kZThreadsPlace) return run(std::integral_constant<uint32_t, kZThreadsPlace>{});
+        }
+        run(std::integral_constant<uint32_t, kZThreads>{});
     };
-    if (wide && place) launch(std::true_type{}, std::true_type{});
-    else if (wide) launch(std::true_type{}, std::false_type{});
-    else if (place) launch(std::false_type{}, std::true_type{});
-    else launch(std::false_type{}, std::false_type{});
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if constexpr (Inverse) {
+        if (repair) return launch(yes, no, no);
+    }
+    if (wide && place) launch(no, yes, yes);
+    else if (wide) launch(no, yes, no);
+    else if (place) launch(no, no, yes);
+    else launch(no, no, no);
 }
 
 template <class T, bool Requant, bool Screen>

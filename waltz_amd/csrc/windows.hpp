@@ -32,6 +32,18 @@ constexpr bool zcol_lds_fits(uint32_t nz, unsigned width) { return zcol_lds_byte
 constexpr bool zcol_place_fits(uint32_t nz, unsigned levels, unsigned width) {
     return zcol_lds_bytes(nz, levels, width, true) <= 65536;
 }
+// Threads of a workgroup of columns, by the workgroups of the launch and their
+// LDS. Where a CU gets no second workgroup, a row of columns is a chain of tiles
+// per wave and lasts the longer the fewer its waves are (260x60x9 float, z first:
+// compress 131 us with 4 waves, 114 with 8, 107 with 16; 200x200x64 float forward
+// 19.3, 16.1, 15.1). Beyond that four are enough (100x2000x64 float inverse 29.5,
+// 35.9, 68.3), except in place where LDS holds the workgroups of a CU to two or
+// three (100x2000x64 double, 64 KiB: 59.6, 51.2, 68.7; 99x3300x3370, 5.7, 4.8 ms;
+// but 60x3300x3370, 38 KiB: 2.5, 2.6).
+constexpr uint32_t kZThreads = 256, kZThreadsPlace = 512, kZThreadsMost = 1024;
+constexpr uint32_t zcol_threads(uint64_t workgroups, bool in_place, uint64_t lds) {
+    return workgroups <= 256 ? kZThreadsMost : in_place && lds > 49152 ? kZThreadsPlace : kZThreads;
+}
 // Whether every one of `levels` levels lifts lines of at least two samples. One
 // sample is its own even and odd neighbour: kernels that address the two halves
 // of a line apart would read past it.

@@ -11,8 +11,8 @@
 
 namespace wz {
 
-// A workgroup of four waves owns a row of 64 columns, all z; a wave takes one tile of the
-// 64 columns at a time, a lane a column, so that a tile's rows, their
+// A workgroup of four waves (more: zcol_threads) owns a row of 64 columns, all z; a
+// wave takes one tile of the 64 columns at a time, a lane a column, so that a tile's rows, their
 // mirrored places and its tests are wave-uniform (scalar): per sample only the
 // lifting itself and its loads and stores reach the vector unit. The finest
 // level reads (forward) or writes (inverse) the field and every high band
@@ -26,8 +26,6 @@ namespace wz {
 // every column staged in LDS and per-lane index arithmetic it was bound by
 // vector issue: 500x500x100 float 108 -> 55 us (forward), 127 -> 61 us
 // (inverse), 384x384x96 double 70 -> 56 us, 73 -> 67 us.
-constexpr uint32_t kZThreads = 256;
-
 // Repair (inverse, compress): the reconstruction is not written; each sample
 // is compared with the original as its tile is lifted, and the native repair
 // records and flag bits go out (one segment per workgroup, columns x nz slots).
@@ -111,18 +109,18 @@ struct ZColumnsOf {
     uint32_t levels;
 };
 
-// Row y, columns x0 .. x0 + 63 by one workgroup of kZThreads threads; `box0`,
+// Row y, columns x0 .. x0 + 63 by one workgroup of `Threads` threads; `box0`,
 // `box1`: zcol_lds_bytes of LDS. Returns whether this lane met nothing to flag
 // (a non-finite sample of a screened pass, or an unmet bound). Wide: volumes
 // past one window, every plane through its own (3370x3300x99 float, 4.4 GB:
 // forward 2.2 ms, 4.0 TB/s). InPlace: src may be dst; the finest level's rows
 // from `from` on wait in `held` (zcol_held_rows of LDS) until all are read.
-template <class T, bool Inverse, bool Repair, bool Wide = false, bool InPlace = false>
+template <class T, bool Inverse, bool Repair, bool Wide = false, bool InPlace = false, uint32_t Threads = kZThreads>
 WZ_D bool zcol_columns(const ZColumnsOf<T>& a, uint32_t y, uint32_t x0, T* box0, T* box1, bool screen,
                        const ZOutput<T>& out, const WaveRepair<T>& rp, uint32_t id, uint32_t* seg_fill,
                        T* held = nullptr) {
     constexpr int Tile = sizeof(T) == 4 ? 16 : 8, P = Tile / 2 + 4;  // (the inverse's is part of the format)
-    constexpr uint32_t W = kZThreads / 64, S = sizeof(T);
+    constexpr uint32_t W = Threads / 64, S = sizeof(T);
     static_assert(!(Repair && Wide), "the codec's fields fit one window");
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const uint32_t x = x0 + lane;
