@@ -178,7 +178,7 @@ WZ_D void exclusive_scan_block(uint32_t* a, uint32_t len, uint32_t* total) {
 }
 
 // Lays out the archive sections and writes the header and the sections'
-// padding (one thread).
+// padding (one thread); without an archive only the result.
 template <class T>
 WZ_D void write_layout(uint8_t* __restrict__ archive, uint64_t capacity, uint32_t n, uint32_t np, uint32_t nq,
                        uint32_t qcapacity, uint8_t flags, uint8_t lx, uint8_t lz, uint8_t bz, double quantum,
@@ -193,7 +193,7 @@ WZ_D void write_layout(uint8_t* __restrict__ archive, uint64_t capacity, uint32_
     res->nq = nq;
     res->end = L.end;
     res->status = st;
-    if (st) return;
+    if (st || !archive) return;
     uint8_t h[32];
     h[0] = flags;
     h[1] = lx;
