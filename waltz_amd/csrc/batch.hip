@@ -493,66 +493,83 @@ __global__ void __launch_bounds__(256) batch_pass_kernel(const JobShape* __restr
     if (__ballot(!fin) && (threadIdx.x & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteOutput));
 }
 
-constexpr uint32_t kRecords = 8;         // repair records per thread and round
 constexpr uint32_t kRpatchBlocks = 2048;  // fixed grid (the record count is known on the device only)
 
+// Records [b0, b1) of all jobs by one wave, N per lane (every 64th): their
+// indexes and errors, then their samples, are all in flight at once.
+template <uint32_t N, class T>
+WZ_D void patch_records(const uint8_t* __restrict__ packed, const JobShape* __restrict__ shape,
+                        const JobRun* __restrict__ run, const uint32_t* __restrict__ np_pfx, uint32_t jobs,
+                        uint32_t b0, uint32_t b1, T* __restrict__ out, uint32_t* status) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t j0 = __builtin_amdgcn_readfirstlane(job_of_wave(np_pfx, jobs, b0));
+    const bool one = b1 <= np_pfx[j0 + 1];  // scalar job data
+    uint32_t j = j0;
+    uint32_t jr[N], at[N];
+    T err[N], v[N];
+    uint64_t o[N];
+    uint32_t kept = 0;  // bit u: record u changes a sample
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) {
+        const uint32_t k = min(b0 + 64u * u + lane, b1 - 1u);
+        // the next job, or (jobs with few records, or none) a search
+        if (!one && k >= np_pfx[j + 1]) j = k < np_pfx[min(j + 2, jobs)] ? j + 1 : job_of(np_pfx, jobs, k);
+        jr[u] = one ? j0 : j;
+        const JobRun& r = run[jr[u]];
+        const uint8_t* a = packed + r.arc;
+        const uint32_t e = k - np_pfx[jr[u]];
+        at[u] = reinterpret_cast<const uint32_t*>(a + r.pi)[e];
+        err[u] = reinterpret_cast<const T*>(a + r.pv)[e];
+    }
+    bool corrupt = false, fin = true;
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) {
+        const bool in = b0 + 64u * u + lane < b1;
+        const JobShape& sh = shape[jr[u]];
+        const uint32_t i = at[u];
+        const bool bad = i >= sh.n || !__builtin_isfinite(err[u]);
+        corrupt = corrupt || (in && bad);
+        const uint32_t x = i % sh.d.nx, y = (i / sh.d.nx) % sh.d.ny, z = i / (sh.d.nx * sh.d.ny);
+        const bool put = in && !bad && x < sh.clip.nx && y < sh.clip.ny && z < sh.clip.nz;
+        kept |= uint32_t(put) << u;
+        o[u] = sh.out + (put ? uint64_t(z) * sh.opz + uint64_t(y) * sh.opy + x : 0u);
+        v[u] = out[o[u]];  // (any sample of the tile, where none is kept)
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) {
+        if (!((kept >> u) & 1u)) continue;
+        const T w = v[u] - err[u];  // cpu/src/codec.cpp:330
+        out[o[u]] = w;
+        fin = fin && __builtin_isfinite(w);
+    }
+    if (corrupt) atomicOr(status, uint32_t(kCorrupt));
+    if (!fin) atomicOr(status, uint32_t(kNonFiniteOutput));
+}
+
+// A record is a chain of two scattered reads, so one after the other the pass
+// was bound by their latency: a wave takes 512 consecutive records (256 float
+// chunks, 96 M samples: 102 us with four in turn per thread, now 80: partial lines
+// read and written at memory), or 64 where that is one round for all of them:
+// then the chain is all there is, and fewer jobs meet in a wave (64 jobs of
+// 64x64 float: 14 us with 512, 4.0 with 64; with four in turn 8.5).
 template <class T>
 __global__ void __launch_bounds__(256) batch_rpatch_kernel(const uint8_t* __restrict__ packed,
                                                            const JobShape* __restrict__ shape,
                                                            const JobRun* __restrict__ run,
                                                            const uint32_t* __restrict__ np_pfx, uint32_t jobs,
                                                            T* __restrict__ out, uint32_t* status) {
-    // a wave takes 64 * kRecords consecutive records, a lane every 64th of
-    // them: their indexes and errors, then their samples, are all in flight
-    // at once. A record is a chain of two scattered reads, so one after the
-    // other the pass was bound by their latency (256 float chunks, 96 M
-    // samples: 102 us, now 80: partial lines read and written at memory).
-    const uint32_t total = np_pfx[jobs], lane = threadIdx.x & 63u;
+    constexpr uint32_t kMany = 8;
+    const uint32_t total = np_pfx[jobs], lanes = gridDim.x * 256u;
     const uint32_t wave = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (uint64_t base = uint64_t(wave) * 64u * kRecords; base < total; base += uint64_t(gridDim.x) * 256u * kRecords) {
-        const uint32_t b0 = uint32_t(base), b1 = min(b0 + 64u * kRecords, total);
-        const uint32_t j0 = __builtin_amdgcn_readfirstlane(job_of_wave(np_pfx, jobs, b0));
-        const bool one = b1 <= np_pfx[j0 + 1];  // the usual case: scalar job data
-        uint32_t j = j0;
-        uint32_t jr[kRecords], at[kRecords];
-        T err[kRecords], v[kRecords];
-        uint64_t o[kRecords];
-        uint32_t kept = 0;  // bit u: record u changes a sample
-#pragma unroll
-        for (uint32_t u = 0; u < kRecords; ++u) {
-            const uint32_t k = min(b0 + 64u * u + lane, b1 - 1u);
-            if (!one)
-                while (k >= np_pfx[j + 1]) ++j;  // jobs without repairs are skipped
-            jr[u] = one ? j0 : j;
-            const JobRun& r = run[jr[u]];
-            const uint8_t* a = packed + r.arc;
-            const uint32_t e = k - np_pfx[jr[u]];
-            at[u] = reinterpret_cast<const uint32_t*>(a + r.pi)[e];
-            err[u] = reinterpret_cast<const T*>(a + r.pv)[e];
-        }
-        bool corrupt = false, fin = true;
-#pragma unroll
-        for (uint32_t u = 0; u < kRecords; ++u) {
-            const bool in = b0 + 64u * u + lane < b1;
-            const JobShape& sh = shape[jr[u]];
-            const uint32_t i = at[u];
-            const bool bad = i >= sh.n || !__builtin_isfinite(err[u]);
-            corrupt = corrupt || (in && bad);
-            const uint32_t x = i % sh.d.nx, y = (i / sh.d.nx) % sh.d.ny, z = i / (sh.d.nx * sh.d.ny);
-            const bool put = in && !bad && x < sh.clip.nx && y < sh.clip.ny && z < sh.clip.nz;
-            kept |= uint32_t(put) << u;
-            o[u] = sh.out + (put ? uint64_t(z) * sh.opz + uint64_t(y) * sh.opy + x : 0u);
-            v[u] = out[o[u]];  // (any sample of the tile, where none is kept)
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kRecords; ++u) {
-            if (!((kept >> u) & 1u)) continue;
-            const T w = v[u] - err[u];  // cpu/src/codec.cpp:330
-            out[o[u]] = w;
-            fin = fin && __builtin_isfinite(w);
-        }
-        if (corrupt) atomicOr(status, uint32_t(kCorrupt));
-        if (!fin) atomicOr(status, uint32_t(kNonFiniteOutput));
+    if (total <= lanes) {
+        const uint32_t b0 = wave * 64u;
+        if (b0 < total) patch_records<1>(packed, shape, run, np_pfx, jobs, b0, min(b0 + 64u, total), out, status);
+        return;
+    }
+    for (uint64_t b = uint64_t(wave) * 64u * kMany; b < total; b += uint64_t(lanes) * kMany) {
+        const uint32_t b0 = uint32_t(b);
+        patch_records<kMany>(packed, shape, run, np_pfx, jobs, b0, uint32_t(min(b + 64u * kMany, uint64_t(total))), out,
+                             status);
     }
 }
 
