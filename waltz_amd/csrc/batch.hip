@@ -44,6 +44,7 @@
 #include "bricks.hpp"
 #include "fused.hpp"
 #include "lifting.hpp"
+#include "planetail.hpp"
 #include "sections.hpp"
 #include "wzp_encode.hpp"
 #include "xystrip.hpp"
@@ -84,13 +85,13 @@ struct JobRun {
 };
 
 struct Pass {
-    uint8_t kind, src, dst, levels;  // levels: of a column pass
-    // volume of a strip pass: 0 the bank's at the job's pitches, l >= 1 the
-    // compact XY box of level l in the tmp0 bank
-    uint8_t src_box, low_box, dst_box, pad;
+    uint8_t kind, src, dst, levels;  // levels: of a column pass, or of a job's XY schedule (plane pass)
+    // volume of a strip or plane pass: 0 the bank's at the job's pitches, l >= 1
+    // the compact XY box of level l in the tmp0 bank
+    uint8_t src_box, low_box, dst_box, level;  // level: the finest of a plane pass
     Dims act;           // box of this pass
     uint32_t ntiles;    // tiles per line
-    uint32_t work;      // work items: threads, or workgroups of a strip / column pass
+    uint32_t work;      // work items: threads, or workgroups of a strip, column or plane pass
     StripPlan strip;
 };
 
@@ -903,10 +904,10 @@ __global__ void __launch_bounds__(256) batch_place_kernel(const JobShape* __rest
 // (Z levels, zcolumns.hpp) over all jobs, each one launch per step. Bound by
 // memory; staging whole planes and columns in LDS was bound by vector issue:
 // 256 chunks (96 M float samples) decoded 1310 -> 862 us, 64 chunks compressed
-// 765 -> 550 us. A workgroup per plane taking the coarse levels in one launch,
-// as the single-field path does, is slower here: there are planes enough to
-// fill a launch per level (decode 835 -> 956 us).
-enum : uint8_t { kPassStrip = 6, kPassZCol = 7 };
+// 765 -> 550 us. Plane passes take each plane of a plane-schedule job through its
+// coarse XY levels, a workgroup per plane: for batches so small that a level's
+// launch is mostly the way to its first load (few_planes).
+enum : uint8_t { kPassStrip = 6, kPassZCol = 7, kPassPlanes = 8 };
 
 // Banks of these passes: input (compress forward), the three work banks, the
 // output (decode) or reconstruction (compress inverse), and where failures go.
@@ -925,13 +926,14 @@ struct Volume {
 };
 template <class T>
 WZ_D Volume<T> volume_of(const StageBanks& b, const JobShape& sh, uint8_t id, uint8_t box) {
-    if (box) {  // odd levels at offset 0, even ones after the level-1 box (the two never alias)
-        uint32_t nx = sh.d.nx, ny = sh.d.ny;
-        for (uint8_t l = 0; l < box; ++l) {
+    if (box) {  // one level's after the other, as xy_box()
+        uint32_t nx = half_len(sh.d.nx), ny = half_len(sh.d.ny);
+        uint64_t first = 0;
+        for (uint8_t l = 1; l < box; ++l) {
+            first += uint64_t(nx) * ny * sh.d.nz;
             nx = half_len(nx);
             ny = half_len(ny);
         }
-        const uint64_t first = (box & 1u) ? 0u : uint64_t(half_len(sh.d.nx)) * half_len(sh.d.ny) * sh.d.nz;
         return {static_cast<T*>(b.tmp0) + sh.bank + first, nx, uint64_t(nx) * ny};
     }
     const uint64_t py = sh.d.nx, pz = uint64_t(sh.d.nx) * sh.d.ny;
@@ -1008,6 +1010,69 @@ __global__ void __launch_bounds__(kZThreads) batch_zcol_kernel(const JobShape* _
     }
 }
 
+constexpr uint32_t kPlaneThreads = 64 * kPlaneTailWaves;
+// The strips of one plane on the waves of one workgroup, y segments of the length
+// with the fewest steps in a row (a segment of sy rows takes sy / 2 + 4).
+WZ_D StripPlan plane_plan(Dims n) {
+    StripPlan best = strip_plan(n, false, 1u, 128u);
+    uint32_t least = ~0u;
+    for (uint32_t sy = 128; sy >= 8; sy >>= 1) {
+        const uint32_t segs = (n.ny + sy - 1) / sy;
+        const uint32_t steps = ((best.strips * segs + kPlaneTailWaves - 1) / kPlaneTailWaves) * (sy / 2 + 4);
+        if (steps >= least) continue;
+        least = steps;
+        best.sy = sy;
+        best.segs = segs;
+    }
+    return best;
+}
+template <class T, bool Inverse>
+__global__ void __launch_bounds__(kPlaneThreads) batch_planes_kernel(const JobShape* __restrict__ shape,
+                                                                     const JobRun* __restrict__ run,
+                                                                     const Pass* __restrict__ pass,
+                                                                     const uint32_t* __restrict__ pfx, uint32_t jobs,
+                                                                     StageBanks b, T fill, uint32_t* status) {
+    const uint32_t id = xcd_place(pfx[jobs]);
+    if (id >= pfx[jobs]) return;
+    const uint32_t j = __builtin_amdgcn_readfirstlane(job_of_wave(pfx, jobs, id));
+    const Pass& ps = pass[j];
+    const uint32_t state = run ? run[j].state : uint32_t(kJobOk);
+    if (state == kJobBad || (state == kJobHole && ps.dst != kOutput)) return;
+    const JobShape& sh = shape[j];
+    const uint32_t z = id - pfx[j], wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t l0 = ps.level, l1 = ps.levels;
+    auto plane = [z](Volume<T> v) { return Volume<T>{v.p + uint64_t(z) * v.pz, v.py, v.pz}; };
+    const Volume<T> home = plane(volume_of<T>(b, sh, kHome, 0));
+    bool fin = true;
+    for (uint32_t k = l0; k < l1; ++k) {
+        const uint32_t l = Inverse ? l1 - 1u - (k - l0) : k;
+        Dims n{sh.d.nx, sh.d.ny, 1};
+        for (uint32_t i = 0; i < l; ++i) n = Dims{half_len(n.nx), half_len(n.ny), 1};
+        const StripPlan plan = plane_plan(n);
+        const Volume<T> low = l + 1 == l1 ? home : plane(volume_of<T>(b, sh, kTmp0, uint8_t(l + 1)));
+        if constexpr (Inverse) {
+            const bool last = l == 0 && ps.dst == kOutput;
+            const Volume<T> dst = plane(volume_of<T>(b, sh, l ? uint8_t(kTmp0) : ps.dst, uint8_t(l)));
+            const Dims kept = last ? Dims{sh.clip.nx, sh.clip.ny, z < sh.clip.nz ? 1u : 0u} : n;
+            const XYInverse<T> a{home.p, home.py, home.pz, low.p, low.py, low.pz, dst.p, dst.py, dst.pz,
+                                 n,      T(0),    T(0),    0u};
+            for (uint32_t i = wave; i < plan.items(); i += kPlaneTailWaves) {
+                StripOutput<T> out{kept, last && state == kJobHole, fill};
+                strip_inverse<T, false>(a, plan, i, out);
+                fin = fin && (out.finite || !last);
+            }
+        } else {
+            const Volume<T> src = plane(volume_of<T>(b, sh, l ? uint8_t(kTmp0) : ps.src, uint8_t(l)));
+            const XYForward<T> a{src.p,  src.py, src.pz, home.p, home.py,
+                                 home.pz, low.p,  low.py, low.pz, n,
+                                 l == 0 && ps.src == kInput ? &b.res[j].status : nullptr};
+            for (uint32_t i = wave; i < plan.items(); i += kPlaneTailWaves) strip_forward<T>(a, plan, i);
+        }
+        __syncthreads();
+    }
+    if (Inverse && __ballot(!fin) && (threadIdx.x & 63u) == 0) atomicOr(status, uint32_t(kNonFiniteOutput));
+}
+
 // ------------------------------------------------------------------ host plan
 Dims halve(Dims d, bool xy, bool z) {
     if (xy) {
@@ -1059,6 +1124,20 @@ Pass strip_pass(const JobShape& sh, uint8_t src, uint8_t src_box, uint8_t low_bo
     p.work = uint32_t((p.strip.items() + 3) / 4);
     return p;
 }
+// XY levels l .. levels - 1 of a plane-schedule job, from `src` (forward) or into
+// `dst` (inverse) where l is 0.
+Pass plane_pass(const JobShape& sh, uint8_t src, uint8_t dst, unsigned l) {
+    Pass p{};
+    p.kind = kPassPlanes;
+    p.src = src;
+    p.dst = dst;
+    p.level = uint8_t(l);
+    p.levels = uint8_t(sh.lx);
+    p.act = sh.d;
+    p.ntiles = 1;
+    p.work = sh.d.nz;
+    return p;
+}
 Pass column_pass(uint8_t src, uint8_t dst, Dims act, unsigned levels) {
     Pass p{};
     p.kind = kPassZCol;
@@ -1107,7 +1186,7 @@ void axis_level(std::vector<Pass>& out, Dims act, std::initializer_list<uint8_t>
 // Z) into scratch and a strip pass (X then Y) back into the home bank. The
 // plane schedule is a strip pass per XY level, through compact boxes, and one
 // column pass for all Z levels when they fit its LDS, else one per level.
-std::vector<Pass> inverse_schedule(const JobShape& sh, unsigned width, uint32_t jobs) {
+std::vector<Pass> inverse_schedule(const JobShape& sh, unsigned width, uint32_t jobs, bool tails) {
     std::vector<Pass> out;
     if (sh.lx == 0 && sh.lz == 0) {
         out.push_back(make_pass(kPassCopy, kHome, kOutput, sh.d, width));
@@ -1138,14 +1217,12 @@ std::vector<Pass> inverse_schedule(const JobShape& sh, unsigned width, uint32_t 
         return out;
     }
     uint8_t at = kHome;  // where the whole volume is
-    for (int l = int(sh.lx) - 1; l >= 0; --l) {
+    if (sh.lx) at = !sh.lz && strip_output_fits(sh, width) ? uint8_t(kOutput) : uint8_t(kTmp1);
+    const unsigned tail = tails ? plane_tail_level(sh.d, sh.lx) : sh.lx;
+    if (tail < sh.lx) out.push_back(plane_pass(sh, kHome, at, tail));
+    for (int l = int(tail) - 1; l >= 0; --l) {
         const uint8_t low = l + 1 == int(sh.lx) ? 0 : uint8_t(l + 1);
-        if (l) {
-            out.push_back(strip_pass(sh, kHome, 0, low, kTmp0, uint8_t(l), xy[l], width, jobs));
-        } else {
-            at = !sh.lz && strip_output_fits(sh, width) ? uint8_t(kOutput) : uint8_t(kTmp1);
-            out.push_back(strip_pass(sh, kHome, 0, low, at, 0, xy[0], width, jobs));
-        }
+        out.push_back(strip_pass(sh, kHome, 0, low, l ? uint8_t(kTmp0) : at, uint8_t(l), xy[l], width, jobs));
     }
     if (sh.lz && zcol_lds_fits(sh.d.nz, width)) {
         const uint8_t dst = column_output_fits(sh, width) ? uint8_t(kOutput) : at == kHome ? uint8_t(kTmp1) : uint8_t(kHome);
@@ -1165,7 +1242,7 @@ std::vector<Pass> inverse_schedule(const JobShape& sh, unsigned width, uint32_t 
 // The forward schedule of transform_forward (cpu/src/transform.cpp:425-456):
 // the first pass reads the job's input, the coefficients end in the home bank.
 // Mirrors inverse_schedule; forward tiles do not change a bit.
-std::vector<Pass> forward_schedule(const JobShape& sh, unsigned width, uint32_t jobs) {
+std::vector<Pass> forward_schedule(const JobShape& sh, unsigned width, uint32_t jobs, bool tails) {
     std::vector<Pass> out;
     if (sh.lx == 0 && sh.lz == 0) {
         out.push_back(make_pass(kPassCopy, kInput, kHome, sh.d, width));
@@ -1208,18 +1285,37 @@ std::vector<Pass> forward_schedule(const JobShape& sh, unsigned width, uint32_t 
             src = zdst;
         }
     }
-    for (unsigned l = 0; l < sh.lx; ++l)
+    const unsigned tail = tails ? plane_tail_level(sh.d, sh.lx) : sh.lx;
+    for (unsigned l = 0; l < tail; ++l)
         out.push_back(strip_pass(sh, l ? uint8_t(kTmp0) : src, uint8_t(l), l + 1 == sh.lx ? 0 : uint8_t(l + 1), kHome, 0,
                                  xy[l], width, jobs));
+    if (tail < sh.lx) out.push_back(plane_pass(sh, tail ? uint8_t(kTmp0) : src, kHome, tail));
     return out;
+}
+
+// Whether a batch's coarse XY levels run as plane passes: there are no other jobs
+// whose launches they would share (eight of the 32^3 .. 64x128x128 mix compress
+// in 246 us with strips, 267 with planes), and the planes fit the device at once
+// (8 waves and up to 100 VGPRs: two workgroups a CU). Strips and planes, compress /
+// decode in us: 64 tiles of 64x64 float 115 / 67, 104 / 58 (with every level in LDS
+// 107 / 65); one of 32x64x64 130 / 71, 114 / 60; 16 of those (512 planes) 151 / 78,
+// 138 / 73; 32 of them 173 / 95, 185 / 100. 16 waves a workgroup gain nothing up to
+// 256 planes and lose above.
+bool few_planes(const std::vector<JobShape>& jobs) {
+    uint64_t planes = 0;
+    for (const JobShape& s : jobs) {
+        if (s.dyadic || plane_tail_level(s.d, s.lx) >= s.lx) return false;
+        planes += s.d.nz;
+    }
+    return planes <= 512;
 }
 
 // One step's launches: every job's pass at that step, and the block prefixes
 // of the per-axis kernel (256-thread blocks of work items), the strip kernel
-// and the column kernel (with its LDS).
+// the column kernel (with its LDS) and the plane kernel.
 struct StepTables {
     std::vector<std::vector<Pass>> pass;                  // [step][job]
-    std::vector<std::vector<uint32_t>> pfx, spfx, zpfx;   // [step][job + 1]
+    std::vector<std::vector<uint32_t>> pfx, spfx, zpfx, ppfx;   // [step][job + 1]
     std::vector<uint32_t> zlds;                           // [step]
 };
 StepTables build_steps(const std::vector<std::vector<Pass>>& sched, uint32_t J, unsigned width) {
@@ -1227,10 +1323,10 @@ StepTables build_steps(const std::vector<std::vector<Pass>>& sched, uint32_t J, 
     for (const auto& v : sched) steps = std::max(steps, v.size());
     StepTables t;
     t.pass.assign(steps, std::vector<Pass>(J));
-    for (auto* p : {&t.pfx, &t.spfx, &t.zpfx}) p->assign(steps, std::vector<uint32_t>(J + 1, 0));
+    for (auto* p : {&t.pfx, &t.spfx, &t.zpfx, &t.ppfx}) p->assign(steps, std::vector<uint32_t>(J + 1, 0));
     t.zlds.assign(steps, 0);
     for (size_t st = 0; st < steps; ++st) {
-        uint64_t blocks = 0, sblocks = 0, zblocks = 0;
+        uint64_t blocks = 0, sblocks = 0, zblocks = 0, pblocks = 0;
         for (uint32_t j = 0; j < J; ++j) {
             Pass ps{};
             ps.kind = kPassNone;
@@ -1239,7 +1335,10 @@ StepTables build_steps(const std::vector<std::vector<Pass>>& sched, uint32_t J, 
             t.pfx[st][j] = uint32_t(blocks);
             t.spfx[st][j] = uint32_t(sblocks);
             t.zpfx[st][j] = uint32_t(zblocks);
-            if (ps.kind == kPassStrip) {
+            t.ppfx[st][j] = uint32_t(pblocks);
+            if (ps.kind == kPassPlanes) {
+                pblocks += ps.work;
+            } else if (ps.kind == kPassStrip) {
                 sblocks += ps.work;
             } else if (ps.kind == kPassZCol) {
                 zblocks += ps.work;
@@ -1248,10 +1347,11 @@ StepTables build_steps(const std::vector<std::vector<Pass>>& sched, uint32_t J, 
                 blocks += (uint64_t(ps.work) + 255) / 256;
             }
         }
-        if (std::max({blocks, sblocks, zblocks}) > 0x7FFFFFF0ull) throw std::invalid_argument("batch launch limit");
+        if (std::max({blocks, sblocks, zblocks, pblocks}) > 0x7FFFFFF0ull) throw std::invalid_argument("batch launch limit");
         t.pfx[st][J] = uint32_t(blocks);
         t.spfx[st][J] = uint32_t(sblocks);
         t.zpfx[st][J] = uint32_t(zblocks);
+        t.ppfx[st][J] = uint32_t(pblocks);
     }
     return t;
 }
@@ -1269,6 +1369,7 @@ struct HostPlan {
     std::vector<uint32_t> chunk_pfx, brick_pfx;
     // chunks of each kind of coder's jobs (one WZP launch each)
     std::vector<uint32_t> cube_pfx, direct_pfx, rank_pfx, mag_pfx;
+    bool tails = false;                       // coarse XY levels as plane passes
     StepTables inv;                           // inverse passes
     uint64_t bank_elems = 0, mag_elems = 0, sign_words = 0, out_elems = 0;
     // compress
@@ -1343,7 +1444,7 @@ void finish_compress_plan(HostPlan& p) {
         tiles += c.tiles;
         pblocks += c.pblocks;
         places += uint64_t(c.tiles) + c.qblocks;
-        sched[j] = forward_schedule(s, w, J);
+        sched[j] = forward_schedule(s, w, J, p.tails);
     }
     if (groups > 0x7FFFFFFFull || tiles > 0x7FFFFFFFull || 2 * pblocks > 0x7FFFFFFFull || places > 0x7FFFFFFFull)
         throw std::invalid_argument("batch launch limit");
@@ -1393,6 +1494,7 @@ void finish_plan(HostPlan& p) {
     p.rank_pfx.assign(J + 1, 0);
     p.mag_pfx.assign(J + 1, 0);
     std::vector<std::vector<Pass>> sched(J);
+    p.tails = few_planes(p.shape);
     uint64_t bank = 0, mag = 0, sign = 0, chunks = 0, bricks = 0, cubes = 0, dchunks = 0, rchunks = 0, mchunks = 0;
     p.rank_geo.clear();
     for (uint32_t j = 0; j < J; ++j) {
@@ -1432,7 +1534,7 @@ void finish_plan(HostPlan& p) {
             mchunks += s.chunks;
             bricks += (uint64_t(s.nbx) * s.nby * s.nbz + kBricksPerBlock - 1) / kBricksPerBlock;  // brick blocks
         }
-        sched[j] = inverse_schedule(s, p.width, J);
+        sched[j] = inverse_schedule(s, p.width, J, p.tails);
     }
     if (chunks > 0x7FFFFFFFull || bricks > 0x7FFFFFFFull) throw std::invalid_argument("batch launch limit");
     p.chunk_pfx[J] = uint32_t(chunks);
@@ -1458,7 +1560,7 @@ struct DevicePlan {
     uint32_t *cube_pfx = nullptr, *direct_pfx = nullptr, *rank_pfx = nullptr, *mag_pfx = nullptr;
     struct DeviceSteps {
         Pass* pass;                     // steps x jobs
-        uint32_t *pfx, *spfx, *zpfx;    // steps x (jobs + 1)
+        uint32_t *pfx, *spfx, *zpfx, *ppfx;    // steps x (jobs + 1)
     } inv{}, fwd{};
     uint32_t* host_status = nullptr;  // pinned
     // compress tables
@@ -1498,7 +1600,7 @@ struct DevicePlan {
         const size_t o_comp = carve(sizeof(JobComp) * J), o_tp = carve(4 * (J + 1)),
                      o_pbp = carve(4 * (J + 1)), o_plp = carve(4 * (J + 1));
         const StepTables* tables[2] = {&p.inv, &p.fwd};
-        size_t o_pass[2], o_pfx[2][3];
+        size_t o_pass[2], o_pfx[2][4];
         for (int k = 0; k < 2; ++k) {
             const size_t S = tables[k]->pass.size();
             o_pass[k] = carve(sizeof(Pass) * J * S);
@@ -1526,18 +1628,19 @@ struct DevicePlan {
         place_pfx = reinterpret_cast<uint32_t*>(mem + o_plp);
         // the steps' tables, flattened (kept until the copies are done, below)
         std::vector<Pass> flat[2];
-        std::vector<uint32_t> prefixes[2][3];
+        std::vector<uint32_t> prefixes[2][4];
         for (int k = 0; k < 2; ++k) {
             DeviceSteps& d = k ? fwd : inv;
             d.pass = reinterpret_cast<Pass*>(mem + o_pass[k]);
-            uint32_t** place[3] = {&d.pfx, &d.spfx, &d.zpfx};
-            const std::vector<std::vector<uint32_t>>* from[3] = {&tables[k]->pfx, &tables[k]->spfx, &tables[k]->zpfx};
+            uint32_t** place[4] = {&d.pfx, &d.spfx, &d.zpfx, &d.ppfx};
+            const std::vector<std::vector<uint32_t>>* from[4] = {&tables[k]->pfx, &tables[k]->spfx, &tables[k]->zpfx,
+                                                                 &tables[k]->ppfx};
             for (const auto& v : tables[k]->pass) flat[k].insert(flat[k].end(), v.begin(), v.end());
             if (!flat[k].empty())
                 hip_check(hipMemcpyAsync(d.pass, flat[k].data(), sizeof(Pass) * flat[k].size(), hipMemcpyHostToDevice,
                                          s),
                           "plan");
-            for (int q = 0; q < 3; ++q) {
+            for (int q = 0; q < 4; ++q) {
                 *place[q] = reinterpret_cast<uint32_t*>(mem + o_pfx[k][q]);
                 for (const auto& v : *from[q]) prefixes[k][q].insert(prefixes[k][q].end(), v.begin(), v.end());
                 if (!prefixes[k][q].empty())
@@ -1565,13 +1668,13 @@ struct DevicePlan {
         hip_check(hipStreamSynchronize(s), "plan upload");
     }
 
-    // The strip and column passes of one step.
+    // The strip, column and plane passes of one step.
     template <class T, bool Inverse>
     void launch_step(size_t st, const JobRun* r, const StageBanks& sb, T fill, uint32_t* status_word,
                      hipStream_t s) const {
         const StepTables& t = Inverse ? host.inv : host.fwd;
         const DeviceSteps& d = Inverse ? inv : fwd;
-        const uint32_t J = host.jobs, strips = t.spfx[st][J], columns = t.zpfx[st][J];
+        const uint32_t J = host.jobs, strips = t.spfx[st][J], columns = t.zpfx[st][J], planes = t.ppfx[st][J];
         if (strips)
             hipLaunchKernelGGL((batch_strip_kernel<T, Inverse>), dim3(8 * ((strips + 7) / 8)), dim3(kStripThreads), 0,
                                s, shape, r, d.pass + st * J, d.spfx + st * (J + 1), J, sb, fill, status_word);
@@ -1579,6 +1682,9 @@ struct DevicePlan {
             hipLaunchKernelGGL((batch_zcol_kernel<T, Inverse>), dim3(8 * ((columns + 7) / 8)), dim3(kZThreads),
                                t.zlds[st], s, shape, r, d.pass + st * J, d.zpfx + st * (J + 1), J, sb, fill,
                                status_word);
+        if (planes)
+            hipLaunchKernelGGL((batch_planes_kernel<T, Inverse>), dim3(8 * ((planes + 7) / 8)), dim3(kPlaneThreads), 0,
+                               s, shape, r, d.pass + st * J, d.ppfx + st * (J + 1), J, sb, fill, status_word);
     }
 
     // Enqueues the batched compress on `s`: no synchronisation, allocation or
