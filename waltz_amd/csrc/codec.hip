@@ -252,7 +252,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
         p.qbm = c.take<uint32_t>(words);
         if (shared_words) p.rbm = c.take<uint32_t>(words);
         p.glen = c.take<uint32_t>(ws.groups);
-        p.counters = c.take<uint32_t>(4);  // ticket, q count, repair total
+        p.counters = c.take<uint32_t>(4);  // (unused), q count, repair total
         p.res = c.take<EncodeResult>(1);
         p.zeroed = reinterpret_cast<uint32_t*>(c.base + z0);
         return std::make_pair(p, c.used - z0);
@@ -284,7 +284,7 @@ uint64_t compress(const T* input, Dims d, double abs_bound, uint8_t* archive, ui
     // it as much as they hid, and the payload placement then collided with the
     // finest level, which needs every CU's two workgroup slots.
     const bool split = requant && coarse_split_fits(g.d, g.lx, sizeof(T));
-    // a plane-schedule field whose inverse runs as fused XY levels quantizes
+    // a plane-schedule field whose inverse runs as strips and columns quantizes
     // and dequantizes the coefficients as they load: nothing written back
     const bool plane_requant = !g.dyadic && plane_fused_fits(g.d, g.lx, g.lz, sizeof(T));
     const WriteBack wb = split || plane_requant ? kWriteNone : requant ? kWriteCoarseBox : kWriteAll;

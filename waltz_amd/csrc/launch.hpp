@@ -52,7 +52,8 @@ struct Level0Emit {
 // tile), or 0 when a list of np entries of `width`-byte values cannot be
 // folded into the finest level's stores for this geometry.
 uint64_t patch_table_words(Dims full, uint32_t np, unsigned width);
-// Returns true when `emit` was carried out inside the last pass; false means the caller must run the equivalent separate pass on `output`.
+// Returns true when `emit` was carried out inside the last pass; false means
+// the caller must run the equivalent separate pass on `output`.
 // requant > 0 (plane-schedule fields with plane_fused_fits only): coeff holds
 // the unquantized coefficients, quantized with this quantum and dequantized
 // as the levels load them.
@@ -97,9 +98,9 @@ void transform_adjoint(T* data, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsig
 // finest level fused with the same requantization and `emit`. Applies when
 // coarse_split_fits (dyadic, >= 2 levels, both leading levels fused).
 bool coarse_split_fits(Dims full, unsigned lxy, unsigned width);
-// Whether the plane schedule's inverse of this geometry runs as fused XY
-// levels and one LDS-staged Z phase; that inverse screens its output for
-// non-finite samples when asked (a kEmitStoreScreen emit without repairs).
+// Whether the plane schedule's inverse of this geometry runs as XY strips and
+// one column pass for the Z phase; that pass screens the output for non-finite
+// samples (a kEmitStoreScreen emit without repairs) or detects the repairs.
 bool plane_fused_fits(Dims full, unsigned lxy, unsigned lz, unsigned width);
 template <class T>
 void inverse_coarse_requant(const T* coeff, T* t0, T* t1, Dims full, unsigned lxy, double quantum, hipStream_t s);
@@ -285,14 +286,14 @@ template <class T>
 void detect_repairs(const T* original, const T* reconstructed, uint32_t n, double bound, SegList r,
                     uint32_t* status, hipStream_t s);
 struct EncodeResult {
-    unsigned long long wzp_bytes;  // written by wzp_encode
+    unsigned long long wzp_bytes;  // written by the payload placement
     unsigned long long end;        // archive bytes
     uint32_t np, nq, status, pad;
 };
 // Orders both side lists by index into the archive sections and writes the
 // 32-byte header and all padding; the result goes to `host` (pinned) as well.
 // `scratch` needs finish_scratch_words(n) u32. `pack` (n <= kFinishSmall only):
-// the encoder's group pass has not run and comes first, in the same launch.
+// the payload placement has not run and comes first, in the same launch.
 constexpr uint32_t kFinishSmall = 1u << 17;  // 16 chunks: one group
 uint64_t finish_scratch_words(uint32_t n);
 template <class T>

@@ -1,12 +1,7 @@
-// Chunk <-> brick map of the paired-brick path. With full 16x16x16 bricks
-// (nx % 32 == 0, ny % 16 == 0, nz % 16 == 0, z band 16) WZP chunk c, i.e.
-// magnitudes [8192c, 8192c + 8192), is exactly bricks 2c and 2c+1 of the
-// row-major brick grid (brick base = brick index * 4096), and the 32 ranks
-// [32t, 32t + 32) of that chunk form one 4x4x2 sub-block: in a 16^3 brick the
-// recursive octant rank (cpu/src/codec.cpp:96-107) has bits
-// z3 y3 x3 z2 y2 x2 z1 y1 x1 z0 y0 x0 from most to least significant, so the
-// low five bits are x0 y0 z0 x1 y1. Host+device so a CPU test checks the map
-// against the recursive rank.
+// Chunk <-> brick maps of the coders that quantize inside the encoder and
+// dequantize inside the decoder: direct_bricks_fit (z bands of a power of two)
+// and rank_bricks_fit (the other fields of full bricks). Host+device so that CPU
+// tests check them against the recursive octant rank (cpu/src/codec.cpp:96-107).
 #pragma once
 
 #include <cstdint>
@@ -20,6 +15,13 @@
 
 namespace wz {
 
+// The map of direct_bricks_fit written out for one kind of field, full 16^3
+// bricks in pairs (no kernel uses it by itself): WZP chunk c, i.e. magnitudes
+// [8192c, 8192c + 8192), is exactly bricks 2c and 2c+1 of the row-major brick
+// grid (brick base = brick index * 4096), and the 32 ranks [32t, 32t + 32) of
+// that chunk form one 4x4x2 sub-block: in a 16^3 brick the recursive rank has
+// bits z3 y3 x3 z2 y2 x2 z1 y1 x1 z0 y0 x0 from most to least significant, so
+// the low five bits are x0 y0 z0 x1 y1.
 constexpr bool pair_bricks_fit(uint32_t nx, uint32_t ny, uint32_t nz, uint32_t bz) {
     return bz == 16 && nx % 32 == 0 && ny % 16 == 0 && nz % 16 == 0 && nx && ny && nz;
 }

@@ -847,7 +847,7 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
     }
     static const int zonly[1] = {2};
     static const int yx[2] = {1, 0};
-    // every XY level as one fused launch: the Z phase (one pass)
+    // every XY level as one launch of strips: the Z phase (one pass)
     // into tmp1, then level l reads its box (tmp1, then the compact boxes in
     // tmp0) and writes its high bands into coeff and its low band into the
     // next box (coeff for the last level)
@@ -938,7 +938,7 @@ template <class T>
 bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy, unsigned lz, bool dyadic,
                   hipStream_t s, const Level0Emit<T>* emit, const Tuning& tu, unsigned base, double requant = 0.0) {
     if (requant > 0 && (dyadic || !plane_fused_fits(full, lxy, lz, sizeof(T))))
-        throw std::logic_error("requantizing inverse without fused XY levels");
+        throw std::logic_error("requantizing inverse without XY strips");
     Passes<T, true> p{coeff, {tmp0, tmp1}, coeff, output == coeff ? nullptr : output, nullptr, s, tu};
     p.base = base;
     if (lxy == 0 && lz == 0) {
@@ -973,7 +973,7 @@ bool inverse_impl(T* coeff, T* output, T* tmp0, T* tmp1, Dims full, unsigned lxy
     for (unsigned l = 0; l < lz; ++l) { zs[l] = act; act = shrink(act, false, true); }
     static const int xyo[2] = {0, 1};
     static const int zonly[1] = {2};
-    // every XY level as one fused launch: level l reads coeff's bands and the
+    // every XY level as one launch of strips: level l reads coeff's bands and the
     // coarser reconstruction (coeff's low quadrant for the coarsest level,
     // then the compact boxes in tmp0) and writes its box to tmp0, the finest
     // into tmp1, from which the Z phase (one pass) writes output

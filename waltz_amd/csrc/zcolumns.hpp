@@ -11,26 +11,31 @@
 
 namespace wz {
 
-// A workgroup of four waves (more: zcol_threads) owns a row of 64 columns, all z; a
-// wave takes one tile of the 64 columns at a time, a lane a column, so that a tile's rows, their
-// mirrored places and its tests are wave-uniform (scalar): per sample only the
-// lifting itself and its loads and stores reach the vector unit. The finest
+// A workgroup of four waves (more: zcol_threads) owns a row of 64 columns, all
+// z; a wave takes one tile of the 64 columns at a time, a lane a column, so
+// that a tile's rows, their mirrored places and its tests are wave-uniform
+// (scalar): per sample only the lifting itself and its loads and stores reach
+// the vector unit. The finest
 // level reads (forward) or writes (inverse) the field and every high band
 // goes between registers and the volume directly; only the low boxes between
 // the levels pass through LDS, alternating between two buffers (box 1 in the
 // first, ceil(nz/2) rows, box 2 in the second, box 3 in the first again), with
 // one barrier per level. Tiles and arithmetic are those of the Z axis passes
-// (lift_forward / lift_inverse folded), so the same bits. src != dst; status:
-// screen for non-finite samples the forward's input or the inverse's output.
-// Bound by memory: it reads and writes the field once, at 3.3-4.0 TB/s. With
-// every column staged in LDS and per-lane index arithmetic it was bound by
-// vector issue: 500x500x100 float 108 -> 55 us (forward), 127 -> 61 us
-// (inverse), 384x384x96 double 70 -> 56 us, 73 -> 67 us.
+// (lift_forward / lift_inverse folded), so the same bits; status: screen for
+// non-finite samples the forward's input or the inverse's output. It reads and
+// writes the field once, at 3.3-4.0 TB/s of the 5.1 that a copy reaches: the
+// halo rows of the tiles and one level after the other. With every column
+// staged in LDS and per-lane index arithmetic it was bound by vector issue:
+// 500x500x100 float 108 -> 55 us (forward), 127 -> 61 us (inverse), 384x384x96
+// double 70 -> 56 us, 73 -> 67 us.
+//
 // Repair (inverse, compress): the reconstruction is not written; each sample
 // is compared with the original as its tile is lifted, and the native repair
 // records and flag bits go out (one segment per workgroup, columns x nz slots).
 // That drops a write and a read of the field and one launch: 384x384x96
-// double, inverse and repair passes 67 + 47 us before.
+// double 68 us, inverse and repair passes 67 + 47 before; where rows share flag
+// words, which are set by atomics then, slower (500x500x100 float 88 us, 2.3 TB/s).
+
 // Decides the samples v[j] (rows z + j of column x, row y) of a wave's tile
 // against their originals, sets their flag bits and appends their records to
 // segment `id`; false when a lane's sample cannot meet the bound. Wave masks
