@@ -61,3 +61,19 @@ def test_phases_of_a_large_volume(shape, lz):
     want = stages.transform(x, 5, lz, False, False)
     stages.transform(x, 5, lz, False, False, out=x)
     assert torch.equal(x, want)
+
+
+# A plane past one window: out of place its forward levels run as strips with a
+# window per row, in place as axis passes with 64-bit addresses.
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,dtype", [((1, 33001, 32603), "float32"), ((1, 16500, 32700), "float64")], ids=str)
+def test_forward_of_a_large_plane(shape, dtype):
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from waltz_amd import stages
+    x = torch.rand(shape, device="cuda", dtype=getattr(torch, dtype), generator=torch.Generator("cuda").manual_seed(4))
+    assert x.numel() * x.element_size() > 1 << 32
+    want = stages.transform(x, 5, 0, False, False)
+    stages.transform(x, 5, 0, False, False, out=x)
+    assert torch.equal(x, want)

@@ -284,10 +284,10 @@ __global__ void __launch_bounds__(kStripThreads) xy_inverse_kernel(XYInverse<T> 
         strip_inverse<T, Requant>(a, p, item, StripStore<T>{});
     }
 }
-template <class T>
+template <class T, bool Wide>
 __global__ void __launch_bounds__(kStripThreads) xy_forward_kernel(XYForward<T> a, StripPlan p) {
     uint32_t item;
-    if (strip_of_wave(p, item)) strip_forward<T>(a, p, item);
+    if (strip_of_wave(p, item)) strip_forward<T, false, Wide>(a, p, item);
 }
 // screen: flag non-finite results
 template <class T>
@@ -302,7 +302,11 @@ void xy_inverse(const XYInverse<T>& a, hipStream_t s, uint32_t* screen = nullptr
 template <class T>
 void xy_forward(const XYForward<T>& a, hipStream_t s) {
     const StripPlan p = strip_plan(a.n, strips_pack(std::max({a.hpz, a.lpz, a.spz}), sizeof(T)));
-    hipLaunchKernelGGL((xy_forward_kernel<T>), dim3(strip_blocks(p)), dim3(kStripThreads), 0, s, a, p);
+    const dim3 grid(strip_blocks(p)), block(kStripThreads);
+    if (fused_plane_fits(std::max({a.hpy, a.lpy, a.spy}), a.n.ny, sizeof(T)))
+        hipLaunchKernelGGL((xy_forward_kernel<T, false>), grid, block, 0, s, a, p);
+    else
+        hipLaunchKernelGGL((xy_forward_kernel<T, true>), grid, block, 0, s, a, p);
 }
 
 // The finest level of a dyadic field (its Z pass done, in `src`) with the
@@ -851,7 +855,7 @@ void transform_forward(const T* input, T* coeff, T* tmp0, T* tmp1, Dims full, un
     // into tmp1, then level l reads its box (tmp1, then the compact boxes in
     // tmp0) and writes its high bands into coeff and its low band into the
     // next box (coeff for the last level)
-    if (strips_fit(full, full.nx, full.ny, lxy, sizeof(T)) && lxy &&
+    if (strip_lines_fit(full, lxy) && fused_plane_fits(full.nx, 1, sizeof(T)) && lxy &&
         (lz ? zcol_fits(full, lz, sizeof(T)) : input != coeff)) {
         const T* src = input;
         uint64_t spy = full.nx, spz = uint64_t(full.nx) * full.ny;
