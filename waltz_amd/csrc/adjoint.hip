@@ -24,8 +24,8 @@
 // writing its box once; low boxes move on in compact copies, so no level is
 // copied back. Against a pass per axis through LDS (and, on small planes, one
 // for X and Y with a halo of 2.4 times its outputs), IDWT^T / DWT^T:
-// 256^3 float 199 -> 112 / 234 -> 132 us, double 439 -> 186 / 508 -> 208;
-// 203x150x61 double 142 -> 62 / 159 -> 69. Memory bounds the finest level,
+// 256^3 float 199 -> 106 / 234 -> 124 us, double 439 -> 184 / 508 -> 206;
+// 203x150x61 double 142 -> 60 / 159 -> 68. Memory bounds the finest level,
 // launches the coarse ones. The passes per axis (adjoint_pass) are left for
 // lines of one sample and planes past a 32-bit window.
 #include <algorithm>
